@@ -345,7 +345,7 @@ static int build_haar_table(int levels, HaarTable &t, std::string &err)
     return WAVI_OK;
 }
 
-// +-1 Haar rows as bit masks for levels 0..3 (inverse, transposed inverse)
+// P's rows as bit masks for levels 0..3
 static void build_haar_masks(HaarMasks tabs[4])
 {
     memset(tabs, 0, 4 * sizeof(HaarMasks));
@@ -354,19 +354,18 @@ static void build_haar_masks(HaarMasks tabs[4])
         for (int m = 1; m <= B; ++m) {
             std::vector<double> Wi;
             wavelet_matrix(m, lev, false, Wi);
-            for (int dir = 0; dir < 2; ++dir)
-                for (int r = 0; r < m; ++r) {
-                    uint16_t nz = 0, neg = 0;
-                    for (int c = 0; c < m; ++c) {
-                        double w = dir == 0 ? Wi[(size_t)r * m + c] : Wi[(size_t)c * m + r];
-                        if (w != 0.0) {
-                            nz |= (uint16_t)(1u << c);
-                            if (w < 0.0) neg |= (uint16_t)(1u << c);
-                        }
+            for (int r = 0; r < m; ++r) {
+                uint16_t nz = 0, neg = 0;
+                for (int c = 0; c < m; ++c) {
+                    const double w = Wi[(size_t)r * m + c];
+                    if (w != 0.0) {
+                        nz |= (uint16_t)(1u << c);
+                        if (w < 0.0) neg |= (uint16_t)(1u << c);
                     }
-                    tabs[lev].nz[dir][m][r] = nz;
-                    tabs[lev].neg[dir][m][r] = neg;
                 }
+                tabs[lev].nz[m][r] = nz;
+                tabs[lev].neg[m][r] = neg;
+            }
         }
     }
 }
@@ -1287,18 +1286,7 @@ static bool cg_one_workgroup(const wavi_ctx *ctx)
     return ctx->cg_mode == WAVI_CG_WORKGROUP;
 }
 
-// The three-kernel coarse CG takes its Haar rows loads first
-// (haar_pm_row_ld; the same bits) on grids of at most this many tiles,
-// where a launch costs one tile's chain of LDS waits.
-constexpr int HAAR_LD_MAX_TILES = 256;
-
-static bool haar_loads_first(const wavi_ctx *ctx)
-{
-    return ctx->g.nbx * ctx->g.nby <= HAAR_LD_MAX_TILES;
-}
-
-// A +-1 Haar transform (dir 1: P, 2: R) of the u and v vectors on the tiles,
-// with the Haar rows loads first where haar_loads_first says so.
+// A +-1 Haar transform (dir 1: P, 2: R) of the u and v vectors on the tiles
 // (accu != nullptr: the result added into accu, accv at the output masks'
 // points instead, outu, outv untouched)
 template <typename T>
@@ -1307,13 +1295,8 @@ static void launch_tile_haar(wavi_ctx *ctx, int dir, const T *inu, const T *inv,
                              T *accu = nullptr, T *accv = nullptr)
 {
     const GridDims &g = ctx->g;
-    const dim3 tg(g.nbx, g.nby);
-    if (haar_loads_first(ctx))
-        hipLaunchKernelGGL((k_tile_haar<T, T, true>), tg, dim3(256), 0, ctx->stream, g, ctx->tab, ctx->S.levels, dir,
-                           inu, inv, min_u, min_v, outu, outv, mout_u, mout_v, accu, accv);
-    else
-        hipLaunchKernelGGL((k_tile_haar<T, T, false>), tg, dim3(256), 0, ctx->stream, g, ctx->tab, ctx->S.levels, dir,
-                           inu, inv, min_u, min_v, outu, outv, mout_u, mout_v, accu, accv);
+    hipLaunchKernelGGL((k_tile_haar<T, T>), dim3(g.nbx, g.nby), dim3(256), 0, ctx->stream, g, ctx->tab, ctx->S.levels,
+                       dir, inu, inv, min_u, min_v, outu, outv, mout_u, mout_v, accu, accv);
 }
 
 // coarse CG on b_c held in w.cr; solution in the warm start w.xc
@@ -1328,7 +1311,6 @@ static int do_coarse_cg(wavi_ctx *ctx, const VSet<T> &w, int *iters)
     ctx->h_flag->done = 0;
     ctx->h_flag->iters = 0;
     const bool pre = ctx->cg_pre;
-    const bool ld = haar_loads_first(ctx);
     // k_cg_apply / k_cg_update return on the stop flag at once after a short
     // previous CG (one that fitted its first chunk): such CGs stop within a
     // chunk, so the launches queued past the stop are many.  Long CGs have
@@ -1370,25 +1352,17 @@ static int do_coarse_cg(wavi_ctx *ctx, const VSet<T> &w, int *iters)
             const int par = q & 1;
             {
                 ProfScope ps(ctx, WAVI_KT_CG_DIR, sampled);
-                if (pre && ld)
-                    hipLaunchKernelGGL((k_cg_dir<T, true, true>), tb, dim3(256), 0, ctx->stream, a, par);
-                else if (pre)
-                    hipLaunchKernelGGL((k_cg_dir<T, true, false>), tb, dim3(256), 0, ctx->stream, a, par);
-                else if (ld)
-                    hipLaunchKernelGGL((k_cg_dir<T, false, true>), tb, dim3(256), 0, ctx->stream, a, par);
+                if (pre)
+                    hipLaunchKernelGGL((k_cg_dir<T, true>), tb, dim3(256), 0, ctx->stream, a, par);
                 else
-                    hipLaunchKernelGGL((k_cg_dir<T, false, false>), tb, dim3(256), 0, ctx->stream, a, par);
+                    hipLaunchKernelGGL((k_cg_dir<T, false>), tb, dim3(256), 0, ctx->stream, a, par);
             }
             {
                 ProfScope ps(ctx, WAVI_KT_CG_APPLY, sampled);
-                if (ld && early)
-                    hipLaunchKernelGGL((k_cg_apply<T, true, true>), tb, dim3(256), 0, ctx->stream, a);
-                else if (ld)
-                    hipLaunchKernelGGL((k_cg_apply<T, true, false>), tb, dim3(256), 0, ctx->stream, a);
-                else if (early)
-                    hipLaunchKernelGGL((k_cg_apply<T, false, true>), tb, dim3(256), 0, ctx->stream, a);
+                if (early)
+                    hipLaunchKernelGGL((k_cg_apply<T, true>), tb, dim3(256), 0, ctx->stream, a);
                 else
-                    hipLaunchKernelGGL((k_cg_apply<T, false, false>), tb, dim3(256), 0, ctx->stream, a);
+                    hipLaunchKernelGGL((k_cg_apply<T, false>), tb, dim3(256), 0, ctx->stream, a);
             }
             {
                 ProfScope ps(ctx, WAVI_KT_CG_UPDATE, sampled);

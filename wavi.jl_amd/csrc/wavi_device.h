@@ -107,17 +107,53 @@ __device__ __forceinline__ double det_pow(double x, double y)
 // ---------------------------------------------------------------------------
 // Canonical reduction trees.  A 256-thread workgroup reduces one value per
 // thread: each 64-wide wavefront sums its lanes with t[e] += t[e+s],
-// s = 32..1 (shuffles, lane e reads lane e+s), and the four wavefront sums
-// combine as (w0 + w2) + (w1 + w3).  The oracle sums in the same order.
-template <typename T>
-__device__ __forceinline__ T tree256(T v, T *lds)
+// s = 32..1 (lane e takes lane e+s), and the four wavefront sums combine as
+// (w0 + w2) + (w1 + w3).  The oracle sums in the same order.
+
+// The value of lane e + S at every lane e < S of a wavefront, the lanes on
+// which lane 0 of the tree depends (other lanes get values that the tree does
+// not use).  A tree is a chain of six such exchanges and most kernels of the
+// FP64 coarse CG have two or three trees in a row, so the exchange's latency
+// counts: register moves (v_permlane32_swap, v_permlane16_swap, DPP
+// row_shl) in place of the LDS permutes of __shfl_down.  Every lane of the
+// wavefront must be active.
+template <int S>
+__device__ __forceinline__ unsigned lane_down_b32(unsigned v)
+{
+    if constexpr (S == 32)
+        return __builtin_amdgcn_permlane32_swap(v, v, false, false)[1];
+    else if constexpr (S == 16)
+        return __builtin_amdgcn_permlane16_swap(v, v, false, false)[1];
+    else
+        return (unsigned)__builtin_amdgcn_mov_dpp((int)v, 0x100 | S, 0xF, 0xF, true);  // row_shl:S
+}
+
+template <int S>
+__device__ __forceinline__ double lane_down(double v)
+{
+    const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+    const unsigned lo = lane_down_b32<S>((unsigned)b), hi = lane_down_b32<S>((unsigned)(b >> 32));
+    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+
+// The tree over one wavefront: its sum in lane 0.
+__device__ __forceinline__ double wave_tree(double v)
+{
+    v = v + lane_down<32>(v);
+    v = v + lane_down<16>(v);
+    v = v + lane_down<8>(v);
+    v = v + lane_down<4>(v);
+    v = v + lane_down<2>(v);
+    return v + lane_down<1>(v);
+}
+
+__device__ __forceinline__ double tree256(double v, double *lds)
 {
     const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
-#pragma unroll
-    for (int s = 32; s > 0; s >>= 1) v = v + __shfl_down(v, s, 64);
+    v = wave_tree(v);
     if (l == 0) lds[w] = v;
     __syncthreads();
-    const T r = (lds[0] + lds[2]) + (lds[1] + lds[3]);
+    const double r = (lds[0] + lds[2]) + (lds[1] + lds[3]);
     __syncthreads();
     return r;
 }
@@ -126,11 +162,8 @@ __device__ __forceinline__ T tree256(T v, T *lds)
 __device__ __forceinline__ void tree256x2(double &a, double &b, double *lds)
 {
     const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
-#pragma unroll
-    for (int s = 32; s > 0; s >>= 1) {
-        a = a + __shfl_down(a, s, 64);
-        b = b + __shfl_down(b, s, 64);
-    }
+    a = wave_tree(a);
+    b = wave_tree(b);
     if (l == 0) {
         lds[w] = a;
         lds[4 + w] = b;
@@ -143,48 +176,42 @@ __device__ __forceinline__ void tree256x2(double &a, double &b, double *lds)
 
 // Fold `np` block partials into 256 lanes (lane L = thread L sums P[L],
 // P[L+256], ... in order; missing terms add +0) and sum the lanes with
-// tree256.  Loads are issued eight at a time.  Every workgroup that calls
-// this obtains the same bits, in all threads.
-__device__ __forceinline__ double lanes_sum(const double *P, int np, double *lds)
+// tree256.  Loads are issued unconditionally at clamped indices, one for a
+// small grid, else eight at a time.  Every workgroup that calls this obtains
+// the same bits, in all threads.
+__device__ __forceinline__ double lane_fold(const double *P, int np)
 {
     const int t = threadIdx.x;
+    if (np <= 256) {
+        const double v = P[t < np ? t : 0];
+        return t < np ? v : 0.0;
+    }
     double acc = 0.0;
     for (int q0 = 0; q0 < np; q0 += 8 * 256) {
         double v[8];
 #pragma unroll
         for (int k = 0; k < 8; ++k) {
             const int q = q0 + t + 256 * k;
-            v[k] = q < np ? P[q] : 0.0;
+            v[k] = P[q < np ? q : 0];
         }
 #pragma unroll
-        for (int k = 0; k < 8; ++k) acc = acc + v[k];
+        for (int k = 0; k < 8; ++k) acc = acc + (q0 + t + 256 * k < np ? v[k] : 0.0);
     }
-    return tree256(acc, lds);
+    return acc;
+}
+
+__device__ __forceinline__ double lanes_sum(const double *P, int np, double *lds)
+{
+    return tree256(lane_fold(P, np), lds);
 }
 
 // lanes_sum of two partial arrays of the same length in one pass.
 __device__ __forceinline__ void lanes_sum2(const double *P, const double *Q, int np, double *lds, double &a,
                                            double &b)
 {
-    const int t = threadIdx.x;
-    double x = 0.0, y = 0.0;
-    for (int q0 = 0; q0 < np; q0 += 8 * 256) {
-        double v[8], w[8];
-#pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            const int q = q0 + t + 256 * k;
-            v[k] = q < np ? P[q] : 0.0;
-            w[k] = q < np ? Q[q] : 0.0;
-        }
-#pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            x = x + v[k];
-            y = y + w[k];
-        }
-    }
-    tree256x2(x, y, lds);
-    a = x;
-    b = y;
+    a = lane_fold(P, np);
+    b = lane_fold(Q, np);
+    tree256x2(a, b, lds);
 }
 
 // ---------------------------------------------------------------------------

@@ -933,7 +933,7 @@ __device__ __forceinline__ void haar_tile(const HaarTable *tab, int dir, T (*til
         tmp[ly][lx] = haar_table_row<T>(tab, dir, m, r, &tile[jb][lx], TILE + 1);
     }
     __syncthreads();
-    // x pass, with the transposed element mapping of haar_pm_tile2m (the
+    // x pass, with the transposed element mapping of the y pass swapped (the
     // lanes of a wave share the column, so rows of one length)
     const int lyx = threadIdx.x & 15, lxx = threadIdx.x >> 4;
     if (i0 + lxx < nxw && j0 + lyx < nyw) {
@@ -991,153 +991,191 @@ __global__ void k_tile_wavelets(GridDims g, const HaarTable *tab, const double *
 }
 
 // ===========================================================================
-// Haar transforms with +-1 coefficients (the inverse and its transpose): each
-// composed row is a pair of 16-bit masks, bit c of `nz` marking a term in
-// column c and bit c of `neg` its sign, one table per `levels` (0..3).
-// Terms are summed in increasing column order, as the oracle sums them.
+// Haar transforms with +-1 coefficients: the inverse P and its transpose R.
+
+// P's rows as bit masks (k_coarse_diag): bit c of `nz` marks a term in column
+// c and bit c of `neg` its sign, one table per `levels` (0..3).
 struct HaarMasks {
-    uint16_t nz[2][17][16];
-    uint16_t neg[2][17][16];
+    uint16_t nz[17][16];
+    uint16_t neg[17][16];
 };
 __constant__ HaarMasks c_haar[4];
 
-template <typename T>
-__device__ __forceinline__ T haar_pm_row(uint32_t nz, uint32_t neg, const T *src, int stride)
+// One 16-point line of P, the composed inverse of wavelet_matrix
+// (src/Wavelets/update_wavelets.jl:38-89) with blocks of B = 2^(LEV+1)
+// points: y_i = sum over c of P[i][c] x_c, the terms added in increasing
+// column order as the oracle adds them.  Of a pair (o, e = o + h) the column
+// e is -1 on the h rows from o and +1 on the h rows from e, and column 0 of a
+// block is +1 on all its rows, so a row has LEV + 2 terms.  A thread computes
+// rows 2w and 2w + 1 of the half line `half` (8 points): the two rows share
+// all columns and differ in one sign.  z: the half line; with LEV = 3 the
+// block is the whole line, whose columns 0 and 8 come before (second half:
+// x_0 + x_8) and around (first half: x_0 first, -x_8 last) the half's own.
+// w is uniform over a wavefront.  Points past the end of the grid must hold
+// zero: their terms then change nothing, which leaves wavelet_matrix's
+// partial blocks.
+template <int LEV, typename T>
+__device__ __forceinline__ void haar_line_P(const T *src, T *dst, int st, int half, int w)
 {
-    T acc = T(0);
-    while (nz) {
-        const int c = __builtin_ctz(nz);
-        const T v = src[c * stride];
-        acc = ((neg >> c) & 1u) ? acc - v : acc + v;
-        nz &= nz - 1u;
-    }
-    return acc;
-}
-
-// haar_pm_row with the B = 2 << levels entries of the row's block loaded
-// first, then added in increasing column order through selects: the same
-// additions as haar_pm_row, so the same bits, with one LDS wait instead of
-// one per term.  The block lies inside the 16 x 16 tile, so every load is in
-// bounds; entries outside the row's terms are loaded and discarded.  Shorter
-// where a tile's latency chain is the launch's cost (grids of few tiles);
-// the extra VALU work costs more than it saves when many tiles share a CU.
-template <typename T, int B>
-__device__ __forceinline__ T haar_pm_row_ld(uint32_t nz, uint32_t neg, const T *src, int stride)
-{
-    T v[B];
-#pragma unroll
-    for (int c = 0; c < B; ++c) v[c] = src[c * stride];
-    T acc = T(0);
-#pragma unroll
-    for (int c = 0; c < B; ++c) {
-        const T t = ((neg >> c) & 1u) ? acc - v[c] : acc + v[c];
-        acc = ((nz >> c) & 1u) ? t : acc;
-    }
-    return acc;
-}
-
-template <typename T, bool LD>
-__device__ __forceinline__ T haar_pm_row_sel(int levels, uint32_t nz, uint32_t neg, const T *src, int stride)
-{
-    if constexpr (!LD) {
-        return haar_pm_row<T>(nz, neg, src, stride);
+    const T *z = src + 8 * half * st;
+    T lo, hi;  // rows 2w and 2w + 1
+    if constexpr (LEV == 0) {
+        const T o = z[2 * w * st], e = z[(2 * w + 1) * st];
+        lo = o - e;
+        hi = o + e;
+    } else if constexpr (LEV == 1) {
+        const T o = z[(w & 2) * 2 * st];
+        if ((w & 1) == 0) {
+            const T e = z[((w & 2) * 2 + 1) * st], m = z[((w & 2) * 2 + 2) * st];
+            lo = (o - e) - m;
+            hi = (o + e) - m;
+        } else {
+            const T m = z[((w & 2) * 2 + 2) * st], e = z[((w & 2) * 2 + 3) * st];
+            const T b = o + m;
+            lo = b - e;
+            hi = b + e;
+        }
     } else {
-        switch (levels) {
-        case 0:
-            return haar_pm_row_ld<T, 2>(nz, neg, src, stride);
-        case 1:
-            return haar_pm_row_ld<T, 4>(nz, neg, src, stride);
-        case 2:
-            return haar_pm_row_ld<T, 8>(nz, neg, src, stride);
-        default:
-            return haar_pm_row_ld<T, 16>(nz, neg, src, stride);
+        T base = src[(LEV == 3 ? 0 : 8 * half) * st], tail = T(0);
+        if constexpr (LEV == 3) {
+            const T x8 = src[8 * st];
+            tail = half ? T(0) : x8;
+            base = half ? base + x8 : base;
+        }
+        if (w == 0) {
+            const T z1 = z[st], z2 = z[2 * st], z4 = z[4 * st];
+            lo = ((base - z1) - z2) - z4;
+            hi = ((base + z1) - z2) - z4;
+        } else if (w == 1) {
+            const T z2 = z[2 * st], z3 = z[3 * st], z4 = z[4 * st];
+            const T b = base + z2;
+            lo = (b - z3) - z4;
+            hi = (b + z3) - z4;
+        } else if (w == 2) {
+            const T z4 = z[4 * st], z5 = z[5 * st], z6 = z[6 * st];
+            const T b = base + z4;
+            lo = (b - z5) - z6;
+            hi = (b + z5) - z6;
+        } else {
+            const T z4 = z[4 * st], z6 = z[6 * st], z7 = z[7 * st];
+            const T b = (base + z4) + z6;
+            lo = b - z7;
+            hi = b + z7;
+        }
+        if constexpr (LEV == 3) {
+            lo = lo - tail;
+            hi = hi - tail;
+        }
+    }
+    T *d = dst + (8 * half + 2 * w) * st;
+    d[0] = lo;
+    d[st] = hi;
+}
+
+// One 16-point line of R = P^T: row o + h of a pair is -1 on the h points
+// from o and +1 on the h points from o + h, row 0 of a block sums the block;
+// terms in increasing order.  A row's leading minus terms are the negated
+// prefix sum of its points, the same roundings as subtracting them one by
+// one, so the long rows share their prefixes.  The four wavefronts take the
+// block sums (LEV = 3: rows 0 and 8, one per half), the rows 4 and 12, the
+// rows 2 and 6 of each half, and the odd rows; a thread of the first adds
+// 16 terms, of the others at most 8.
+template <int LEV, typename T>
+__device__ __forceinline__ void haar_line_R(const T *src, T *dst, int st, int half, int w)
+{
+    const T *z = src + 8 * half * st;
+    T *d = dst + 8 * half * st;
+    if (w == 0) {
+        if constexpr (LEV == 3) {
+            T x[16];
+#pragma unroll
+            for (int c = 0; c < 16; ++c) x[c] = src[c * st];
+            T a = x[0];
+#pragma unroll
+            for (int c = 1; c < 8; ++c) a = a + x[c];
+            a = half ? -a : a;
+#pragma unroll
+            for (int c = 8; c < 16; ++c) a = a + x[c];
+            d[0] = a;
+        } else {
+            T x[8];
+#pragma unroll
+            for (int c = 0; c < 8; ++c) x[c] = z[c * st];
+            constexpr int B = 2 << LEV;
+#pragma unroll
+            for (int o = 0; o < 8; o += B) {
+                T a = x[o];
+#pragma unroll
+                for (int c = 1; c < B; ++c) a = a + x[o + c];
+                d[o * st] = a;
+            }
+        }
+    } else if (w == 1) {
+        if constexpr (LEV >= 2) {
+            T x[8];
+#pragma unroll
+            for (int c = 0; c < 8; ++c) x[c] = z[c * st];
+            const T a = ((x[0] + x[1]) + x[2]) + x[3];
+            d[4 * st] = (((x[4] - a) + x[5]) + x[6]) + x[7];
+        }
+    } else if (w == 2) {
+        if constexpr (LEV >= 1) {
+            T x[8];
+#pragma unroll
+            for (int c = 0; c < 8; ++c) x[c] = z[c * st];
+            d[2 * st] = (x[2] - (x[0] + x[1])) + x[3];
+            d[6 * st] = (x[6] - (x[4] + x[5])) + x[7];
+        }
+    } else {
+#pragma unroll
+        for (int o = 0; o < 8; o += 2) {
+            const T a = z[o * st], b = z[(o + 1) * st];
+            d[(o + 1) * st] = b - a;
         }
     }
 }
 
-// The row masks one thread reads in the two passes of a transform of the u
-// and the v tile of block (i0, j0), all loaded at once (so that they can be
-// loaded with a kernel's other inputs instead of one round trip per pass).
-// The y pass computes element (ly, lx) = (tid >> 4, tid & 15), the x pass
-// element (tid & 15, tid >> 4): the lanes of a wave then share the row of
-// their y pass and the column of their x pass, and with it the number of
-// terms, so the long rows (16 terms in the transposed inverse at 3 levels)
-// fall in one wave of four in both passes.
-struct HaarRowMasks {
-    uint32_t yz_u, yn_u, yz_v, yn_v;  // y pass: terms and signs, u and v tile
-    uint32_t xz_u, xn_u, xz_v, xn_v;  // x pass
-};
+// A u tile and a v tile side by side, as the transforms read them.
+template <typename T>
+using TilePair = T[2][TILE][TILE + 1];
 
-// p[k] where ok, else 0, with the load issued unconditionally (index 0
-// where !ok).
-__device__ __forceinline__ uint32_t haar_mask_or0(bool ok, const uint16_t *p, int k)
+// P (R = false) or R of the u and the v tile of one block, in place, with m
+// as scratch: the y lines, then the x lines (the order KroneckerProduct mul!
+// takes for square factors).  Every wavefront covers all 32 lines of both
+// tiles, a half line per lane, and takes its own rows of each line, so the
+// code of a wavefront is straight and the operands of a row are read from
+// LDS once, all before the first is used.  The rows as bit masks walked term
+// by term (one row per thread, 16 dependent LDS reads in the longest)
+// cost k_cg_apply 9,200 of its 16,600 cycles on a lone tile.
+// Points past the grid's end must hold zero.  Ends with a barrier.
+template <bool R, int LEV, typename T>
+__device__ __forceinline__ void haar_pair_lev(TilePair<T> &t, TilePair<T> &m)
 {
-    const uint32_t v = p[ok ? k : 0];
-    return ok ? v : 0u;
-}
-
-__device__ __forceinline__ HaarRowMasks haar_row_masks(int levels, int dir, int i0, int j0, const GridDims &g,
-                                                       bool has_u, bool has_v)
-{
-    // the y pass's element (ly, lx)
-    const int lx = threadIdx.x & 15, ly = threadIdx.x >> 4;
-    const int B = 2 << levels;
-    const int i = i0 + lx, j = j0 + ly;
-    const int jb = ly & ~(B - 1), ry = ly - jb;
-    const bool ou = has_u && i < g.nxu && j < g.nyu, ov = has_v && i < g.nxv && j < g.nyv;
-    const uint16_t *nz = &c_haar[levels].nz[dir][0][0], *ng = &c_haar[levels].neg[dir][0][0];
-    const int yu = min(g.nyu - (j0 + jb), B) * 16 + ry, yv = min(g.nyv - (j0 + jb), B) * 16 + ry;
-    // the x pass's element (lyx, lxx)
-    const int lyx = threadIdx.x & 15, lxx = threadIdx.x >> 4;
-    const int ix = i0 + lxx, jx = j0 + lyx, ibx = lxx & ~(B - 1), rxx = lxx - ibx;
-    const bool oux = has_u && ix < g.nxu && jx < g.nyu, ovx = has_v && ix < g.nxv && jx < g.nyv;
-    const int xux = min(g.nxu - (i0 + ibx), B) * 16 + rxx, xvx = min(g.nxv - (i0 + ibx), B) * 16 + rxx;
-    HaarRowMasks m;
-    m.yz_u = haar_mask_or0(ou, nz, yu);
-    m.yn_u = haar_mask_or0(ou, ng, yu);
-    m.yz_v = haar_mask_or0(ov, nz, yv);
-    m.yn_v = haar_mask_or0(ov, ng, yv);
-    m.xz_u = haar_mask_or0(oux, nz, xux);
-    m.xn_u = haar_mask_or0(oux, ng, xux);
-    m.xz_v = haar_mask_or0(ovx, nz, xvx);
-    m.xn_v = haar_mask_or0(ovx, ng, xvx);
-    return m;
-}
-
-// The same transform on the u tile and the v tile of one block at once, with
-// the row masks given (haar_row_masks; LD: the rows as haar_pm_row_ld).
-template <typename T, bool LD = false>
-__device__ __forceinline__ void haar_pm_tile2m(int levels, const HaarRowMasks &hm, T (*tu)[TILE + 1],
-                                               T (*mu)[TILE + 1], T (*tv)[TILE + 1], T (*mv)[TILE + 1], int i0,
-                                               int j0, const GridDims &g, bool has_u, bool has_v)
-{
-    const int lx = threadIdx.x & 15, ly = threadIdx.x >> 4;
-    const int B = 2 << levels;
-    const int i = i0 + lx, j = j0 + ly;
-    const int jb = ly & ~(B - 1);
-    if (has_u && i < g.nxu && j < g.nyu)
-        mu[ly][lx] = haar_pm_row_sel<T, LD>(levels, hm.yz_u, hm.yn_u, &tu[jb][lx], TILE + 1);
-    if (has_v && i < g.nxv && j < g.nyv)
-        mv[ly][lx] = haar_pm_row_sel<T, LD>(levels, hm.yz_v, hm.yn_v, &tv[jb][lx], TILE + 1);
+    const int l = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int q = l & 15, comp = (l >> 4) & 1, half = l >> 5;
+    if constexpr (R)
+        haar_line_R<LEV, T>(&t[comp][0][q], &m[comp][0][q], TILE + 1, half, w);
+    else
+        haar_line_P<LEV, T>(&t[comp][0][q], &m[comp][0][q], TILE + 1, half, w);
     __syncthreads();
-    // the x pass with the transposed element mapping (haar_row_masks)
-    const int lyx = threadIdx.x & 15, lxx = threadIdx.x >> 4;
-    const int ix = i0 + lxx, jx = j0 + lyx, ibx = lxx & ~(B - 1);
-    if (has_u && ix < g.nxu && jx < g.nyu)
-        tu[lyx][lxx] = haar_pm_row_sel<T, LD>(levels, hm.xz_u, hm.xn_u, &mu[lyx][ibx], 1);
-    if (has_v && ix < g.nxv && jx < g.nyv)
-        tv[lyx][lxx] = haar_pm_row_sel<T, LD>(levels, hm.xz_v, hm.xn_v, &mv[lyx][ibx], 1);
+    if constexpr (R)
+        haar_line_R<LEV, T>(&m[comp][q][0], &t[comp][q][0], 1, half, w);
+    else
+        haar_line_P<LEV, T>(&m[comp][q][0], &t[comp][q][0], 1, half, w);
     __syncthreads();
 }
 
-// haar_pm_tile2m with the masks loaded here.
-template <typename T, bool LD = false>
-__device__ __forceinline__ void haar_pm_tile2(int levels, int dir, T (*tu)[TILE + 1], T (*mu)[TILE + 1],
-                                              T (*tv)[TILE + 1], T (*mv)[TILE + 1], int i0, int j0, const GridDims &g,
-                                              bool has_u, bool has_v)
+template <bool R, typename T>
+__device__ __forceinline__ void haar_pair(int levels, TilePair<T> &t, TilePair<T> &m)
 {
-    const HaarRowMasks hm = haar_row_masks(levels, dir, i0, j0, g, has_u, has_v);
-    haar_pm_tile2m<T, LD>(levels, hm, tu, mu, tv, mv, i0, j0, g, has_u, has_v);
+    if (levels == 3)
+        haar_pair_lev<R, 3, T>(t, m);
+    else if (levels == 2)
+        haar_pair_lev<R, 2, T>(t, m);
+    else if (levels == 1)
+        haar_pair_lev<R, 1, T>(t, m);
+    else
+        haar_pair_lev<R, 0, T>(t, m);
 }
 
 // ===========================================================================
@@ -1337,11 +1375,11 @@ __device__ __forceinline__ void optile_store(const StageRegs<T> &r, OpTile<T> &s
 }
 
 // The whole tile operator with prefetch: stage t, compute intermediates,
-// outputs into tu / tv (zero off the inner masks).  Ends with a barrier.
+// outputs into t (zero off the inner masks).  Ends with a barrier.
 template <typename T>
 __device__ __forceinline__ void optile_apply(const GridDims &g, const OpCoef<T> &c, const T *tU, const T *tV,
                                              int i0, int j0, const PointCoef<T> &pc, OpTile<T> &s,
-                                             T (*tu)[TILE + 1], T (*tv)[TILE + 1])
+                                             TilePair<T> &t)
 {
     StageRegs<T> sr;
     CellCoef<T> c0, c1;
@@ -1354,8 +1392,8 @@ __device__ __forceinline__ void optile_apply(const GridDims &g, const OpCoef<T> 
     cell_compute(c, c1, threadIdx.x + 256, s);
     __syncthreads();
     const int lx = threadIdx.x & 15, ly = threadIdx.x >> 4;
-    tu[ly][lx] = (pc.oku && pc.ui) ? optile_u(c, s, pc, lx, ly) : T(0);
-    tv[ly][lx] = (pc.okv && pc.vi) ? optile_v(c, s, pc, lx, ly) : T(0);
+    t[0][ly][lx] = (pc.oku && pc.ui) ? optile_u(c, s, pc, lx, ly) : T(0);
+    t[1][ly][lx] = (pc.okv && pc.vi) ? optile_v(c, s, pc, lx, ly) : T(0);
     __syncthreads();
 }
 
@@ -2000,16 +2038,14 @@ __device__ __forceinline__ int band_tile(const GridDims &g, int L, int &bx, int 
     return L;
 }
 
-// c = R A t for the tile: A into tu / tv, then the transposed inverse Haar,
-// zero off the wavelet masks.
-template <typename T, bool LD = false>
-__device__ __forceinline__ void tile_apply_restrict(const CGArgs<T> &a, int i0, int j0, bool has_u, bool has_v,
-                                                    const PointCoef<T> &pc, OpTile<T> &s, T (*tu)[TILE + 1],
-                                                    T (*mu)[TILE + 1], T (*tv)[TILE + 1], T (*mv)[TILE + 1])
+// c = R A t for the tile: A into `t`, then the transposed inverse Haar (c at
+// the wavelet masks' points).
+template <typename T>
+__device__ __forceinline__ void tile_apply_restrict(const CGArgs<T> &a, int i0, int j0, const PointCoef<T> &pc,
+                                                    OpTile<T> &s, TilePair<T> &t, TilePair<T> &m)
 {
-    const HaarRowMasks hm = haar_row_masks(a.levels, 1, i0, j0, a.g, has_u, has_v);
-    optile_apply(a.g, a.c, a.tu, a.tv, i0, j0, pc, s, tu, tv);
-    haar_pm_tile2m<T, LD>(a.levels, hm, tu, mu, tv, mv, i0, j0, a.g, has_u, has_v);
+    optile_apply(a.g, a.c, a.tu, a.tv, i0, j0, pc, s, t);
+    haar_pair<true, T>(a.levels, t, m);
 }
 
 // setup (t = P x0 computed beforehand): r = b - R A t (b arrives in r),
@@ -2019,7 +2055,7 @@ template <typename T, bool PRE>
 __global__ void __launch_bounds__(256) k_cg_setup(CGArgs<T> a)
 {
     __shared__ OpTile<T> s;
-    __shared__ T tu[TILE][TILE + 1], mu[TILE][TILE + 1], tv[TILE][TILE + 1], mv[TILE][TILE + 1];
+    __shared__ TilePair<T> t, m;
     __shared__ double lds[8];
     const GridDims &g = a.g;
     const int L = xcd_tile(a.nblk);
@@ -2043,10 +2079,10 @@ __global__ void __launch_bounds__(256) k_cg_setup(CGArgs<T> a)
     PointCoef<T> pc;
     point_prefetch(g, a.c, a.mwu, a.mwv, i0 + lx, j0 + ly, has_u, has_v, pc);
     const T bu = pc.oku ? a.ru[pc.ku] : T(0), bv = pc.okv ? a.rv[pc.kv] : T(0);
-    tile_apply_restrict<T>(a, i0, j0, has_u, has_v, pc, s, tu, mu, tv, mv);
+    tile_apply_restrict<T>(a, i0, j0, pc, s, t, m);
     double r2u = 0.0, b2u = 0.0, r2v = 0.0, b2v = 0.0, z2u = 0.0, z2v = 0.0;
     if (pc.oku) {
-        const T r = bu - (pc.mwu ? tu[ly][lx] : T(0));
+        const T r = bu - (pc.mwu ? t[0][ly][lx] : T(0));
         a.ru[pc.ku] = r;
         a.pu[pc.ku] = T(0);
         r2u = (double)r * (double)r;
@@ -2054,7 +2090,7 @@ __global__ void __launch_bounds__(256) k_cg_setup(CGArgs<T> a)
         if constexpr (PRE) z2u = (double)r * (a.dinvu[pc.ku] * (double)r);
     }
     if (pc.okv) {
-        const T r = bv - (pc.mwv ? tv[ly][lx] : T(0));
+        const T r = bv - (pc.mwv ? t[1][ly][lx] : T(0));
         a.rv[pc.kv] = r;
         a.pv[pc.kv] = T(0);
         r2v = (double)r * (double)r;
@@ -2097,12 +2133,11 @@ __device__ __forceinline__ V cg_scalar(const V *p)
 // u = r + beta u with beta = res^2 / prev^2 (PRE: u = D^-1 r + beta u with
 // beta = rz / prev rz), t = P u.  The stop decision is
 // recomputed from the partials each time, so it needs no flag: after a stop
-// the partials are frozen and it[1 - par] repeats the count.  LD: the Haar
-// rows loads first (haar_pm_row_ld), the same bits.
-template <typename T, bool PRE, bool LD = false>
+// the partials are frozen and it[1 - par] repeats the count.
+template <typename T, bool PRE>
 __device__ __forceinline__ bool cg_dir_tile(const CGArgs<T> &a, int par, const int L)
 {
-    __shared__ T tu[TILE][TILE + 1], mu[TILE][TILE + 1], tv[TILE][TILE + 1], mv[TILE][TILE + 1];
+    __shared__ TilePair<T> t, m;
     __shared__ double lds[8];
     const GridDims &g = a.g;
     if (L >= g.nbx * g.nby) return false;
@@ -2121,7 +2156,6 @@ __device__ __forceinline__ bool cg_dir_tile(const CGArgs<T> &a, int par, const i
     const T rv = ld_or(okv, a.rv, kv, T(0)), pv = ld_or(okv, a.pv, kv, T(0));
     const bool mwu = ld_or(oku, a.mwu, ku, (uint8_t)0) != 0, mwv = ld_or(okv, a.mwv, kv, (uint8_t)0) != 0;
     const bool iu = ld_or(oku, a.ui, ku, (uint8_t)0) != 0, iv = ld_or(okv, a.vi, kv, (uint8_t)0) != 0;
-    const HaarRowMasks hm = haar_row_masks(a.levels, 0, i0, j0, g, has_u, has_v);
     double dzu = 0.0, dzv = 0.0, rz = 0.0, prev_rz = 0.0;
     if constexpr (PRE) {
         dzu = ld_or(oku, a.dinvu, ku, 0.0);
@@ -2182,12 +2216,12 @@ __device__ __forceinline__ bool cg_dir_tile(const CGArgs<T> &a, int par, const i
             unv = rv + beta * pv;
         a.pv[kv] = unv;
     }
-    tu[ly][lx] = mwu ? unu : T(0);
-    tv[ly][lx] = mwv ? unv : T(0);
+    t[0][ly][lx] = mwu ? unu : T(0);
+    t[1][ly][lx] = mwv ? unv : T(0);
     __syncthreads();
-    haar_pm_tile2m<T, LD>(a.levels, hm, tu, mu, tv, mv, i0, j0, g, has_u, has_v);
-    if (oku) a.tu[ku] = iu ? tu[ly][lx] : T(0);
-    if (okv) a.tv[kv] = iv ? tv[ly][lx] : T(0);
+    haar_pair<false, T>(a.levels, t, m);
+    if (oku) a.tu[ku] = iu ? t[0][ly][lx] : T(0);
+    if (okv) a.tv[kv] = iv ? t[1][ly][lx] : T(0);
     return false;
 }
 
@@ -2196,11 +2230,11 @@ __device__ __forceinline__ bool cg_dir_tile(const CGArgs<T> &a, int par, const i
 // stores in full: after a stop only k_cg_update reads c and the partials, and
 // it changes nothing then; a return on the flag would put its round trip
 // before every load of the launch.
-template <typename T, bool LD = false, bool EARLY = true>
+template <typename T, bool EARLY = true>
 __device__ __forceinline__ void cg_apply_tile(const CGArgs<T> &a, const int L)
 {
     __shared__ OpTile<T> s;
-    __shared__ T tu[TILE][TILE + 1], mu[TILE][TILE + 1], tv[TILE][TILE + 1], mv[TILE][TILE + 1];
+    __shared__ TilePair<T> t, m;
     __shared__ double lds[8];
     const GridDims &g = a.g;
     if (L >= g.nbx * g.nby) return;
@@ -2213,15 +2247,15 @@ __device__ __forceinline__ void cg_apply_tile(const CGArgs<T> &a, const int L)
     PointCoef<T> pc;
     point_prefetch(g, a.c, a.mwu, a.mwv, i0 + lx, j0 + ly, has_u, has_v, pc);
     const T pu = ld_or(pc.oku, a.pu, pc.ku, T(0)), pv = ld_or(pc.okv, a.pv, pc.kv, T(0));
-    tile_apply_restrict<T, LD>(a, i0, j0, has_u, has_v, pc, s, tu, mu, tv, mv);
+    tile_apply_restrict<T>(a, i0, j0, pc, s, t, m);
     double du = 0.0, dv = 0.0;
     if (pc.oku) {
-        const T cv = pc.mwu ? tu[ly][lx] : T(0);
+        const T cv = pc.mwu ? t[0][ly][lx] : T(0);
         a.qu[pc.ku] = cv;
         du = (double)(pu * cv);
     }
     if (pc.okv) {
-        const T cv = pc.mwv ? tv[ly][lx] : T(0);
+        const T cv = pc.mwv ? t[1][ly][lx] : T(0);
         a.qv[pc.kv] = cv;
         dv = (double)(pv * cv);
     }
@@ -2301,16 +2335,16 @@ __device__ __forceinline__ void cg_update_tile(const CGArgs<T> &a, int par, cons
     }
 }
 
-template <typename T, bool PRE, bool LD>
+template <typename T, bool PRE>
 __global__ void __launch_bounds__(256) k_cg_dir(CGArgs<T> a, int par)
 {
-    (void)cg_dir_tile<T, PRE, LD>(a, par, xcd_tile(a.nblk));
+    (void)cg_dir_tile<T, PRE>(a, par, xcd_tile(a.nblk));
 }
 
-template <typename T, bool LD, bool EARLY>
+template <typename T, bool EARLY>
 __global__ void __launch_bounds__(256) k_cg_apply(CGArgs<T> a)
 {
-    cg_apply_tile<T, LD, EARLY>(a, xcd_tile(a.nblk));
+    cg_apply_tile<T, EARLY>(a, xcd_tile(a.nblk));
 }
 
 template <typename T, bool PRE, bool EARLY>
@@ -2355,13 +2389,13 @@ __global__ void __launch_bounds__(256) k_coarse_diag(GridDims g, OpCoef<double> 
     double fy = 0.0;
     if (jb == kjb && j0 + ly < nyw) {
         const int my = min(nyw - (j0 + jb), B), col = ky - kjb;
-        const uint32_t nz = c_haar[levels].nz[0][my][ly - jb], ng = c_haar[levels].neg[0][my][ly - jb];
+        const uint32_t nz = c_haar[levels].nz[my][ly - jb], ng = c_haar[levels].neg[my][ly - jb];
         if ((nz >> col) & 1u) fy = ((ng >> col) & 1u) ? -1.0 : 1.0;
     }
     const int ib = lx & ~(B - 1);
     const int mx = i0 + lx < nxw ? min(nxw - (i0 + ib), B) : 0;
-    const uint32_t nzx = mx > 0 ? c_haar[levels].nz[0][mx][lx - ib] : 0u;
-    const uint32_t ngx = mx > 0 ? c_haar[levels].neg[0][mx][lx - ib] : 0u;
+    const uint32_t nzx = mx > 0 ? c_haar[levels].nz[mx][lx - ib] : 0u;
+    const uint32_t ngx = mx > 0 ? c_haar[levels].neg[mx][lx - ib] : 0u;
     // zero windows (the halo and the other component stay zero)
     for (int q = threadIdx.x; q < 18 * 19; q += 256) {
         (&s.U[0][0])[q] = 0.0;
@@ -2601,7 +2635,7 @@ template <bool PRE>
 __global__ void __launch_bounds__(256) k_cgm_setup(CGMArgs a)
 {
     __shared__ OpTile<float> s;
-    __shared__ float tu[TILE][TILE + 1], mu[TILE][TILE + 1], tv[TILE][TILE + 1], mv[TILE][TILE + 1];
+    __shared__ TilePair<float> t, m;
     __shared__ double lds[8];
     const GridDims &g = a.g;
     const int L = xcd_tile(a.nblk);
@@ -2631,14 +2665,14 @@ __global__ void __launch_bounds__(256) k_cgm_setup(CGMArgs a)
     point_prefetch(g, a.c, a.mwu, a.mwv, i0 + lx, j0 + ly, has_u, has_v, pc);
     const float bu = pc.oku ? a.bu[pc.ku] : 0.f, bv = pc.okv ? a.bv[pc.kv] : 0.f;
     const float xu = pc.oku ? a.x0u[pc.ku] : 0.f, xv = pc.okv ? a.x0v[pc.kv] : 0.f;
-    optile_apply(g, a.c, a.t0u, a.t0v, i0, j0, pc, s, tu, tv);
-    haar_pm_tile2<float>(a.levels, 1, tu, mu, tv, mv, i0, j0, g, has_u, has_v);
+    optile_apply(g, a.c, a.t0u, a.t0v, i0, j0, pc, s, t);
+    haar_pair<true, float>(a.levels, t, m);
     float ru = 0.f, rv = 0.f;
     double b2u = 0.0, b2v = 0.0;
     // Jacobi: the rings hold P D^-1 r and ||b||^2 is the D^-1 norm
     const float dzu = PRE && pc.oku ? F[CGM_DINV * ns + o] : 1.f, dzv = PRE && pc.okv ? F[(CGM_DINV + 1) * ns + o] : 1.f;
     if (pc.oku) {
-        ru = bu - (pc.mwu ? tu[ly][lx] : 0.f);
+        ru = bu - (pc.mwu ? t[0][ly][lx] : 0.f);
         F[CGM_R * ns + o] = ru;
         F[CGM_P * ns + o] = 0.f;
         F[CGM_S * ns + o] = 0.f;
@@ -2646,7 +2680,7 @@ __global__ void __launch_bounds__(256) k_cgm_setup(CGMArgs a)
         b2u = PRE ? (double)bu * ((double)dzu * (double)bu) : (double)bu * (double)bu;
     }
     if (pc.okv) {
-        rv = bv - (pc.mwv ? tv[ly][lx] : 0.f);
+        rv = bv - (pc.mwv ? t[1][ly][lx] : 0.f);
         F[(CGM_R + 1) * ns + o] = rv;
         F[(CGM_P + 1) * ns + o] = 0.f;
         F[(CGM_S + 1) * ns + o] = 0.f;
@@ -2654,12 +2688,12 @@ __global__ void __launch_bounds__(256) k_cgm_setup(CGMArgs a)
         b2v = PRE ? (double)bv * ((double)dzv * (double)bv) : (double)bv * (double)bv;
     }
     // each thread rewrites only its own entry; the transform ended with a barrier
-    tu[ly][lx] = pc.mwu ? (PRE ? dzu * ru : ru) : 0.f;
-    tv[ly][lx] = pc.mwv ? (PRE ? dzv * rv : rv) : 0.f;
+    t[0][ly][lx] = pc.mwu ? (PRE ? dzu * ru : ru) : 0.f;
+    t[1][ly][lx] = pc.mwv ? (PRE ? dzv * rv : rv) : 0.f;
     __syncthreads();
-    haar_pm_tile2<float>(a.levels, 0, tu, mu, tv, mv, i0, j0, g, has_u, has_v);
-    if (pc.oku) ring_put(a.R, ring_at(0, g.nbx * g.nby, tile_id, 0, 0), lx, ly, pc.ui ? tu[ly][lx] : 0.f);
-    if (pc.okv) ring_put(a.R, ring_at(0, g.nbx * g.nby, tile_id, 0, 1), lx, ly, pc.vi ? tv[ly][lx] : 0.f);
+    haar_pair<false, float>(a.levels, t, m);
+    if (pc.oku) ring_put(a.R, ring_at(0, g.nbx * g.nby, tile_id, 0, 0), lx, ly, pc.ui ? t[0][ly][lx] : 0.f);
+    if (pc.okv) ring_put(a.R, ring_at(0, g.nbx * g.nby, tile_id, 0, 1), lx, ly, pc.vi ? t[1][ly][lx] : 0.f);
     tree256x2(b2u, b2v, lds);
     if (threadIdx.x == 0) {
         if (has_u) a.Pb[bx + g.nbxu * by] = b2u;
@@ -3201,30 +3235,26 @@ __device__ __forceinline__ bool mask_or_all(const uint8_t *mask, const void *any
 // +-1 transform only) the result is added into accu, accv at the points of
 // the output masks instead (x += P y, as an add of the masked output would
 // do), and outu, outv are not written.
-template <typename Tin, typename Tout, bool LD = false>
+template <typename Tin, typename Tout>
 __global__ void k_tile_haar(GridDims g, const HaarTable *tab, int levels, int dir,
                             const Tin *inu, const Tin *inv, const uint8_t *min_u, const uint8_t *min_v,
                             Tout *outu, Tout *outv, const uint8_t *mout_u, const uint8_t *mout_v,
                             Tout *accu = nullptr, Tout *accv = nullptr)
 {
-    __shared__ Tout tile[TILE][TILE + 1];
-    __shared__ Tout tmp[TILE][TILE + 1];
-    __shared__ Tout tile_v[TILE][TILE + 1];
-    __shared__ Tout tmp_v[TILE][TILE + 1];
+    __shared__ TilePair<Tout> t, m;
     const int lx = threadIdx.x & 15, ly = threadIdx.x >> 4;
     const int bx = blockIdx.x, by = blockIdx.y;
     const int i0 = bx * TILE, j0 = by * TILE;
     const int i = i0 + lx, j = j0 + ly;
     const bool has_u = bx < g.nbxu && by < g.nbyu, has_v = bx < g.nbxv && by < g.nbyv;
     if (dir != 0) {
-        // the +-1 transforms: the u and the v tile together, every input,
-        // mask and row mask loaded first (ld_or, haar_row_masks)
+        // the +-1 transforms: the u and the v tile together, every input
+        // and mask loaded first (ld_or)
         const int ku = i + g.nxu * j, kv = i + g.nxv * j;
         const bool oku = has_u && i < g.nxu && j < g.nyu, okv = has_v && i < g.nxv && j < g.nyv;
         const Tin xu = ld_or(oku, inu, ku, Tin(0)), xv = ld_or(okv, inv, kv, Tin(0));
         const bool iu = mask_or_all(min_u, inu, oku, ku), iv = mask_or_all(min_v, inv, okv, kv);
         const bool ou = mask_or_all(mout_u, inu, oku, ku), ov = mask_or_all(mout_v, inv, okv, kv);
-        const HaarRowMasks hm = haar_row_masks(levels, dir - 1, i0, j0, g, has_u, has_v);
         // the accumulation target's values, loaded with the inputs (a uniform
         // branch: their first use is after the transform)
         const bool acc = accu != nullptr;
@@ -3233,35 +3263,38 @@ __global__ void k_tile_haar(GridDims g, const HaarTable *tab, int levels, int di
             au = ld_or(oku, accu, ku, Tout(0));
             av = ld_or(okv, accv, kv, Tout(0));
         }
-        tile[ly][lx] = (oku && iu) ? (Tout)xu : Tout(0);
-        tile_v[ly][lx] = (okv && iv) ? (Tout)xv : Tout(0);
+        t[0][ly][lx] = (oku && iu) ? (Tout)xu : Tout(0);
+        t[1][ly][lx] = (okv && iv) ? (Tout)xv : Tout(0);
         __syncthreads();
-        haar_pm_tile2m<Tout, LD>(levels, hm, tile, tmp, tile_v, tmp_v, i0, j0, g, has_u, has_v);
+        if (dir == 1)
+            haar_pair<false, Tout>(levels, t, m);
+        else
+            haar_pair<true, Tout>(levels, t, m);
         if (acc) {
-            if (oku && ou) accu[ku] = au + tile[ly][lx];
-            if (okv && ov) accv[kv] = av + tile_v[ly][lx];
+            if (oku && ou) accu[ku] = au + t[0][ly][lx];
+            if (okv && ov) accv[kv] = av + t[1][ly][lx];
         } else {
-            if (oku) outu[ku] = ou ? tile[ly][lx] : Tout(0);
-            if (okv) outv[kv] = ov ? tile_v[ly][lx] : Tout(0);
+            if (oku) outu[ku] = ou ? t[0][ly][lx] : Tout(0);
+            if (okv) outv[kv] = ov ? t[1][ly][lx] : Tout(0);
         }
         return;
     }
     if (has_u) {
         int k = i + g.nxu * j;
         bool ok = i < g.nxu && j < g.nyu;
-        tile[ly][lx] = (ok && (!min_u || min_u[k])) ? (Tout)inu[k] : Tout(0);
+        t[0][ly][lx] = (ok && (!min_u || min_u[k])) ? (Tout)inu[k] : Tout(0);
         __syncthreads();
-        haar_tile<Tout>(tab, 0, tile, tmp, i0, j0, g.nxu, g.nyu);
-        if (ok) outu[k] = (!mout_u || mout_u[k]) ? tile[ly][lx] : Tout(0);
+        haar_tile<Tout>(tab, 0, t[0], m[0], i0, j0, g.nxu, g.nyu);
+        if (ok) outu[k] = (!mout_u || mout_u[k]) ? t[0][ly][lx] : Tout(0);
         __syncthreads();
     }
     if (has_v) {
         int k = i + g.nxv * j;
         bool ok = i < g.nxv && j < g.nyv;
-        tile[ly][lx] = (ok && (!min_v || min_v[k])) ? (Tout)inv[k] : Tout(0);
+        t[0][ly][lx] = (ok && (!min_v || min_v[k])) ? (Tout)inv[k] : Tout(0);
         __syncthreads();
-        haar_tile<Tout>(tab, 0, tile, tmp, i0, j0, g.nxv, g.nyv);
-        if (ok) outv[k] = (!mout_v || mout_v[k]) ? tile[ly][lx] : Tout(0);
+        haar_tile<Tout>(tab, 0, t[0], m[0], i0, j0, g.nxv, g.nyv);
+        if (ok) outv[k] = (!mout_v || mout_v[k]) ? t[0][ly][lx] : Tout(0);
         __syncthreads();
     }
 }
