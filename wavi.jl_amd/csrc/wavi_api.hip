@@ -76,6 +76,7 @@ struct wavi_ctx {
     // masks (uint8, device)
     uint8_t *hm = nullptr, *hfix = nullptr, *um = nullptr, *vm = nullptr, *cm = nullptr;
     uint8_t *ui = nullptr, *vi = nullptr, *ufix = nullptr, *vfix = nullptr, *mwu = nullptr, *mwv = nullptr;
+    uint8_t *mcu = nullptr, *mcv = nullptr;  // FP64 coarse CG: packed masks (k_cg_setup)
     bool has_fixed = false;     // any u_isfixed / v_isfixed point
     std::vector<uint8_t> h_ui, h_vi;  // host copies of the inner masks
     double *adj_base = nullptr;       // adjoint workspace, kept between gradient calls
@@ -600,6 +601,8 @@ int wavi_ctx_create(const wavi_grid_desc *grid, const wavi_phys_params *phys, co
     CREATECHK(alloc8(&ctx->vfix, vfix));
     CREATECHK(alloc8(&ctx->mwu, ones_u));  // UWavelets mask = trues (UWavelets.jl:38)
     CREATECHK(alloc8(&ctx->mwv, ones_v));
+    CREATECHK(alloc8(&ctx->mcu, ones_u));
+    CREATECHK(alloc8(&ctx->mcv, ones_v));
 
     for (int id = 0; id < WAVI_NFIELDS; ++id) {
         if (id == WAVI_WU_MASK || id == WAVI_WV_MASK) continue;
@@ -709,7 +712,7 @@ static void ctx_free(wavi_ctx *ctx)
 {
     if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
     for (uint8_t *p : {ctx->hm, ctx->hfix, ctx->um, ctx->vm, ctx->cm, ctx->ui, ctx->vi, ctx->ufix, ctx->vfix,
-                       ctx->mwu, ctx->mwv, ctx->saved_mwu, ctx->saved_mwv})
+                       ctx->mwu, ctx->mwv, ctx->mcu, ctx->mcv, ctx->saved_mwu, ctx->saved_mwv})
         if (p) (void)hipFree(p);
     for (int id = 0; id < WAVI_NFIELDS; ++id)
         if (ctx->f[id]) (void)hipFree(ctx->f[id]);
@@ -1214,6 +1217,8 @@ static CGArgs<T> cg_args(wavi_ctx *ctx, const VSet<T> &w)
     a.mwv = ctx->mwv;
     a.ui = ctx->ui;
     a.vi = ctx->vi;
+    a.mcu = ctx->mcu;
+    a.mcv = ctx->mcv;
     a.xu = w.xc.u;
     a.xv = w.xc.v;
     a.ru = w.cr.u;

@@ -1288,31 +1288,9 @@ __device__ __forceinline__ void cell_compute(const OpCoef<T> &c, const CellCoef<
 template <typename T>
 struct PointCoef {
     T bu, hu, bv, hv;
-    bool oku, okv, ui, um, vi, vm, mwu, mwv;
+    bool oku, okv, ui, um, vi, vm;
     int ku, kv;
 };
-
-template <typename T>
-__device__ __forceinline__ void point_prefetch(const GridDims &g, const OpCoef<T> &c, const uint8_t *mwu,
-                                               const uint8_t *mwv, int i, int j, bool has_u, bool has_v,
-                                               PointCoef<T> &pc)
-{
-    pc.oku = has_u && i < g.nxu && j < g.nyu;
-    pc.okv = has_v && i < g.nxv && j < g.nyv;
-    pc.ku = i + g.nxu * j;
-    pc.kv = i + g.nxv * j;
-    // loads issued unconditionally (ld_or)
-    pc.ui = ld_or(pc.oku, c.ui, pc.ku, (uint8_t)0) != 0;
-    pc.um = ld_or(pc.oku, c.um, pc.ku, (uint8_t)0) != 0;
-    pc.bu = ld_or(pc.oku, c.bu, pc.ku, T(0));
-    pc.hu = ld_or(pc.oku, c.hu, pc.ku, T(0));
-    pc.mwu = ld_or(pc.oku, mwu, pc.ku, (uint8_t)0) != 0;
-    pc.vi = ld_or(pc.okv, c.vi, pc.kv, (uint8_t)0) != 0;
-    pc.vm = ld_or(pc.okv, c.vm, pc.kv, (uint8_t)0) != 0;
-    pc.bv = ld_or(pc.okv, c.bv, pc.kv, T(0));
-    pc.hv = ld_or(pc.okv, c.hv, pc.kv, T(0));
-    pc.mwv = ld_or(pc.okv, mwv, pc.kv, (uint8_t)0) != 0;
-}
 
 // fx at the u point (i0 + x, j0 + y), whose value is s.U[y + 1][x + 1] and
 // whose cell (i, j) is s.rxx[y + 1][x + 1]
@@ -1337,70 +1315,217 @@ __device__ __forceinline__ T optile_v(const OpCoef<T> &c, const S &s, const Poin
     return ((d_ryy_dy + d_rxy_dx) - tauby) - pc.hv * d_extra_dy;
 }
 
-// Stage one tile of a fine vector: each thread loads its (at most two)
-// staging entries into registers; optile_store puts them in LDS.
-template <typename T>
-struct StageRegs {
-    T u0, v0, u1, v1;
+// The operator on a tile of u and v outputs from global memory.  What bounds
+// these kernels on any grid is the number of load and LDS instructions of a
+// wavefront, so each operand is loaded once: a thread loads its own u and v
+// point (value, thickness, drag, mask bits) and its own h cell and corner;
+// wavefront 3 adds the 64 points of the four sides of the one-point halo,
+// wavefront 2 the two halo corners that are read (u at (16, -1), v at
+// (-1, 16)), wavefront 0 the 33 cells before the tile.  13 to 19 loads a
+// wavefront instead of 42 with the window walked by 256 threads and every
+// cell loading its four thicknesses and six masks.  The fluxes h u and h v
+// of the implicit term are formed once per point, masked, and staged.
+// heta_h, dimp and heta_c are zero off the h and c masks, so those masks are
+// not read.  The arithmetic is that of op_u / op_v.
+
+// Mask bits of a u or v point: 1 inner, 2 u / v mask, 4 wavelet mask.
+enum { MB_INNER = 1, MB_POINT = 2, MB_WAVELET = 4 };
+
+// ... from the separate masks (mw may be null: bit 4 clear)
+template <bool MW>
+struct MaskSep {
+    const uint8_t *ui, *um, *vi, *vm, *mwu, *mwv;
+    __device__ __forceinline__ unsigned u(bool ok, int k) const
+    {
+        const int q = ok ? k : 0;
+        const unsigned a = ui[q], b = um[q], w = MW ? mwu[q] : 0;
+        return ok ? (a ? MB_INNER : 0u) | (b ? MB_POINT : 0u) | (w ? MB_WAVELET : 0u) : 0u;
+    }
+    __device__ __forceinline__ unsigned v(bool ok, int k) const
+    {
+        const int q = ok ? k : 0;
+        const unsigned a = vi[q], b = vm[q], w = MW ? mwv[q] : 0;
+        return ok ? (a ? MB_INNER : 0u) | (b ? MB_POINT : 0u) | (w ? MB_WAVELET : 0u) : 0u;
+    }
 };
 
+// ... packed, one byte per point
+struct MaskPacked {
+    const uint8_t *mu, *mv;
+    __device__ __forceinline__ unsigned u(bool ok, int k) const
+    {
+        const unsigned a = mu[ok ? k : 0];
+        return ok ? a : 0u;
+    }
+    __device__ __forceinline__ unsigned v(bool ok, int k) const
+    {
+        const unsigned a = mv[ok ? k : 0];
+        return ok ? a : 0u;
+    }
+};
+
+// Window point (x, y) is (i0 - 1 + x, j0 - 1 + y); cell (x, y) has the same
+// origin.  The transforms' tiles share the window's room: the window is read
+// last before the barrier that the outputs follow.
 template <typename T>
-__device__ __forceinline__ void optile_fetch(const GridDims &g, const T *U, const T *V, int i0, int j0,
-                                             StageRegs<T> &r)
+struct OpLds {
+    union {
+        struct {
+            T U[18][19], V[18][19], QX[18][19], QY[18][19];
+        } w;
+        struct {
+            TilePair<T> t, m;
+        } h;
+    };
+    T rxx[17][18], ryy[17][18], ext[17][18], rxy[17][18];
+};
+
+// What a thread holds of its tile.
+template <typename T>
+struct OpOwn {
+    T u, v, hu, hv, bu, bv;
+    T heta, dimp, hetac;
+    unsigned mu, mv;  // mask bits
+    bool oku, okv;
+    int ku, kv;
+};
+
+// h cell (a, b) and its corner: 0 outside their grids
+template <typename T>
+__device__ __forceinline__ void op_cell_load(const GridDims &g, const OpCoef<T> &c, int a, int b, T &heta, T &dimp,
+                                             T &hetac)
 {
-    const int q0 = threadIdx.x, q1 = threadIdx.x + 256;
-    {
-        const int x = q0 % 18, y = q0 / 18, i = i0 - 1 + x, j = j0 - 1 + y;
-        r.u0 = ld_or(i >= 0 && i < g.nxu && j >= 0 && j < g.nyu, U, i + g.nxu * j, T(0));
-        r.v0 = ld_or(i >= 0 && i < g.nxv && j >= 0 && j < g.nyv, V, i + g.nxv * j, T(0));
+    const bool cell = a >= 0 && a < g.nx && b >= 0 && b < g.ny;
+    const bool corner = a >= 0 && a < g.nx - 1 && b >= 0 && b < g.ny - 1;
+    heta = ld_or(cell, c.heta_h, a + g.nx * b, T(0));
+    dimp = ld_or(cell, c.dimp, a + g.nx * b, T(0));
+    hetac = ld_or(corner, c.heta_c, a + (g.nx - 1) * b, T(0));
+}
+
+// Intermediates of cell (x, y) (the expressions of op_rxx, op_ryy, op_extra,
+// op_rxy).  Cell (0, 0) reads one absent window point of each kind and corner
+// (16, 16) another; no output reads what they feed.
+template <typename T>
+__device__ __forceinline__ void op_cell(const OpCoef<T> &c, OpLds<T> &s, int x, int y, T heta, T dimp, T hetac)
+{
+    const T u0 = s.w.U[y][x], u1 = s.w.U[y][x + 1], v0 = s.w.V[y][x], v1 = s.w.V[y + 1][x];
+    const T dudx = c.rdx * u1 - c.rdx * u0;
+    const T dvdy = c.rdy * v1 - c.rdy * v0;
+    const T divq = (c.rdx * s.w.QX[y][x + 1] - c.rdx * s.w.QX[y][x]) + (c.rdy * s.w.QY[y + 1][x] - c.rdy * s.w.QY[y][x]);
+    const T dudy = c.rdy * s.w.U[y + 1][x + 1] - c.rdy * u1;
+    const T dvdx = c.rdx * s.w.V[y + 1][x + 1] - c.rdx * v1;
+    s.rxx[y][x] = T(2) * (heta * (T(2) * dudx + dvdy));
+    s.ryy[y][x] = T(2) * (heta * (T(2) * dvdy + dudx));
+    s.ext[y][x] = dimp * divq;
+    s.rxy[y][x] = hetac * (dudy + dvdx);
+}
+
+// Load the tile of (xu, xv) and its coefficients and compute the cells'
+// intermediates (ends with a barrier, after which the window is free).
+template <typename T, class M>
+__device__ __forceinline__ void op_tile(const GridDims &g, const OpCoef<T> &c, const M &mask, const T *xu, const T *xv,
+                                        int i0, int j0, OpLds<T> &s, OpOwn<T> &o)
+{
+    const int lx = threadIdx.x & 15, ly = threadIdx.x >> 4, l = threadIdx.x & 63;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int i = i0 + lx, j = j0 + ly;
+    o.oku = i < g.nxu && j < g.nyu;
+    o.okv = i < g.nxv && j < g.nyv;
+    o.ku = i + g.nxu * j;
+    o.kv = i + g.nxv * j;
+    o.u = ld_or(o.oku, xu, o.ku, T(0));
+    o.v = ld_or(o.okv, xv, o.kv, T(0));
+    o.hu = ld_or(o.oku, c.hu, o.ku, T(0));
+    o.hv = ld_or(o.okv, c.hv, o.kv, T(0));
+    o.mu = mask.u(o.oku, o.ku);
+    o.mv = mask.v(o.okv, o.kv);
+    // halo points: U and V at (ux, uy), (vx, vy) of the window
+    int ux = 17, uy = 0, vx = 0, vy = 17;
+    T hu = T(0), hv = T(0), hhu = T(0), hhv = T(0);
+    unsigned hmu = 0, hmv = 0;
+    if (w >= 2) {
+        if (w == 3) {
+            const int q = 1 + (l & 15), far = (l & 16) ? 17 : 0;
+            ux = vx = l < 32 ? far : q;
+            uy = vy = l < 32 ? q : far;
+        }
+        const int iu = i0 - 1 + ux, ju = j0 - 1 + uy, iv = i0 - 1 + vx, jv = j0 - 1 + vy;
+        const bool in = w == 3 || l == 0;
+        const bool okhu = in && iu >= 0 && iu < g.nxu && ju >= 0 && ju < g.nyu;
+        const bool okhv = in && iv >= 0 && iv < g.nxv && jv >= 0 && jv < g.nyv;
+        const int khu = iu + g.nxu * ju, khv = iv + g.nxv * jv;
+        hu = ld_or(okhu, xu, khu, T(0));
+        hv = ld_or(okhv, xv, khv, T(0));
+        hhu = ld_or(okhu, c.hu, khu, T(0));
+        hhv = ld_or(okhv, c.hv, khv, T(0));
+        hmu = mask.u(okhu, khu);
+        hmv = mask.v(okhv, khv);
     }
-    {
-        const int x = q1 % 18, y = q1 / 18, i = i0 - 1 + x, j = j0 - 1 + y;
-        const bool in = q1 < 324;
-        r.u1 = ld_or(in && i >= 0 && i < g.nxu && j >= 0 && j < g.nyu, U, i + g.nxu * j, T(0));
-        r.v1 = ld_or(in && i >= 0 && i < g.nxv && j >= 0 && j < g.nyv, V, i + g.nxv * j, T(0));
+    op_cell_load(g, c, i, j, o.heta, o.dimp, o.hetac);
+    // the cells before the tile: (0, 0..16), (1..16, 0)
+    const int ex = l < 17 ? 0 : l - 16, ey = l < 17 ? l : 0;
+    T eh = T(0), ed = T(0), ec = T(0);
+    if (w == 0) op_cell_load(g, c, l < 33 ? i0 - 1 + ex : -1, j0 - 1 + ey, eh, ed, ec);
+    o.bu = ld_or(o.oku, c.bu, o.ku, T(0));
+    o.bv = ld_or(o.okv, c.bv, o.kv, T(0));
+    s.w.U[ly + 1][lx + 1] = o.u;
+    s.w.V[ly + 1][lx + 1] = o.v;
+    s.w.QX[ly + 1][lx + 1] = (o.mu & MB_POINT) ? o.hu * o.u : T(0);
+    s.w.QY[ly + 1][lx + 1] = (o.mv & MB_POINT) ? o.hv * o.v : T(0);
+    if (w == 3 || (w == 2 && l == 0)) {
+        s.w.U[uy][ux] = hu;
+        s.w.V[vy][vx] = hv;
+        s.w.QX[uy][ux] = (hmu & MB_POINT) ? hhu * hu : T(0);
+        s.w.QY[vy][vx] = (hmv & MB_POINT) ? hhv * hv : T(0);
     }
+    __syncthreads();
+    op_cell(c, s, lx + 1, ly + 1, o.heta, o.dimp, o.hetac);
+    if (w == 0 && l < 33) op_cell(c, s, ex, ey, eh, ed, ec);
+    __syncthreads();
+}
+
+// A x at the thread's u point and v point (inner or not)
+template <typename T>
+__device__ __forceinline__ T op_out_u(const OpCoef<T> &c, const OpLds<T> &s, const OpOwn<T> &o)
+{
+    const int x = threadIdx.x & 15, y = threadIdx.x >> 4;
+    const T d_rxx_dx = c.rdx * s.rxx[y + 1][x + 1] - c.rdx * s.rxx[y + 1][x];
+    const T d_rxy_dy = c.rdy * s.rxy[y + 1][x] - c.rdy * s.rxy[y][x];
+    const T taubx = (o.mu & MB_POINT) ? o.bu * o.u : T(0);
+    const T d_extra_dx = c.rdx * s.ext[y + 1][x + 1] - c.rdx * s.ext[y + 1][x];
+    return ((d_rxx_dx + d_rxy_dy) - taubx) - o.hu * d_extra_dx;
 }
 
 template <typename T>
-__device__ __forceinline__ void optile_store(const StageRegs<T> &r, OpTile<T> &s)
+__device__ __forceinline__ T op_out_v(const OpCoef<T> &c, const OpLds<T> &s, const OpOwn<T> &o)
 {
-    const int q0 = threadIdx.x, q1 = threadIdx.x + 256;
-    s.U[q0 / 18][q0 % 18] = r.u0;
-    s.V[q0 / 18][q0 % 18] = r.v0;
-    if (q1 < 324) {
-        s.U[q1 / 18][q1 % 18] = r.u1;
-        s.V[q1 / 18][q1 % 18] = r.v1;
-    }
+    const int x = threadIdx.x & 15, y = threadIdx.x >> 4;
+    const T d_ryy_dy = c.rdy * s.ryy[y + 1][x + 1] - c.rdy * s.ryy[y][x + 1];
+    const T d_rxy_dx = c.rdx * s.rxy[y][x + 1] - c.rdx * s.rxy[y][x];
+    const T tauby = (o.mv & MB_POINT) ? o.bv * o.v : T(0);
+    const T d_extra_dy = c.rdy * s.ext[y + 1][x + 1] - c.rdy * s.ext[y][x + 1];
+    return ((d_ryy_dy + d_rxy_dx) - tauby) - o.hv * d_extra_dy;
 }
 
-// The whole tile operator with prefetch: stage t, compute intermediates,
-// outputs into t (zero off the inner masks).  Ends with a barrier.
-template <typename T>
-__device__ __forceinline__ void optile_apply(const GridDims &g, const OpCoef<T> &c, const T *tU, const T *tV,
-                                             int i0, int j0, const PointCoef<T> &pc, OpTile<T> &s,
-                                             TilePair<T> &t)
+// R A x of the tile into s.h.t (A zero off the inner masks; valid at the
+// wavelet masks' points), x on the fine grid.  Ends with a barrier.
+template <typename T, class M>
+__device__ __forceinline__ void op_restrict_tile(const GridDims &g, const OpCoef<T> &c, const M &mask, int levels,
+                                                 const T *xu, const T *xv, int i0, int j0, OpLds<T> &s, OpOwn<T> &o)
 {
-    StageRegs<T> sr;
-    CellCoef<T> c0, c1;
-    optile_fetch(g, tU, tV, i0, j0, sr);
-    cell_prefetch(g, c, i0, j0, threadIdx.x, c0);
-    cell_prefetch(g, c, i0, j0, threadIdx.x + 256, c1);
-    optile_store(sr, s);
-    __syncthreads();
-    cell_compute(c, c0, threadIdx.x, s);
-    cell_compute(c, c1, threadIdx.x + 256, s);
-    __syncthreads();
     const int lx = threadIdx.x & 15, ly = threadIdx.x >> 4;
-    t[0][ly][lx] = (pc.oku && pc.ui) ? optile_u(c, s, pc, lx, ly) : T(0);
-    t[1][ly][lx] = (pc.okv && pc.vi) ? optile_v(c, s, pc, lx, ly) : T(0);
+    op_tile(g, c, mask, xu, xv, i0, j0, s, o);
+    const T yu = (o.mu & MB_INNER) ? op_out_u(c, s, o) : T(0), yv = (o.mv & MB_INNER) ? op_out_v(c, s, o) : T(0);
+    s.h.t[0][ly][lx] = yu;
+    s.h.t[1][ly][lx] = yv;
     __syncthreads();
+    haar_pair<true, T>(levels, s.h.t, s.h.m);
 }
 
 // ===========================================================================
 // Operator application and residual on 16 x 16 tiles of u and v points: the
 // tile stages its inputs with a one-point halo and its coefficients once
-// (OpTile), computes every intermediate once, and each thread evaluates its
+// (op_tile), computes every intermediate once, and each thread evaluates its
 // u and its v point.  The arithmetic is that of op_u / op_v, so the results
 // equal the per-point forms bit for bit.  Launched as nblk workgroups
 // (xcd_band_tile).
@@ -1430,7 +1555,6 @@ __device__ __forceinline__ void point_prefetch_op(const GridDims &g, const OpCoe
     pc.okv = has_v && i < g.nxv && j < g.nyv;
     pc.ku = i + g.nxu * j;
     pc.kv = i + g.nxv * j;
-    pc.mwu = pc.mwv = false;
     // loads issued unconditionally (ld_or)
     pc.ui = ld_or(pc.oku, c.ui, pc.ku, (uint8_t)0) != 0;
     pc.um = ld_or(pc.oku, c.um, pc.ku, (uint8_t)0) != 0;
@@ -1442,38 +1566,18 @@ __device__ __forceinline__ void point_prefetch_op(const GridDims &g, const OpCoe
     pc.hv = ld_or(pc.okv, c.hv, pc.kv, T(0));
 }
 
-// Stage the tile's window of x and its intermediates (ends with a barrier).
-template <typename T>
-__device__ __forceinline__ void optile_prepare(const GridDims &g, const OpCoef<T> &c, const T *xu, const T *xv,
-                                               int i0, int j0, OpTile<T> &s)
-{
-    StageRegs<T> sr;
-    CellCoef<T> c0, c1;
-    optile_fetch(g, xu, xv, i0, j0, sr);
-    cell_prefetch(g, c, i0, j0, threadIdx.x, c0);
-    cell_prefetch(g, c, i0, j0, threadIdx.x + 256, c1);
-    optile_store(sr, s);
-    __syncthreads();
-    cell_compute(c, c0, threadIdx.x, s);
-    cell_compute(c, c1, threadIdx.x + 256, s);
-    __syncthreads();
-}
-
 // y = A x at inner points, 0 elsewhere
 template <typename T>
 __global__ void __launch_bounds__(256) k_op(GridDims g, OpCoef<T> c, const T *xu, const T *xv, T *yu, T *yv,
                                             int nblk)
 {
-    __shared__ OpTile<T> s;
+    __shared__ OpLds<T> s;
     int bx, by;
     if (!xcd_band_tile(g.nbx, g.nby, nblk, true, bx, by)) return;
-    const bool has_u = bx < g.nbxu && by < g.nbyu, has_v = bx < g.nbxv && by < g.nbyv;
-    const int i0 = bx * TILE, j0 = by * TILE, lx = threadIdx.x & 15, ly = threadIdx.x >> 4;
-    PointCoef<T> pc;
-    point_prefetch_op(g, c, i0 + lx, j0 + ly, has_u, has_v, pc);
-    optile_prepare(g, c, xu, xv, i0, j0, s);
-    if (pc.oku) yu[pc.ku] = pc.ui ? optile_u(c, s, pc, lx, ly) : T(0);
-    if (pc.okv) yv[pc.kv] = pc.vi ? optile_v(c, s, pc, lx, ly) : T(0);
+    OpOwn<T> o;
+    op_tile(g, c, MaskSep<false>{c.ui, c.um, c.vi, c.vm, nullptr, nullptr}, xu, xv, bx * TILE, by * TILE, s, o);
+    if (o.oku) yu[o.ku] = (o.mu & MB_INNER) ? op_out_u(c, s, o) : T(0);
+    if (o.okv) yv[o.kv] = (o.mv & MB_INNER) ? op_out_v(c, s, o) : T(0);
 }
 
 // r = b - A x at inner points (get_resid!, utilities.jl:549-552); per-tile
@@ -1486,22 +1590,23 @@ __global__ void __launch_bounds__(256) k_tile_resid(GridDims g, OpCoef<T> c, con
                                                     const T *bv, T *ru, T *rv, double *Pr, double *Pb, int nblk,
                                                     T *fu = nullptr, T *fv = nullptr)
 {
-    __shared__ OpTile<T> s;
+    __shared__ OpLds<T> s;
     __shared__ double lds[8];
     int bx, by;
     if (!xcd_band_tile(g.nbx, g.nby, nblk, true, bx, by)) return;
     const bool has_u = bx < g.nbxu && by < g.nbyu, has_v = bx < g.nbxv && by < g.nbyv;
-    const int i0 = bx * TILE, j0 = by * TILE, lx = threadIdx.x & 15, ly = threadIdx.x >> 4;
-    PointCoef<T> pc;
-    point_prefetch_op(g, c, i0 + lx, j0 + ly, has_u, has_v, pc);
-    const T b_u = ld_or(pc.oku, bu, pc.ku, T(0)), b_v = ld_or(pc.okv, bv, pc.kv, T(0));
-    optile_prepare(g, c, xu, xv, i0, j0, s);
+    // the thread's right-hand side, loaded before the operator's barriers
+    const int i = bx * TILE + (threadIdx.x & 15), j = by * TILE + (threadIdx.x >> 4);
+    const T b_u = ld_or(i < g.nxu && j < g.nyu, bu, i + g.nxu * j, T(0));
+    const T b_v = ld_or(i < g.nxv && j < g.nyv, bv, i + g.nxv * j, T(0));
+    OpOwn<T> o;
+    op_tile(g, c, MaskSep<false>{c.ui, c.um, c.vi, c.vm, nullptr, nullptr}, xu, xv, bx * TILE, by * TILE, s, o);
     if (has_u) {
         double r2 = 0.0, b2 = 0.0;
-        if (pc.oku) {
-            const T r = pc.ui ? b_u - optile_u(c, s, pc, lx, ly) : T(0);
-            ru[pc.ku] = r;
-            if (fu && pc.ui) fu[pc.ku] = r;
+        if (o.oku) {
+            const T r = (o.mu & MB_INNER) ? b_u - op_out_u(c, s, o) : T(0);
+            ru[o.ku] = r;
+            if (fu && (o.mu & MB_INNER)) fu[o.ku] = r;
             r2 = (double)r * (double)r;
             b2 = (double)b_u * (double)b_u;
         }
@@ -1513,18 +1618,18 @@ __global__ void __launch_bounds__(256) k_tile_resid(GridDims g, OpCoef<T> c, con
     }
     if (has_v) {
         double r2 = 0.0, b2 = 0.0;
-        if (pc.okv) {
-            const T r = pc.vi ? b_v - optile_v(c, s, pc, lx, ly) : T(0);
-            rv[pc.kv] = r;
-            if (fv && pc.vi) fv[pc.kv] = r;
+        if (o.okv) {
+            const T r = (o.mv & MB_INNER) ? b_v - op_out_v(c, s, o) : T(0);
+            rv[o.kv] = r;
+            if (fv && (o.mv & MB_INNER)) fv[o.kv] = r;
             r2 = (double)r * (double)r;
             b2 = (double)b_v * (double)b_v;
         }
         tree256x2(r2, b2, lds);
         if (threadIdx.x == 0) {
-            const int o = g.nbxu * g.nbyu + bx + g.nbxv * by;
-            Pr[o] = r2;
-            if (Pb) Pb[o] = b2;
+            const int q = g.nbxu * g.nbyu + bx + g.nbxv * by;
+            Pr[q] = r2;
+            if (Pb) Pb[q] = b2;
         }
     }
 }
@@ -1603,7 +1708,7 @@ __global__ void __launch_bounds__(256) k_smooth4(GridDims g, OpCoef<T> c, const 
         pc.okv = q < S::PX * S::PY && i >= 0 && j >= 0 && i < g.nxv && j < g.nyv;
         pc.ku = i + g.nxu * j;
         pc.kv = i + g.nxv * j;
-        pc.ui = pc.um = pc.vi = pc.vm = pc.mwu = pc.mwv = false;
+        pc.ui = pc.um = pc.vi = pc.vm = false;
         pc.bu = pc.hu = pc.bv = pc.hv = T(0);
         sp[k].bu = sp[k].du = sp[k].bv = sp[k].dv = T(0);
         T u = T(0), v = T(0);
@@ -1760,7 +1865,7 @@ __global__ void __launch_bounds__(SMG_THREADS) k_smooth_grid(GridDims g, OpCoef<
         pc.okv = q < PX * PY && i >= 0 && j >= 0 && i < g.nxv && j < g.nyv;
         pc.ku = i + g.nxu * j;
         pc.kv = i + g.nxv * j;
-        pc.ui = pc.um = pc.vi = pc.vm = pc.mwu = pc.mwv = false;
+        pc.ui = pc.um = pc.vi = pc.vm = false;
         pc.bu = pc.hu = pc.bv = pc.hv = T(0);
         sp[k].bu = sp[k].du = sp[k].bv = sp[k].dv = T(0);
         T u = T(0), v = T(0);
@@ -2005,6 +2110,7 @@ struct CGArgs {
     OpCoef<T> c;
     int levels;
     const uint8_t *mwu, *mwv, *ui, *vi;
+    uint8_t *mcu, *mcv;  // packed mask bits (MB_*) of the u and v points, written by k_cg_setup
     T *xu, *xv;       // solution (warm start in, result out)
     T *ru, *rv;       // residual (right-hand side on entry to setup)
     T *pu, *pv;       // search direction u
@@ -2038,24 +2144,13 @@ __device__ __forceinline__ int band_tile(const GridDims &g, int L, int &bx, int 
     return L;
 }
 
-// c = R A t for the tile: A into `t`, then the transposed inverse Haar (c at
-// the wavelet masks' points).
-template <typename T>
-__device__ __forceinline__ void tile_apply_restrict(const CGArgs<T> &a, int i0, int j0, const PointCoef<T> &pc,
-                                                    OpTile<T> &s, TilePair<T> &t, TilePair<T> &m)
-{
-    optile_apply(a.g, a.c, a.tu, a.tv, i0, j0, pc, s, t);
-    haar_pair<true, T>(a.levels, t, m);
-}
-
 // setup (t = P x0 computed beforehand): r = b - R A t (b arrives in r),
-// u = 0, partials of ||r0||^2 and ||b||^2 (PRE: also of (r0, D^-1 r0));
-// resets the scalars.
+// u = 0, partials of ||r0||^2 and ||b||^2 (PRE: also of (r0, D^-1 r0)),
+// the packed masks of the iterations; resets the scalars.
 template <typename T, bool PRE>
 __global__ void __launch_bounds__(256) k_cg_setup(CGArgs<T> a)
 {
-    __shared__ OpTile<T> s;
-    __shared__ TilePair<T> t, m;
+    __shared__ OpLds<T> s;
     __shared__ double lds[8];
     const GridDims &g = a.g;
     const int L = xcd_tile(a.nblk);
@@ -2076,26 +2171,30 @@ __global__ void __launch_bounds__(256) k_cg_setup(CGArgs<T> a)
     const bool has_u = bx < g.nbxu && by < g.nbyu, has_v = bx < g.nbxv && by < g.nbyv;
     const int i0 = bx * TILE, j0 = by * TILE;
     const int lx = threadIdx.x & 15, ly = threadIdx.x >> 4;
-    PointCoef<T> pc;
-    point_prefetch(g, a.c, a.mwu, a.mwv, i0 + lx, j0 + ly, has_u, has_v, pc);
-    const T bu = pc.oku ? a.ru[pc.ku] : T(0), bv = pc.okv ? a.rv[pc.kv] : T(0);
-    tile_apply_restrict<T>(a, i0, j0, pc, s, t, m);
+    const int i = i0 + lx, j = j0 + ly;
+    const T bu = ld_or(i < g.nxu && j < g.nyu, a.ru, i + g.nxu * j, T(0));
+    const T bv = ld_or(i < g.nxv && j < g.nyv, a.rv, i + g.nxv * j, T(0));
+    OpOwn<T> o;
+    op_restrict_tile(g, a.c, MaskSep<true>{a.ui, a.c.um, a.vi, a.c.vm, a.mwu, a.mwv}, a.levels, a.tu, a.tv, i0, j0, s,
+                     o);
+    if (o.oku) a.mcu[o.ku] = (uint8_t)o.mu;
+    if (o.okv) a.mcv[o.kv] = (uint8_t)o.mv;
     double r2u = 0.0, b2u = 0.0, r2v = 0.0, b2v = 0.0, z2u = 0.0, z2v = 0.0;
-    if (pc.oku) {
-        const T r = bu - (pc.mwu ? t[0][ly][lx] : T(0));
-        a.ru[pc.ku] = r;
-        a.pu[pc.ku] = T(0);
+    if (o.oku) {
+        const T r = bu - ((o.mu & MB_WAVELET) ? s.h.t[0][ly][lx] : T(0));
+        a.ru[o.ku] = r;
+        a.pu[o.ku] = T(0);
         r2u = (double)r * (double)r;
         b2u = (double)bu * (double)bu;
-        if constexpr (PRE) z2u = (double)r * (a.dinvu[pc.ku] * (double)r);
+        if constexpr (PRE) z2u = (double)r * (a.dinvu[o.ku] * (double)r);
     }
-    if (pc.okv) {
-        const T r = bv - (pc.mwv ? t[1][ly][lx] : T(0));
-        a.rv[pc.kv] = r;
-        a.pv[pc.kv] = T(0);
+    if (o.okv) {
+        const T r = bv - ((o.mv & MB_WAVELET) ? s.h.t[1][ly][lx] : T(0));
+        a.rv[o.kv] = r;
+        a.pv[o.kv] = T(0);
         r2v = (double)r * (double)r;
         b2v = (double)bv * (double)bv;
-        if constexpr (PRE) z2v = (double)r * (a.dinvv[pc.kv] * (double)r);
+        if constexpr (PRE) z2v = (double)r * (a.dinvv[o.kv] * (double)r);
     }
     tree256x2(r2u, r2v, lds);
     tree256x2(b2u, b2v, lds);
@@ -2107,10 +2206,10 @@ __global__ void __launch_bounds__(256) k_cg_setup(CGArgs<T> a)
             if constexpr (PRE) a.Pz[bx + g.nbxu * by] = z2u;
         }
         if (has_v) {
-            const int o = g.nbxu * g.nbyu + bx + g.nbxv * by;
-            a.Pr[o] = r2v;
-            a.Pb[o] = b2v;
-            if constexpr (PRE) a.Pz[o] = z2v;
+            const int q = g.nbxu * g.nbyu + bx + g.nbxv * by;
+            a.Pr[q] = r2v;
+            a.Pb[q] = b2v;
+            if constexpr (PRE) a.Pz[q] = z2v;
         }
     }
 }
@@ -2154,8 +2253,8 @@ __device__ __forceinline__ bool cg_dir_tile(const CGArgs<T> &a, int par, const i
     const double told = cg_scalar(&a.st->tol), prev_res = cg_scalar(&a.st->res[1 - par]);
     const T ru = ld_or(oku, a.ru, ku, T(0)), pu = ld_or(oku, a.pu, ku, T(0));
     const T rv = ld_or(okv, a.rv, kv, T(0)), pv = ld_or(okv, a.pv, kv, T(0));
-    const bool mwu = ld_or(oku, a.mwu, ku, (uint8_t)0) != 0, mwv = ld_or(okv, a.mwv, kv, (uint8_t)0) != 0;
-    const bool iu = ld_or(oku, a.ui, ku, (uint8_t)0) != 0, iv = ld_or(okv, a.vi, kv, (uint8_t)0) != 0;
+    const unsigned mu = ld_or(oku, (const uint8_t *)a.mcu, ku, (uint8_t)0);
+    const unsigned mv = ld_or(okv, (const uint8_t *)a.mcv, kv, (uint8_t)0);
     double dzu = 0.0, dzv = 0.0, rz = 0.0, prev_rz = 0.0;
     if constexpr (PRE) {
         dzu = ld_or(oku, a.dinvu, ku, 0.0);
@@ -2216,12 +2315,12 @@ __device__ __forceinline__ bool cg_dir_tile(const CGArgs<T> &a, int par, const i
             unv = rv + beta * pv;
         a.pv[kv] = unv;
     }
-    t[0][ly][lx] = mwu ? unu : T(0);
-    t[1][ly][lx] = mwv ? unv : T(0);
+    t[0][ly][lx] = (mu & MB_WAVELET) ? unu : T(0);
+    t[1][ly][lx] = (mv & MB_WAVELET) ? unv : T(0);
     __syncthreads();
     haar_pair<false, T>(a.levels, t, m);
-    if (oku) a.tu[ku] = iu ? t[0][ly][lx] : T(0);
-    if (okv) a.tv[kv] = iv ? t[1][ly][lx] : T(0);
+    if (oku) a.tu[ku] = (mu & MB_INNER) ? t[0][ly][lx] : T(0);
+    if (okv) a.tv[kv] = (mv & MB_INNER) ? t[1][ly][lx] : T(0);
     return false;
 }
 
@@ -2233,8 +2332,7 @@ __device__ __forceinline__ bool cg_dir_tile(const CGArgs<T> &a, int par, const i
 template <typename T, bool EARLY = true>
 __device__ __forceinline__ void cg_apply_tile(const CGArgs<T> &a, const int L)
 {
-    __shared__ OpTile<T> s;
-    __shared__ TilePair<T> t, m;
+    __shared__ OpLds<T> s;
     __shared__ double lds[8];
     const GridDims &g = a.g;
     if (L >= g.nbx * g.nby) return;
@@ -2244,19 +2342,20 @@ __device__ __forceinline__ void cg_apply_tile(const CGArgs<T> &a, const int L)
     const bool has_u = bx < g.nbxu && by < g.nbyu, has_v = bx < g.nbxv && by < g.nbyv;
     const int i0 = bx * TILE, j0 = by * TILE;
     const int lx = threadIdx.x & 15, ly = threadIdx.x >> 4;
-    PointCoef<T> pc;
-    point_prefetch(g, a.c, a.mwu, a.mwv, i0 + lx, j0 + ly, has_u, has_v, pc);
-    const T pu = ld_or(pc.oku, a.pu, pc.ku, T(0)), pv = ld_or(pc.okv, a.pv, pc.kv, T(0));
-    tile_apply_restrict<T>(a, i0, j0, pc, s, t, m);
+    const int i = i0 + lx, j = j0 + ly;
+    const T pu = ld_or(i < g.nxu && j < g.nyu, a.pu, i + g.nxu * j, T(0));
+    const T pv = ld_or(i < g.nxv && j < g.nyv, a.pv, i + g.nxv * j, T(0));
+    OpOwn<T> o;
+    op_restrict_tile(g, a.c, MaskPacked{a.mcu, a.mcv}, a.levels, a.tu, a.tv, i0, j0, s, o);
     double du = 0.0, dv = 0.0;
-    if (pc.oku) {
-        const T cv = pc.mwu ? t[0][ly][lx] : T(0);
-        a.qu[pc.ku] = cv;
+    if (o.oku) {
+        const T cv = (o.mu & MB_WAVELET) ? s.h.t[0][ly][lx] : T(0);
+        a.qu[o.ku] = cv;
         du = (double)(pu * cv);
     }
-    if (pc.okv) {
-        const T cv = pc.mwv ? t[1][ly][lx] : T(0);
-        a.qv[pc.kv] = cv;
+    if (o.okv) {
+        const T cv = (o.mv & MB_WAVELET) ? s.h.t[1][ly][lx] : T(0);
+        a.qv[o.kv] = cv;
         dv = (double)(pv * cv);
     }
     tree256x2(du, dv, lds);
@@ -2634,8 +2733,7 @@ struct CGMArgs {
 template <bool PRE>
 __global__ void __launch_bounds__(256) k_cgm_setup(CGMArgs a)
 {
-    __shared__ OpTile<float> s;
-    __shared__ TilePair<float> t, m;
+    __shared__ OpLds<float> s;
     __shared__ double lds[8];
     const GridDims &g = a.g;
     const int L = xcd_tile(a.nblk);
@@ -2660,40 +2758,43 @@ __global__ void __launch_bounds__(256) k_cgm_setup(CGMArgs a)
     const int i0 = bx * TILE, j0 = by * TILE;
     const int lx = threadIdx.x & 15, ly = threadIdx.x >> 4;
     float *F = a.Lo.F;
-    const unsigned ns = a.Lo.ns, o = a.Lo.at(i0 + lx, j0 + ly);
-    PointCoef<float> pc;
-    point_prefetch(g, a.c, a.mwu, a.mwv, i0 + lx, j0 + ly, has_u, has_v, pc);
-    const float bu = pc.oku ? a.bu[pc.ku] : 0.f, bv = pc.okv ? a.bv[pc.kv] : 0.f;
-    const float xu = pc.oku ? a.x0u[pc.ku] : 0.f, xv = pc.okv ? a.x0v[pc.kv] : 0.f;
-    optile_apply(g, a.c, a.t0u, a.t0v, i0, j0, pc, s, t);
-    haar_pair<true, float>(a.levels, t, m);
+    const unsigned ns = a.Lo.ns, at = a.Lo.at(i0 + lx, j0 + ly);
+    const int i = i0 + lx, j = j0 + ly;
+    const bool oku = i < g.nxu && j < g.nyu, okv = i < g.nxv && j < g.nyv;
+    const int ku = i + g.nxu * j, kv = i + g.nxv * j;
+    const float bu = ld_or(oku, a.bu, ku, 0.f), bv = ld_or(okv, a.bv, kv, 0.f);
+    const float xu = ld_or(oku, a.x0u, ku, 0.f), xv = ld_or(okv, a.x0v, kv, 0.f);
+    OpOwn<float> o;
+    op_restrict_tile(g, a.c, MaskSep<true>{a.c.ui, a.c.um, a.c.vi, a.c.vm, a.mwu, a.mwv}, a.levels, a.t0u, a.t0v, i0,
+                     j0, s, o);
+    TilePair<float> &t = s.h.t, &m = s.h.m;
     float ru = 0.f, rv = 0.f;
     double b2u = 0.0, b2v = 0.0;
     // Jacobi: the rings hold P D^-1 r and ||b||^2 is the D^-1 norm
-    const float dzu = PRE && pc.oku ? F[CGM_DINV * ns + o] : 1.f, dzv = PRE && pc.okv ? F[(CGM_DINV + 1) * ns + o] : 1.f;
-    if (pc.oku) {
-        ru = bu - (pc.mwu ? t[0][ly][lx] : 0.f);
-        F[CGM_R * ns + o] = ru;
-        F[CGM_P * ns + o] = 0.f;
-        F[CGM_S * ns + o] = 0.f;
-        F[CGM_X * ns + o] = xu;
+    const float dzu = PRE && oku ? F[CGM_DINV * ns + at] : 1.f, dzv = PRE && okv ? F[(CGM_DINV + 1) * ns + at] : 1.f;
+    if (oku) {
+        ru = bu - ((o.mu & MB_WAVELET) ? t[0][ly][lx] : 0.f);
+        F[CGM_R * ns + at] = ru;
+        F[CGM_P * ns + at] = 0.f;
+        F[CGM_S * ns + at] = 0.f;
+        F[CGM_X * ns + at] = xu;
         b2u = PRE ? (double)bu * ((double)dzu * (double)bu) : (double)bu * (double)bu;
     }
-    if (pc.okv) {
-        rv = bv - (pc.mwv ? t[1][ly][lx] : 0.f);
-        F[(CGM_R + 1) * ns + o] = rv;
-        F[(CGM_P + 1) * ns + o] = 0.f;
-        F[(CGM_S + 1) * ns + o] = 0.f;
-        F[(CGM_X + 1) * ns + o] = xv;
+    if (okv) {
+        rv = bv - ((o.mv & MB_WAVELET) ? t[1][ly][lx] : 0.f);
+        F[(CGM_R + 1) * ns + at] = rv;
+        F[(CGM_P + 1) * ns + at] = 0.f;
+        F[(CGM_S + 1) * ns + at] = 0.f;
+        F[(CGM_X + 1) * ns + at] = xv;
         b2v = PRE ? (double)bv * ((double)dzv * (double)bv) : (double)bv * (double)bv;
     }
     // each thread rewrites only its own entry; the transform ended with a barrier
-    t[0][ly][lx] = pc.mwu ? (PRE ? dzu * ru : ru) : 0.f;
-    t[1][ly][lx] = pc.mwv ? (PRE ? dzv * rv : rv) : 0.f;
+    t[0][ly][lx] = (o.mu & MB_WAVELET) ? (PRE ? dzu * ru : ru) : 0.f;
+    t[1][ly][lx] = (o.mv & MB_WAVELET) ? (PRE ? dzv * rv : rv) : 0.f;
     __syncthreads();
     haar_pair<false, float>(a.levels, t, m);
-    if (pc.oku) ring_put(a.R, ring_at(0, g.nbx * g.nby, tile_id, 0, 0), lx, ly, pc.ui ? t[0][ly][lx] : 0.f);
-    if (pc.okv) ring_put(a.R, ring_at(0, g.nbx * g.nby, tile_id, 0, 1), lx, ly, pc.vi ? t[1][ly][lx] : 0.f);
+    if (oku) ring_put(a.R, ring_at(0, g.nbx * g.nby, tile_id, 0, 0), lx, ly, (o.mu & MB_INNER) ? t[0][ly][lx] : 0.f);
+    if (okv) ring_put(a.R, ring_at(0, g.nbx * g.nby, tile_id, 0, 1), lx, ly, (o.mv & MB_INNER) ? t[1][ly][lx] : 0.f);
     tree256x2(b2u, b2v, lds);
     if (threadIdx.x == 0) {
         if (has_u) a.Pb[bx + g.nbxu * by] = b2u;
