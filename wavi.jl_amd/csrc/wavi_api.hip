@@ -1223,12 +1223,12 @@ static CGArgs<T> cg_args(wavi_ctx *ctx, const VSet<T> &w)
     a.xv = w.xc.v;
     a.ru = w.cr.u;
     a.rv = w.cr.v;
-    a.pu = w.cp.u;
-    a.pv = w.cp.v;
+    a.pu[0] = w.cp.u;
+    a.pv[0] = w.cp.v;
+    a.pu[1] = w.ct.u;
+    a.pv[1] = w.ct.v;
     a.qu = w.cq.u;
     a.qv = w.cq.v;
-    a.tu = w.ct.u;
-    a.tv = w.ct.v;
     a.Pr = ctx->Pr0;
     a.Pd = ctx->Pd;
     a.Pb = ctx->Pb;
@@ -1253,7 +1253,7 @@ static bool use_cg_graph()
     return on;
 }
 
-// Iterations (launches, or triplets of launches in FP64) of coarse-CG chunk
+// Iterations (launches, or pairs of launches in FP64) of coarse-CG chunk
 // k.  The host reads the stop report of chunk k - 1 once chunk k is queued,
 // so one chunk keeps the GPU busy while the host waits, and every launch
 // queued past the stop runs as a no-op (the kernels read the stop from the
@@ -1304,6 +1304,30 @@ static void launch_tile_haar(wavi_ctx *ctx, int dir, const T *inu, const T *inv,
                        dir, inu, inv, min_u, min_v, outu, outv, mout_u, mout_v, accu, accv);
 }
 
+// The kernels of the FP64 coarse CG at the context's Haar level,
+// Jacobi-preconditioned inside a linear solve (ctx->cg_pre).
+template <typename T, bool PRE>
+static void launch_cg_step_p(wavi_ctx *ctx, dim3 tb, const CGArgs<T> &a, int par)
+{
+    switch (ctx->S.levels) {
+    case 0: hipLaunchKernelGGL((k_cg_step<T, PRE, 0>), tb, dim3(256), 0, ctx->stream, a, par); break;
+    case 1: hipLaunchKernelGGL((k_cg_step<T, PRE, 1>), tb, dim3(256), 0, ctx->stream, a, par); break;
+    case 2: hipLaunchKernelGGL((k_cg_step<T, PRE, 2>), tb, dim3(256), 0, ctx->stream, a, par); break;
+    default: hipLaunchKernelGGL((k_cg_step<T, PRE, 3>), tb, dim3(256), 0, ctx->stream, a, par); break;
+    }
+}
+
+template <typename T, bool PRE>
+static void launch_cg_solve1_p(wavi_ctx *ctx, const CGArgs<T> &a)
+{
+    switch (ctx->S.levels) {
+    case 0: hipLaunchKernelGGL((k_cg_solve1<T, PRE, 0>), dim3(1), dim3(256), 0, ctx->stream, a); break;
+    case 1: hipLaunchKernelGGL((k_cg_solve1<T, PRE, 1>), dim3(1), dim3(256), 0, ctx->stream, a); break;
+    case 2: hipLaunchKernelGGL((k_cg_solve1<T, PRE, 2>), dim3(1), dim3(256), 0, ctx->stream, a); break;
+    default: hipLaunchKernelGGL((k_cg_solve1<T, PRE, 3>), dim3(1), dim3(256), 0, ctx->stream, a); break;
+    }
+}
+
 // coarse CG on b_c held in w.cr; solution in the warm start w.xc
 template <typename T>
 static int do_coarse_cg(wavi_ctx *ctx, const VSet<T> &w, int *iters)
@@ -1312,13 +1336,13 @@ static int do_coarse_cg(wavi_ctx *ctx, const VSet<T> &w, int *iters)
     dim3 tg(g.nbx, g.nby), tb(ctx->nblk);
     CGArgs<T> a = cg_args(ctx, w);
     // t = P x0
-    launch_tile_haar<T>(ctx, 1, a.xu, a.xv, ctx->mwu, ctx->mwv, a.tu, a.tv, ctx->ui, ctx->vi);
+    launch_tile_haar<T>(ctx, 1, a.xu, a.xv, ctx->mwu, ctx->mwv, a.pu[1], a.pv[1], ctx->ui, ctx->vi);
     ctx->h_flag->done = 0;
     ctx->h_flag->iters = 0;
     const bool pre = ctx->cg_pre;
-    // k_cg_apply / k_cg_update return on the stop flag at once after a short
-    // previous CG (one that fitted its first chunk): such CGs stop within a
-    // chunk, so the launches queued past the stop are many.  Long CGs have
+    // k_cg_update returns on the stop flag at once after a short previous CG
+    // (one that fitted its first chunk): such CGs stop within a chunk, so the
+    // launches queued past the stop are many.  Long CGs have
     // about one, and their launches do without the flag's round trip.
     const bool early = ctx->cg_prev < CG_CHUNK;
     if (pre)
@@ -1329,9 +1353,9 @@ static int do_coarse_cg(wavi_ctx *ctx, const VSet<T> &w, int *iters)
     volatile CGMHostFlag *hf = ctx->h_flag;
     if (cg_one_workgroup(ctx)) {
         if (pre)
-            hipLaunchKernelGGL((k_cg_solve1<T, true>), dim3(1), dim3(256), 0, ctx->stream, a);
+            launch_cg_solve1_p<T, true>(ctx, a);
         else
-            hipLaunchKernelGGL((k_cg_solve1<T, false>), dim3(1), dim3(256), 0, ctx->stream, a);
+            launch_cg_solve1_p<T, false>(ctx, a);
         HIPCHK(hipGetLastError());
         HIPCHK(hipStreamSynchronize(ctx->stream));
         if (!hf->done) {
@@ -1341,8 +1365,8 @@ static int do_coarse_cg(wavi_ctx *ctx, const VSet<T> &w, int *iters)
         *iters = hf->iters;
         return WAVI_OK;
     }
-    // Triplet q performs iteration q unless the CG has stopped; triplet
-    // maxiter always stops, so no more are needed.  Triplets are queued in
+    // Launch pair q performs iteration q unless the CG has stopped; pair
+    // maxiter always stops, so no more are needed.  Pairs are queued in
     // chunks (cg_chunk_len); the host reads the stop report between chunks
     // and queues no more after a stop.
     const int nq = ctx->S.maxiter_coarse + 1;
@@ -1356,18 +1380,11 @@ static int do_coarse_cg(wavi_ctx *ctx, const VSet<T> &w, int *iters)
         for (int s = 0; s < n; ++s, ++q) {
             const int par = q & 1;
             {
-                ProfScope ps(ctx, WAVI_KT_CG_DIR, sampled);
-                if (pre)
-                    hipLaunchKernelGGL((k_cg_dir<T, true>), tb, dim3(256), 0, ctx->stream, a, par);
-                else
-                    hipLaunchKernelGGL((k_cg_dir<T, false>), tb, dim3(256), 0, ctx->stream, a, par);
-            }
-            {
                 ProfScope ps(ctx, WAVI_KT_CG_APPLY, sampled);
-                if (early)
-                    hipLaunchKernelGGL((k_cg_apply<T, true>), tb, dim3(256), 0, ctx->stream, a);
+                if (pre)
+                    launch_cg_step_p<T, true>(ctx, tb, a, par);
                 else
-                    hipLaunchKernelGGL((k_cg_apply<T, false>), tb, dim3(256), 0, ctx->stream, a);
+                    launch_cg_step_p<T, false>(ctx, tb, a, par);
             }
             {
                 ProfScope ps(ctx, WAVI_KT_CG_UPDATE, sampled);
@@ -1396,7 +1413,7 @@ static int do_coarse_cg(wavi_ctx *ctx, const VSet<T> &w, int *iters)
         HIPCHK(hipStreamSynchronize(ctx->stream));
         prof_collect(ctx);
     }
-    // triplet q iterates when q < iters
+    // pair q iterates when q < iters
     burst_collect(ctx, WAVI_KT_CG_ITER_FP64, hf->done ? hf->iters - 1 : -1);
     if (!hf->done) {
         ctx->err = "coarse CG did not terminate";

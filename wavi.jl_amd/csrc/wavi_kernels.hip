@@ -1364,9 +1364,22 @@ struct MaskPacked {
     }
 };
 
+// The coarse values around a tile from which k_cg_step forms P u on the
+// halo (HALO_N of haar_halo_offset per side, 5 at three levels).
+template <typename T>
+struct HaloLds {
+    T x[2][10][17];   // component; columns left (0..4) and right (5..9), rows by y
+    T y[2][10][16];   // rows below and above, by x
+    T c[2][5][5];     // the corner block, [y][x]
+    T lx[2][10][17];  // y sums of x
+    T ly[2][2][16];   // y sums of y: rows -1 and 16, by x
+    T lc[2][5];       // y sums of c
+};
+
 // Window point (x, y) is (i0 - 1 + x, j0 - 1 + y); cell (x, y) has the same
-// origin.  The transforms' tiles share the window's room: the window is read
-// last before the barrier that the outputs follow.
+// origin.  The window's room also holds the tiles of R (h; the window is
+// read last before the barrier that the outputs follow) and, before it, the
+// coarse halo (n); the cells' room holds the tiles of P (p) before them.
 template <typename T>
 struct OpLds {
     union {
@@ -1376,8 +1389,16 @@ struct OpLds {
         struct {
             TilePair<T> t, m;
         } h;
+        HaloLds<T> n;
     };
-    T rxx[17][18], ryy[17][18], ext[17][18], rxy[17][18];
+    union {
+        struct {
+            T rxx[17][18], ryy[17][18], ext[17][18], rxy[17][18];
+        };
+        struct {
+            TilePair<T> t, m;
+        } p;
+    };
 };
 
 // What a thread holds of its tile.
@@ -1420,68 +1441,127 @@ __device__ __forceinline__ void op_cell(const OpCoef<T> &c, OpLds<T> &s, int x, 
     s.rxy[y][x] = hetac * (dudy + dvdx);
 }
 
-// Load the tile of (xu, xv) and its coefficients and compute the cells'
-// intermediates (ends with a barrier, after which the window is free).
+// Halo points a thread stages: u at (ux, uy) and v at (vx, vy) of the window.
+// op_halo_sides: wavefront 3 the four sides, wavefront 2 the corners.
+struct HaloPos {
+    int ux, uy, vx, vy;
+    bool hu, hv;  // holds a u / a v halo point
+};
+
+// Side point l (0..63: left and right columns by y, bottom and top rows by x)
+__device__ __forceinline__ void halo_side(int l, int &x, int &y)
+{
+    const int q = 1 + (l & 15), far = (l & 16) ? 17 : 0;
+    x = l < 32 ? far : q;
+    y = l < 32 ? q : far;
+}
+
+__device__ __forceinline__ HaloPos op_halo_sides(int w, int l)
+{
+    HaloPos h{17, 0, 0, 17, w == 3 || (w == 2 && l == 0), w == 3 || (w == 2 && l == 0)};
+    if (w == 3) {
+        halo_side(l, h.ux, h.uy);
+        h.vx = h.ux;
+        h.vy = h.uy;
+    }
+    return h;
+}
+
+// Coefficients of a tile besides its points' values: the thread's own point
+// and cell, its halo points' thicknesses and masks, and the cell before the
+// tile that it computes (wavefront 0, lanes 0..32: (0, 0..16), (1..16, 0)).
+template <typename T>
+struct OpCoefRegs {
+    T hhu, hhv;
+    unsigned hmu, hmv;
+    T eh, ed, ec;
+    int ex, ey;
+};
+
 template <typename T, class M>
-__device__ __forceinline__ void op_tile(const GridDims &g, const OpCoef<T> &c, const M &mask, const T *xu, const T *xv,
-                                        int i0, int j0, OpLds<T> &s, OpOwn<T> &o)
+__device__ __forceinline__ void op_coef_load(const GridDims &g, const OpCoef<T> &c, const M &mask, int i0, int j0,
+                                             const HaloPos &h, bool halo_wave, OpOwn<T> &o, OpCoefRegs<T> &r)
 {
     const int lx = threadIdx.x & 15, ly = threadIdx.x >> 4, l = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int i = i0 + lx, j = j0 + ly;
-    o.oku = i < g.nxu && j < g.nyu;
-    o.okv = i < g.nxv && j < g.nyv;
-    o.ku = i + g.nxu * j;
-    o.kv = i + g.nxv * j;
-    o.u = ld_or(o.oku, xu, o.ku, T(0));
-    o.v = ld_or(o.okv, xv, o.kv, T(0));
     o.hu = ld_or(o.oku, c.hu, o.ku, T(0));
     o.hv = ld_or(o.okv, c.hv, o.kv, T(0));
-    o.mu = mask.u(o.oku, o.ku);
-    o.mv = mask.v(o.okv, o.kv);
-    // halo points: U and V at (ux, uy), (vx, vy) of the window
-    int ux = 17, uy = 0, vx = 0, vy = 17;
-    T hu = T(0), hv = T(0), hhu = T(0), hhv = T(0);
-    unsigned hmu = 0, hmv = 0;
-    if (w >= 2) {
-        if (w == 3) {
-            const int q = 1 + (l & 15), far = (l & 16) ? 17 : 0;
-            ux = vx = l < 32 ? far : q;
-            uy = vy = l < 32 ? q : far;
-        }
-        const int iu = i0 - 1 + ux, ju = j0 - 1 + uy, iv = i0 - 1 + vx, jv = j0 - 1 + vy;
-        const bool in = w == 3 || l == 0;
-        const bool okhu = in && iu >= 0 && iu < g.nxu && ju >= 0 && ju < g.nyu;
-        const bool okhv = in && iv >= 0 && iv < g.nxv && jv >= 0 && jv < g.nyv;
-        const int khu = iu + g.nxu * ju, khv = iv + g.nxv * jv;
-        hu = ld_or(okhu, xu, khu, T(0));
-        hv = ld_or(okhv, xv, khv, T(0));
-        hhu = ld_or(okhu, c.hu, khu, T(0));
-        hhv = ld_or(okhv, c.hv, khv, T(0));
-        hmu = mask.u(okhu, khu);
-        hmv = mask.v(okhv, khv);
+    r.hhu = r.hhv = T(0);
+    r.hmu = r.hmv = 0;
+    if (halo_wave) {
+        const int iu = i0 - 1 + h.ux, ju = j0 - 1 + h.uy, iv = i0 - 1 + h.vx, jv = j0 - 1 + h.vy;
+        const bool oku = h.hu && iu >= 0 && iu < g.nxu && ju >= 0 && ju < g.nyu;
+        const bool okv = h.hv && iv >= 0 && iv < g.nxv && jv >= 0 && jv < g.nyv;
+        r.hhu = ld_or(oku, c.hu, iu + g.nxu * ju, T(0));
+        r.hhv = ld_or(okv, c.hv, iv + g.nxv * jv, T(0));
+        r.hmu = mask.u(oku, iu + g.nxu * ju);
+        r.hmv = mask.v(okv, iv + g.nxv * jv);
     }
-    op_cell_load(g, c, i, j, o.heta, o.dimp, o.hetac);
-    // the cells before the tile: (0, 0..16), (1..16, 0)
-    const int ex = l < 17 ? 0 : l - 16, ey = l < 17 ? l : 0;
-    T eh = T(0), ed = T(0), ec = T(0);
-    if (w == 0) op_cell_load(g, c, l < 33 ? i0 - 1 + ex : -1, j0 - 1 + ey, eh, ed, ec);
+    op_cell_load(g, c, i0 + lx, j0 + ly, o.heta, o.dimp, o.hetac);
+    r.ex = l < 17 ? 0 : l - 16;
+    r.ey = l < 17 ? l : 0;
+    r.eh = r.ed = r.ec = T(0);
+    if (w == 0) op_cell_load(g, c, l < 33 ? i0 - 1 + r.ex : -1, j0 - 1 + r.ey, r.eh, r.ed, r.ec);
     o.bu = ld_or(o.oku, c.bu, o.ku, T(0));
     o.bv = ld_or(o.okv, c.bv, o.kv, T(0));
+}
+
+// Stage the window (the thread's own point and its halo points hu, hv) and
+// compute the cells' intermediates.  Ends with a barrier, after which the
+// window is free.
+template <typename T>
+__device__ __forceinline__ void op_cells(const OpCoef<T> &c, const HaloPos &h, T hu, T hv, const OpOwn<T> &o,
+                                         const OpCoefRegs<T> &r, OpLds<T> &s)
+{
+    const int lx = threadIdx.x & 15, ly = threadIdx.x >> 4;
     s.w.U[ly + 1][lx + 1] = o.u;
     s.w.V[ly + 1][lx + 1] = o.v;
     s.w.QX[ly + 1][lx + 1] = (o.mu & MB_POINT) ? o.hu * o.u : T(0);
     s.w.QY[ly + 1][lx + 1] = (o.mv & MB_POINT) ? o.hv * o.v : T(0);
-    if (w == 3 || (w == 2 && l == 0)) {
-        s.w.U[uy][ux] = hu;
-        s.w.V[vy][vx] = hv;
-        s.w.QX[uy][ux] = (hmu & MB_POINT) ? hhu * hu : T(0);
-        s.w.QY[vy][vx] = (hmv & MB_POINT) ? hhv * hv : T(0);
+    if (h.hu) {
+        s.w.U[h.uy][h.ux] = hu;
+        s.w.QX[h.uy][h.ux] = (r.hmu & MB_POINT) ? r.hhu * hu : T(0);
+    }
+    if (h.hv) {
+        s.w.V[h.vy][h.vx] = hv;
+        s.w.QY[h.vy][h.vx] = (r.hmv & MB_POINT) ? r.hhv * hv : T(0);
     }
     __syncthreads();
     op_cell(c, s, lx + 1, ly + 1, o.heta, o.dimp, o.hetac);
-    if (w == 0 && l < 33) op_cell(c, s, ex, ey, eh, ed, ec);
+    if (threadIdx.x < 33) op_cell(c, s, r.ex, r.ey, r.eh, r.ed, r.ec);
     __syncthreads();
+}
+
+__device__ __forceinline__ void op_own_index(const GridDims &g, int i, int j, bool &oku, bool &okv, int &ku, int &kv)
+{
+    oku = i < g.nxu && j < g.nyu;
+    okv = i < g.nxv && j < g.nyv;
+    ku = i + g.nxu * j;
+    kv = i + g.nxv * j;
+}
+
+// Load the tile of (xu, xv) and its coefficients and compute the cells'
+// intermediates.
+template <typename T, class M>
+__device__ __forceinline__ void op_tile(const GridDims &g, const OpCoef<T> &c, const M &mask, const T *xu, const T *xv,
+                                        int i0, int j0, OpLds<T> &s, OpOwn<T> &o)
+{
+    const int l = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    op_own_index(g, i0 + (threadIdx.x & 15), j0 + (threadIdx.x >> 4), o.oku, o.okv, o.ku, o.kv);
+    o.u = ld_or(o.oku, xu, o.ku, T(0));
+    o.v = ld_or(o.okv, xv, o.kv, T(0));
+    o.mu = mask.u(o.oku, o.ku);
+    o.mv = mask.v(o.okv, o.kv);
+    const HaloPos h = op_halo_sides(w, l);
+    T hu = T(0), hv = T(0);
+    if (w >= 2) {
+        const int iu = i0 - 1 + h.ux, ju = j0 - 1 + h.uy, iv = i0 - 1 + h.vx, jv = j0 - 1 + h.vy;
+        hu = ld_or(h.hu && iu >= 0 && iu < g.nxu && ju >= 0 && ju < g.nyu, xu, iu + g.nxu * ju, T(0));
+        hv = ld_or(h.hv && iv >= 0 && iv < g.nxv && jv >= 0 && jv < g.nyv, xv, iv + g.nxv * jv, T(0));
+    }
+    OpCoefRegs<T> r;
+    op_coef_load(g, c, mask, i0, j0, h, w >= 2, o, r);
+    op_cells(c, h, hu, hv, o, r, s);
 }
 
 // A x at the thread's u point and v point (inner or not)
@@ -2075,8 +2155,8 @@ __global__ void k_scale_uv(double *u, int nu, double *v, int nv, double a)
 
 // ===========================================================================
 // Coarse CG: IterativeSolvers.cg! on A_c = R A P (update_preconditioners.jl:73)
-// with x0 the cached warm start: three kernels per iteration and no host
-// round trip.  Kernels that end in a reduction write one partial per 16x16
+// with x0 the cached warm start: two kernels per iteration (one per global
+// sum) and no host round trip.  Kernels that end in a reduction write one partial per 16x16
 // block; the next kernel folds them with the canonical tree in every
 // workgroup (all get the same bits), so no workgroup waits for another inside
 // a kernel.  Scalars a kernel publishes are double-buffered by iteration
@@ -2096,12 +2176,13 @@ struct CGMHostFlag {
 };
 
 struct CGScalars {
-    double res[2];    // residual norm by iteration parity (written by k_cg_dir)
+    double res[2];    // residual norm by iteration parity (written by k_cg_step)
     double tol;       // max(reltol ||r0||, abstol)
+    double alpha;     // step length whose x += alpha u is still to be applied (written by k_cg_update)
     int it[2];        // iterations done, by parity
-    int done;         // sticky stop flag, written only by k_cg_dir
+    int done;         // sticky stop flag, written only by k_cg_step
     int iters;        // iterations at termination
-    double rz[2];     // Jacobi-preconditioned CG: (r, D^-1 r) by parity (written by k_cg_dir)
+    double rz[2];     // Jacobi-preconditioned CG: (r, D^-1 r) by parity (written by k_cg_step)
 };
 
 template <typename T>
@@ -2113,9 +2194,8 @@ struct CGArgs {
     uint8_t *mcu, *mcv;  // packed mask bits (MB_*) of the u and v points, written by k_cg_setup
     T *xu, *xv;       // solution (warm start in, result out)
     T *ru, *rv;       // residual (right-hand side on entry to setup)
-    T *pu, *pv;       // search direction u
+    T *pu[2], *pv[2]; // search direction u by iteration parity (set 1 holds P x0 during the set-up)
     T *qu, *qv;       // c = A_c u
-    T *tu, *tv;       // P u on the fine grid
     double *Pr, *Pd, *Pb;
     double *Pz;                       // Jacobi: partials of (r, D^-1 r)
     const double *dinvu, *dinvv;      // Jacobi: 1 / |diag(A_c)|, 0 off the wavelet masks
@@ -2160,6 +2240,7 @@ __global__ void __launch_bounds__(256) k_cg_setup(CGArgs<T> a)
         a.st->iters = 0;
         a.st->it[0] = 0;
         a.st->it[1] = 0;
+        a.st->alpha = 0.0;
         // also reset on the stream: launches queued past the previous
         // CG's stop, which rewrite the report, may still have been running
         // when the host reset it
@@ -2175,7 +2256,7 @@ __global__ void __launch_bounds__(256) k_cg_setup(CGArgs<T> a)
     const T bu = ld_or(i < g.nxu && j < g.nyu, a.ru, i + g.nxu * j, T(0));
     const T bv = ld_or(i < g.nxv && j < g.nyv, a.rv, i + g.nxv * j, T(0));
     OpOwn<T> o;
-    op_restrict_tile(g, a.c, MaskSep<true>{a.ui, a.c.um, a.vi, a.c.vm, a.mwu, a.mwv}, a.levels, a.tu, a.tv, i0, j0, s,
+    op_restrict_tile(g, a.c, MaskSep<true>{a.ui, a.c.um, a.vi, a.c.vm, a.mwu, a.mwv}, a.levels, a.pu[1], a.pv[1], i0, j0, s,
                      o);
     if (o.oku) a.mcu[o.ku] = (uint8_t)o.mu;
     if (o.okv) a.mcv[o.kv] = (uint8_t)o.mv;
@@ -2183,7 +2264,7 @@ __global__ void __launch_bounds__(256) k_cg_setup(CGArgs<T> a)
     if (o.oku) {
         const T r = bu - ((o.mu & MB_WAVELET) ? s.h.t[0][ly][lx] : T(0));
         a.ru[o.ku] = r;
-        a.pu[o.ku] = T(0);
+        a.pu[0][o.ku] = T(0);
         r2u = (double)r * (double)r;
         b2u = (double)bu * (double)bu;
         if constexpr (PRE) z2u = (double)r * (a.dinvu[o.ku] * (double)r);
@@ -2191,7 +2272,7 @@ __global__ void __launch_bounds__(256) k_cg_setup(CGArgs<T> a)
     if (o.okv) {
         const T r = bv - ((o.mv & MB_WAVELET) ? s.h.t[1][ly][lx] : T(0));
         a.rv[o.kv] = r;
-        a.pv[o.kv] = T(0);
+        a.pv[0][o.kv] = T(0);
         r2v = (double)r * (double)r;
         b2v = (double)bv * (double)bv;
         if constexpr (PRE) z2v = (double)r * (a.dinvv[o.kv] * (double)r);
@@ -2228,46 +2309,150 @@ __device__ __forceinline__ V cg_scalar(const V *p)
     return p[z];
 }
 
-// part 1 (iteration parity par): residual norm and stop test, then
-// u = r + beta u with beta = res^2 / prev^2 (PRE: u = D^-1 r + beta u with
-// beta = rz / prev rz), t = P u.  The stop decision is
-// recomputed from the partials each time, so it needs no flag: after a stop
-// the partials are frozen and it[1 - par] repeats the count.
-template <typename T, bool PRE>
-__device__ __forceinline__ bool cg_dir_tile(const CGArgs<T> &a, int par, const int L)
+// Offset of the k-th coarse row (or column) that the point next to a tile
+// takes from the neighbour, relative to the tile's first: below (k < 5) the
+// neighbour's last point 15, whose row of P has the terms 16 - B, .., 8, 12,
+// 14, 15 (all +1), above (k >= 5) its first point 0 with the terms 0, 1, 2, 4,
+// 8 (+1, then all -1).  N = LEV + 2 of them, in increasing order.
+template <int LEV>
+__device__ __forceinline__ int haar_halo_offset(int k)
 {
-    __shared__ TilePair<T> t, m;
+    return k < 5 ? -((2 << LEV) >> k) : 16 + ((1 << (k - 5)) >> 1);
+}
+
+// The row of P that haar_halo_offset's terms v[0..N) (stride st) make: the
+// last point of a block (neg = false) or its first.
+template <int LEV, typename T>
+__device__ __forceinline__ T haar_halo_sum(const T *v, int st, bool neg)
+{
+    T x[LEV + 2];
+#pragma unroll
+    for (int k = 0; k < LEV + 2; ++k) x[k] = v[k * st];
+    T a = x[0];
+#pragma unroll
+    for (int k = 1; k < LEV + 2; ++k) a = a + (neg ? -x[k] : x[k]);
+    return a;
+}
+
+// Row i of P on a 16-point line: x_0 of the block, then in increasing column
+// order the details e_h = (i's pair point at distance h) of the set bits of i
+// (h descending, +1) and of the clear bits (h ascending, -1).
+template <int LEV, typename T>
+__device__ __forceinline__ T haar_row_P(const T *src, int i)
+{
+    T d[LEV + 1];
+#pragma unroll
+    for (int k = 0; k <= LEV; ++k) d[k] = src[(i & ~((2 << k) - 1)) + (1 << k)];
+    T a = src[i & ~((2 << LEV) - 1)];
+#pragma unroll
+    for (int k = LEV; k >= 0; --k) a = (i >> k) & 1 ? a + d[k] : a;
+#pragma unroll
+    for (int k = 0; k <= LEV; ++k) a = (i >> k) & 1 ? a : a - d[k];
+    return a;
+}
+
+// part 1 (iteration parity par): residual norm and stop test; x += alpha u
+// of the previous iteration; u = r + beta u with beta = res^2 / prev^2 (PRE:
+// u = D^-1 r + beta u with beta = rz / prev rz); c = R A P u and the partials
+// of dot(u, c).  The stop decision is recomputed from the partials each time,
+// so it needs no flag: after a stop the partials are frozen and it[1 - par]
+// repeats the count; alpha is then zero, so x is not changed again.
+//
+// A needs P u on the tile and a one-point halo.  The tile's own part is the
+// block transform of its own u.  A halo point needs N = LEV + 2 coarse rows
+// and columns of the neighbour's u, which the tile forms itself from r and
+// the previous u (the neighbours' 4 x 16 x N values per component and one
+// N x N corner block; the previous and the new u are double-buffered by
+// parity, so no tile reads what another writes).  Every value adds its terms
+// in the order of the block transform, so it has the neighbour's bits.  With
+// the direction in a launch of its own, P u went through memory and the
+// iteration had a third kernel boundary (at least 2.5 us on this chip).
+template <typename T, bool PRE, int LEV>
+__device__ __forceinline__ bool cg_step_tile(const CGArgs<T> &a, int par, const int L)
+{
+    constexpr int N = LEV + 2;
+    __shared__ OpLds<T> s;
     __shared__ double lds[8];
     const GridDims &g = a.g;
     if (L >= g.nbx * g.nby) return false;
     int bx, by;
     band_tile(g, L, bx, by);
     const bool has_u = bx < g.nbxu && by < g.nbyu, has_v = bx < g.nbxv && by < g.nbyv;
-    const int lx = threadIdx.x & 15, ly = threadIdx.x >> 4;
+    const int lx = threadIdx.x & 15, ly = threadIdx.x >> 4, l = threadIdx.x & 63;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int i0 = bx * TILE, j0 = by * TILE;
-    const int i = i0 + lx, j = j0 + ly;
-    const bool oku = has_u && i < g.nxu && j < g.nyu, okv = has_v && i < g.nxv && j < g.nyv;
-    const int ku = i + g.nxu * j, kv = i + g.nxv * j;
-    // independent loads first
+    OpOwn<T> o;
+    op_own_index(g, i0 + lx, j0 + ly, o.oku, o.okv, o.ku, o.kv);
+    const T *pu_old = a.pu[par], *pv_old = a.pv[par];
+    const MaskPacked mask{a.mcu, a.mcv};
+    // loads in the order of first use: scalars and partials, the tile's
+    // vectors, the coarse halo, the coefficients
     const int it = cg_scalar(&a.st->it[par]);
     const double told = cg_scalar(&a.st->tol), prev_res = cg_scalar(&a.st->res[1 - par]);
-    const T ru = ld_or(oku, a.ru, ku, T(0)), pu = ld_or(oku, a.pu, ku, T(0));
-    const T rv = ld_or(okv, a.rv, kv, T(0)), pv = ld_or(okv, a.pv, kv, T(0));
-    const unsigned mu = ld_or(oku, (const uint8_t *)a.mcu, ku, (uint8_t)0);
-    const unsigned mv = ld_or(okv, (const uint8_t *)a.mcv, kv, (uint8_t)0);
-    double dzu = 0.0, dzv = 0.0, rz = 0.0, prev_rz = 0.0;
+    const T alpha = (T)cg_scalar(&a.st->alpha);
+    double rz = 0.0, prev_rz = 0.0, fold_r, fold_z = 0.0;
+    fold_r = lane_fold(a.Pr, g.npart);
     if constexpr (PRE) {
-        dzu = ld_or(oku, a.dinvu, ku, 0.0);
-        dzv = ld_or(okv, a.dinvv, kv, 0.0);
         prev_rz = cg_scalar(&a.st->rz[1 - par]);
+        fold_z = lane_fold(a.Pz, g.npart);
     }
+    const T ru = ld_or(o.oku, a.ru, o.ku, T(0)), pu = ld_or(o.oku, pu_old, o.ku, T(0));
+    const T rv = ld_or(o.okv, a.rv, o.kv, T(0)), pv = ld_or(o.okv, pv_old, o.kv, T(0));
+    const T xu = ld_or(o.oku, a.xu, o.ku, T(0)), xv = ld_or(o.okv, a.xv, o.kv, T(0));
+    o.mu = mask.u(o.oku, o.ku);
+    o.mv = mask.v(o.okv, o.kv);
+    double dzu = 0.0, dzv = 0.0;
+    if constexpr (PRE) {
+        dzu = ld_or(o.oku, a.dinvu, o.ku, 0.0);
+        dzv = ld_or(o.okv, a.dinvv, o.kv, 0.0);
+    }
+    // the coarse halo: wavefronts 0, 1 the columns left and right of the tile
+    // (u, v) and the corner block, 2, 3 the rows below and above; entry
+    // c = l / 16 + 4 k of 10, point l % 16 along it
+    const bool hv_wave = (w & 1) != 0, rows = w >= 2;
+    const T *hr = hv_wave ? a.rv : a.ru, *hp = hv_wave ? pv_old : pu_old;
+    const uint8_t *hm = hv_wave ? a.mcv : a.mcu;
+    const double *hd = hv_wave ? a.dinvv : a.dinvu;
+    const int hnx = hv_wave ? g.nxv : g.nxu, hny = hv_wave ? g.nyv : g.nyu;
+    T nr[3], np[3];
+    double nd[3];
+    unsigned nm[3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        const int c = (l >> 4) + 4 * k, q = l & 15;
+        int di = rows ? q : haar_halo_offset<LEV>(c), dj = rows ? haar_halo_offset<LEV>(c) : q;
+        bool in = c < 5 ? c < N : (c < 10 && c - 5 < N);
+        if (k == 2 && l >= 32) {  // the corner block: u below right, v above left
+            const int e = l - 32, cx = e % 5, cy = e / 5;
+            di = haar_halo_offset<LEV>(hv_wave ? cx : cx + 5);
+            dj = haar_halo_offset<LEV>(hv_wave ? cy + 5 : cy);
+            in = !rows && e < 25 && cx < N && cy < N;
+        }
+        const int i = i0 + di, j = j0 + dj;
+        const bool ok = in && i >= 0 && i < hnx && j >= 0 && j < hny;
+        nr[k] = ld_or(ok, hr, i + hnx * j, T(0));
+        np[k] = ld_or(ok, hp, i + hnx * j, T(0));
+        nm[k] = ld_or(ok, hm, i + hnx * j, (uint8_t)0);
+        nd[k] = PRE ? ld_or(ok, hd, i + hnx * j, 0.0) : 0.0;
+    }
+    // halo points: wavefront 3 the sides' u, wavefront 2 their v, wavefront 1
+    // the corners (u lane 0, v lane 1)
+    HaloPos h{17, 0, 0, 17, w == 3 || (w == 1 && l == 0), w == 2 || (w == 1 && l == 1)};
+    if (w >= 2) {
+        halo_side(l, h.ux, h.uy);
+        h.vx = h.ux;
+        h.vy = h.uy;
+    }
+    OpCoefRegs<T> cr;
+    op_coef_load(g, a.c, mask, i0, j0, h, w >= 1, o, cr);
     double res;
     if constexpr (PRE) {
-        double r2;
-        lanes_sum2(a.Pr, a.Pz, g.npart, lds, r2, rz);
+        double r2 = fold_r;
+        rz = fold_z;
+        tree256x2(r2, rz, lds);
         res = sqrt(r2);
     } else {
-        res = sqrt(lanes_sum(a.Pr, g.npart, lds));
+        res = sqrt(tree256(fold_r, lds));
     }
     double tol;
     if (it == 0) {
@@ -2292,6 +2477,10 @@ __device__ __forceinline__ bool cg_dir_tile(const CGArgs<T> &a, int par, const i
             }
         }
     }
+    if (alpha != T(0)) {
+        if (o.oku) a.xu[o.ku] = xu + alpha * pu;
+        if (o.okv) a.xv[o.kv] = xv + alpha * pv;
+    }
     if (done) return true;
     T beta;
     if constexpr (PRE) {
@@ -2300,124 +2489,152 @@ __device__ __forceinline__ bool cg_dir_tile(const CGArgs<T> &a, int par, const i
         const double prev = it == 0 ? 1.0 : prev_res;
         beta = (T)((res * res) / (prev * prev));
     }
-    T unu = T(0), unv = T(0);
-    if (oku) {
+    auto direction = [&](T r, T p, double dz) -> T {
         if constexpr (PRE)
-            unu = (T)(dzu * (double)ru) + beta * pu;
+            return (T)(dz * (double)r) + beta * p;
         else
-            unu = ru + beta * pu;
-        a.pu[ku] = unu;
+            return r + beta * p;
+    };
+    const T unu = direction(ru, pu, dzu), unv = direction(rv, pv, dzv);
+    if (o.oku) a.pu[1 - par][o.ku] = unu;
+    if (o.okv) a.pv[1 - par][o.kv] = unv;
+    s.p.t[0][ly][lx] = (o.mu & MB_WAVELET) ? unu : T(0);
+    s.p.t[1][ly][lx] = (o.mv & MB_WAVELET) ? unv : T(0);
+    {
+        const int comp = hv_wave ? 1 : 0;
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            const int c = (l >> 4) + 4 * k, q = l & 15;
+            const T x = (nm[k] & MB_WAVELET) ? direction(nr[k], np[k], nd[k]) : T(0);
+            if (k < 2 || l < 32) {
+                if (rows)
+                    s.n.y[comp][c][q] = x;
+                else
+                    s.n.x[comp][c][q] = x;
+            } else if (!rows && l < 57) {
+                (&s.n.c[comp][0][0])[l - 32] = x;
+            }
+        }
     }
-    if (okv) {
-        if constexpr (PRE)
-            unv = (T)(dzv * (double)rv) + beta * pv;
-        else
-            unv = rv + beta * pv;
-        a.pv[kv] = unv;
-    }
-    t[0][ly][lx] = (mu & MB_WAVELET) ? unu : T(0);
-    t[1][ly][lx] = (mv & MB_WAVELET) ? unv : T(0);
     __syncthreads();
-    haar_pair<false, T>(a.levels, t, m);
-    if (oku) a.tu[ku] = (mu & MB_INNER) ? t[0][ly][lx] : T(0);
-    if (okv) a.tv[kv] = (mv & MB_INNER) ? t[1][ly][lx] : T(0);
-    return false;
-}
-
-// part 2: c = R A t and partials of dot(u, c).  EARLY: return at once after
-// a stop (written only by earlier kernels).  Otherwise the launch runs and
-// stores in full: after a stop only k_cg_update reads c and the partials, and
-// it changes nothing then; a return on the flag would put its round trip
-// before every load of the launch.
-template <typename T, bool EARLY = true>
-__device__ __forceinline__ void cg_apply_tile(const CGArgs<T> &a, const int L)
-{
-    __shared__ OpLds<T> s;
-    __shared__ double lds[8];
-    const GridDims &g = a.g;
-    if (L >= g.nbx * g.nby) return;
-    if (EARLY && a.st->done) return;
-    int bx, by;
-    band_tile(g, L, bx, by);
-    const bool has_u = bx < g.nbxu && by < g.nbyu, has_v = bx < g.nbxv && by < g.nbyv;
-    const int i0 = bx * TILE, j0 = by * TILE;
-    const int lx = threadIdx.x & 15, ly = threadIdx.x >> 4;
-    const int i = i0 + lx, j = j0 + ly;
-    const T pu = ld_or(i < g.nxu && j < g.nyu, a.pu, i + g.nxu * j, T(0));
-    const T pv = ld_or(i < g.nxv && j < g.nyv, a.pv, i + g.nxv * j, T(0));
-    OpOwn<T> o;
-    op_restrict_tile(g, a.c, MaskPacked{a.mcu, a.mcv}, a.levels, a.tu, a.tv, i0, j0, s, o);
+    // y pass: the tile's lines; the columns' lines (lanes 0..39, a half line
+    // each); rows -1 and 16 of the neighbours below and above; the corners
+    {
+        const int q = l & 15, comp = (l >> 4) & 1, half = l >> 5;
+        haar_line_P<LEV, T>(&s.p.t[comp][0][q], &s.p.m[comp][0][q], TILE + 1, half, w);
+        if (l < 40) {
+            const int line = l < 20 ? l : l - 20, lh = l < 20 ? 0 : 1;
+            haar_line_P<LEV, T>(&s.n.x[0][0][0] + 17 * line, &s.n.lx[0][0][0] + 17 * line, 1, lh, w);
+        }
+        if (l < 16) {
+            const int cp = w & 1, side = w >> 1;
+            s.n.ly[cp][side][l] = haar_halo_sum<LEV, T>(&s.n.y[cp][5 * side][l], 16, side != 0);
+        } else if (w < 2 && l < 21) {
+            s.n.lc[w][l - 16] = haar_halo_sum<LEV, T>(&s.n.c[w][0][l - 16], 5, w == 1);
+        }
+    }
+    __syncthreads();
+    // x pass: the tile's lines and the halo points
+    T hu = T(0), hv = T(0);
+    {
+        const int q = l & 15, comp = (l >> 4) & 1, half = l >> 5;
+        haar_line_P<LEV, T>(&s.p.m[comp][q][0], &s.p.t[comp][q][0], 1, half, w);
+        if (w >= 2) {
+            const int cp = w == 3 ? 0 : 1, side = (l >> 4) & 1;
+            T x;
+            if (l < 32)
+                x = haar_halo_sum<LEV, T>(&s.n.lx[cp][5 * side][q], 17, side != 0);
+            else
+                x = haar_row_P<LEV, T>(&s.n.ly[cp][side][0], q);
+            hu = (cr.hmu & MB_INNER) ? x : T(0);
+            hv = (cr.hmv & MB_INNER) ? x : T(0);
+        } else if (w == 1 && l < 2) {
+            const T x = haar_halo_sum<LEV, T>(&s.n.lc[l][0], 1, l == 0);
+            hu = (cr.hmu & MB_INNER) ? x : T(0);
+            hv = (cr.hmv & MB_INNER) ? x : T(0);
+        }
+    }
+    __syncthreads();
+    o.u = (o.mu & MB_INNER) ? s.p.t[0][ly][lx] : T(0);
+    o.v = (o.mv & MB_INNER) ? s.p.t[1][ly][lx] : T(0);
+    op_cells(a.c, h, hu, hv, o, cr, s);
+    s.h.t[0][ly][lx] = (o.mu & MB_INNER) ? op_out_u(a.c, s, o) : T(0);
+    s.h.t[1][ly][lx] = (o.mv & MB_INNER) ? op_out_v(a.c, s, o) : T(0);
+    __syncthreads();
+    haar_pair_lev<true, LEV, T>(s.h.t, s.h.m);
     double du = 0.0, dv = 0.0;
     if (o.oku) {
         const T cv = (o.mu & MB_WAVELET) ? s.h.t[0][ly][lx] : T(0);
         a.qu[o.ku] = cv;
-        du = (double)(pu * cv);
+        du = (double)(unu * cv);
     }
     if (o.okv) {
         const T cv = (o.mv & MB_WAVELET) ? s.h.t[1][ly][lx] : T(0);
         a.qv[o.kv] = cv;
-        dv = (double)(pv * cv);
+        dv = (double)(unv * cv);
     }
     tree256x2(du, dv, lds);
     if (threadIdx.x == 0) {
         if (has_u) a.Pd[bx + g.nbxu * by] = du;
         if (has_v) a.Pd[g.nbxu * g.nbyu + bx + g.nbxv * by] = dv;
     }
+    return false;
 }
 
-// part 3: alpha = res^2 / dot(u, c) (PRE: rz / dot(u, c)), x += alpha u,
-// r -= alpha c, partials of ||r||^2 (PRE: and of (r, D^-1 r)) and the
-// iteration count.  EARLY: return at once after a stop.  Otherwise a launch
-// after a stop stores x, r, their partials and the count unchanged (selected
-// by the flag, which is then needed only at the stores), so that the flag's
-// round trip does not precede the loads.
+// part 2: alpha = res^2 / dot(u, c) (PRE: rz / dot(u, c)), left for the next
+// k_cg_step's x += alpha u; r -= alpha c, partials of ||r||^2 (PRE: and of
+// (r, D^-1 r)) and the iteration count.  After a stop alpha is set to zero.
+// EARLY: and nothing else is done.  Otherwise a launch after a stop stores r,
+// its partials and the count unchanged (selected by the flag, which is then
+// needed only at the stores), so that the flag's round trip does not precede
+// the loads.
 template <typename T, bool PRE, bool EARLY = true>
 __device__ __forceinline__ void cg_update_tile(const CGArgs<T> &a, int par, const int L)
 {
     __shared__ double lds[8];
     const GridDims &g = a.g;
     if (L >= g.nbx * g.nby) return;
-    if (EARLY && a.st->done) return;
+    if (EARLY && a.st->done) {
+        if (threadIdx.x == 0) a.st->alpha = 0.0;
+        return;
+    }
     const bool stopped = !EARLY && cg_scalar(&a.st->done) != 0;
     int bx, by;
     band_tile(g, L, bx, by);
     const bool has_u = bx < g.nbxu && by < g.nbyu, has_v = bx < g.nbxv && by < g.nbyv;
-    const int lx = threadIdx.x & 15, ly = threadIdx.x >> 4;
-    const int i = bx * TILE + lx, j = by * TILE + ly;
-    const bool oku = has_u && i < g.nxu && j < g.nyu, okv = has_v && i < g.nxv && j < g.nyv;
-    const int ku = i + g.nxu * j, kv = i + g.nxv * j;
+    bool oku, okv;
+    int ku, kv;
+    op_own_index(g, bx * TILE + (threadIdx.x & 15), by * TILE + (threadIdx.x >> 4), oku, okv, ku, kv);
     const int it = cg_scalar(&a.st->it[par]);
     const double res = cg_scalar(&a.st->res[par]);
-    const T xu = ld_or(oku, a.xu, ku, T(0)), pu = ld_or(oku, a.pu, ku, T(0)), ru = ld_or(oku, a.ru, ku, T(0)),
-            qu = ld_or(oku, a.qu, ku, T(0));
-    const T xv = ld_or(okv, a.xv, kv, T(0)), pv = ld_or(okv, a.pv, kv, T(0)), rv = ld_or(okv, a.rv, kv, T(0)),
-            qv = ld_or(okv, a.qv, kv, T(0));
+    const double fold = lane_fold(a.Pd, g.npart);
+    const T ru = ld_or(oku, a.ru, ku, T(0)), qu = ld_or(oku, a.qu, ku, T(0));
+    const T rv = ld_or(okv, a.rv, kv, T(0)), qv = ld_or(okv, a.qv, kv, T(0));
     double dzu = 0.0, dzv = 0.0, rzc = 0.0;
     if constexpr (PRE) {
         dzu = ld_or(oku, a.dinvu, ku, 0.0);
         dzv = ld_or(okv, a.dinvv, kv, 0.0);
         rzc = cg_scalar(&a.st->rz[par]);
     }
-    const double dot = lanes_sum(a.Pd, g.npart, lds);
+    const double dot = tree256(fold, lds);
     T alpha;
     if constexpr (PRE)
         alpha = (T)(rzc / dot);
     else
         alpha = (T)((res * res) / dot);
-    if (threadIdx.x == 0) a.st->it[1 - par] = stopped ? it : it + 1;
+    if (threadIdx.x == 0) {
+        a.st->it[1 - par] = stopped ? it : it + 1;
+        a.st->alpha = stopped ? 0.0 : (double)alpha;
+    }
     double r2u = 0.0, r2v = 0.0, z2u = 0.0, z2v = 0.0;
     if (oku) {
-        const T x = xu + alpha * pu, rn = ru - alpha * qu;
-        a.xu[ku] = stopped ? xu : x;
-        const T r = stopped ? ru : rn;
+        const T rn = ru - alpha * qu, r = stopped ? ru : rn;
         a.ru[ku] = r;
         r2u = (double)r * (double)r;
         if constexpr (PRE) z2u = (double)r * (dzu * (double)r);
     }
     if (okv) {
-        const T x = xv + alpha * pv, rn = rv - alpha * qv;
-        a.xv[kv] = stopped ? xv : x;
-        const T r = stopped ? rv : rn;
+        const T rn = rv - alpha * qv, r = stopped ? rv : rn;
         a.rv[kv] = r;
         r2v = (double)r * (double)r;
         if constexpr (PRE) z2v = (double)r * (dzv * (double)r);
@@ -2434,16 +2651,10 @@ __device__ __forceinline__ void cg_update_tile(const CGArgs<T> &a, int par, cons
     }
 }
 
-template <typename T, bool PRE>
-__global__ void __launch_bounds__(256) k_cg_dir(CGArgs<T> a, int par)
+template <typename T, bool PRE, int LEV>
+__global__ void __launch_bounds__(256) k_cg_step(CGArgs<T> a, int par)
 {
-    (void)cg_dir_tile<T, PRE>(a, par, xcd_tile(a.nblk));
-}
-
-template <typename T, bool EARLY>
-__global__ void __launch_bounds__(256) k_cg_apply(CGArgs<T> a)
-{
-    cg_apply_tile<T, EARLY>(a, xcd_tile(a.nblk));
+    (void)cg_step_tile<T, PRE, LEV>(a, par, xcd_tile(a.nblk));
 }
 
 template <typename T, bool PRE, bool EARLY>
@@ -2531,11 +2742,11 @@ __global__ void __launch_bounds__(256) k_coarse_diag(GridDims g, OpCoef<double> 
 // the workgroup runs each part of an iteration on every tile in turn, so
 // the barrier between two tiles stands in for the kernel boundary.  Tiles
 // read only what earlier parts wrote and write only their own points,
-// partials and parity slots, so the results are those of the three
+// partials and parity slots, so the results are those of the two
 // launches per iteration, bit for bit.  Ends at the stop, which every
 // thread of every tile decides alike from the same partials and scalars,
 // after maxiter + 1 iterations at most.
-template <typename T, bool PRE>
+template <typename T, bool PRE, int LEV>
 __global__ void __launch_bounds__(256) k_cg_solve1(CGArgs<T> a)
 {
     const int ntile = a.g.nbx * a.g.nby;
@@ -2543,14 +2754,10 @@ __global__ void __launch_bounds__(256) k_cg_solve1(CGArgs<T> a)
         const int par = q & 1;
         bool stop = false;
         for (int L = 0; L < ntile; ++L) {
-            stop = cg_dir_tile<T, PRE>(a, par, L);
+            stop = cg_step_tile<T, PRE, LEV>(a, par, L);
             __syncthreads();
         }
         if (stop) break;
-        for (int L = 0; L < ntile; ++L) {
-            cg_apply_tile<T>(a, L);
-            __syncthreads();
-        }
         for (int L = 0; L < ntile; ++L) {
             cg_update_tile<T, PRE>(a, par, L);
             __syncthreads();
