@@ -17,6 +17,7 @@
 #include <system_error>
 #include <thread>
 #include <tuple>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/wavi_hip.h"
@@ -61,7 +62,7 @@ struct DevVecT {
 template <typename T>
 struct VSet {
     T *heta_h = nullptr, *heta_c = nullptr, *dimp = nullptr;
-    DevVecT<T> h, beff, e, r, d, rho, t, cr, cp, cq, ct, xc;
+    DevVecT<T> h, beff, e, r, d, rho, t, cr, ct, xc;
 };
 
 struct wavi_ctx {
@@ -76,7 +77,6 @@ struct wavi_ctx {
     // masks (uint8, device)
     uint8_t *hm = nullptr, *hfix = nullptr, *um = nullptr, *vm = nullptr, *cm = nullptr;
     uint8_t *ui = nullptr, *vi = nullptr, *ufix = nullptr, *vfix = nullptr, *mwu = nullptr, *mwv = nullptr;
-    uint8_t *mcu = nullptr, *mcv = nullptr;  // FP64 coarse CG: packed masks (k_cg_setup)
     bool has_fixed = false;     // any u_isfixed / v_isfixed point
     std::vector<uint8_t> h_ui, h_vi;  // host copies of the inner masks
     double *adj_base = nullptr;       // adjoint workspace, kept between gradient calls
@@ -94,7 +94,11 @@ struct wavi_ctx {
     // Picard / V-cycle vectors (full u/v grids)
     DevVec x, b, r, e, d, rho, t, f3, fixedv;
     // coarse CG vectors
-    DevVec cr, cp, cq, ct;
+    DevVec cr, ct;
+    // FP64 coarse CG: its arena (CGLayout)
+    double2 *arena64 = nullptr;
+    uint8_t *marena64 = nullptr;
+    unsigned px64 = 0, ns64 = 0;
     VSet<float> v32;
     // mixed-precision coarse CG: s, w, the parity-buffered images P r, P s,
     // P w and partials of (r, r) and (w, r)
@@ -601,8 +605,6 @@ int wavi_ctx_create(const wavi_grid_desc *grid, const wavi_phys_params *phys, co
     CREATECHK(alloc8(&ctx->vfix, vfix));
     CREATECHK(alloc8(&ctx->mwu, ones_u));  // UWavelets mask = trues (UWavelets.jl:38)
     CREATECHK(alloc8(&ctx->mwv, ones_v));
-    CREATECHK(alloc8(&ctx->mcu, ones_u));
-    CREATECHK(alloc8(&ctx->mcv, ones_v));
 
     for (int id = 0; id < WAVI_NFIELDS; ++id) {
         if (id == WAVI_WU_MASK || id == WAVI_WV_MASK) continue;
@@ -635,7 +637,7 @@ int wavi_ctx_create(const wavi_grid_desc *grid, const wavi_phys_params *phys, co
     CREATECHK(zalloc(&ctx->heta_c, ctx->nc > 0 ? ctx->nc : 1));
     CREATECHK(zalloc(&ctx->dimp, ctx->nh));
     for (DevVec *dv : {&ctx->x, &ctx->b, &ctx->r, &ctx->e, &ctx->d, &ctx->rho, &ctx->t, &ctx->f3, &ctx->fixedv,
-                       &ctx->cr, &ctx->cp, &ctx->cq, &ctx->ct}) {
+                       &ctx->cr, &ctx->ct}) {
         CREATECHK(zalloc(&dv->u, ctx->nu));
         CREATECHK(zalloc(&dv->v, ctx->nv));
     }
@@ -660,6 +662,20 @@ int wavi_ctx_create(const wavi_grid_desc *grid, const wavi_phys_params *phys, co
     CREATECHK(hipEventCreateWithFlags(&ctx->ev_ls, hipEventDisableTiming));
     for (hipEvent_t &e : ctx->ev_tune) CREATECHK(hipEventCreate(&e));
     CREATECHK(hipEventCreateWithFlags(&ctx->ev_ls_done, hipEventDisableTiming));
+    if (precision_mode == WAVI_PRECISION_FP64) {
+        const size_t px = (size_t)TILE * (g.nbx + 2), ns = px * TILE * (g.nby + 2);
+        if (ns * sizeof(double2) > UINT32_MAX) {
+            ctx->err = "grid too large for the coarse solver's 32-bit offsets";
+            return fail(WAVI_EARG);
+        }
+        ctx->px64 = (unsigned)px;
+        ctx->ns64 = (unsigned)ns;
+        const size_t bytes = ns * (CG_NPAIR * sizeof(double2) + sizeof(double));
+        CREATECHK(hipMalloc(&ctx->arena64, bytes));
+        CREATECHK(hipMemset(ctx->arena64, 0, bytes));
+        CREATECHK(hipMalloc(&ctx->marena64, ns));
+        CREATECHK(hipMemset(ctx->marena64, 0, ns));
+    }
     if (precision_mode == WAVI_PRECISION_MIXED) {
         VSet<float> &w = ctx->v32;
         auto falloc = [&](float **p, size_t n) -> hipError_t {
@@ -670,7 +686,7 @@ int wavi_ctx_create(const wavi_grid_desc *grid, const wavi_phys_params *phys, co
         CREATECHK(falloc(&w.heta_h, ctx->nh));
         CREATECHK(falloc(&w.heta_c, ctx->nc > 0 ? ctx->nc : 1));
         CREATECHK(falloc(&w.dimp, ctx->nh));
-        for (DevVecT<float> *dv : {&w.h, &w.beff, &w.e, &w.r, &w.d, &w.rho, &w.t, &w.cr, &w.cp, &w.cq, &w.ct, &w.xc}) {
+        for (DevVecT<float> *dv : {&w.h, &w.beff, &w.e, &w.r, &w.d, &w.rho, &w.t, &w.cr, &w.ct, &w.xc}) {
             CREATECHK(falloc(&dv->u, ctx->nu));
             CREATECHK(falloc(&dv->v, ctx->nv));
         }
@@ -712,7 +728,7 @@ static void ctx_free(wavi_ctx *ctx)
 {
     if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
     for (uint8_t *p : {ctx->hm, ctx->hfix, ctx->um, ctx->vm, ctx->cm, ctx->ui, ctx->vi, ctx->ufix, ctx->vfix,
-                       ctx->mwu, ctx->mwv, ctx->mcu, ctx->mcv, ctx->saved_mwu, ctx->saved_mwv})
+                       ctx->mwu, ctx->mwv, ctx->saved_mwu, ctx->saved_mwv})
         if (p) (void)hipFree(p);
     for (int id = 0; id < WAVI_NFIELDS; ++id)
         if (ctx->f[id]) (void)hipFree(ctx->f[id]);
@@ -722,7 +738,7 @@ static void ctx_free(wavi_ctx *ctx)
                       ctx->Pn, ctx->Pz, ctx->cdinv.u, ctx->cdinv.v, ctx->quad})
         if (p) (void)hipFree(p);
     for (DevVec *dv : {&ctx->x, &ctx->b, &ctx->r, &ctx->e, &ctx->d, &ctx->rho, &ctx->t, &ctx->f3, &ctx->fixedv,
-                       &ctx->cr, &ctx->cp, &ctx->cq, &ctx->ct}) {
+                       &ctx->cr, &ctx->ct}) {
         if (dv->u) (void)hipFree(dv->u);
         if (dv->v) (void)hipFree(dv->v);
     }
@@ -730,12 +746,13 @@ static void ctx_free(wavi_ctx *ctx)
         VSet<float> &w = ctx->v32;
         for (float *p : {w.heta_h, w.heta_c, w.dimp})
             if (p) (void)hipFree(p);
-        for (DevVecT<float> *dv : {&w.h, &w.beff, &w.e, &w.r, &w.d, &w.rho, &w.t, &w.cr, &w.cp, &w.cq, &w.ct, &w.xc}) {
+        for (DevVecT<float> *dv : {&w.h, &w.beff, &w.e, &w.r, &w.d, &w.rho, &w.t, &w.cr, &w.ct, &w.xc}) {
             if (dv->u) (void)hipFree(dv->u);
             if (dv->v) (void)hipFree(dv->v);
         }
     }
-    for (void *p : {(void *)ctx->arena, (void *)ctx->marena, (void *)ctx->Pgd, (void *)ctx->rings})
+    for (void *p : {(void *)ctx->arena, (void *)ctx->marena, (void *)ctx->Pgd, (void *)ctx->rings, (void *)ctx->arena64,
+                    (void *)ctx->marena64})
         if (p) (void)hipFree(p);
     if (ctx->stm) (void)hipFree(ctx->stm);
     if (ctx->h_flag) (void)hipHostFree(ctx->h_flag);
@@ -1025,8 +1042,6 @@ static VSet<double> vset64(wavi_ctx *ctx)
     w.rho = {ctx->rho.u, ctx->rho.v};
     w.t = {ctx->t.u, ctx->t.v};
     w.cr = {ctx->cr.u, ctx->cr.v};
-    w.cp = {ctx->cp.u, ctx->cp.v};
-    w.cq = {ctx->cq.u, ctx->cq.v};
     w.ct = {ctx->ct.u, ctx->ct.v};
     w.xc = {ctx->f[WAVI_WU_CORRECTION_COARSE], ctx->f[WAVI_WV_CORRECTION_COARSE]};
     return w;
@@ -1206,35 +1221,20 @@ static int do_smoother(wavi_ctx *ctx, const VSet<T> &w, const int order[4])
 // Longest chunk of coarse-CG launches queued at once (cg_chunk_len).
 constexpr int CG_CHUNK = 32;
 
-template <typename T>
-static CGArgs<T> cg_args(wavi_ctx *ctx, const VSet<T> &w)
+static CGArgs cg_args(wavi_ctx *ctx)
 {
-    CGArgs<T> a;
+    CGArgs a;
     a.g = ctx->g;
-    a.c = coef_of(ctx, w);
-    a.levels = ctx->S.levels;
-    a.mwu = ctx->mwu;
-    a.mwv = ctx->mwv;
-    a.ui = ctx->ui;
-    a.vi = ctx->vi;
-    a.mcu = ctx->mcu;
-    a.mcv = ctx->mcv;
-    a.xu = w.xc.u;
-    a.xv = w.xc.v;
-    a.ru = w.cr.u;
-    a.rv = w.cr.v;
-    a.pu[0] = w.cp.u;
-    a.pv[0] = w.cp.v;
-    a.pu[1] = w.ct.u;
-    a.pv[1] = w.ct.v;
-    a.qu = w.cq.u;
-    a.qv = w.cq.v;
+    a.Lo.F = ctx->arena64;
+    a.Lo.M = ctx->marena64;
+    a.Lo.px = ctx->px64;
+    a.Lo.ns = ctx->ns64;
+    a.rdx = ctx->rdx;
+    a.rdy = ctx->rdy;
     a.Pr = ctx->Pr0;
     a.Pd = ctx->Pd;
     a.Pb = ctx->Pb;
     a.Pz = ctx->Pz;
-    a.dinvu = ctx->cdinv.u;
-    a.dinvv = ctx->cdinv.v;
     a.st = ctx->st;
     a.hflag = ctx->d_flag;
     a.tol_coarse = ctx->S.tol_coarse;
@@ -1242,6 +1242,26 @@ static CGArgs<T> cg_args(wavi_ctx *ctx, const VSet<T> &w)
     a.maxiter = ctx->S.maxiter_coarse;
     a.nblk = ctx->nblk;
     return a;
+}
+
+static CGIo cg_io(wavi_ctx *ctx, const VSet<double> &w)
+{
+    CGIo io;
+    io.c = coef_of(ctx, w);
+    io.levels = ctx->S.levels;
+    io.mwu = ctx->mwu;
+    io.mwv = ctx->mwv;
+    io.bu = w.cr.u;
+    io.bv = w.cr.v;
+    io.xu = w.xc.u;
+    io.xv = w.xc.v;
+    io.tu = w.ct.u;
+    io.tv = w.ct.v;
+    io.dinvu = ctx->cdinv.u;
+    io.dinvv = ctx->cdinv.v;
+    io.eu = w.e.u;
+    io.ev = w.e.v;
+    return io;
 }
 
 // Full chunks of CG iterations replay one captured HIP graph per context
@@ -1306,37 +1326,41 @@ static void launch_tile_haar(wavi_ctx *ctx, int dir, const T *inu, const T *inv,
 
 // The kernels of the FP64 coarse CG at the context's Haar level,
 // Jacobi-preconditioned inside a linear solve (ctx->cg_pre).
-template <typename T, bool PRE>
-static void launch_cg_step_p(wavi_ctx *ctx, dim3 tb, const CGArgs<T> &a, int par)
+template <bool PRE>
+static void launch_cg_step_p(wavi_ctx *ctx, dim3 tb, const CGArgs &a, int par)
 {
     switch (ctx->S.levels) {
-    case 0: hipLaunchKernelGGL((k_cg_step<T, PRE, 0>), tb, dim3(256), 0, ctx->stream, a, par); break;
-    case 1: hipLaunchKernelGGL((k_cg_step<T, PRE, 1>), tb, dim3(256), 0, ctx->stream, a, par); break;
-    case 2: hipLaunchKernelGGL((k_cg_step<T, PRE, 2>), tb, dim3(256), 0, ctx->stream, a, par); break;
-    default: hipLaunchKernelGGL((k_cg_step<T, PRE, 3>), tb, dim3(256), 0, ctx->stream, a, par); break;
+    case 0: hipLaunchKernelGGL((k_cg_step<PRE, 0>), tb, dim3(256), 0, ctx->stream, a, par); break;
+    case 1: hipLaunchKernelGGL((k_cg_step<PRE, 1>), tb, dim3(256), 0, ctx->stream, a, par); break;
+    case 2: hipLaunchKernelGGL((k_cg_step<PRE, 2>), tb, dim3(256), 0, ctx->stream, a, par); break;
+    default: hipLaunchKernelGGL((k_cg_step<PRE, 3>), tb, dim3(256), 0, ctx->stream, a, par); break;
     }
 }
 
-template <typename T, bool PRE>
-static void launch_cg_solve1_p(wavi_ctx *ctx, const CGArgs<T> &a)
+template <bool PRE>
+static void launch_cg_solve1_p(wavi_ctx *ctx, const CGArgs &a)
 {
     switch (ctx->S.levels) {
-    case 0: hipLaunchKernelGGL((k_cg_solve1<T, PRE, 0>), dim3(1), dim3(256), 0, ctx->stream, a); break;
-    case 1: hipLaunchKernelGGL((k_cg_solve1<T, PRE, 1>), dim3(1), dim3(256), 0, ctx->stream, a); break;
-    case 2: hipLaunchKernelGGL((k_cg_solve1<T, PRE, 2>), dim3(1), dim3(256), 0, ctx->stream, a); break;
-    default: hipLaunchKernelGGL((k_cg_solve1<T, PRE, 3>), dim3(1), dim3(256), 0, ctx->stream, a); break;
+    case 0: hipLaunchKernelGGL((k_cg_solve1<PRE, 0>), dim3(1), dim3(256), 0, ctx->stream, a); break;
+    case 1: hipLaunchKernelGGL((k_cg_solve1<PRE, 1>), dim3(1), dim3(256), 0, ctx->stream, a); break;
+    case 2: hipLaunchKernelGGL((k_cg_solve1<PRE, 2>), dim3(1), dim3(256), 0, ctx->stream, a); break;
+    default: hipLaunchKernelGGL((k_cg_solve1<PRE, 3>), dim3(1), dim3(256), 0, ctx->stream, a); break;
     }
 }
 
-// coarse CG on b_c held in w.cr; solution in the warm start w.xc
 template <typename T>
-static int do_coarse_cg(wavi_ctx *ctx, const VSet<T> &w, int *iters)
+static int do_coarse_cg(wavi_ctx *ctx, const VSet<T> &w, int *iters);
+
+// FP64 coarse CG on b_c held in w.cr from the warm start w.xc; the solution
+// stays in the arena until k_cg_finish.
+template <>
+int do_coarse_cg<double>(wavi_ctx *ctx, const VSet<double> &w, int *iters)
 {
-    const GridDims &g = ctx->g;
-    dim3 tg(g.nbx, g.nby), tb(ctx->nblk);
-    CGArgs<T> a = cg_args(ctx, w);
+    dim3 tb(ctx->nblk);
+    const CGArgs a = cg_args(ctx);
+    const CGIo io = cg_io(ctx, w);
     // t = P x0
-    launch_tile_haar<T>(ctx, 1, a.xu, a.xv, ctx->mwu, ctx->mwv, a.pu[1], a.pv[1], ctx->ui, ctx->vi);
+    launch_tile_haar<double>(ctx, 1, w.xc.u, w.xc.v, ctx->mwu, ctx->mwv, w.ct.u, w.ct.v, ctx->ui, ctx->vi);
     ctx->h_flag->done = 0;
     ctx->h_flag->iters = 0;
     const bool pre = ctx->cg_pre;
@@ -1346,16 +1370,16 @@ static int do_coarse_cg(wavi_ctx *ctx, const VSet<T> &w, int *iters)
     // about one, and their launches do without the flag's round trip.
     const bool early = ctx->cg_prev < CG_CHUNK;
     if (pre)
-        hipLaunchKernelGGL((k_cg_setup<T, true>), tb, dim3(256), 0, ctx->stream, a);
+        hipLaunchKernelGGL(k_cg_setup<true>, tb, dim3(256), 0, ctx->stream, a, io);
     else
-        hipLaunchKernelGGL((k_cg_setup<T, false>), tb, dim3(256), 0, ctx->stream, a);
+        hipLaunchKernelGGL(k_cg_setup<false>, tb, dim3(256), 0, ctx->stream, a, io);
     HIPCHK(hipGetLastError());
     volatile CGMHostFlag *hf = ctx->h_flag;
     if (cg_one_workgroup(ctx)) {
         if (pre)
-            launch_cg_solve1_p<T, true>(ctx, a);
+            launch_cg_solve1_p<true>(ctx, a);
         else
-            launch_cg_solve1_p<T, false>(ctx, a);
+            launch_cg_solve1_p<false>(ctx, a);
         HIPCHK(hipGetLastError());
         HIPCHK(hipStreamSynchronize(ctx->stream));
         if (!hf->done) {
@@ -1382,20 +1406,20 @@ static int do_coarse_cg(wavi_ctx *ctx, const VSet<T> &w, int *iters)
             {
                 ProfScope ps(ctx, WAVI_KT_CG_APPLY, sampled);
                 if (pre)
-                    launch_cg_step_p<T, true>(ctx, tb, a, par);
+                    launch_cg_step_p<true>(ctx, tb, a, par);
                 else
-                    launch_cg_step_p<T, false>(ctx, tb, a, par);
+                    launch_cg_step_p<false>(ctx, tb, a, par);
             }
             {
                 ProfScope ps(ctx, WAVI_KT_CG_UPDATE, sampled);
                 if (pre && early)
-                    hipLaunchKernelGGL((k_cg_update<T, true, true>), tb, dim3(256), 0, ctx->stream, a, par);
+                    hipLaunchKernelGGL((k_cg_update<true, true>), tb, dim3(256), 0, ctx->stream, a, par);
                 else if (pre)
-                    hipLaunchKernelGGL((k_cg_update<T, true, false>), tb, dim3(256), 0, ctx->stream, a, par);
+                    hipLaunchKernelGGL((k_cg_update<true, false>), tb, dim3(256), 0, ctx->stream, a, par);
                 else if (early)
-                    hipLaunchKernelGGL((k_cg_update<T, false, true>), tb, dim3(256), 0, ctx->stream, a, par);
+                    hipLaunchKernelGGL((k_cg_update<false, true>), tb, dim3(256), 0, ctx->stream, a, par);
                 else
-                    hipLaunchKernelGGL((k_cg_update<T, false, false>), tb, dim3(256), 0, ctx->stream, a, par);
+                    hipLaunchKernelGGL((k_cg_update<false, false>), tb, dim3(256), 0, ctx->stream, a, par);
             }
         }
         burst_end(ctx, bev, q - 1, n);
@@ -1665,7 +1689,10 @@ static int vcycle_post(wavi_ctx *ctx, const VSet<T> &w)
     const GridDims &g = ctx->g;
     dim3 tg(g.nbx, g.nby);
     // e += P x_c
-    launch_tile_haar<T>(ctx, 1, w.xc.u, w.xc.v, ctx->mwu, ctx->mwv, w.t.u, w.t.v, ctx->ui, ctx->vi, w.e.u, w.e.v);
+    if constexpr (std::is_same<T, double>::value)
+        hipLaunchKernelGGL(k_cg_finish, dim3(ctx->nblk), dim3(256), 0, ctx->stream, cg_args(ctx), cg_io(ctx, w));
+    else
+        launch_tile_haar<T>(ctx, 1, w.xc.u, w.xc.v, ctx->mwu, ctx->mwv, w.t.u, w.t.v, ctx->ui, ctx->vi, w.e.u, w.e.v);
     CHK(do_smoother(ctx, w, rev));
     HIPCHK(hipGetLastError());
     return WAVI_OK;

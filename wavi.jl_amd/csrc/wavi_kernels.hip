@@ -10,6 +10,7 @@
 // the u grid and of the v grid (grid (nbx, nby)); they own the Haar blocks
 // (levels <= 3) and write one reduction partial per block.  Other kernels
 // are flat (256 threads, one point each).
+#include <type_traits>
 #include "wavi_device.h"
 
 namespace wavi {
@@ -1349,27 +1350,12 @@ struct MaskSep {
     }
 };
 
-// ... packed, one byte per point
-struct MaskPacked {
-    const uint8_t *mu, *mv;
-    __device__ __forceinline__ unsigned u(bool ok, int k) const
-    {
-        const unsigned a = mu[ok ? k : 0];
-        return ok ? a : 0u;
-    }
-    __device__ __forceinline__ unsigned v(bool ok, int k) const
-    {
-        const unsigned a = mv[ok ? k : 0];
-        return ok ? a : 0u;
-    }
-};
-
 // The coarse values around a tile from which k_cg_step forms P u on the
 // halo (HALO_N of haar_halo_offset per side, 5 at three levels).
 template <typename T>
 struct HaloLds {
-    T x[2][10][17];   // component; columns left (0..4) and right (5..9), rows by y
-    T y[2][10][16];   // rows below and above, by x
+    T x[2][10][17];   // component; columns left (0..4) and right (5..9), by y
+    T y[2][10][16];   // rows below (0..4) and above (5..9), by x
     T c[2][5][5];     // the corner block, [y][x]
     T lx[2][10][17];  // y sums of x
     T ly[2][2][16];   // y sums of y: rows -1 and 16, by x
@@ -1401,7 +1387,8 @@ struct OpLds {
     };
 };
 
-// What a thread holds of its tile.
+// What a thread holds of its tile.  The thicknesses and drags are zero off the
+// u and v masks (an inner point is on its mask).
 template <typename T>
 struct OpOwn {
     T u, v, hu, hv, bu, bv;
@@ -1427,14 +1414,14 @@ __device__ __forceinline__ void op_cell_load(const GridDims &g, const OpCoef<T> 
 // op_rxy).  Cell (0, 0) reads one absent window point of each kind and corner
 // (16, 16) another; no output reads what they feed.
 template <typename T>
-__device__ __forceinline__ void op_cell(const OpCoef<T> &c, OpLds<T> &s, int x, int y, T heta, T dimp, T hetac)
+__device__ __forceinline__ void op_cell(T rdx, T rdy, OpLds<T> &s, int x, int y, T heta, T dimp, T hetac)
 {
     const T u0 = s.w.U[y][x], u1 = s.w.U[y][x + 1], v0 = s.w.V[y][x], v1 = s.w.V[y + 1][x];
-    const T dudx = c.rdx * u1 - c.rdx * u0;
-    const T dvdy = c.rdy * v1 - c.rdy * v0;
-    const T divq = (c.rdx * s.w.QX[y][x + 1] - c.rdx * s.w.QX[y][x]) + (c.rdy * s.w.QY[y + 1][x] - c.rdy * s.w.QY[y][x]);
-    const T dudy = c.rdy * s.w.U[y + 1][x + 1] - c.rdy * u1;
-    const T dvdx = c.rdx * s.w.V[y + 1][x + 1] - c.rdx * v1;
+    const T dudx = rdx * u1 - rdx * u0;
+    const T dvdy = rdy * v1 - rdy * v0;
+    const T divq = (rdx * s.w.QX[y][x + 1] - rdx * s.w.QX[y][x]) + (rdy * s.w.QY[y + 1][x] - rdy * s.w.QY[y][x]);
+    const T dudy = rdy * s.w.U[y + 1][x + 1] - rdy * u1;
+    const T dvdx = rdx * s.w.V[y + 1][x + 1] - rdx * v1;
     s.rxx[y][x] = T(2) * (heta * (T(2) * dudx + dvdy));
     s.ryy[y][x] = T(2) * (heta * (T(2) * dvdy + dudx));
     s.ext[y][x] = dimp * divq;
@@ -1468,15 +1455,23 @@ __device__ __forceinline__ HaloPos op_halo_sides(int w, int l)
 }
 
 // Coefficients of a tile besides its points' values: the thread's own point
-// and cell, its halo points' thicknesses and masks, and the cell before the
-// tile that it computes (wavefront 0, lanes 0..32: (0, 0..16), (1..16, 0)).
+// and cell, its halo points' thicknesses (zero off the masks), and the cell
+// before the tile that it computes (wavefront 0, lanes 0..32: (0, 0..16), (1..16, 0)).
 template <typename T>
 struct OpCoefRegs {
     T hhu, hhv;
-    unsigned hmu, hmv;
     T eh, ed, ec;
     int ex, ey;
 };
+
+// ... and where that cell is
+template <typename T>
+__device__ __forceinline__ void op_extra_cell(int l, OpCoefRegs<T> &r)
+{
+    r.ex = l < 17 ? 0 : l - 16;
+    r.ey = l < 17 ? l : 0;
+    r.eh = r.ed = r.ec = T(0);
+}
 
 template <typename T, class M>
 __device__ __forceinline__ void op_coef_load(const GridDims &g, const OpCoef<T> &c, const M &mask, int i0, int j0,
@@ -1484,51 +1479,49 @@ __device__ __forceinline__ void op_coef_load(const GridDims &g, const OpCoef<T> 
 {
     const int lx = threadIdx.x & 15, ly = threadIdx.x >> 4, l = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    o.hu = ld_or(o.oku, c.hu, o.ku, T(0));
-    o.hv = ld_or(o.okv, c.hv, o.kv, T(0));
+    const T ohu = ld_or(o.oku, c.hu, o.ku, T(0)), ohv = ld_or(o.okv, c.hv, o.kv, T(0));
     r.hhu = r.hhv = T(0);
-    r.hmu = r.hmv = 0;
     if (halo_wave) {
         const int iu = i0 - 1 + h.ux, ju = j0 - 1 + h.uy, iv = i0 - 1 + h.vx, jv = j0 - 1 + h.vy;
         const bool oku = h.hu && iu >= 0 && iu < g.nxu && ju >= 0 && ju < g.nyu;
         const bool okv = h.hv && iv >= 0 && iv < g.nxv && jv >= 0 && jv < g.nyv;
-        r.hhu = ld_or(oku, c.hu, iu + g.nxu * ju, T(0));
-        r.hhv = ld_or(okv, c.hv, iv + g.nxv * jv, T(0));
-        r.hmu = mask.u(oku, iu + g.nxu * ju);
-        r.hmv = mask.v(okv, iv + g.nxv * jv);
+        const T u = ld_or(oku, c.hu, iu + g.nxu * ju, T(0)), v = ld_or(okv, c.hv, iv + g.nxv * jv, T(0));
+        r.hhu = (mask.u(oku, iu + g.nxu * ju) & MB_POINT) ? u : T(0);
+        r.hhv = (mask.v(okv, iv + g.nxv * jv) & MB_POINT) ? v : T(0);
     }
     op_cell_load(g, c, i0 + lx, j0 + ly, o.heta, o.dimp, o.hetac);
-    r.ex = l < 17 ? 0 : l - 16;
-    r.ey = l < 17 ? l : 0;
-    r.eh = r.ed = r.ec = T(0);
+    op_extra_cell(l, r);
     if (w == 0) op_cell_load(g, c, l < 33 ? i0 - 1 + r.ex : -1, j0 - 1 + r.ey, r.eh, r.ed, r.ec);
-    o.bu = ld_or(o.oku, c.bu, o.ku, T(0));
-    o.bv = ld_or(o.okv, c.bv, o.kv, T(0));
+    const T obu = ld_or(o.oku, c.bu, o.ku, T(0)), obv = ld_or(o.okv, c.bv, o.kv, T(0));
+    o.hu = (o.mu & MB_POINT) ? ohu : T(0);
+    o.hv = (o.mv & MB_POINT) ? ohv : T(0);
+    o.bu = (o.mu & MB_POINT) ? obu : T(0);
+    o.bv = (o.mv & MB_POINT) ? obv : T(0);
 }
 
 // Stage the window (the thread's own point and its halo points hu, hv) and
 // compute the cells' intermediates.  Ends with a barrier, after which the
 // window is free.
 template <typename T>
-__device__ __forceinline__ void op_cells(const OpCoef<T> &c, const HaloPos &h, T hu, T hv, const OpOwn<T> &o,
+__device__ __forceinline__ void op_cells(T rdx, T rdy, const HaloPos &h, T hu, T hv, const OpOwn<T> &o,
                                          const OpCoefRegs<T> &r, OpLds<T> &s)
 {
     const int lx = threadIdx.x & 15, ly = threadIdx.x >> 4;
     s.w.U[ly + 1][lx + 1] = o.u;
     s.w.V[ly + 1][lx + 1] = o.v;
-    s.w.QX[ly + 1][lx + 1] = (o.mu & MB_POINT) ? o.hu * o.u : T(0);
-    s.w.QY[ly + 1][lx + 1] = (o.mv & MB_POINT) ? o.hv * o.v : T(0);
+    s.w.QX[ly + 1][lx + 1] = o.hu * o.u;
+    s.w.QY[ly + 1][lx + 1] = o.hv * o.v;
     if (h.hu) {
         s.w.U[h.uy][h.ux] = hu;
-        s.w.QX[h.uy][h.ux] = (r.hmu & MB_POINT) ? r.hhu * hu : T(0);
+        s.w.QX[h.uy][h.ux] = r.hhu * hu;
     }
     if (h.hv) {
         s.w.V[h.vy][h.vx] = hv;
-        s.w.QY[h.vy][h.vx] = (r.hmv & MB_POINT) ? r.hhv * hv : T(0);
+        s.w.QY[h.vy][h.vx] = r.hhv * hv;
     }
     __syncthreads();
-    op_cell(c, s, lx + 1, ly + 1, o.heta, o.dimp, o.hetac);
-    if (threadIdx.x < 33) op_cell(c, s, r.ex, r.ey, r.eh, r.ed, r.ec);
+    op_cell(rdx, rdy, s, lx + 1, ly + 1, o.heta, o.dimp, o.hetac);
+    if (threadIdx.x < 33) op_cell(rdx, rdy, s, r.ex, r.ey, r.eh, r.ed, r.ec);
     __syncthreads();
 }
 
@@ -1561,29 +1554,29 @@ __device__ __forceinline__ void op_tile(const GridDims &g, const OpCoef<T> &c, c
     }
     OpCoefRegs<T> r;
     op_coef_load(g, c, mask, i0, j0, h, w >= 2, o, r);
-    op_cells(c, h, hu, hv, o, r, s);
+    op_cells(c.rdx, c.rdy, h, hu, hv, o, r, s);
 }
 
 // A x at the thread's u point and v point (inner or not)
 template <typename T>
-__device__ __forceinline__ T op_out_u(const OpCoef<T> &c, const OpLds<T> &s, const OpOwn<T> &o)
+__device__ __forceinline__ T op_out_u(T rdx, T rdy, const OpLds<T> &s, const OpOwn<T> &o)
 {
     const int x = threadIdx.x & 15, y = threadIdx.x >> 4;
-    const T d_rxx_dx = c.rdx * s.rxx[y + 1][x + 1] - c.rdx * s.rxx[y + 1][x];
-    const T d_rxy_dy = c.rdy * s.rxy[y + 1][x] - c.rdy * s.rxy[y][x];
-    const T taubx = (o.mu & MB_POINT) ? o.bu * o.u : T(0);
-    const T d_extra_dx = c.rdx * s.ext[y + 1][x + 1] - c.rdx * s.ext[y + 1][x];
+    const T d_rxx_dx = rdx * s.rxx[y + 1][x + 1] - rdx * s.rxx[y + 1][x];
+    const T d_rxy_dy = rdy * s.rxy[y + 1][x] - rdy * s.rxy[y][x];
+    const T taubx = o.bu * o.u;
+    const T d_extra_dx = rdx * s.ext[y + 1][x + 1] - rdx * s.ext[y + 1][x];
     return ((d_rxx_dx + d_rxy_dy) - taubx) - o.hu * d_extra_dx;
 }
 
 template <typename T>
-__device__ __forceinline__ T op_out_v(const OpCoef<T> &c, const OpLds<T> &s, const OpOwn<T> &o)
+__device__ __forceinline__ T op_out_v(T rdx, T rdy, const OpLds<T> &s, const OpOwn<T> &o)
 {
     const int x = threadIdx.x & 15, y = threadIdx.x >> 4;
-    const T d_ryy_dy = c.rdy * s.ryy[y + 1][x + 1] - c.rdy * s.ryy[y][x + 1];
-    const T d_rxy_dx = c.rdx * s.rxy[y][x + 1] - c.rdx * s.rxy[y][x];
-    const T tauby = (o.mv & MB_POINT) ? o.bv * o.v : T(0);
-    const T d_extra_dy = c.rdy * s.ext[y + 1][x + 1] - c.rdy * s.ext[y][x + 1];
+    const T d_ryy_dy = rdy * s.ryy[y + 1][x + 1] - rdy * s.ryy[y][x + 1];
+    const T d_rxy_dx = rdx * s.rxy[y][x + 1] - rdx * s.rxy[y][x];
+    const T tauby = o.bv * o.v;
+    const T d_extra_dy = rdy * s.ext[y + 1][x + 1] - rdy * s.ext[y][x + 1];
     return ((d_ryy_dy + d_rxy_dx) - tauby) - o.hv * d_extra_dy;
 }
 
@@ -1595,7 +1588,7 @@ __device__ __forceinline__ void op_restrict_tile(const GridDims &g, const OpCoef
 {
     const int lx = threadIdx.x & 15, ly = threadIdx.x >> 4;
     op_tile(g, c, mask, xu, xv, i0, j0, s, o);
-    const T yu = (o.mu & MB_INNER) ? op_out_u(c, s, o) : T(0), yv = (o.mv & MB_INNER) ? op_out_v(c, s, o) : T(0);
+    const T yu = (o.mu & MB_INNER) ? op_out_u(c.rdx, c.rdy, s, o) : T(0), yv = (o.mv & MB_INNER) ? op_out_v(c.rdx, c.rdy, s, o) : T(0);
     s.h.t[0][ly][lx] = yu;
     s.h.t[1][ly][lx] = yv;
     __syncthreads();
@@ -1656,8 +1649,8 @@ __global__ void __launch_bounds__(256) k_op(GridDims g, OpCoef<T> c, const T *xu
     if (!xcd_band_tile(g.nbx, g.nby, nblk, true, bx, by)) return;
     OpOwn<T> o;
     op_tile(g, c, MaskSep<false>{c.ui, c.um, c.vi, c.vm, nullptr, nullptr}, xu, xv, bx * TILE, by * TILE, s, o);
-    if (o.oku) yu[o.ku] = (o.mu & MB_INNER) ? op_out_u(c, s, o) : T(0);
-    if (o.okv) yv[o.kv] = (o.mv & MB_INNER) ? op_out_v(c, s, o) : T(0);
+    if (o.oku) yu[o.ku] = (o.mu & MB_INNER) ? op_out_u(c.rdx, c.rdy, s, o) : T(0);
+    if (o.okv) yv[o.kv] = (o.mv & MB_INNER) ? op_out_v(c.rdx, c.rdy, s, o) : T(0);
 }
 
 // r = b - A x at inner points (get_resid!, utilities.jl:549-552); per-tile
@@ -1684,7 +1677,7 @@ __global__ void __launch_bounds__(256) k_tile_resid(GridDims g, OpCoef<T> c, con
     if (has_u) {
         double r2 = 0.0, b2 = 0.0;
         if (o.oku) {
-            const T r = (o.mu & MB_INNER) ? b_u - op_out_u(c, s, o) : T(0);
+            const T r = (o.mu & MB_INNER) ? b_u - op_out_u(c.rdx, c.rdy, s, o) : T(0);
             ru[o.ku] = r;
             if (fu && (o.mu & MB_INNER)) fu[o.ku] = r;
             r2 = (double)r * (double)r;
@@ -1699,7 +1692,7 @@ __global__ void __launch_bounds__(256) k_tile_resid(GridDims g, OpCoef<T> c, con
     if (has_v) {
         double r2 = 0.0, b2 = 0.0;
         if (o.okv) {
-            const T r = (o.mv & MB_INNER) ? b_v - op_out_v(c, s, o) : T(0);
+            const T r = (o.mv & MB_INNER) ? b_v - op_out_v(c.rdx, c.rdy, s, o) : T(0);
             rv[o.kv] = r;
             if (fv && (o.mv & MB_INNER)) fv[o.kv] = r;
             r2 = (double)r * (double)r;
@@ -2185,25 +2178,72 @@ struct CGScalars {
     double rz[2];     // Jacobi-preconditioned CG: (r, D^-1 r) by parity (written by k_cg_step)
 };
 
-template <typename T>
+// The FP64 coarse CG works in an arena of zero-padded 2-D arrays shared by
+// the u grid, the v grid and the h cells: point (i, j) at (i + 16) + px (j +
+// 16), px = 16 (nbx + 2), with a border of one tile that stays zero.  A tile's
+// rows are then aligned, u and v of a point come in one 16-byte load, every
+// window, halo and store is unconditional at a 32-bit offset from a uniform
+// base, and what a tile stores past the end of a grid is zero.  Guarded
+// loads from the compact arrays at clamped indices took about half of the
+// VALU instructions of an iteration.  k_cg_setup fills it.
+enum CGPair {        // (u, v) pairs, ns each
+    CG_R = 0,        // residual r
+    CG_P = 1,        // search direction u, by iteration parity (two arrays)
+    CG_X = 3,        // solution
+    CG_Q = 4,        // c = A_c u
+    CG_H = 5,        // thickness on u and v points, 0 off the masks
+    CG_B = 6,        // beta_eff on u and v points, 0 off the masks
+    CG_CELL = 7,     // per h cell: (h*eta_av, dimp)
+    CG_DINV = 8,     // Jacobi: 1 / |diag(A_c)|, 0 off the wavelet masks
+    CG_NPAIR = 9
+};
+enum { CB_INNER_U = 1, CB_INNER_V = 2, CB_WAVELET_U = 4, CB_WAVELET_V = 8 };  // mask bits of a point
+
+struct CGLayout {
+    double2 *F;       // pair array A at F + A * ns, then the corners' h*eta_av (ns doubles)
+    uint8_t *M;       // mask bits (CB_*)
+    unsigned px, ns;  // row pitch, array stride
+    __device__ __forceinline__ unsigned at(int i, int j) const
+    {
+        return (unsigned)(i + TILE) + __umul24(px, (unsigned)(j + TILE));
+    }
+    __device__ __forceinline__ double2 *pair(int a) const { return F + (size_t)a * ns; }
+    __device__ __forceinline__ double *corner() const { return reinterpret_cast<double *>(F + (size_t)CG_NPAIR * ns); }
+};
+
+// Element k of an array below 4 GiB, addressed by a 32-bit byte offset from
+// its uniform base (the scalar-base form of the global loads and stores).
+template <typename V>
+__device__ __forceinline__ V &elem32(V *p, unsigned k)
+{
+    typedef typename std::conditional<std::is_const<V>::value, const char, char>::type C;
+    return *reinterpret_cast<V *>(reinterpret_cast<C *>(p) + (size_t)(unsigned)(k * (unsigned)sizeof(V)));
+}
+
 struct CGArgs {
     GridDims g;
-    OpCoef<T> c;
-    int levels;
-    const uint8_t *mwu, *mwv, *ui, *vi;
-    uint8_t *mcu, *mcv;  // packed mask bits (MB_*) of the u and v points, written by k_cg_setup
-    T *xu, *xv;       // solution (warm start in, result out)
-    T *ru, *rv;       // residual (right-hand side on entry to setup)
-    T *pu[2], *pv[2]; // search direction u by iteration parity (set 1 holds P x0 during the set-up)
-    T *qu, *qv;       // c = A_c u
+    CGLayout Lo;
+    double rdx, rdy;
     double *Pr, *Pd, *Pb;
     double *Pz;                       // Jacobi: partials of (r, D^-1 r)
-    const double *dinvu, *dinvv;      // Jacobi: 1 / |diag(A_c)|, 0 off the wavelet masks
     CGScalars *st;
     CGMHostFlag *hflag;   // host-mapped stop report
     double tol_coarse, reltol;
     int maxiter;
     int nblk;         // launched workgroups, a multiple of 8
+};
+
+// What the set-up and the end of the CG read and write besides: the compact
+// arrays.
+struct CGIo {
+    OpCoef<double> c;
+    int levels;
+    const uint8_t *mwu, *mwv;
+    const double *bu, *bv;            // right-hand side
+    double *xu, *xv;                  // warm start in, solution out
+    const double *tu, *tv;            // P x0
+    const double *dinvu, *dinvv;      // Jacobi: 1 / |diag(A_c)|, 0 off the wavelet masks
+    double *eu, *ev;                  // the V-cycle's correction, += P x
 };
 
 // XCD-aware tile order: workgroups are dispatched round-robin over the 8
@@ -2224,13 +2264,13 @@ __device__ __forceinline__ int band_tile(const GridDims &g, int L, int &bx, int 
     return L;
 }
 
-// setup (t = P x0 computed beforehand): r = b - R A t (b arrives in r),
-// u = 0, partials of ||r0||^2 and ||b||^2 (PRE: also of (r0, D^-1 r0)),
-// the packed masks of the iterations; resets the scalars.
-template <typename T, bool PRE>
-__global__ void __launch_bounds__(256) k_cg_setup(CGArgs<T> a)
+// setup (t = P x0 computed beforehand): r = b - R A t, x = x0, u = 0, the
+// coefficients and mask bits into the arena, partials of ||r0||^2 and ||b||^2
+// (PRE: also of (r0, D^-1 r0)); resets the scalars.
+template <bool PRE>
+__global__ void __launch_bounds__(256) k_cg_setup(CGArgs a, CGIo io)
 {
-    __shared__ OpLds<T> s;
+    __shared__ OpLds<double> s;
     __shared__ double lds[8];
     const GridDims &g = a.g;
     const int L = xcd_tile(a.nblk);
@@ -2252,34 +2292,34 @@ __global__ void __launch_bounds__(256) k_cg_setup(CGArgs<T> a)
     const bool has_u = bx < g.nbxu && by < g.nbyu, has_v = bx < g.nbxv && by < g.nbyv;
     const int i0 = bx * TILE, j0 = by * TILE;
     const int lx = threadIdx.x & 15, ly = threadIdx.x >> 4;
-    const int i = i0 + lx, j = j0 + ly;
-    const T bu = ld_or(i < g.nxu && j < g.nyu, a.ru, i + g.nxu * j, T(0));
-    const T bv = ld_or(i < g.nxv && j < g.nyv, a.rv, i + g.nxv * j, T(0));
-    OpOwn<T> o;
-    op_restrict_tile(g, a.c, MaskSep<true>{a.ui, a.c.um, a.vi, a.c.vm, a.mwu, a.mwv}, a.levels, a.pu[1], a.pv[1], i0, j0, s,
-                     o);
-    if (o.oku) a.mcu[o.ku] = (uint8_t)o.mu;
-    if (o.okv) a.mcv[o.kv] = (uint8_t)o.mv;
-    double r2u = 0.0, b2u = 0.0, r2v = 0.0, b2v = 0.0, z2u = 0.0, z2v = 0.0;
-    if (o.oku) {
-        const T r = bu - ((o.mu & MB_WAVELET) ? s.h.t[0][ly][lx] : T(0));
-        a.ru[o.ku] = r;
-        a.pu[0][o.ku] = T(0);
-        r2u = (double)r * (double)r;
-        b2u = (double)bu * (double)bu;
-        if constexpr (PRE) z2u = (double)r * (a.dinvu[o.ku] * (double)r);
-    }
-    if (o.okv) {
-        const T r = bv - ((o.mv & MB_WAVELET) ? s.h.t[1][ly][lx] : T(0));
-        a.rv[o.kv] = r;
-        a.pv[0][o.kv] = T(0);
-        r2v = (double)r * (double)r;
-        b2v = (double)bv * (double)bv;
-        if constexpr (PRE) z2v = (double)r * (a.dinvv[o.kv] * (double)r);
-    }
+    OpOwn<double> o;
+    op_own_index(g, i0 + lx, j0 + ly, o.oku, o.okv, o.ku, o.kv);
+    const double bu = ld_or(o.oku, io.bu, o.ku, 0.0), bv = ld_or(o.okv, io.bv, o.kv, 0.0);
+    const double xu = ld_or(o.oku, io.xu, o.ku, 0.0), xv = ld_or(o.okv, io.xv, o.kv, 0.0);
+    const double zu = PRE ? ld_or(o.oku, io.dinvu, o.ku, 0.0) : 0.0, zv = PRE ? ld_or(o.okv, io.dinvv, o.kv, 0.0) : 0.0;
+    const OpCoef<double> &c = io.c;
+    op_restrict_tile(g, c, MaskSep<true>{c.ui, c.um, c.vi, c.vm, io.mwu, io.mwv}, io.levels, io.tu, io.tv, i0, j0, s, o);
+    const double ru = (o.mu & MB_WAVELET) ? bu - s.h.t[0][ly][lx] : bu, rv = (o.mv & MB_WAVELET) ? bv - s.h.t[1][ly][lx] : bv;
+    const unsigned at = a.Lo.at(i0 + lx, j0 + ly);
+    elem32(a.Lo.pair(CG_R), at) = make_double2(ru, rv);
+    elem32(a.Lo.pair(CG_P), at) = make_double2(0.0, 0.0);
+    elem32(a.Lo.pair(CG_X), at) = make_double2(xu, xv);
+    elem32(a.Lo.pair(CG_H), at) = make_double2(o.hu, o.hv);
+    elem32(a.Lo.pair(CG_B), at) = make_double2(o.bu, o.bv);
+    elem32(a.Lo.pair(CG_CELL), at) = make_double2(o.heta, o.dimp);
+    if constexpr (PRE) elem32(a.Lo.pair(CG_DINV), at) = make_double2(zu, zv);
+    elem32(a.Lo.corner(), at) = o.hetac;
+    elem32(a.Lo.M, at) = (uint8_t)(((o.mu & MB_INNER) ? CB_INNER_U : 0) | ((o.mv & MB_INNER) ? CB_INNER_V : 0) |
+                           ((o.mu & MB_WAVELET) ? CB_WAVELET_U : 0) | ((o.mv & MB_WAVELET) ? CB_WAVELET_V : 0));
+    double r2u = ru * ru, r2v = rv * rv, b2u = bu * bu, b2v = bv * bv;
     tree256x2(r2u, r2v, lds);
     tree256x2(b2u, b2v, lds);
-    if constexpr (PRE) tree256x2(z2u, z2v, lds);
+    double z2u = 0.0, z2v = 0.0;
+    if constexpr (PRE) {
+        z2u = ru * (zu * ru);
+        z2v = rv * (zv * rv);
+        tree256x2(z2u, z2v, lds);
+    }
     if (threadIdx.x == 0) {
         if (has_u) {
             a.Pr[bx + g.nbxu * by] = r2u;
@@ -2293,6 +2333,34 @@ __global__ void __launch_bounds__(256) k_cg_setup(CGArgs<T> a)
             if constexpr (PRE) a.Pz[q] = z2v;
         }
     }
+}
+
+// The end of the CG: x back into the compact warm start, and e += P x at the
+// inner points.
+__global__ void __launch_bounds__(256) k_cg_finish(CGArgs a, CGIo io)
+{
+    __shared__ TilePair<double> t, m;
+    const GridDims &g = a.g;
+    const int L = xcd_tile(a.nblk);
+    if (L >= g.nbx * g.nby) return;
+    int bx, by;
+    band_tile(g, L, bx, by);
+    const int lx = threadIdx.x & 15, ly = threadIdx.x >> 4, i = bx * TILE + lx, j = by * TILE + ly;
+    bool oku, okv;
+    int ku, kv;
+    op_own_index(g, i, j, oku, okv, ku, kv);
+    const unsigned at = a.Lo.at(i, j);
+    const double2 x = elem32(a.Lo.pair(CG_X), at);
+    const unsigned mb = elem32(a.Lo.M, at);
+    const double eu = ld_or(oku, (const double *)io.eu, ku, 0.0), ev = ld_or(okv, (const double *)io.ev, kv, 0.0);
+    if (oku) io.xu[ku] = x.x;
+    if (okv) io.xv[kv] = x.y;
+    t[0][ly][lx] = (mb & CB_WAVELET_U) ? x.x : 0.0;
+    t[1][ly][lx] = (mb & CB_WAVELET_V) ? x.y : 0.0;
+    __syncthreads();
+    haar_pair<false, double>(io.levels, t, m);
+    if (mb & CB_INNER_U) io.eu[ku] = eu + t[0][ly][lx];
+    if (mb & CB_INNER_V) io.ev[kv] = ev + t[1][ly][lx];
 }
 
 // A CG scalar written by an earlier kernel, read as a vector load: a scalar
@@ -2310,14 +2378,14 @@ __device__ __forceinline__ V cg_scalar(const V *p)
 }
 
 // Offset of the k-th coarse row (or column) that the point next to a tile
-// takes from the neighbour, relative to the tile's first: below (k < 5) the
-// neighbour's last point 15, whose row of P has the terms 16 - B, .., 8, 12,
-// 14, 15 (all +1), above (k >= 5) its first point 0 with the terms 0, 1, 2, 4,
-// 8 (+1, then all -1).  N = LEV + 2 of them, in increasing order.
+// takes from the neighbour, relative to the tile's first: before the tile
+// the neighbour's last point 15, whose row of P has the terms 16 - B, .., 8,
+// 12, 14, 15 (all +1), after it the neighbour's first point 0 with the terms
+// 0, 1, 2, 4, 8 (+1, then all -1).  N = LEV + 2 of them, in increasing order.
 template <int LEV>
-__device__ __forceinline__ int haar_halo_offset(int k)
+__device__ __forceinline__ int haar_halo_offset(bool after, int k)
 {
-    return k < 5 ? -((2 << LEV) >> k) : 16 + ((1 << (k - 5)) >> 1);
+    return after ? 16 + ((1 << k) >> 1) : -((2 << LEV) >> k);
 }
 
 // The row of P that haar_halo_offset's terms v[0..N) (stride st) make: the
@@ -2367,9 +2435,12 @@ __device__ __forceinline__ T haar_row_P(const T *src, int i)
 // in the order of the block transform, so it has the neighbour's bits.  With
 // the direction in a launch of its own, P u went through memory and the
 // iteration had a third kernel boundary (at least 2.5 us on this chip).
-template <typename T, bool PRE, int LEV>
-__device__ __forceinline__ bool cg_step_tile(const CGArgs<T> &a, int par, const int L)
+// u and c are zero off the wavelet masks by construction (b, and with it r, u
+// and D^-1, are).
+template <bool PRE, int LEV>
+__device__ __forceinline__ bool cg_step_tile(const CGArgs &a, int par, const int L)
 {
+    using T = double;
     constexpr int N = LEV + 2;
     __shared__ OpLds<T> s;
     __shared__ double lds[8];
@@ -2377,64 +2448,47 @@ __device__ __forceinline__ bool cg_step_tile(const CGArgs<T> &a, int par, const 
     if (L >= g.nbx * g.nby) return false;
     int bx, by;
     band_tile(g, L, bx, by);
-    const bool has_u = bx < g.nbxu && by < g.nbyu, has_v = bx < g.nbxv && by < g.nbyv;
     const int lx = threadIdx.x & 15, ly = threadIdx.x >> 4, l = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int i0 = bx * TILE, j0 = by * TILE;
-    OpOwn<T> o;
-    op_own_index(g, i0 + lx, j0 + ly, o.oku, o.okv, o.ku, o.kv);
-    const T *pu_old = a.pu[par], *pv_old = a.pv[par];
-    const MaskPacked mask{a.mcu, a.mcv};
+    const CGLayout &Lo = a.Lo;
+    const unsigned at0 = Lo.at(i0, j0), at = at0 + lx + __umul24(Lo.px, (unsigned)ly);
+    const double2 *R = Lo.pair(CG_R), *P = Lo.pair(CG_P + par), *D = Lo.pair(CG_DINV);
     // loads in the order of first use: scalars and partials, the tile's
     // vectors, the coarse halo, the coefficients
     const int it = cg_scalar(&a.st->it[par]);
     const double told = cg_scalar(&a.st->tol), prev_res = cg_scalar(&a.st->res[1 - par]);
-    const T alpha = (T)cg_scalar(&a.st->alpha);
+    const T alpha = cg_scalar(&a.st->alpha);
     double rz = 0.0, prev_rz = 0.0, fold_r, fold_z = 0.0;
     fold_r = lane_fold(a.Pr, g.npart);
     if constexpr (PRE) {
         prev_rz = cg_scalar(&a.st->rz[1 - par]);
         fold_z = lane_fold(a.Pz, g.npart);
     }
-    const T ru = ld_or(o.oku, a.ru, o.ku, T(0)), pu = ld_or(o.oku, pu_old, o.ku, T(0));
-    const T rv = ld_or(o.okv, a.rv, o.kv, T(0)), pv = ld_or(o.okv, pv_old, o.kv, T(0));
-    const T xu = ld_or(o.oku, a.xu, o.ku, T(0)), xv = ld_or(o.okv, a.xv, o.kv, T(0));
-    o.mu = mask.u(o.oku, o.ku);
-    o.mv = mask.v(o.okv, o.kv);
-    double dzu = 0.0, dzv = 0.0;
-    if constexpr (PRE) {
-        dzu = ld_or(o.oku, a.dinvu, o.ku, 0.0);
-        dzv = ld_or(o.okv, a.dinvv, o.kv, 0.0);
+    const double2 r = elem32(R, at), p = elem32(P, at), x = elem32(Lo.pair(CG_X), at);
+    const double2 dz = PRE ? elem32(D, at) : make_double2(0.0, 0.0);
+    const unsigned mb = elem32(Lo.M, at);
+    // the coarse halo, one side per wavefront (left, right, below, above):
+    // line k = l / 16 of N, point l % 16 along it; the fifth line and the
+    // corner blocks (u below right, v above left) in a second round
+    const bool rows = w >= 2, after = (w & 1) != 0;
+    int di, dj;
+    {
+        const int c = haar_halo_offset<LEV>(after, l >> 4), q = l & 15;
+        di = rows ? q : c;
+        dj = rows ? c : q;
     }
-    // the coarse halo: wavefronts 0, 1 the columns left and right of the tile
-    // (u, v) and the corner block, 2, 3 the rows below and above; entry
-    // c = l / 16 + 4 k of 10, point l % 16 along it
-    const bool hv_wave = (w & 1) != 0, rows = w >= 2;
-    const T *hr = hv_wave ? a.rv : a.ru, *hp = hv_wave ? pv_old : pu_old;
-    const uint8_t *hm = hv_wave ? a.mcv : a.mcu;
-    const double *hd = hv_wave ? a.dinvv : a.dinvu;
-    const int hnx = hv_wave ? g.nxv : g.nxu, hny = hv_wave ? g.nyv : g.nyu;
-    T nr[3], np[3];
-    double nd[3];
-    unsigned nm[3];
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-        const int c = (l >> 4) + 4 * k, q = l & 15;
-        int di = rows ? q : haar_halo_offset<LEV>(c), dj = rows ? haar_halo_offset<LEV>(c) : q;
-        bool in = c < 5 ? c < N : (c < 10 && c - 5 < N);
-        if (k == 2 && l >= 32) {  // the corner block: u below right, v above left
-            const int e = l - 32, cx = e % 5, cy = e / 5;
-            di = haar_halo_offset<LEV>(hv_wave ? cx : cx + 5);
-            dj = haar_halo_offset<LEV>(hv_wave ? cy + 5 : cy);
-            in = !rows && e < 25 && cx < N && cy < N;
-        }
-        const int i = i0 + di, j = j0 + dj;
-        const bool ok = in && i >= 0 && i < hnx && j >= 0 && j < hny;
-        nr[k] = ld_or(ok, hr, i + hnx * j, T(0));
-        np[k] = ld_or(ok, hp, i + hnx * j, T(0));
-        nm[k] = ld_or(ok, hm, i + hnx * j, (uint8_t)0);
-        nd[k] = PRE ? ld_or(ok, hd, i + hnx * j, 0.0) : 0.0;
+    const unsigned h0 = at0 + (unsigned)(di + (int)__mul24((int)Lo.px, dj));
+    const double2 nr0 = elem32(R, h0), np0 = elem32(P, h0), nd0 = PRE ? elem32(D, h0) : make_double2(0.0, 0.0);
+    const int e = l - 16, cx = e % 5, cy = e / 5;  // corner entry of lanes 16..40 of wavefronts 0 (v) and 1 (u)
+    const bool corner = w < 2 && e >= 0 && e < 25;
+    {
+        const int c = haar_halo_offset<LEV>(after, 4), q = l & 15;
+        di = corner ? haar_halo_offset<LEV>(after, cx) : (rows ? q : c);
+        dj = corner ? haar_halo_offset<LEV>(!after, cy) : (rows ? c : q);
     }
+    const unsigned h1 = at0 + (unsigned)(di + (int)__mul24((int)Lo.px, dj));
+    const double2 nr1 = elem32(R, h1), np1 = elem32(P, h1), nd1 = PRE ? elem32(D, h1) : make_double2(0.0, 0.0);
     // halo points: wavefront 3 the sides' u, wavefront 2 their v, wavefront 1
     // the corners (u lane 0, v lane 1)
     HaloPos h{17, 0, 0, 17, w == 3 || (w == 1 && l == 0), w == 2 || (w == 1 && l == 1)};
@@ -2443,8 +2497,34 @@ __device__ __forceinline__ bool cg_step_tile(const CGArgs<T> &a, int par, const 
         h.vx = h.ux;
         h.vy = h.uy;
     }
+    OpOwn<T> o;
     OpCoefRegs<T> cr;
-    op_coef_load(g, a.c, mask, i0, j0, h, w >= 1, o, cr);
+    cr.hhu = cr.hhv = 0.0;
+    const double2 oh = elem32(Lo.pair(CG_H), at);
+    unsigned hmb = 0;
+    if (w >= 1) {
+        const int hx = h.hu ? h.ux : h.vx, hy = h.hu ? h.uy : h.vy;
+        const unsigned ha = at0 + (unsigned)(hx - 1 + (int)__mul24((int)Lo.px, hy - 1));
+        cr.hhu = cr.hhv = elem32(reinterpret_cast<const double *>(Lo.pair(CG_H)), 2 * ha + (h.hu ? 0 : 1));
+        hmb = elem32(Lo.M, ha);
+    }
+    const double2 cell = elem32(Lo.pair(CG_CELL), at);
+    o.hetac = elem32(Lo.corner(), at);
+    op_extra_cell(l, cr);
+    if (w == 0) {
+        const unsigned ea = at0 + (unsigned)(cr.ex - 1 + (int)__mul24((int)Lo.px, cr.ey - 1));
+        const double2 ce = elem32(Lo.pair(CG_CELL), ea);
+        cr.ec = elem32(Lo.corner(), ea);
+        cr.eh = ce.x;
+        cr.ed = ce.y;
+    }
+    const double2 ob = elem32(Lo.pair(CG_B), at);
+    o.hu = oh.x;
+    o.hv = oh.y;
+    o.bu = ob.x;
+    o.bv = ob.y;
+    o.heta = cell.x;
+    o.dimp = cell.y;
     double res;
     if constexpr (PRE) {
         double r2 = fold_r;
@@ -2477,42 +2557,43 @@ __device__ __forceinline__ bool cg_step_tile(const CGArgs<T> &a, int par, const 
             }
         }
     }
-    if (alpha != T(0)) {
-        if (o.oku) a.xu[o.ku] = xu + alpha * pu;
-        if (o.okv) a.xv[o.kv] = xv + alpha * pv;
-    }
+    if (alpha != 0.0) elem32(Lo.pair(CG_X), at) = make_double2(x.x + alpha * p.x, x.y + alpha * p.y);
     if (done) return true;
     T beta;
     if constexpr (PRE) {
-        beta = it == 0 ? T(0) : (T)(rz / prev_rz);
+        beta = it == 0 ? T(0) : rz / prev_rz;
     } else {
         const double prev = it == 0 ? 1.0 : prev_res;
-        beta = (T)((res * res) / (prev * prev));
+        beta = (res * res) / (prev * prev);
     }
-    auto direction = [&](T r, T p, double dz) -> T {
+    auto direction = [&](double2 rr, double2 pp, double2 zz) -> double2 {
         if constexpr (PRE)
-            return (T)(dz * (double)r) + beta * p;
+            return make_double2(zz.x * rr.x + beta * pp.x, zz.y * rr.y + beta * pp.y);
         else
-            return r + beta * p;
+            return make_double2(rr.x + beta * pp.x, rr.y + beta * pp.y);
     };
-    const T unu = direction(ru, pu, dzu), unv = direction(rv, pv, dzv);
-    if (o.oku) a.pu[1 - par][o.ku] = unu;
-    if (o.okv) a.pv[1 - par][o.kv] = unv;
-    s.p.t[0][ly][lx] = (o.mu & MB_WAVELET) ? unu : T(0);
-    s.p.t[1][ly][lx] = (o.mv & MB_WAVELET) ? unv : T(0);
+    const double2 un = direction(r, p, dz);
+    elem32(Lo.pair(CG_P + 1 - par), at) = un;
+    s.p.t[0][ly][lx] = un.x;
+    s.p.t[1][ly][lx] = un.y;
     {
-        const int comp = hv_wave ? 1 : 0;
-#pragma unroll
-        for (int k = 0; k < 3; ++k) {
-            const int c = (l >> 4) + 4 * k, q = l & 15;
-            const T x = (nm[k] & MB_WAVELET) ? direction(nr[k], np[k], nd[k]) : T(0);
-            if (k < 2 || l < 32) {
-                if (rows)
-                    s.n.y[comp][c][q] = x;
-                else
-                    s.n.x[comp][c][q] = x;
-            } else if (!rows && l < 57) {
-                (&s.n.c[comp][0][0])[l - 32] = x;
+        const int k = (w & 1) * 5 + (l >> 4), q = l & 15;
+        const double2 n0 = direction(nr0, np0, nd0), n1 = direction(nr1, np1, nd1);
+        if (rows) {
+            s.n.y[0][k][q] = n0.x;
+            s.n.y[1][k][q] = n0.y;
+            if (l < 16) {
+                s.n.y[0][k + 4][q] = n1.x;
+                s.n.y[1][k + 4][q] = n1.y;
+            }
+        } else {
+            s.n.x[0][k][q] = n0.x;
+            s.n.x[1][k][q] = n0.y;
+            if (l < 16) {
+                s.n.x[0][k + 4][q] = n1.x;
+                s.n.x[1][k + 4][q] = n1.y;
+            } else if (corner) {
+                s.n.c[1 - w][cy][cx] = w == 1 ? n1.x : n1.y;
             }
         }
     }
@@ -2535,48 +2616,39 @@ __device__ __forceinline__ bool cg_step_tile(const CGArgs<T> &a, int par, const 
     }
     __syncthreads();
     // x pass: the tile's lines and the halo points
-    T hu = T(0), hv = T(0);
+    T hu = 0.0, hv = 0.0;
     {
         const int q = l & 15, comp = (l >> 4) & 1, half = l >> 5;
         haar_line_P<LEV, T>(&s.p.m[comp][q][0], &s.p.t[comp][q][0], 1, half, w);
         if (w >= 2) {
             const int cp = w == 3 ? 0 : 1, side = (l >> 4) & 1;
-            T x;
+            T y;
             if (l < 32)
-                x = haar_halo_sum<LEV, T>(&s.n.lx[cp][5 * side][q], 17, side != 0);
+                y = haar_halo_sum<LEV, T>(&s.n.lx[cp][5 * side][q], 17, side != 0);
             else
-                x = haar_row_P<LEV, T>(&s.n.ly[cp][side][0], q);
-            hu = (cr.hmu & MB_INNER) ? x : T(0);
-            hv = (cr.hmv & MB_INNER) ? x : T(0);
+                y = haar_row_P<LEV, T>(&s.n.ly[cp][side][0], q);
+            hu = hv = (hmb & (w == 3 ? CB_INNER_U : CB_INNER_V)) ? y : 0.0;
         } else if (w == 1 && l < 2) {
-            const T x = haar_halo_sum<LEV, T>(&s.n.lc[l][0], 1, l == 0);
-            hu = (cr.hmu & MB_INNER) ? x : T(0);
-            hv = (cr.hmv & MB_INNER) ? x : T(0);
+            const T y = haar_halo_sum<LEV, T>(&s.n.lc[l][0], 1, l == 0);
+            hu = hv = (hmb & (l == 0 ? CB_INNER_U : CB_INNER_V)) ? y : 0.0;
         }
     }
     __syncthreads();
-    o.u = (o.mu & MB_INNER) ? s.p.t[0][ly][lx] : T(0);
-    o.v = (o.mv & MB_INNER) ? s.p.t[1][ly][lx] : T(0);
-    op_cells(a.c, h, hu, hv, o, cr, s);
-    s.h.t[0][ly][lx] = (o.mu & MB_INNER) ? op_out_u(a.c, s, o) : T(0);
-    s.h.t[1][ly][lx] = (o.mv & MB_INNER) ? op_out_v(a.c, s, o) : T(0);
+    o.u = (mb & CB_INNER_U) ? s.p.t[0][ly][lx] : 0.0;
+    o.v = (mb & CB_INNER_V) ? s.p.t[1][ly][lx] : 0.0;
+    op_cells(a.rdx, a.rdy, h, hu, hv, o, cr, s);
+    s.h.t[0][ly][lx] = (mb & CB_INNER_U) ? op_out_u(a.rdx, a.rdy, s, o) : 0.0;
+    s.h.t[1][ly][lx] = (mb & CB_INNER_V) ? op_out_v(a.rdx, a.rdy, s, o) : 0.0;
     __syncthreads();
     haar_pair_lev<true, LEV, T>(s.h.t, s.h.m);
-    double du = 0.0, dv = 0.0;
-    if (o.oku) {
-        const T cv = (o.mu & MB_WAVELET) ? s.h.t[0][ly][lx] : T(0);
-        a.qu[o.ku] = cv;
-        du = (double)(unu * cv);
-    }
-    if (o.okv) {
-        const T cv = (o.mv & MB_WAVELET) ? s.h.t[1][ly][lx] : T(0);
-        a.qv[o.kv] = cv;
-        dv = (double)(unv * cv);
-    }
+    const double2 c = make_double2((mb & CB_WAVELET_U) ? s.h.t[0][ly][lx] : 0.0,
+                                   (mb & CB_WAVELET_V) ? s.h.t[1][ly][lx] : 0.0);
+    elem32(Lo.pair(CG_Q), at) = c;
+    double du = un.x * c.x, dv = un.y * c.y;
     tree256x2(du, dv, lds);
     if (threadIdx.x == 0) {
-        if (has_u) a.Pd[bx + g.nbxu * by] = du;
-        if (has_v) a.Pd[g.nbxu * g.nbyu + bx + g.nbxv * by] = dv;
+        if (bx < g.nbxu && by < g.nbyu) a.Pd[bx + g.nbxu * by] = du;
+        if (bx < g.nbxv && by < g.nbyv) a.Pd[g.nbxu * g.nbyu + bx + g.nbxv * by] = dv;
     }
     return false;
 }
@@ -2588,8 +2660,8 @@ __device__ __forceinline__ bool cg_step_tile(const CGArgs<T> &a, int par, const 
 // its partials and the count unchanged (selected by the flag, which is then
 // needed only at the stores), so that the flag's round trip does not precede
 // the loads.
-template <typename T, bool PRE, bool EARLY = true>
-__device__ __forceinline__ void cg_update_tile(const CGArgs<T> &a, int par, const int L)
+template <bool PRE, bool EARLY = true>
+__device__ __forceinline__ void cg_update_tile(const CGArgs &a, int par, const int L)
 {
     __shared__ double lds[8];
     const GridDims &g = a.g;
@@ -2601,66 +2673,53 @@ __device__ __forceinline__ void cg_update_tile(const CGArgs<T> &a, int par, cons
     const bool stopped = !EARLY && cg_scalar(&a.st->done) != 0;
     int bx, by;
     band_tile(g, L, bx, by);
-    const bool has_u = bx < g.nbxu && by < g.nbyu, has_v = bx < g.nbxv && by < g.nbyv;
-    bool oku, okv;
-    int ku, kv;
-    op_own_index(g, bx * TILE + (threadIdx.x & 15), by * TILE + (threadIdx.x >> 4), oku, okv, ku, kv);
+    const unsigned at = a.Lo.at(bx * TILE + (threadIdx.x & 15), by * TILE + (threadIdx.x >> 4));
     const int it = cg_scalar(&a.st->it[par]);
     const double res = cg_scalar(&a.st->res[par]);
     const double fold = lane_fold(a.Pd, g.npart);
-    const T ru = ld_or(oku, a.ru, ku, T(0)), qu = ld_or(oku, a.qu, ku, T(0));
-    const T rv = ld_or(okv, a.rv, kv, T(0)), qv = ld_or(okv, a.qv, kv, T(0));
-    double dzu = 0.0, dzv = 0.0, rzc = 0.0;
-    if constexpr (PRE) {
-        dzu = ld_or(oku, a.dinvu, ku, 0.0);
-        dzv = ld_or(okv, a.dinvv, kv, 0.0);
-        rzc = cg_scalar(&a.st->rz[par]);
-    }
+    const double2 r = elem32(a.Lo.pair(CG_R), at), q = elem32(a.Lo.pair(CG_Q), at);
+    const double2 dz = PRE ? elem32(a.Lo.pair(CG_DINV), at) : make_double2(0.0, 0.0);
+    double rzc = 0.0;
+    if constexpr (PRE) rzc = cg_scalar(&a.st->rz[par]);
     const double dot = tree256(fold, lds);
-    T alpha;
-    if constexpr (PRE)
-        alpha = (T)(rzc / dot);
-    else
-        alpha = (T)((res * res) / dot);
+    const double alpha = (PRE ? rzc : res * res) / dot;
     if (threadIdx.x == 0) {
         a.st->it[1 - par] = stopped ? it : it + 1;
-        a.st->alpha = stopped ? 0.0 : (double)alpha;
+        a.st->alpha = stopped ? 0.0 : alpha;
     }
-    double r2u = 0.0, r2v = 0.0, z2u = 0.0, z2v = 0.0;
-    if (oku) {
-        const T rn = ru - alpha * qu, r = stopped ? ru : rn;
-        a.ru[ku] = r;
-        r2u = (double)r * (double)r;
-        if constexpr (PRE) z2u = (double)r * (dzu * (double)r);
-    }
-    if (okv) {
-        const T rn = rv - alpha * qv, r = stopped ? rv : rn;
-        a.rv[kv] = r;
-        r2v = (double)r * (double)r;
-        if constexpr (PRE) z2v = (double)r * (dzv * (double)r);
-    }
+    double2 rn = make_double2(r.x - alpha * q.x, r.y - alpha * q.y);
+    if (stopped) rn = r;
+    elem32(a.Lo.pair(CG_R), at) = rn;
+    double r2u = rn.x * rn.x, r2v = rn.y * rn.y, z2u = 0.0, z2v = 0.0;
     tree256x2(r2u, r2v, lds);
-    if constexpr (PRE) tree256x2(z2u, z2v, lds);
+    if constexpr (PRE) {
+        z2u = rn.x * (dz.x * rn.x);
+        z2v = rn.y * (dz.y * rn.y);
+        tree256x2(z2u, z2v, lds);
+    }
     if (threadIdx.x == 0) {
-        if (has_u) a.Pr[bx + g.nbxu * by] = r2u;
-        if (has_v) a.Pr[g.nbxu * g.nbyu + bx + g.nbxv * by] = r2v;
-        if constexpr (PRE) {
-            if (has_u) a.Pz[bx + g.nbxu * by] = z2u;
-            if (has_v) a.Pz[g.nbxu * g.nbyu + bx + g.nbxv * by] = z2v;
+        if (bx < g.nbxu && by < g.nbyu) {
+            a.Pr[bx + g.nbxu * by] = r2u;
+            if constexpr (PRE) a.Pz[bx + g.nbxu * by] = z2u;
+        }
+        if (bx < g.nbxv && by < g.nbyv) {
+            const int q2 = g.nbxu * g.nbyu + bx + g.nbxv * by;
+            a.Pr[q2] = r2v;
+            if constexpr (PRE) a.Pz[q2] = z2v;
         }
     }
 }
 
-template <typename T, bool PRE, int LEV>
-__global__ void __launch_bounds__(256) k_cg_step(CGArgs<T> a, int par)
+template <bool PRE, int LEV>
+__global__ void __launch_bounds__(256) k_cg_step(CGArgs a, int par)
 {
-    (void)cg_step_tile<T, PRE, LEV>(a, par, xcd_tile(a.nblk));
+    (void)cg_step_tile<PRE, LEV>(a, par, xcd_tile(a.nblk));
 }
 
-template <typename T, bool PRE, bool EARLY>
-__global__ void __launch_bounds__(256) k_cg_update(CGArgs<T> a, int par)
+template <bool PRE, bool EARLY>
+__global__ void __launch_bounds__(256) k_cg_update(CGArgs a, int par)
 {
-    cg_update_tile<T, PRE, EARLY>(a, par, xcd_tile(a.nblk));
+    cg_update_tile<PRE, EARLY>(a, par, xcd_tile(a.nblk));
 }
 
 // Diagonal of the coarse-CG operator A_c = M_w R M_i A M_i P M_w
@@ -2746,20 +2805,20 @@ __global__ void __launch_bounds__(256) k_coarse_diag(GridDims g, OpCoef<double> 
 // launches per iteration, bit for bit.  Ends at the stop, which every
 // thread of every tile decides alike from the same partials and scalars,
 // after maxiter + 1 iterations at most.
-template <typename T, bool PRE, int LEV>
-__global__ void __launch_bounds__(256) k_cg_solve1(CGArgs<T> a)
+template <bool PRE, int LEV>
+__global__ void __launch_bounds__(256) k_cg_solve1(CGArgs a)
 {
     const int ntile = a.g.nbx * a.g.nby;
     for (int q = 0; q <= a.maxiter; ++q) {
         const int par = q & 1;
         bool stop = false;
         for (int L = 0; L < ntile; ++L) {
-            stop = cg_step_tile<T, PRE, LEV>(a, par, L);
+            stop = cg_step_tile<PRE, LEV>(a, par, L);
             __syncthreads();
         }
         if (stop) break;
         for (int L = 0; L < ntile; ++L) {
-            cg_update_tile<T, PRE>(a, par, L);
+            cg_update_tile<PRE>(a, par, L);
             __syncthreads();
         }
     }
