@@ -1326,15 +1326,38 @@ static void launch_tile_haar(wavi_ctx *ctx, int dir, const T *inu, const T *inv,
 
 // The kernels of the FP64 coarse CG at the context's Haar level,
 // Jacobi-preconditioned inside a linear solve (ctx->cg_pre).
-template <bool PRE>
+// Partials that a lane of the CG's folds loads with the kernels' other
+// inputs: all of them on grids of up to 2048 partials (npart: one per tile
+// and component).
+constexpr int CG_FOLD_LARGE = 8;
+
+template <bool PRE, int FOLD>
 static void launch_cg_step_p(wavi_ctx *ctx, dim3 tb, const CGArgs &a, int par)
 {
     switch (ctx->S.levels) {
-    case 0: hipLaunchKernelGGL((k_cg_step<PRE, 0>), tb, dim3(256), 0, ctx->stream, a, par); break;
-    case 1: hipLaunchKernelGGL((k_cg_step<PRE, 1>), tb, dim3(256), 0, ctx->stream, a, par); break;
-    case 2: hipLaunchKernelGGL((k_cg_step<PRE, 2>), tb, dim3(256), 0, ctx->stream, a, par); break;
-    default: hipLaunchKernelGGL((k_cg_step<PRE, 3>), tb, dim3(256), 0, ctx->stream, a, par); break;
+    case 0: hipLaunchKernelGGL((k_cg_step<PRE, 0, FOLD>), tb, dim3(256), 0, ctx->stream, a, par); break;
+    case 1: hipLaunchKernelGGL((k_cg_step<PRE, 1, FOLD>), tb, dim3(256), 0, ctx->stream, a, par); break;
+    case 2: hipLaunchKernelGGL((k_cg_step<PRE, 2, FOLD>), tb, dim3(256), 0, ctx->stream, a, par); break;
+    default: hipLaunchKernelGGL((k_cg_step<PRE, 3, FOLD>), tb, dim3(256), 0, ctx->stream, a, par); break;
     }
+}
+
+template <bool PRE>
+static void launch_cg_step(wavi_ctx *ctx, dim3 tb, const CGArgs &a, int par)
+{
+    if (ctx->g.npart <= 256)
+        launch_cg_step_p<PRE, 1>(ctx, tb, a, par);
+    else
+        launch_cg_step_p<PRE, CG_FOLD_LARGE>(ctx, tb, a, par);
+}
+
+template <bool PRE, bool EARLY>
+static void launch_cg_update(wavi_ctx *ctx, dim3 tb, const CGArgs &a, int par)
+{
+    if (ctx->g.npart <= 256)
+        hipLaunchKernelGGL((k_cg_update<PRE, EARLY, 1>), tb, dim3(256), 0, ctx->stream, a, par);
+    else
+        hipLaunchKernelGGL((k_cg_update<PRE, EARLY, CG_FOLD_LARGE>), tb, dim3(256), 0, ctx->stream, a, par);
 }
 
 template <bool PRE>
@@ -1406,20 +1429,20 @@ int do_coarse_cg<double>(wavi_ctx *ctx, const VSet<double> &w, int *iters)
             {
                 ProfScope ps(ctx, WAVI_KT_CG_APPLY, sampled);
                 if (pre)
-                    launch_cg_step_p<true>(ctx, tb, a, par);
+                    launch_cg_step<true>(ctx, tb, a, par);
                 else
-                    launch_cg_step_p<false>(ctx, tb, a, par);
+                    launch_cg_step<false>(ctx, tb, a, par);
             }
             {
                 ProfScope ps(ctx, WAVI_KT_CG_UPDATE, sampled);
                 if (pre && early)
-                    hipLaunchKernelGGL((k_cg_update<true, true>), tb, dim3(256), 0, ctx->stream, a, par);
+                    launch_cg_update<true, true>(ctx, tb, a, par);
                 else if (pre)
-                    hipLaunchKernelGGL((k_cg_update<true, false>), tb, dim3(256), 0, ctx->stream, a, par);
+                    launch_cg_update<true, false>(ctx, tb, a, par);
                 else if (early)
-                    hipLaunchKernelGGL((k_cg_update<false, true>), tb, dim3(256), 0, ctx->stream, a, par);
+                    launch_cg_update<false, true>(ctx, tb, a, par);
                 else
-                    hipLaunchKernelGGL((k_cg_update<false, false>), tb, dim3(256), 0, ctx->stream, a, par);
+                    launch_cg_update<false, false>(ctx, tb, a, par);
             }
         }
         burst_end(ctx, bev, q - 1, n);

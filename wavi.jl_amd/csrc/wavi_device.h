@@ -147,19 +147,26 @@ __device__ __forceinline__ double wave_tree(double v)
     return v + lane_down<1>(v);
 }
 
-__device__ __forceinline__ double tree256(double v, double *lds)
+// tree256_open: without the last barrier; lds must not be written again before
+// the next one.
+__device__ __forceinline__ double tree256_open(double v, double *lds)
 {
     const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
     v = wave_tree(v);
     if (l == 0) lds[w] = v;
     __syncthreads();
-    const double r = (lds[0] + lds[2]) + (lds[1] + lds[3]);
+    return (lds[0] + lds[2]) + (lds[1] + lds[3]);
+}
+
+__device__ __forceinline__ double tree256(double v, double *lds)
+{
+    const double r = tree256_open(v, lds);
     __syncthreads();
     return r;
 }
 
 // Two independent trees in one pass.
-__device__ __forceinline__ void tree256x2(double &a, double &b, double *lds)
+__device__ __forceinline__ void tree256x2_open(double &a, double &b, double *lds)
 {
     const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
     a = wave_tree(a);
@@ -171,33 +178,55 @@ __device__ __forceinline__ void tree256x2(double &a, double &b, double *lds)
     __syncthreads();
     a = (lds[0] + lds[2]) + (lds[1] + lds[3]);
     b = (lds[4] + lds[6]) + (lds[5] + lds[7]);
+}
+
+__device__ __forceinline__ void tree256x2(double &a, double &b, double *lds)
+{
+    tree256x2_open(a, b, lds);
     __syncthreads();
 }
 
 // Fold `np` block partials into 256 lanes (lane L = thread L sums P[L],
 // P[L+256], ... in order; missing terms add +0) and sum the lanes with
-// tree256.  Loads are issued unconditionally at clamped indices, one for a
-// small grid, else eight at a time.  Every workgroup that calls this obtains
-// the same bits, in all threads.
+// tree256.  The first K partials of a lane are loaded by load() (no branch,
+// so that other loads can follow before the first is waited for), any more
+// by sum().  Every workgroup that sums the same partials obtains the same
+// bits, in all threads.
+template <int K>
+struct LaneFold {
+    double v[K];
+    __device__ __forceinline__ void load(const double *P, int np)
+    {
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            const unsigned q = threadIdx.x + 256u * k;
+            v[k] = P[q < (unsigned)np ? q : 0u];
+        }
+    }
+    __device__ __forceinline__ double sum(const double *P, int np) const
+    {
+        double acc = (int)threadIdx.x < np ? v[0] : 0.0;
+#pragma unroll
+        for (int k = 1; k < K; ++k) acc = acc + ((int)threadIdx.x + 256 * k < np ? v[k] : 0.0);
+        for (int q0 = 256 * K; q0 < np; q0 += 8 * 256) {
+            double u[8];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                const int q = q0 + (int)threadIdx.x + 256 * k;
+                u[k] = P[q < np ? q : 0];
+            }
+#pragma unroll
+            for (int k = 0; k < 8; ++k) acc = acc + (q0 + (int)threadIdx.x + 256 * k < np ? u[k] : 0.0);
+        }
+        return acc;
+    }
+};
+
 __device__ __forceinline__ double lane_fold(const double *P, int np)
 {
-    const int t = threadIdx.x;
-    if (np <= 256) {
-        const double v = P[t < np ? t : 0];
-        return t < np ? v : 0.0;
-    }
-    double acc = 0.0;
-    for (int q0 = 0; q0 < np; q0 += 8 * 256) {
-        double v[8];
-#pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            const int q = q0 + t + 256 * k;
-            v[k] = P[q < np ? q : 0];
-        }
-#pragma unroll
-        for (int k = 0; k < 8; ++k) acc = acc + (q0 + t + 256 * k < np ? v[k] : 0.0);
-    }
-    return acc;
+    LaneFold<1> f;
+    f.load(P, np);
+    return f.sum(P, np);
 }
 
 __device__ __forceinline__ double lanes_sum(const double *P, int np, double *lds)

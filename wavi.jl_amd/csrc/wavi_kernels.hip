@@ -1002,75 +1002,83 @@ struct HaarMasks {
 };
 __constant__ HaarMasks c_haar[4];
 
+// acc + v or acc - v (neg), with the sign as an exact factor: one instruction,
+// rounded as the addition.
+__device__ __forceinline__ double add_sign(double acc, double v, bool neg) { return __builtin_fma(neg ? -1.0 : 1.0, v, acc); }
+__device__ __forceinline__ float add_sign(float acc, float v, bool neg) { return __builtin_fmaf(neg ? -1.0f : 1.0f, v, acc); }
+
 // One 16-point line of P, the composed inverse of wavelet_matrix
 // (src/Wavelets/update_wavelets.jl:38-89) with blocks of B = 2^(LEV+1)
 // points: y_i = sum over c of P[i][c] x_c, the terms added in increasing
-// column order as the oracle adds them.  Of a pair (o, e = o + h) the column
-// e is -1 on the h rows from o and +1 on the h rows from e, and column 0 of a
-// block is +1 on all its rows, so a row has LEV + 2 terms.  A thread computes
-// rows 2w and 2w + 1 of the half line `half` (8 points): the two rows share
-// all columns and differ in one sign.  z: the half line; with LEV = 3 the
-// block is the whole line, whose columns 0 and 8 come before (second half:
-// x_0 + x_8) and around (first half: x_0 first, -x_8 last) the half's own.
-// w is uniform over a wavefront.  Points past the end of the grid must hold
-// zero: their terms then change nothing, which leaves wavelet_matrix's
-// partial blocks.
+// column order as the oracle adds them.  Row i has the block's column 0 and
+// one column e_h = o + h per pair (o, e_h) that i belongs to, h = 1 .. B/2: +1
+// where i is on the pair's upper half (bit h of i set), else -1.  In
+// increasing order these are the e_h of the set bits, then of the clear ones.
+// A thread computes rows 2w and 2w + 1 of the half line `half` (8 points): the
+// two rows share all columns and differ in one sign.  With LEV = 3 the block
+// is the whole line: its columns 0 and 8 come first in the second half (x_0 +
+// x_8), and in the first half x_0 first and -x_8 last.  w is uniform over a
+// wavefront, so columns and signs are, and the wavefronts share one code;
+// load and rows are apart so that the operands of several lines can be in
+// flight.  Points past the end of the grid must hold zero: their terms then
+// change nothing, which leaves wavelet_matrix's partial blocks.
 template <int LEV, typename T>
-__device__ __forceinline__ void haar_line_P(const T *src, T *dst, int st, int half, int w)
-{
-    const T *z = src + 8 * half * st;
-    T lo, hi;  // rows 2w and 2w + 1
-    if constexpr (LEV == 0) {
-        const T o = z[2 * w * st], e = z[(2 * w + 1) * st];
-        lo = o - e;
-        hi = o + e;
-    } else if constexpr (LEV == 1) {
-        const T o = z[(w & 2) * 2 * st];
-        if ((w & 1) == 0) {
-            const T e = z[((w & 2) * 2 + 1) * st], m = z[((w & 2) * 2 + 2) * st];
-            lo = (o - e) - m;
-            hi = (o + e) - m;
+struct HaarLineP {
+    static constexpr int S = LEV < 2 ? LEV + 1 : 3;  // columns of a row inside the half line
+    T base, x8, v[S];
+    __device__ __forceinline__ void load(const T *src, int st, int half, int w)
+    {
+        const T *z = src + 8 * half * st;
+        x8 = T(0);
+        if constexpr (LEV == 0) {
+            base = z[2 * w * st];
+            v[0] = z[(2 * w + 1) * st];
+        } else if constexpr (LEV == 1) {
+            const int o = 2 * (w & 2);
+            base = z[o * st];
+            v[0] = z[(o + 1 + (w & 1)) * st];
+            v[1] = z[(o + 2 + (w & 1)) * st];
         } else {
-            const T m = z[((w & 2) * 2 + 2) * st], e = z[((w & 2) * 2 + 3) * st];
-            const T b = o + m;
-            lo = b - e;
-            hi = b + e;
+            // columns by w: 1 2 4, 2 3 4, 4 5 6, 4 6 7
+            const int k0 = w == 0 ? 1 : (w == 1 ? 2 : 4);
+            const int k1 = w == 0 ? 2 : (w == 1 ? 3 : (w == 2 ? 5 : 6)), k2 = w < 2 ? 4 : (w == 2 ? 6 : 7);
+            base = LEV == 3 ? src[0] : z[0];
+            if constexpr (LEV == 3) x8 = src[8 * st];
+            v[0] = z[k0 * st];
+            v[1] = z[k1 * st];
+            v[2] = z[k2 * st];
         }
-    } else {
-        T base = src[(LEV == 3 ? 0 : 8 * half) * st], tail = T(0);
+    }
+    __device__ __forceinline__ void rows(T *dst, int st, int half, int w) const
+    {
+        T b = base, tail = T(0);
         if constexpr (LEV == 3) {
-            const T x8 = src[8 * st];
+            b = half ? b + x8 : b;
             tail = half ? T(0) : x8;
-            base = half ? base + x8 : base;
         }
-        if (w == 0) {
-            const T z1 = z[st], z2 = z[2 * st], z4 = z[4 * st];
-            lo = ((base - z1) - z2) - z4;
-            hi = ((base + z1) - z2) - z4;
-        } else if (w == 1) {
-            const T z2 = z[2 * st], z3 = z[3 * st], z4 = z[4 * st];
-            const T b = base + z2;
-            lo = (b - z3) - z4;
-            hi = (b + z3) - z4;
-        } else if (w == 2) {
-            const T z4 = z[4 * st], z5 = z[5 * st], z6 = z[6 * st];
-            const T b = base + z4;
-            lo = (b - z5) - z6;
-            hi = (b + z5) - z6;
-        } else {
-            const T z4 = z[4 * st], z6 = z[6 * st], z7 = z[7 * st];
-            const T b = (base + z4) + z6;
-            lo = b - z7;
-            hi = b + z7;
+        const int plus = LEV == 0 ? 0 : (LEV == 1 ? (w & 1) : (w & 1) + (w >> 1));  // + signs of row 2w
+        T lo = b, hi = b;
+#pragma unroll
+        for (int k = 0; k < S; ++k) {
+            lo = add_sign(lo, v[k], k >= plus);
+            hi = add_sign(hi, v[k], k >= plus + 1);
         }
         if constexpr (LEV == 3) {
             lo = lo - tail;
             hi = hi - tail;
         }
+        T *d = dst + (8 * half + 2 * w) * st;
+        d[0] = lo;
+        d[st] = hi;
     }
-    T *d = dst + (8 * half + 2 * w) * st;
-    d[0] = lo;
-    d[st] = hi;
+};
+
+template <int LEV, typename T>
+__device__ __forceinline__ void haar_line_P(const T *src, T *dst, int st, int half, int w)
+{
+    HaarLineP<LEV, T> p;
+    p.load(src, st, half, w);
+    p.rows(dst, st, half, w);
 }
 
 // One 16-point line of R = P^T: row o + h of a pair is -1 on the h points
@@ -1387,12 +1395,26 @@ struct OpLds {
     };
 };
 
+// Intermediates of one cell.
+template <typename T>
+struct OpCell {
+    T rxx, ryy, ext, rxy;
+    __device__ __forceinline__ void store(OpLds<T> &s, int x, int y) const
+    {
+        s.rxx[y][x] = rxx;
+        s.ryy[y][x] = ryy;
+        s.ext[y][x] = ext;
+        s.rxy[y][x] = rxy;
+    }
+};
+
 // What a thread holds of its tile.  The thicknesses and drags are zero off the
 // u and v masks (an inner point is on its mask).
 template <typename T>
 struct OpOwn {
     T u, v, hu, hv, bu, bv;
     T heta, dimp, hetac;
+    OpCell<T> cell;   // the intermediates of its cell
     unsigned mu, mv;  // mask bits
     bool oku, okv;
     int ku, kv;
@@ -1413,19 +1435,18 @@ __device__ __forceinline__ void op_cell_load(const GridDims &g, const OpCoef<T> 
 // Intermediates of cell (x, y) (the expressions of op_rxx, op_ryy, op_extra,
 // op_rxy).  Cell (0, 0) reads one absent window point of each kind and corner
 // (16, 16) another; no output reads what they feed.
+// u, v, qx, qy: the window at (x, y)
 template <typename T>
-__device__ __forceinline__ void op_cell(T rdx, T rdy, OpLds<T> &s, int x, int y, T heta, T dimp, T hetac)
+__device__ __forceinline__ OpCell<T> op_cell(T rdx, T rdy, const OpLds<T> &s, int x, int y, T u, T v, T qx, T qy,
+                                             T heta, T dimp, T hetac)
 {
-    const T u0 = s.w.U[y][x], u1 = s.w.U[y][x + 1], v0 = s.w.V[y][x], v1 = s.w.V[y + 1][x];
-    const T dudx = rdx * u1 - rdx * u0;
-    const T dvdy = rdy * v1 - rdy * v0;
-    const T divq = (rdx * s.w.QX[y][x + 1] - rdx * s.w.QX[y][x]) + (rdy * s.w.QY[y + 1][x] - rdy * s.w.QY[y][x]);
+    const T u1 = s.w.U[y][x + 1], v1 = s.w.V[y + 1][x];
+    const T dudx = rdx * u1 - rdx * u;
+    const T dvdy = rdy * v1 - rdy * v;
+    const T divq = (rdx * s.w.QX[y][x + 1] - rdx * qx) + (rdy * s.w.QY[y + 1][x] - rdy * qy);
     const T dudy = rdy * s.w.U[y + 1][x + 1] - rdy * u1;
     const T dvdx = rdx * s.w.V[y + 1][x + 1] - rdx * v1;
-    s.rxx[y][x] = T(2) * (heta * (T(2) * dudx + dvdy));
-    s.ryy[y][x] = T(2) * (heta * (T(2) * dvdy + dudx));
-    s.ext[y][x] = dimp * divq;
-    s.rxy[y][x] = hetac * (dudy + dvdx);
+    return {T(2) * (heta * (T(2) * dudx + dvdy)), T(2) * (heta * (T(2) * dvdy + dudx)), dimp * divq, hetac * (dudy + dvdx)};
 }
 
 // Halo points a thread stages: u at (ux, uy) and v at (vx, vy) of the window.
@@ -1468,7 +1489,7 @@ struct OpCoefRegs {
 template <typename T>
 __device__ __forceinline__ void op_extra_cell(int l, OpCoefRegs<T> &r)
 {
-    r.ex = l < 17 ? 0 : l - 16;
+    r.ex = l < 17 ? 0 : (l < 33 ? l - 16 : 16);
     r.ey = l < 17 ? l : 0;
     r.eh = r.ed = r.ec = T(0);
 }
@@ -1491,7 +1512,7 @@ __device__ __forceinline__ void op_coef_load(const GridDims &g, const OpCoef<T> 
     }
     op_cell_load(g, c, i0 + lx, j0 + ly, o.heta, o.dimp, o.hetac);
     op_extra_cell(l, r);
-    if (w == 0) op_cell_load(g, c, l < 33 ? i0 - 1 + r.ex : -1, j0 - 1 + r.ey, r.eh, r.ed, r.ec);
+    if (w == 0) op_cell_load(g, c, i0 - 1 + r.ex, j0 - 1 + r.ey, r.eh, r.ed, r.ec);
     const T obu = ld_or(o.oku, c.bu, o.ku, T(0)), obv = ld_or(o.okv, c.bv, o.kv, T(0));
     o.hu = (o.mu & MB_POINT) ? ohu : T(0);
     o.hv = (o.mv & MB_POINT) ? ohv : T(0);
@@ -1503,14 +1524,15 @@ __device__ __forceinline__ void op_coef_load(const GridDims &g, const OpCoef<T> 
 // compute the cells' intermediates.  Ends with a barrier, after which the
 // window is free.
 template <typename T>
-__device__ __forceinline__ void op_cells(T rdx, T rdy, const HaloPos &h, T hu, T hv, const OpOwn<T> &o,
+__device__ __forceinline__ void op_cells(T rdx, T rdy, const HaloPos &h, T hu, T hv, OpOwn<T> &o,
                                          const OpCoefRegs<T> &r, OpLds<T> &s)
 {
     const int lx = threadIdx.x & 15, ly = threadIdx.x >> 4;
     s.w.U[ly + 1][lx + 1] = o.u;
     s.w.V[ly + 1][lx + 1] = o.v;
-    s.w.QX[ly + 1][lx + 1] = o.hu * o.u;
-    s.w.QY[ly + 1][lx + 1] = o.hv * o.v;
+    const T qx = o.hu * o.u, qy = o.hv * o.v;
+    s.w.QX[ly + 1][lx + 1] = qx;
+    s.w.QY[ly + 1][lx + 1] = qy;
     if (h.hu) {
         s.w.U[h.uy][h.ux] = hu;
         s.w.QX[h.uy][h.ux] = r.hhu * hu;
@@ -1520,8 +1542,14 @@ __device__ __forceinline__ void op_cells(T rdx, T rdy, const HaloPos &h, T hu, T
         s.w.QY[h.vy][h.vx] = r.hhv * hv;
     }
     __syncthreads();
-    op_cell(rdx, rdy, s, lx + 1, ly + 1, o.heta, o.dimp, o.hetac);
-    if (threadIdx.x < 33) op_cell(rdx, rdy, s, r.ex, r.ey, r.eh, r.ed, r.ec);
+    o.cell = op_cell(rdx, rdy, s, lx + 1, ly + 1, o.u, o.v, qx, qy, o.heta, o.dimp, o.hetac);
+    if (__builtin_amdgcn_readfirstlane(threadIdx.x) == 0) {
+        // lanes past the 33 cells before the tile repeat the last
+        const OpCell<T> first = op_cell(rdx, rdy, s, r.ex, r.ey, s.w.U[r.ey][r.ex], s.w.V[r.ey][r.ex],
+                                        s.w.QX[r.ey][r.ex], s.w.QY[r.ey][r.ex], r.eh, r.ed, r.ec);
+        first.store(s, r.ex, r.ey);
+    }
+    o.cell.store(s, lx + 1, ly + 1);
     __syncthreads();
 }
 
@@ -1562,10 +1590,10 @@ template <typename T>
 __device__ __forceinline__ T op_out_u(T rdx, T rdy, const OpLds<T> &s, const OpOwn<T> &o)
 {
     const int x = threadIdx.x & 15, y = threadIdx.x >> 4;
-    const T d_rxx_dx = rdx * s.rxx[y + 1][x + 1] - rdx * s.rxx[y + 1][x];
+    const T d_rxx_dx = rdx * o.cell.rxx - rdx * s.rxx[y + 1][x];
     const T d_rxy_dy = rdy * s.rxy[y + 1][x] - rdy * s.rxy[y][x];
     const T taubx = o.bu * o.u;
-    const T d_extra_dx = rdx * s.ext[y + 1][x + 1] - rdx * s.ext[y + 1][x];
+    const T d_extra_dx = rdx * o.cell.ext - rdx * s.ext[y + 1][x];
     return ((d_rxx_dx + d_rxy_dy) - taubx) - o.hu * d_extra_dx;
 }
 
@@ -1573,10 +1601,10 @@ template <typename T>
 __device__ __forceinline__ T op_out_v(T rdx, T rdy, const OpLds<T> &s, const OpOwn<T> &o)
 {
     const int x = threadIdx.x & 15, y = threadIdx.x >> 4;
-    const T d_ryy_dy = rdy * s.ryy[y + 1][x + 1] - rdy * s.ryy[y][x + 1];
+    const T d_ryy_dy = rdy * o.cell.ryy - rdy * s.ryy[y][x + 1];
     const T d_rxy_dx = rdx * s.rxy[y][x + 1] - rdx * s.rxy[y][x];
     const T tauby = o.bv * o.v;
-    const T d_extra_dy = rdy * s.ext[y + 1][x + 1] - rdy * s.ext[y][x + 1];
+    const T d_extra_dy = rdy * o.cell.ext - rdy * s.ext[y][x + 1];
     return ((d_ryy_dy + d_rxy_dx) - tauby) - o.hv * d_extra_dy;
 }
 
@@ -2388,35 +2416,58 @@ __device__ __forceinline__ int haar_halo_offset(bool after, int k)
     return after ? 16 + ((1 << k) >> 1) : -((2 << LEV) >> k);
 }
 
-// The row of P that haar_halo_offset's terms v[0..N) (stride st) make: the
-// last point of a block (neg = false) or its first.
+// A row of P on the terms at v + off[0..N): + for the first `plus` details,
+// then -.
 template <int LEV, typename T>
-__device__ __forceinline__ T haar_halo_sum(const T *v, int st, bool neg)
-{
+struct HaarRow {
     T x[LEV + 2];
+    __device__ __forceinline__ void load(const T *v, const int (&off)[LEV + 2])
+    {
 #pragma unroll
-    for (int k = 0; k < LEV + 2; ++k) x[k] = v[k * st];
-    T a = x[0];
+        for (int k = 0; k < LEV + 2; ++k) x[k] = v[off[k]];
+    }
+    __device__ __forceinline__ T sum(int plus) const
+    {
+        T a = x[0];
 #pragma unroll
-    for (int k = 1; k < LEV + 2; ++k) a = a + (neg ? -x[k] : x[k]);
-    return a;
+        for (int k = 0; k <= LEV; ++k) a = add_sign(a, x[k + 1], k >= plus);
+        return a;
+    }
+};
+
+// The terms of haar_halo_offset (stride st): the last point of a block (all +)
+// or its first (all -).
+template <int LEV>
+__device__ __forceinline__ void haar_halo_terms(int st, int (&off)[LEV + 2])
+{
+#pragma unroll
+    for (int k = 0; k < LEV + 2; ++k) off[k] = k * st;
 }
 
-// Row i of P on a 16-point line: x_0 of the block, then in increasing column
-// order the details e_h = (i's pair point at distance h) of the set bits of i
-// (h descending, +1) and of the clear bits (h ascending, -1).
-template <int LEV, typename T>
-__device__ __forceinline__ T haar_row_P(const T *src, int i)
+// The terms of row i of a 16-point line in increasing column order: the
+// block's first, the e_h of i's set bits (h descending), then of its clear
+// bits (h ascending).  Returns the number of set bits.
+template <int LEV>
+__device__ __forceinline__ int haar_row_terms(int i, int (&off)[LEV + 2])
 {
-    T d[LEV + 1];
+    off[0] = i & ~((2 << LEV) - 1);
+    int plus = 0;
 #pragma unroll
-    for (int k = 0; k <= LEV; ++k) d[k] = src[(i & ~((2 << k) - 1)) + (1 << k)];
-    T a = src[i & ~((2 << LEV) - 1)];
+    for (int h = 0; h <= LEV; ++h) plus += (i >> h) & 1;
+    int up = 0;
 #pragma unroll
-    for (int k = LEV; k >= 0; --k) a = (i >> k) & 1 ? a + d[k] : a;
+    for (int k = 1; k < LEV + 2; ++k) off[k] = 0;
 #pragma unroll
-    for (int k = 0; k <= LEV; ++k) a = (i >> k) & 1 ? a : a - d[k];
-    return a;
+    for (int h = LEV; h >= 0; --h) {  // slot of e_h: set bits count down from h = LEV, clear bits come last in reverse
+        const bool set = (i >> h) & 1;
+        const int e = (i & ~((2 << h) - 1)) + (1 << h);
+        const int clear_below = h - (plus - up - (set ? 1 : 0));  // clear bits under h
+        const int slot = 1 + (set ? up : plus + clear_below);
+#pragma unroll
+        for (int k = 1; k < LEV + 2; ++k) off[k] = slot == k ? e : off[k];
+        up += set ? 1 : 0;
+    }
+    return plus;
 }
 
 // part 1 (iteration parity par): residual norm and stop test; x += alpha u
@@ -2437,13 +2488,13 @@ __device__ __forceinline__ T haar_row_P(const T *src, int i)
 // iteration had a third kernel boundary (at least 2.5 us on this chip).
 // u and c are zero off the wavelet masks by construction (b, and with it r, u
 // and D^-1, are).
-template <bool PRE, int LEV>
+template <bool PRE, int LEV, int FOLD>
 __device__ __forceinline__ bool cg_step_tile(const CGArgs &a, int par, const int L)
 {
     using T = double;
     constexpr int N = LEV + 2;
     __shared__ OpLds<T> s;
-    __shared__ double lds[8];
+    __shared__ double lds[20];  // a slot per sum
     const GridDims &g = a.g;
     if (L >= g.nbx * g.nby) return false;
     int bx, by;
@@ -2459,11 +2510,12 @@ __device__ __forceinline__ bool cg_step_tile(const CGArgs &a, int par, const int
     const int it = cg_scalar(&a.st->it[par]);
     const double told = cg_scalar(&a.st->tol), prev_res = cg_scalar(&a.st->res[1 - par]);
     const T alpha = cg_scalar(&a.st->alpha);
-    double rz = 0.0, prev_rz = 0.0, fold_r, fold_z = 0.0;
-    fold_r = lane_fold(a.Pr, g.npart);
+    double rz = 0.0, prev_rz = 0.0;
+    LaneFold<FOLD> fr, fz;
+    fr.load(a.Pr, g.npart);
     if constexpr (PRE) {
         prev_rz = cg_scalar(&a.st->rz[1 - par]);
-        fold_z = lane_fold(a.Pz, g.npart);
+        fz.load(a.Pz, g.npart);
     }
     const double2 r = elem32(R, at), p = elem32(P, at), x = elem32(Lo.pair(CG_X), at);
     const double2 dz = PRE ? elem32(D, at) : make_double2(0.0, 0.0);
@@ -2525,18 +2577,26 @@ __device__ __forceinline__ bool cg_step_tile(const CGArgs &a, int par, const int
     o.bv = ob.y;
     o.heta = cell.x;
     o.dimp = cell.y;
+    // the halo point's terms in the x pass (wavefronts 2, 3)
+    int hoff[N], hplus;
+    if (l < 32) {
+        haar_halo_terms<LEV>(17, hoff);
+        hplus = l < 16 ? LEV + 1 : 0;
+    } else {
+        hplus = haar_row_terms<LEV>(l & 15, hoff);
+    }
     double res;
     if constexpr (PRE) {
-        double r2 = fold_r;
-        rz = fold_z;
-        tree256x2(r2, rz, lds);
+        double r2 = fr.sum(a.Pr, g.npart);
+        rz = fz.sum(a.Pz, g.npart);
+        tree256x2_open(r2, rz, lds);
         res = sqrt(r2);
     } else {
-        res = sqrt(tree256(fold_r, lds));
+        res = sqrt(tree256_open(fr.sum(a.Pr, g.npart), lds));
     }
     double tol;
     if (it == 0) {
-        const double abstol = a.tol_coarse * sqrt(lanes_sum(a.Pb, g.npart, lds));
+        const double abstol = a.tol_coarse * sqrt(tree256_open(lane_fold(a.Pb, g.npart), lds + 8));
         tol = a.reltol * res;
         if (abstol > tol) tol = abstol;
     } else {
@@ -2598,39 +2658,53 @@ __device__ __forceinline__ bool cg_step_tile(const CGArgs &a, int par, const int
         }
     }
     __syncthreads();
-    // y pass: the tile's lines; the columns' lines (lanes 0..39, a half line
-    // each); rows -1 and 16 of the neighbours below and above; the corners
+    // y pass: the tile's lines; the columns' lines (40 half lines; lanes
+    // 40..63 repeat the first); rows -1 and 16 of the neighbours below and
+    // above (lanes 0..15) and the corners (16..20 of wavefronts 0, 1).  The
+    // operands of all three are read before the first is used.
     {
         const int q = l & 15, comp = (l >> 4) & 1, half = l >> 5;
-        haar_line_P<LEV, T>(&s.p.t[comp][0][q], &s.p.m[comp][0][q], TILE + 1, half, w);
-        if (l < 40) {
-            const int line = l < 20 ? l : l - 20, lh = l < 20 ? 0 : 1;
-            haar_line_P<LEV, T>(&s.n.x[0][0][0] + 17 * line, &s.n.lx[0][0][0] + 17 * line, 1, lh, w);
-        }
-        if (l < 16) {
-            const int cp = w & 1, side = w >> 1;
-            s.n.ly[cp][side][l] = haar_halo_sum<LEV, T>(&s.n.y[cp][5 * side][l], 16, side != 0);
-        } else if (w < 2 && l < 21) {
-            s.n.lc[w][l - 16] = haar_halo_sum<LEV, T>(&s.n.c[w][0][l - 16], 5, w == 1);
-        }
+        const int hl = l < 40 ? l : l - 40, line = hl < 20 ? hl : hl - 20, lh = hl < 20 ? 0 : 1;
+        const int cp = w & 1, side = w >> 1;
+        const bool edge = l < 16;
+        const T *se = edge ? &s.n.y[cp][5 * side][l] : &s.n.c[cp][0][l < 20 ? l - 16 : 4];
+        int off[N];
+        haar_halo_terms<LEV>(edge ? 16 : 5, off);
+        HaarLineP<LEV, T> own, hal;
+        HaarRow<LEV, T> row;
+        own.load(&s.p.t[comp][0][q], TILE + 1, half, w);
+        hal.load(&s.n.x[0][0][0] + 17 * line, 1, lh, w);
+        row.load(se, off);
+        own.rows(&s.p.m[comp][0][q], TILE + 1, half, w);
+        hal.rows(&s.n.lx[0][0][0] + 17 * line, 1, lh, w);
+        const T y = row.sum((edge ? side != 0 : w == 1) ? 0 : LEV + 1);
+        if (edge)
+            s.n.ly[cp][side][l] = y;
+        else if (w < 2 && l < 21)
+            s.n.lc[w][l - 16] = y;
     }
     __syncthreads();
     // x pass: the tile's lines and the halo points
     T hu = 0.0, hv = 0.0;
     {
         const int q = l & 15, comp = (l >> 4) & 1, half = l >> 5;
-        haar_line_P<LEV, T>(&s.p.m[comp][q][0], &s.p.t[comp][q][0], 1, half, w);
+        HaarLineP<LEV, T> own;
+        own.load(&s.p.m[comp][q][0], 1, half, w);
         if (w >= 2) {
             const int cp = w == 3 ? 0 : 1, side = (l >> 4) & 1;
-            T y;
-            if (l < 32)
-                y = haar_halo_sum<LEV, T>(&s.n.lx[cp][5 * side][q], 17, side != 0);
-            else
-                y = haar_row_P<LEV, T>(&s.n.ly[cp][side][0], q);
+            HaarRow<LEV, T> row;
+            row.load(l < 32 ? &s.n.lx[cp][5 * side][q] : &s.n.ly[cp][side][0], hoff);
+            own.rows(&s.p.t[comp][q][0], 1, half, w);
+            const T y = row.sum(hplus);
             hu = hv = (hmb & (w == 3 ? CB_INNER_U : CB_INNER_V)) ? y : 0.0;
-        } else if (w == 1 && l < 2) {
-            const T y = haar_halo_sum<LEV, T>(&s.n.lc[l][0], 1, l == 0);
-            hu = hv = (hmb & (l == 0 ? CB_INNER_U : CB_INNER_V)) ? y : 0.0;
+        } else {
+            int off[N];
+            haar_halo_terms<LEV>(1, off);
+            HaarRow<LEV, T> row;
+            row.load(&s.n.lc[l == 0 ? 0 : 1][0], off);
+            own.rows(&s.p.t[comp][q][0], 1, half, w);
+            const T y = row.sum(l == 0 ? 0 : LEV + 1);
+            hu = hv = (hmb & (l == 0 ? CB_INNER_U : CB_INNER_V)) ? y : 0.0;  // staged by wavefront 1's lanes 0, 1
         }
     }
     __syncthreads();
@@ -2645,7 +2719,7 @@ __device__ __forceinline__ bool cg_step_tile(const CGArgs &a, int par, const int
                                    (mb & CB_WAVELET_V) ? s.h.t[1][ly][lx] : 0.0);
     elem32(Lo.pair(CG_Q), at) = c;
     double du = un.x * c.x, dv = un.y * c.y;
-    tree256x2(du, dv, lds);
+    tree256x2_open(du, dv, lds + 12);
     if (threadIdx.x == 0) {
         if (bx < g.nbxu && by < g.nbyu) a.Pd[bx + g.nbxu * by] = du;
         if (bx < g.nbxv && by < g.nbyv) a.Pd[g.nbxu * g.nbyu + bx + g.nbxv * by] = dv;
@@ -2660,10 +2734,10 @@ __device__ __forceinline__ bool cg_step_tile(const CGArgs &a, int par, const int
 // its partials and the count unchanged (selected by the flag, which is then
 // needed only at the stores), so that the flag's round trip does not precede
 // the loads.
-template <bool PRE, bool EARLY = true>
+template <bool PRE, bool EARLY, int FOLD>
 __device__ __forceinline__ void cg_update_tile(const CGArgs &a, int par, const int L)
 {
-    __shared__ double lds[8];
+    __shared__ double lds[20];  // a slot per sum
     const GridDims &g = a.g;
     if (L >= g.nbx * g.nby) return;
     if (EARLY && a.st->done) {
@@ -2676,12 +2750,13 @@ __device__ __forceinline__ void cg_update_tile(const CGArgs &a, int par, const i
     const unsigned at = a.Lo.at(bx * TILE + (threadIdx.x & 15), by * TILE + (threadIdx.x >> 4));
     const int it = cg_scalar(&a.st->it[par]);
     const double res = cg_scalar(&a.st->res[par]);
-    const double fold = lane_fold(a.Pd, g.npart);
+    LaneFold<FOLD> fd;
+    fd.load(a.Pd, g.npart);
     const double2 r = elem32(a.Lo.pair(CG_R), at), q = elem32(a.Lo.pair(CG_Q), at);
     const double2 dz = PRE ? elem32(a.Lo.pair(CG_DINV), at) : make_double2(0.0, 0.0);
     double rzc = 0.0;
     if constexpr (PRE) rzc = cg_scalar(&a.st->rz[par]);
-    const double dot = tree256(fold, lds);
+    const double dot = tree256_open(fd.sum(a.Pd, g.npart), lds);
     const double alpha = (PRE ? rzc : res * res) / dot;
     if (threadIdx.x == 0) {
         a.st->it[1 - par] = stopped ? it : it + 1;
@@ -2691,11 +2766,11 @@ __device__ __forceinline__ void cg_update_tile(const CGArgs &a, int par, const i
     if (stopped) rn = r;
     elem32(a.Lo.pair(CG_R), at) = rn;
     double r2u = rn.x * rn.x, r2v = rn.y * rn.y, z2u = 0.0, z2v = 0.0;
-    tree256x2(r2u, r2v, lds);
+    tree256x2_open(r2u, r2v, lds + 4);
     if constexpr (PRE) {
         z2u = rn.x * (dz.x * rn.x);
         z2v = rn.y * (dz.y * rn.y);
-        tree256x2(z2u, z2v, lds);
+        tree256x2_open(z2u, z2v, lds + 12);
     }
     if (threadIdx.x == 0) {
         if (bx < g.nbxu && by < g.nbyu) {
@@ -2710,16 +2785,16 @@ __device__ __forceinline__ void cg_update_tile(const CGArgs &a, int par, const i
     }
 }
 
-template <bool PRE, int LEV>
+template <bool PRE, int LEV, int FOLD>
 __global__ void __launch_bounds__(256) k_cg_step(CGArgs a, int par)
 {
-    (void)cg_step_tile<PRE, LEV>(a, par, xcd_tile(a.nblk));
+    (void)cg_step_tile<PRE, LEV, FOLD>(a, par, xcd_tile(a.nblk));
 }
 
-template <bool PRE, bool EARLY>
+template <bool PRE, bool EARLY, int FOLD>
 __global__ void __launch_bounds__(256) k_cg_update(CGArgs a, int par)
 {
-    cg_update_tile<PRE, EARLY>(a, par, xcd_tile(a.nblk));
+    cg_update_tile<PRE, EARLY, FOLD>(a, par, xcd_tile(a.nblk));
 }
 
 // Diagonal of the coarse-CG operator A_c = M_w R M_i A M_i P M_w
@@ -2813,12 +2888,12 @@ __global__ void __launch_bounds__(256) k_cg_solve1(CGArgs a)
         const int par = q & 1;
         bool stop = false;
         for (int L = 0; L < ntile; ++L) {
-            stop = cg_step_tile<PRE, LEV>(a, par, L);
+            stop = cg_step_tile<PRE, LEV, 1>(a, par, L);
             __syncthreads();
         }
         if (stop) break;
         for (int L = 0; L < ntile; ++L) {
-            cg_update_tile<PRE>(a, par, L);
+            cg_update_tile<PRE, true, 1>(a, par, L);
             __syncthreads();
         }
     }
