@@ -102,13 +102,13 @@ struct wavi_ctx {
     VSet<float> v32;
     // mixed-precision coarse CG: s, w, the parity-buffered images P r, P s,
     // P w and partials of (r, r) and (w, r)
-    // mixed coarse CG: one FP32 arena (enum CGMArray) and a mask-byte arena
+    // mixed coarse CG: one FP32 arena (enum CGMPair) and a mask-byte arena
     // in the padded layout of pitch px and array stride ns
-    float *arena = nullptr;
+    float2 *arena = nullptr;
     uint8_t *marena = nullptr;
     unsigned px = 0, ns = 0;
     float2 *Pgd = nullptr;  // [2][npad] (r, r) and (w, r) partials by parity
-    float *rings = nullptr; // ring images [2][tiles + 1][3][2][64]
+    float *rings = nullptr; // ring images: [2][tiles + 1][64] float4, then as many float2 (CGMRings)
     int npad = 0;
     CGMScalars *stm = nullptr;
     CGMHostFlag *h_flag = nullptr;  // pinned, host-mapped stop report of the mixed coarse CG
@@ -663,7 +663,7 @@ int wavi_ctx_create(const wavi_grid_desc *grid, const wavi_phys_params *phys, co
     for (hipEvent_t &e : ctx->ev_tune) CREATECHK(hipEventCreate(&e));
     CREATECHK(hipEventCreateWithFlags(&ctx->ev_ls_done, hipEventDisableTiming));
     if (precision_mode == WAVI_PRECISION_FP64) {
-        const size_t px = (size_t)TILE * (g.nbx + 2), ns = px * TILE * (g.nby + 2);
+        const size_t px = (size_t)TILE * (g.nbx + 1), ns = px * TILE * (g.nby + 2);
         if (ns * sizeof(double2) > UINT32_MAX) {
             ctx->err = "grid too large for the coarse solver's 32-bit offsets";
             return fail(WAVI_EARG);
@@ -690,13 +690,14 @@ int wavi_ctx_create(const wavi_grid_desc *grid, const wavi_phys_params *phys, co
             CREATECHK(falloc(&dv->u, ctx->nu));
             CREATECHK(falloc(&dv->v, ctx->nv));
         }
-        ctx->px = (unsigned)((TILE * g.nbx + 2 + 31) / 32 * 32);
-        ctx->ns = ctx->px * (unsigned)(TILE * g.nby + 2);
-        CREATECHK(falloc(&ctx->arena, (size_t)CGM_NARRAY * ctx->ns));
-        CREATECHK(hipMalloc(&ctx->marena, 2 * (size_t)ctx->ns));
-        CREATECHK(hipMemset(ctx->marena, 0, 2 * (size_t)ctx->ns));
+        ctx->px = (unsigned)(TILE * (g.nbx + 1));
+        ctx->ns = ctx->px * (unsigned)(TILE * g.nby + 3);
+        CREATECHK(hipMalloc(&ctx->arena, (2 * CGM_NPAIR + 1) * (size_t)ctx->ns * sizeof(float)));
+        CREATECHK(hipMemset(ctx->arena, 0, (2 * CGM_NPAIR + 1) * (size_t)ctx->ns * sizeof(float)));
+        CREATECHK(hipMalloc(&ctx->marena, ctx->ns));
+        CREATECHK(hipMemset(ctx->marena, 0, ctx->ns));
         ctx->npad = (g.nbx * g.nby + 1023) / 1024 * 1024;
-        CREATECHK(falloc(&ctx->rings, 2 * (size_t)(g.nbx * g.nby + 1) * 6 * 64));
+        CREATECHK(falloc(&ctx->rings, 2 * (size_t)(g.nbx * g.nby + 1) * 64 * 6));
         CREATECHK(hipMalloc(&ctx->Pgd, 2 * (size_t)ctx->npad * sizeof(float2)));
         CREATECHK(hipMemset(ctx->Pgd, 0, 2 * (size_t)ctx->npad * sizeof(float2)));
         CREATECHK(hipMalloc(&ctx->stm, sizeof(CGMScalars)));
@@ -1503,12 +1504,21 @@ static void launch_cgm_iter(wavi_ctx *ctx, dim3 tb, const CGMIterArgs &a)
         launch_cgm_iter_p<PAR, INIT, false>(ctx, tb, a);
 }
 
+static CGMRings cgm_rings(const wavi_ctx *ctx)
+{
+    const size_t n = 2 * (size_t)(ctx->g.nbx * ctx->g.nby + 1) * 64;
+    CGMRings R;
+    R.rs = reinterpret_cast<float4 *>(ctx->rings);
+    R.w = reinterpret_cast<float2 *>(ctx->rings + 4 * n);
+    return R;
+}
+
 // The arguments of k_cgm_iter, fixed for the context.
 static CGMIterArgs cgm_iter_args(wavi_ctx *ctx)
 {
     CGMIterArgs ia;
     ia.Lo = cgm_layout(ctx);
-    ia.R = ctx->rings;
+    ia.R = cgm_rings(ctx);
     ia.Pgd = ctx->Pgd;
     ia.st = ctx->stm;
     ia.hflag = ctx->d_flag;
@@ -1529,61 +1539,60 @@ static CGMIterArgs cgm_iter_args(wavi_ctx *ctx)
     return ia;
 }
 
-// Set-up of the mixed coarse CG on b_c in w.cr with the warm start w.xc:
-// coefficients and masks into the arena, P x0, r0 = b - A_c x0, the
-// scalars and the host stop report reset.
-static int cgm_prepare(wavi_ctx *ctx, const VSet<float> &w)
+static CGMArgs cgm_args(wavi_ctx *ctx, const VSet<float> &w)
 {
-    const GridDims &g = ctx->g;
-    dim3 tg(g.nbx, g.nby), tb(ctx->nblk);
-    const CGMLayout Lo = cgm_layout(ctx);
-    const OpCoef<float> c = coef_of(ctx, w);
-    hipLaunchKernelGGL(k_cgm_pack, flat(std::max(ctx->nh, std::max(ctx->nu, ctx->nv))), dim3(256), 0, ctx->stream, g,
-                       c, ctx->mwu, ctx->mwv, Lo, ctx->cg_pre ? (const double *)ctx->cdinv.u : nullptr,
-                       ctx->cg_pre ? (const double *)ctx->cdinv.v : nullptr);
-    // P x0
-    launch_tile_haar<float>(ctx, 1, w.xc.u, w.xc.v, ctx->mwu, ctx->mwv, w.ct.u, w.ct.v, ctx->ui, ctx->vi);
     CGMArgs sa;
-    sa.g = g;
-    sa.c = c;
-    sa.Lo = Lo;
+    sa.g = ctx->g;
+    sa.c = coef_of(ctx, w);
+    sa.Lo = cgm_layout(ctx);
     sa.levels = ctx->S.levels;
     sa.mwu = ctx->mwu;
     sa.mwv = ctx->mwv;
     sa.bu = w.cr.u;
     sa.bv = w.cr.v;
-    sa.x0u = w.xc.u;
-    sa.x0v = w.xc.v;
+    sa.xu = w.xc.u;
+    sa.xv = w.xc.v;
     sa.t0u = w.ct.u;
     sa.t0v = w.ct.v;
-    sa.R = ctx->rings;
+    sa.dinvu = ctx->cdinv.u;
+    sa.dinvv = ctx->cdinv.v;
+    sa.eu = w.e.u;
+    sa.ev = w.e.v;
+    sa.R = cgm_rings(ctx);
     sa.Pb = ctx->Pb;
     sa.st = ctx->stm;
     sa.hflag = ctx->d_flag;
     sa.nblk = ctx->nblk;
+    return sa;
+}
+
+// Set-up of the mixed coarse CG on b_c in w.cr with the warm start w.xc:
+// P x0, then k_cgm_setup (the arena, r0 = b - A_c x0, the scalars and the
+// host stop report).
+static int cgm_prepare(wavi_ctx *ctx, const VSet<float> &w)
+{
+    launch_tile_haar<float>(ctx, 1, w.xc.u, w.xc.v, ctx->mwu, ctx->mwv, w.ct.u, w.ct.v, ctx->ui, ctx->vi);
     ctx->h_flag->done = 0;
     ctx->h_flag->iters = 0;
+    const CGMArgs sa = cgm_args(ctx, w);
     if (ctx->cg_pre)
-        hipLaunchKernelGGL(k_cgm_setup<true>, tb, dim3(256), 0, ctx->stream, sa);
+        hipLaunchKernelGGL(k_cgm_setup<true>, dim3(ctx->nblk), dim3(256), 0, ctx->stream, sa);
     else
-        hipLaunchKernelGGL(k_cgm_setup<false>, tb, dim3(256), 0, ctx->stream, sa);
+        hipLaunchKernelGGL(k_cgm_setup<false>, dim3(ctx->nblk), dim3(256), 0, ctx->stream, sa);
     HIPCHK(hipGetLastError());
     return WAVI_OK;
 }
 
 // Mixed-precision coarse CG (Chronopoulos-Gear form, one launch per
-// iteration) on b_c held in v32.cr; solution in the warm start v32.xc.  The
-// CG works in the padded arena: k_cgm_pack fills the coefficients and masks,
-// k_cgm_setup the vectors, k_cgm_unpack returns the solution.
+// iteration) on b_c held in v32.cr from the warm start v32.xc.  The solution
+// stays in the arena until k_cgm_finish.
 static int rdv_coarse_cg(wavi_ctx *ctx, const VSet<float> &w, int *iters);
 
 template <>
 int do_coarse_cg<float>(wavi_ctx *ctx, const VSet<float> &w, int *iters)
 {
     if (ctx->rdv) return rdv_coarse_cg(ctx, w, iters);
-    const GridDims &g = ctx->g;
     dim3 tb(ctx->nblk);
-    const CGMLayout Lo = cgm_layout(ctx);
     CHK(cgm_prepare(ctx, w));
     const CGMIterArgs ia = cgm_iter_args(ctx);
     volatile CGMHostFlag *hf = ctx->h_flag;
@@ -1599,9 +1608,6 @@ int do_coarse_cg<float>(wavi_ctx *ctx, const VSet<float> &w, int *iters)
         case 6: hipLaunchKernelGGL((k_cgm_solve1<2, true>), dim3(1), dim3(256), 0, ctx->stream, ia); break;
         default: hipLaunchKernelGGL((k_cgm_solve1<3, true>), dim3(1), dim3(256), 0, ctx->stream, ia); break;
         }
-        HIPCHK(hipGetLastError());
-        hipLaunchKernelGGL(k_cgm_unpack, flat(std::max(ctx->nu, ctx->nv)), dim3(256), 0, ctx->stream, g, Lo, w.xc.u,
-                           w.xc.v);
         HIPCHK(hipGetLastError());
         HIPCHK(hipStreamSynchronize(ctx->stream));
         if (!hf->done) {
@@ -1660,9 +1666,6 @@ int do_coarse_cg<float>(wavi_ctx *ctx, const VSet<float> &w, int *iters)
         }
         ++k;
     }
-    hipLaunchKernelGGL(k_cgm_unpack, flat(std::max(ctx->nu, ctx->nv)), dim3(256), 0, ctx->stream, g, Lo, w.xc.u,
-                       w.xc.v);
-    HIPCHK(hipGetLastError());
     // A stop seen between chunks needs no wait for the launches queued past
     // it (they change nothing); the timing events do.
     if (!hf->done || ctx->prof) {
@@ -1715,7 +1718,7 @@ static int vcycle_post(wavi_ctx *ctx, const VSet<T> &w)
     if constexpr (std::is_same<T, double>::value)
         hipLaunchKernelGGL(k_cg_finish, dim3(ctx->nblk), dim3(256), 0, ctx->stream, cg_args(ctx), cg_io(ctx, w));
     else
-        launch_tile_haar<T>(ctx, 1, w.xc.u, w.xc.v, ctx->mwu, ctx->mwv, w.t.u, w.t.v, ctx->ui, ctx->vi, w.e.u, w.e.v);
+        hipLaunchKernelGGL(k_cgm_finish, dim3(ctx->nblk), dim3(256), 0, ctx->stream, cgm_args(ctx, w));
     CHK(do_smoother(ctx, w, rev));
     HIPCHK(hipGetLastError());
     return WAVI_OK;
@@ -2521,9 +2524,6 @@ static int rdv_coarse_cg(wavi_ctx *ctx, const VSet<float> &w, int *iters)
         R.cv.wait(lk, [&] { return ctx->rdv_done; });
     }
     CHK(ctx->rdv_rc);
-    hipLaunchKernelGGL(k_cgm_unpack, flat(std::max(ctx->nu, ctx->nv)), dim3(256), 0, ctx->stream, ctx->g,
-                       cgm_layout(ctx), w.xc.u, w.xc.v);
-    HIPCHK(hipGetLastError());
     *iters = ctx->rdv_iters;
     return WAVI_OK;
 }
@@ -2581,9 +2581,6 @@ static int lockstep_picard(std::vector<LockMember> &M, LockTables &R, int it, in
             wavi_ctx *ctx = M[k].ctx;
             M[k].cg = iters[jj];
             const VSet<float> &w = ctx->v32;
-            hipLaunchKernelGGL(k_cgm_unpack, flat(std::max(ctx->nu, ctx->nv)), dim3(256), 0, ctx->stream, ctx->g,
-                               cgm_layout(ctx), w.xc.u, w.xc.v);
-            HIPCHK(hipGetLastError());
             CHK(vcycle_post(ctx, w));
             CHK(vcycle_widen(ctx));
             CHK(precondition_update(ctx));
@@ -2749,7 +2746,7 @@ constexpr size_t LOCK_ARENA_BYTES = (size_t)128 << 20;
 
 static size_t arena_bytes(const wavi_ctx *ctx)
 {
-    return (size_t)CGM_NARRAY * ctx->ns * sizeof(float) + 2 * (size_t)ctx->ns;
+    return ((2 * CGM_NPAIR + 1) * sizeof(float) + 1) * (size_t)ctx->ns;
 }
 
 // The members of a batch that share coarse-CG launches, in member order.

@@ -2208,7 +2208,8 @@ struct CGScalars {
 
 // The FP64 coarse CG works in an arena of zero-padded 2-D arrays shared by
 // the u grid, the v grid and the h cells: point (i, j) at (i + 16) + px (j +
-// 16), px = 16 (nbx + 2), with a border of one tile that stays zero.  A tile's
+// 16), px = 16 (nbx + 1), with a border of one tile that stays zero (the next
+// row's left border is a row's right one).  A tile's
 // rows are then aligned, u and v of a point come in one 16-byte load, every
 // window, halo and store is unconditional at a 32-bit offset from a uniform
 // base, and what a tile stores past the end of a grid is zero.  Guarded
@@ -2363,32 +2364,37 @@ __global__ void __launch_bounds__(256) k_cg_setup(CGArgs a, CGIo io)
     }
 }
 
-// The end of the CG: x back into the compact warm start, and e += P x at the
-// inner points.
-__global__ void __launch_bounds__(256) k_cg_finish(CGArgs a, CGIo io)
+// The end of a CG on one tile: (x, y) = the solution at the thread's point,
+// back into the compact warm start, and e += P x at the inner points.
+template <typename T>
+__device__ __forceinline__ void cg_finish_tile(const GridDims &g, int levels, int bx, int by, T x, T y, unsigned mb,
+                                               T *xu, T *xv, T *eu, T *ev)
 {
-    __shared__ TilePair<double> t, m;
-    const GridDims &g = a.g;
-    const int L = xcd_tile(a.nblk);
-    if (L >= g.nbx * g.nby) return;
-    int bx, by;
-    band_tile(g, L, bx, by);
-    const int lx = threadIdx.x & 15, ly = threadIdx.x >> 4, i = bx * TILE + lx, j = by * TILE + ly;
+    __shared__ TilePair<T> t, m;
+    const int lx = threadIdx.x & 15, ly = threadIdx.x >> 4;
     bool oku, okv;
     int ku, kv;
-    op_own_index(g, i, j, oku, okv, ku, kv);
-    const unsigned at = a.Lo.at(i, j);
-    const double2 x = elem32(a.Lo.pair(CG_X), at);
-    const unsigned mb = elem32(a.Lo.M, at);
-    const double eu = ld_or(oku, (const double *)io.eu, ku, 0.0), ev = ld_or(okv, (const double *)io.ev, kv, 0.0);
-    if (oku) io.xu[ku] = x.x;
-    if (okv) io.xv[kv] = x.y;
-    t[0][ly][lx] = (mb & CB_WAVELET_U) ? x.x : 0.0;
-    t[1][ly][lx] = (mb & CB_WAVELET_V) ? x.y : 0.0;
+    op_own_index(g, bx * TILE + lx, by * TILE + ly, oku, okv, ku, kv);
+    const T e_u = ld_or(oku, (const T *)eu, ku, T(0)), e_v = ld_or(okv, (const T *)ev, kv, T(0));
+    if (oku) xu[ku] = x;
+    if (okv) xv[kv] = y;
+    t[0][ly][lx] = (mb & CB_WAVELET_U) ? x : T(0);
+    t[1][ly][lx] = (mb & CB_WAVELET_V) ? y : T(0);
     __syncthreads();
-    haar_pair<false, double>(io.levels, t, m);
-    if (mb & CB_INNER_U) io.eu[ku] = eu + t[0][ly][lx];
-    if (mb & CB_INNER_V) io.ev[kv] = ev + t[1][ly][lx];
+    haar_pair<false, T>(levels, t, m);
+    if (mb & CB_INNER_U) eu[ku] = e_u + t[0][ly][lx];
+    if (mb & CB_INNER_V) ev[kv] = e_v + t[1][ly][lx];
+}
+
+__global__ void __launch_bounds__(256) k_cg_finish(CGArgs a, CGIo io)
+{
+    const int L = xcd_tile(a.nblk);
+    if (L >= a.g.nbx * a.g.nby) return;
+    int bx, by;
+    band_tile(a.g, L, bx, by);
+    const unsigned at = a.Lo.at(bx * TILE + (int)(threadIdx.x & 15), by * TILE + (int)(threadIdx.x >> 4));
+    const double2 x = elem32(a.Lo.pair(CG_X), at);
+    cg_finish_tile<double>(a.g, io.levels, bx, by, x.x, x.y, elem32(a.Lo.M, at), io.xu, io.xv, io.eu, io.ev);
 }
 
 // A CG scalar written by an earlier kernel, read as a vector load: a scalar
@@ -2919,11 +2925,11 @@ __global__ void __launch_bounds__(256) k_cg_solve1(CGArgs a)
 // 1 - PAR, so no workgroup reads what another workgroup of the same launch
 // writes.
 //
-// Layout: every array of the CG lives in one FP32 arena in a zero-padded 2-D
-// layout shared by the u grid, the v grid and the h cells: point (i, j) at
-// (i + 1) + px (j + 1), with a zero border of one point and room for whole
-// tiles, so that windows, halos and tile stores need no bounds tests (what a
-// tile stores past the end of a grid is zero).
+// Layout: as the FP64 CG's arena in FP32: (u, v) pairs in zero-padded 2-D
+// arrays shared by the u grid, the v grid and the h cells, point (i, j) at
+// (i + 16) + px (j + 1), px = 16 (nbx + 1), so that a tile's rows are whole
+// aligned 128-byte lines and windows, halos and tile stores need no bounds
+// tests (what a tile stores past the end of a grid is zero).
 
 struct CGMState {
     double igamma;  // 1 / ||r||^2 at the start of the launch that wrote this state
@@ -2940,43 +2946,38 @@ struct CGMScalars {
     int iters;      // iterations at the stop
 };
 
-// Arena arrays (component u; the v component is the next array).
-enum CGMArray {
+// Arena arrays: (u, v) pairs, ns points each; then the corners' h*eta_av.
+enum CGMPair {
     CGM_R = 0,       // residual r
-    CGM_W = 2,       // w = A_c r
-    CGM_P = 4,       // search direction p
-    CGM_S = 6,       // s = A_c p
-    CGM_X = 8,       // solution
-    CGM_HU = 10,     // thickness on u / v points, 0 off the masks
-    CGM_BU = 12,     // beta_eff on u / v points, 0 off the masks
-    CGM_CELL = 14,   // per h cell: (h*eta_av on the h mask, dimp) pairs (two arrays' room)
-    CGM_CORNER = 16, // per h cell: corner h*eta_av (0 off the c grid and mask)
-    CGM_DINV = 17,   // Jacobi-preconditioned CG: 1 / |diag(A_c)| on u / v points, 0 off the masks
-    CGM_NARRAY = 19
+    CGM_W = 1,       // w = A_c r
+    CGM_P = 2,       // search direction p
+    CGM_S = 3,       // s = A_c p
+    CGM_X = 4,       // solution
+    CGM_H = 5,       // thickness on u and v points, 0 off the masks
+    CGM_B = 6,       // beta_eff on u and v points, 0 off the masks
+    CGM_CELL = 7,    // per h cell: (h*eta_av, dimp)
+    CGM_DINV = 8,    // Jacobi-preconditioned CG: 1 / |diag(A_c)|, 0 off the wavelet masks
+    CGM_NPAIR = 9
 };
 
-// Ring images, compact per tile: for each parity, tile (ntile + 1 tiles, the
-// last one all zero and never written, standing in for tiles past the edge),
-// kind (0 P r, 1 P s, 2 P w) and component, 64 slots: the tile's bottom row
-// (y = 0, slots 0-15 by x), top row (y = 15, 16-31), left column (x = 0,
-// 32-47 by y) and right column (x = 15, 48-63).  A side of a neighbour's halo
-// is then 16 consecutive floats.
-__device__ __forceinline__ unsigned ring_at(int par, int ntile, int tile, int kind, int comp)
-{
-    return ((unsigned)(par * (ntile + 1) + tile) * 6u + (unsigned)(2 * kind + comp)) * 64u;
-}
+// Ring images, compact per tile: for each parity and tile (ntile + 1 tiles,
+// the last one all zero and never written, standing in for tiles past the
+// edge) 64 slots: the tile's bottom row (y = 0, slots 0-15 by x), top row
+// (y = 15, 16-31), left column (x = 0, 32-47 by y) and right column (x = 15,
+// 48-63).  A slot holds (P r, P s) of u and v as one float4 and P w as one
+// float2, so a side of a neighbour's halo is 16 consecutive ones of each.
+struct CGMRings {
+    float4 *rs;  // (P r)_u, (P r)_v, (P s)_u, (P s)_v
+    float2 *w;   // (P w)_u, (P w)_v
+};
 
-// Store v at the ring slots of tile position (x, y) (a corner has two).
-__device__ __forceinline__ void ring_put(float *R, unsigned base, int x, int y, float v)
+__device__ __forceinline__ unsigned ring_at(int par, int ntile, int tile)
 {
-    if (y == 0) R[base + x] = v;
-    if (y == 15) R[base + 16 + x] = v;
-    if (x == 0) R[base + 32 + y] = v;
-    if (x == 15) R[base + 48 + y] = v;
+    return (unsigned)(par * (ntile + 1) + tile) * 64u;
 }
 
 // The ring slots of tile position (x, y): a row slot and a column slot, -1
-// where there is none.
+// where there is none (a corner has two).
 struct RingSlots {
     int row, col;
     __device__ __forceinline__ RingSlots(int x, int y)
@@ -2984,93 +2985,50 @@ struct RingSlots {
         row = y == 0 ? x : (y == 15 ? 16 + x : -1);
         col = x == 0 ? 32 + y : (x == 15 ? 48 + y : -1);
     }
-    __device__ __forceinline__ void put(float *R, unsigned base, float v) const
+    template <typename V>
+    __device__ __forceinline__ void put(V *R, V v) const
     {
-        if (row >= 0) R[base + (unsigned)row] = v;
-        if (col >= 0) R[base + (unsigned)col] = v;
+        if (row >= 0) R[row] = v;
+        if (col >= 0) R[col] = v;
     }
 };
 
 struct CGMLayout {
-    float *F;       // FP32 arena, array A at F + A * ns
-    uint8_t *M;     // mask bits (bit 0 inner point, bit 1 wavelet mask): u at M, v at M + ns
+    float2 *F;      // pair array A at F + A * ns, then the corners (ns floats)
+    uint8_t *M;     // mask bits (CB_*)
     unsigned px;    // row pitch
-    unsigned ns;    // array stride (px * rows)
-    __device__ __forceinline__ unsigned at(int i, int j) const { return (unsigned)(i + 1) + px * (unsigned)(j + 1); }
+    unsigned ns;    // array stride
+    __device__ __forceinline__ unsigned at(int i, int j) const
+    {
+        return (unsigned)(i + TILE) + __umul24(px, (unsigned)(j + 1));
+    }
+    __device__ __forceinline__ float2 *pair(int a) const { return F + (size_t)a * ns; }
+    __device__ __forceinline__ float *corner() const { return reinterpret_cast<float *>(F + (size_t)CGM_NPAIR * ns); }
 };
 
-// Coefficients and masks into the arena (once per V-cycle); 0 off the masks.
-__global__ void k_cgm_pack(GridDims g, OpCoef<float> c, const uint8_t *mwu, const uint8_t *mwv, CGMLayout Lo,
-                           const double *dinvu, const double *dinvv)
-{
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    const int nh = g.nx * g.ny, nu = g.nxu * g.nyu, nv = g.nxv * g.nyv;
-    float *F = Lo.F;
-    const unsigned ns = Lo.ns;
-    // every load first (ld_or): the stores into the arena come after, since
-    // the compiler cannot move a load past them
-    const bool kh = k < nh, ku = k < nu, kv = k < nv;
-    const int a = k % g.nx, b = k / g.nx;
-    const bool okc = kh && a < g.nx - 1 && b < g.ny - 1;
-    const int kc = a + (g.nx - 1) * b;
-    const bool cmc = ld_or(okc, c.cm, kc, (uint8_t)0) != 0, hmk = ld_or(kh, c.hm, k, (uint8_t)0) != 0;
-    const float hcc = ld_or(okc, c.heta_c, kc, 0.f), hhk = ld_or(kh, c.heta_h, k, 0.f), dpk = ld_or(kh, c.dimp, k, 0.f);
-    const bool umk = ld_or(ku, c.um, k, (uint8_t)0) != 0, uik = ld_or(ku, c.ui, k, (uint8_t)0) != 0;
-    const bool mwuk = ld_or(ku, mwu, k, (uint8_t)0) != 0;
-    const float huk = ld_or(ku, c.hu, k, 0.f), buk = ld_or(ku, c.bu, k, 0.f);
-    const bool vmk = ld_or(kv, c.vm, k, (uint8_t)0) != 0, vik = ld_or(kv, c.vi, k, (uint8_t)0) != 0;
-    const bool mwvk = ld_or(kv, mwv, k, (uint8_t)0) != 0;
-    const float hvk = ld_or(kv, c.hv, k, 0.f), bvk = ld_or(kv, c.bv, k, 0.f);
-    const double dzu = dinvu ? ld_or(ku, dinvu, k, 0.0) : 0.0, dzv = dinvv ? ld_or(kv, dinvv, k, 0.0) : 0.0;
-    if (kh) {
-        const float hc = okc ? (cmc ? hcc : 0.f) : 0.f;
-        const unsigned o = Lo.at(a, b);
-        reinterpret_cast<float2 *>(F + CGM_CELL * ns)[o] = make_float2(hmk ? hhk : 0.f, dpk);
-        F[CGM_CORNER * ns + o] = hc;
-    }
-    if (ku) {
-        const unsigned o = Lo.at(k % g.nxu, k / g.nxu);
-        F[CGM_HU * ns + o] = umk ? huk : 0.f;
-        F[CGM_BU * ns + o] = umk ? buk : 0.f;
-        Lo.M[o] = (uint8_t)((uik ? 1 : 0) | (mwuk ? 2 : 0));
-        if (dinvu) F[CGM_DINV * ns + o] = (float)fmin(dzu, 1e30);  // finite in FP32
-    }
-    if (kv) {
-        const unsigned o = Lo.at(k % g.nxv, k / g.nxv);
-        F[(CGM_HU + 1) * ns + o] = vmk ? hvk : 0.f;
-        F[(CGM_BU + 1) * ns + o] = vmk ? bvk : 0.f;
-        Lo.M[ns + o] = (uint8_t)((vik ? 1 : 0) | (mwvk ? 2 : 0));
-        if (dinvv) F[(CGM_DINV + 1) * ns + o] = (float)fmin(dzv, 1e30);  // finite in FP32
-    }
-}
-
-// The solution back into the context's compact vectors.
-__global__ void k_cgm_unpack(GridDims g, CGMLayout Lo, float *xu, float *xv)
-{
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k < g.nxu * g.nyu) xu[k] = Lo.F[CGM_X * Lo.ns + Lo.at(k % g.nxu, k / g.nxu)];
-    if (k < g.nxv * g.nyv) xv[k] = Lo.F[(CGM_X + 1) * Lo.ns + Lo.at(k % g.nxv, k / g.nxv)];
-}
-
+// What the set-up and the end of the mixed CG read and write: the compact
+// arrays.
 struct CGMArgs {
     GridDims g;
-    OpCoef<float> c;         // compact coefficients (setup)
+    OpCoef<float> c;
     CGMLayout Lo;
     int levels;
     const uint8_t *mwu, *mwv;
-    const float *bu, *bv;    // right-hand side (compact)
-    const float *x0u, *x0v;  // warm start (compact)
-    const float *t0u, *t0v;  // P x0 (compact)
-    float *R;                // ring images
+    const float *bu, *bv;    // right-hand side
+    float *xu, *xv;          // warm start in, solution out
+    const float *t0u, *t0v;  // P x0
+    const double *dinvu, *dinvv;  // Jacobi: 1 / |diag(A_c)|
+    float *eu, *ev;          // the V-cycle's correction, += P x
+    CGMRings R;
     double *Pb;              // partials of ||b||^2 per u / v block
     CGMScalars *st;
     CGMHostFlag *hflag;      // host-mapped stop report, reset here
     int nblk;
 };
 
-// setup (P x0 computed beforehand): r0 = b - R A P x0, p = s = 0, x = x0 in
-// the arena, P r0 into the P r rings of set 0, partials of ||b||^2; resets
-// the scalars.
+// setup (P x0 computed beforehand): r0 = b - R A P x0, p = s = 0, x = x0, the
+// coefficients and mask bits into the arena, P r0 into the rings of set 0,
+// partials of ||b||^2; resets the scalars.
 template <bool PRE>
 __global__ void __launch_bounds__(256) k_cgm_setup(CGMArgs a)
 {
@@ -3098,49 +3056,57 @@ __global__ void __launch_bounds__(256) k_cgm_setup(CGMArgs a)
     const bool has_u = bx < g.nbxu && by < g.nbyu, has_v = bx < g.nbxv && by < g.nbyv;
     const int i0 = bx * TILE, j0 = by * TILE;
     const int lx = threadIdx.x & 15, ly = threadIdx.x >> 4;
-    float *F = a.Lo.F;
-    const unsigned ns = a.Lo.ns, at = a.Lo.at(i0 + lx, j0 + ly);
-    const int i = i0 + lx, j = j0 + ly;
-    const bool oku = i < g.nxu && j < g.nyu, okv = i < g.nxv && j < g.nyv;
-    const int ku = i + g.nxu * j, kv = i + g.nxv * j;
-    const float bu = ld_or(oku, a.bu, ku, 0.f), bv = ld_or(okv, a.bv, kv, 0.f);
-    const float xu = ld_or(oku, a.x0u, ku, 0.f), xv = ld_or(okv, a.x0v, kv, 0.f);
     OpOwn<float> o;
-    op_restrict_tile(g, a.c, MaskSep<true>{a.c.ui, a.c.um, a.c.vi, a.c.vm, a.mwu, a.mwv}, a.levels, a.t0u, a.t0v, i0,
-                     j0, s, o);
-    TilePair<float> &t = s.h.t, &m = s.h.m;
-    float ru = 0.f, rv = 0.f;
-    double b2u = 0.0, b2v = 0.0;
+    op_own_index(g, i0 + lx, j0 + ly, o.oku, o.okv, o.ku, o.kv);
+    const float bu = ld_or(o.oku, a.bu, o.ku, 0.f), bv = ld_or(o.okv, a.bv, o.kv, 0.f);
+    const float xu = ld_or(o.oku, (const float *)a.xu, o.ku, 0.f), xv = ld_or(o.okv, (const float *)a.xv, o.kv, 0.f);
     // Jacobi: the rings hold P D^-1 r and ||b||^2 is the D^-1 norm
-    const float dzu = PRE && oku ? F[CGM_DINV * ns + at] : 1.f, dzv = PRE && okv ? F[(CGM_DINV + 1) * ns + at] : 1.f;
-    if (oku) {
-        ru = bu - ((o.mu & MB_WAVELET) ? t[0][ly][lx] : 0.f);
-        F[CGM_R * ns + at] = ru;
-        F[CGM_P * ns + at] = 0.f;
-        F[CGM_S * ns + at] = 0.f;
-        F[CGM_X * ns + at] = xu;
-        b2u = PRE ? (double)bu * ((double)dzu * (double)bu) : (double)bu * (double)bu;
-    }
-    if (okv) {
-        rv = bv - ((o.mv & MB_WAVELET) ? t[1][ly][lx] : 0.f);
-        F[(CGM_R + 1) * ns + at] = rv;
-        F[(CGM_P + 1) * ns + at] = 0.f;
-        F[(CGM_S + 1) * ns + at] = 0.f;
-        F[(CGM_X + 1) * ns + at] = xv;
-        b2v = PRE ? (double)bv * ((double)dzv * (double)bv) : (double)bv * (double)bv;
-    }
+    const float dzu = PRE ? (float)fmin(ld_or(o.oku, a.dinvu, o.ku, 0.0), 1e30) : 1.f;  // finite in FP32
+    const float dzv = PRE ? (float)fmin(ld_or(o.okv, a.dinvv, o.kv, 0.0), 1e30) : 1.f;
+    const OpCoef<float> &c = a.c;
+    op_restrict_tile(g, c, MaskSep<true>{c.ui, c.um, c.vi, c.vm, a.mwu, a.mwv}, a.levels, a.t0u, a.t0v, i0, j0, s, o);
+    TilePair<float> &t = s.h.t, &m = s.h.m;
+    const float ru = o.oku ? bu - ((o.mu & MB_WAVELET) ? t[0][ly][lx] : 0.f) : 0.f;
+    const float rv = o.okv ? bv - ((o.mv & MB_WAVELET) ? t[1][ly][lx] : 0.f) : 0.f;
+    const unsigned at = a.Lo.at(i0 + lx, j0 + ly);
+    elem32(a.Lo.pair(CGM_R), at) = make_float2(ru, rv);
+    elem32(a.Lo.pair(CGM_P), at) = make_float2(0.f, 0.f);
+    elem32(a.Lo.pair(CGM_S), at) = make_float2(0.f, 0.f);
+    elem32(a.Lo.pair(CGM_X), at) = make_float2(xu, xv);
+    elem32(a.Lo.pair(CGM_H), at) = make_float2(o.hu, o.hv);
+    elem32(a.Lo.pair(CGM_B), at) = make_float2(o.bu, o.bv);
+    elem32(a.Lo.pair(CGM_CELL), at) = make_float2(o.heta, o.dimp);
+    if constexpr (PRE) elem32(a.Lo.pair(CGM_DINV), at) = make_float2(dzu, dzv);
+    elem32(a.Lo.corner(), at) = o.hetac;
+    elem32(a.Lo.M, at) = (uint8_t)(((o.mu & MB_INNER) ? CB_INNER_U : 0) | ((o.mv & MB_INNER) ? CB_INNER_V : 0) |
+                           ((o.mu & MB_WAVELET) ? CB_WAVELET_U : 0) | ((o.mv & MB_WAVELET) ? CB_WAVELET_V : 0));
+    double b2u = PRE ? (double)bu * ((double)dzu * (double)bu) : (double)bu * (double)bu;
+    double b2v = PRE ? (double)bv * ((double)dzv * (double)bv) : (double)bv * (double)bv;
     // each thread rewrites only its own entry; the transform ended with a barrier
     t[0][ly][lx] = (o.mu & MB_WAVELET) ? (PRE ? dzu * ru : ru) : 0.f;
     t[1][ly][lx] = (o.mv & MB_WAVELET) ? (PRE ? dzv * rv : rv) : 0.f;
     __syncthreads();
     haar_pair<false, float>(a.levels, t, m);
-    if (oku) ring_put(a.R, ring_at(0, g.nbx * g.nby, tile_id, 0, 0), lx, ly, (o.mu & MB_INNER) ? t[0][ly][lx] : 0.f);
-    if (okv) ring_put(a.R, ring_at(0, g.nbx * g.nby, tile_id, 0, 1), lx, ly, (o.mv & MB_INNER) ? t[1][ly][lx] : 0.f);
+    RingSlots(lx, ly).put(a.R.rs + ring_at(0, g.nbx * g.nby, tile_id),
+                          make_float4((o.mu & MB_INNER) ? t[0][ly][lx] : 0.f, (o.mv & MB_INNER) ? t[1][ly][lx] : 0.f, 0.f, 0.f));
     tree256x2(b2u, b2v, lds);
     if (threadIdx.x == 0) {
         if (has_u) a.Pb[bx + g.nbxu * by] = b2u;
         if (has_v) a.Pb[g.nbxu * g.nbyu + bx + g.nbxv * by] = b2v;
     }
+}
+
+// The end of the mixed CG: x back into the compact warm start, and e += P x
+// at the inner points.
+__global__ void __launch_bounds__(256) k_cgm_finish(CGMArgs a)
+{
+    const int L = xcd_tile(a.nblk);
+    if (L >= a.g.nbx * a.g.nby) return;
+    int bx, by;
+    band_tile(a.g, L, bx, by);
+    const unsigned at = a.Lo.at(bx * TILE + (int)(threadIdx.x & 15), by * TILE + (int)(threadIdx.x >> 4));
+    const float2 x = elem32(a.Lo.pair(CGM_X), at);
+    cg_finish_tile<float>(a.g, a.levels, bx, by, x.x, x.y, elem32(a.Lo.M, at), a.xu, a.xv, a.eu, a.ev);
 }
 
 // Block Haar transforms of 16-point lines held one point per lane (pos = the
@@ -3216,24 +3182,6 @@ __device__ __forceinline__ void haar_lines_R(float &v0, float &v1, int pos)
     if constexpr (LEV >= 3) haar_stage_dpp<8>(v0, v1, haar_sign_R<8>(pos));
 }
 
-// Halo point h (0..67) of the 18 x 18 window: window coordinates.
-__device__ __forceinline__ void halo_xy(int h, int &x, int &y)
-{
-    if (h < 18) {
-        x = h;
-        y = 0;
-    } else if (h < 36) {
-        x = h - 18;
-        y = 17;
-    } else if (h < 52) {
-        x = 0;
-        y = h - 35;
-    } else {
-        x = 17;
-        y = h - 51;
-    }
-}
-
 // Sum over a 16-lane row in FP32, left in every lane of the row.
 __device__ __forceinline__ float row_sum16f(float v)
 {
@@ -3246,7 +3194,7 @@ __device__ __forceinline__ float row_sum16f(float v)
 
 struct CGMIterArgs {
     CGMLayout Lo;
-    float *R;               // ring images
+    CGMRings R;
     float2 *Pgd;            // [2][npad]: per tile (r, r) and (w, r) partials by parity (0 past the tiles)
     CGMScalars *st;
     CGMHostFlag *hflag;     // host-mapped stop report
@@ -3270,17 +3218,22 @@ struct CGMIterArgs {
 // delta = (w, u); D^-1 is pointwise, so u, D^-1 s and D^-1 w are formed
 // where they are used and the rings hold P D^-1 r, P D^-1 s, P D^-1 w (the
 // halo of P u_new is then the same linear step).
+//
+// Each operand is loaded and staged once: a thread loads the pairs of its
+// own point and its own cell, wavefront 3 the halo's four sides, wavefront 2
+// the two halo corners that are read, wavefront 0 the 33 cells before the
+// tile; an h cell's four intermediates go through LDS as one float4.
 template <int PAR, bool INIT, int LEV, bool PRE>
 __device__ __forceinline__ bool cgm_iter_tile(const CGMIterArgs &a, const int L)
 {
     static_assert(!INIT || PAR == 0, "the initial launch reads set 0");
     struct Smem {
-        float U[18][19], V[18][19];      // window of P r (u and v points)
-        float HU[18][19], HV[18][19];    // thickness windows, 0 off the masks
-        float rxx[17][18], ryy[17][18], ext[17][18], rxy[17][18];
-        float T[4][TILE][TILE + 1];      // transposes of the block transforms
-        uint8_t mb[2][TILE][TILE + 1];   // mask bits of the tile
-        float dz[PRE ? 2 : 1][TILE][TILE + 1];  // Jacobi: 1 / |diag(A_c)| of the tile
+        float2 UV[18][19];               // window of P r (u and v points)
+        float2 H[18][19];                // thickness window, 0 off the masks
+        float4 cell[17][18];             // r_xx, r_yy, r_xy and the implicit term
+        float2 T[2][TILE][TILE + 1];     // transposes of the block transforms
+        float2 dz[PRE ? TILE : 1][TILE + 1];  // Jacobi: 1 / |diag(A_c)| of the tile
+        uint8_t mb[TILE][TILE + 4];      // mask bits of the tile
         double red0[8];
         float red1[8];
         double red2[8];
@@ -3289,7 +3242,8 @@ __device__ __forceinline__ bool cgm_iter_tile(const CGMIterArgs &a, const int L)
     const GridDims &g = a.g;
     const int ntile = g.nbx * g.nby;
     if (L >= ntile) return false;
-    const int tid = threadIdx.x;
+    const int tid = threadIdx.x, l = tid & 63;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     int bx, by;
     const int tile_id = band_tile(g, L, bx, by);
     const int i0 = bx * TILE, j0 = by * TILE;
@@ -3302,23 +3256,19 @@ __device__ __forceinline__ bool cgm_iter_tile(const CGMIterArgs &a, const int L)
     // (alpha_{k-1} + alpha_k beta_k) p_{k-1} + alpha_k r_k, and a stop after
     // an even iteration applies the pending alpha_{k-1} p_{k-1}.
     constexpr bool XUPD = PAR == 0;
-    const unsigned px = a.Lo.px, ns = a.Lo.ns;
-    float *F = a.Lo.F;
-    const uint8_t *M = a.Lo.M;
+    const CGMLayout &Lo = a.Lo;
     const float rdx = a.rdx, rdy = a.rdy;
-    // Array A is the uniform base F + A ns; a point is a 32-bit byte offset
-    // into it (the scalar-base addressing of global loads and stores).
-    auto arr = [&](int A) { return F + (size_t)A * ns; };
-    auto el = [](float *base, unsigned boff) -> float & { return *reinterpret_cast<float *>(reinterpret_cast<char *>(base) + boff); };
-    // window entry (x, y) is arena offset wb + x + px y
     // (24-bit products: a 32-bit multiply-add is emitted as a 64-bit one whose
     // unused high addend can be a register with a load in flight)
-    const unsigned wb = (unsigned)i0 + __umul24(px, (unsigned)j0);
-    const unsigned o = wb + (unsigned)(lx + 1) + __umul24(px, (unsigned)(ly + 1));   // own point
-    const unsigned ob = 4u * o;
+    const unsigned at0 = Lo.at(i0, j0), at = at0 + (unsigned)lx + __umul24(Lo.px, (unsigned)ly);
+    auto cload = [&](int A, unsigned k) -> float2 { return elem32((const float2 *)Lo.pair(A), k); };
+    auto cstore = [&](int A, float2 v) {
+        st_nt(reinterpret_cast<double *>(&elem32(Lo.pair(A), at)),
+              __hiloint2double(__float_as_int(v.y), __float_as_int(v.x)));
+    };
     // ---- loads, all issued before the first use, in the order they are
     // needed: the wait for a load also waits for every load issued before
-    // it, so the partials come first and the coefficient windows last
+    // it, so the partials come first and the coefficients last
     const CGMState S = a.st->s[PAR];
     // partials of the previous launch
     float2 pv[4];
@@ -3326,62 +3276,52 @@ __device__ __forceinline__ bool cgm_iter_tile(const CGMIterArgs &a, const int L)
 #pragma unroll
         for (int e = 0; e < 4; ++e) pv[e] = a.Pgd[PAR * a.npad + tid + 256 * e];
     }
-    const uint8_t mbu = M[o], mbv = (M + ns)[o];
-    float r_u = el(arr(CGM_R), ob), r_v = el(arr(CGM_R + 1), ob);
-    float w_u0 = 0.f, p_u0 = 0.f, s_u0 = 0.f, x_u0 = 0.f, w_v0 = 0.f, p_v0 = 0.f, s_v0 = 0.f, x_v0 = 0.f;
+    const unsigned mb = elem32((const uint8_t *)Lo.M, at);
+    float2 r = cload(CGM_R, at), w0 = make_float2(0.f, 0.f), p0 = w0, s0 = w0, x0 = w0, dz = make_float2(1.f, 1.f);
     if (!INIT) {
-        w_u0 = el(arr(CGM_W), ob);
-        w_v0 = el(arr(CGM_W + 1), ob);
-        p_u0 = el(arr(CGM_P), ob);
-        p_v0 = el(arr(CGM_P + 1), ob);
-        s_u0 = el(arr(CGM_S), ob);
-        s_v0 = el(arr(CGM_S + 1), ob);
-        if (XUPD) {
-            x_u0 = el(arr(CGM_X), ob);
-            x_v0 = el(arr(CGM_X + 1), ob);
+        w0 = cload(CGM_W, at);
+        p0 = cload(CGM_P, at);
+        s0 = cload(CGM_S, at);
+        if (XUPD) x0 = cload(CGM_X, at);
+    }
+    if constexpr (PRE) dz = cload(CGM_DINV, at);
+    // halo point (hx, hy) of the window from the neighbours' rings: slot
+    // hslot of the tile (bx + hdx, by + hdy)
+    const bool corner = w == 2 && l < 2;  // lane 0: (17, 0), of which u is read; lane 1: (0, 17), v
+    const bool halo = w == 3 || corner;
+    int hx = l == 0 ? 17 : 0, hy = l == 0 ? 0 : 17;
+    float4 hrs = make_float4(0.f, 0.f, 0.f, 0.f);
+    float2 hw = make_float2(0.f, 0.f), hH = hw;
+    if (w >= 2) {
+        const int q = l & 15, side = l >> 4;
+        int hdx = l == 0 ? 1 : -1, hdy = -hdx, hslot = l == 0 ? 16 : 15;
+        if (w == 3) {
+            halo_side(l, hx, hy);
+            hdx = side == 0 ? -1 : (side == 1 ? 1 : 0);
+            hdy = side == 2 ? -1 : (side == 3 ? 1 : 0);
+            hslot = q + (side == 0 ? 48 : (side == 1 ? 32 : (side == 2 ? 16 : 0)));
         }
+        const int nbxx = bx + hdx, nbyy = by + hdy;
+        const int ntl = (nbxx >= 0 && nbxx < g.nbx && nbyy >= 0 && nbyy < g.nby) ? nbxx + g.nbx * nbyy : ntile;
+        const unsigned hr_at = ring_at(PAR, ntile, ntl) + (unsigned)hslot;
+        hrs = elem32((const float4 *)a.R.rs, hr_at);
+        if (!INIT) hw = elem32((const float2 *)a.R.w, hr_at);
+        hH = cload(CGM_H, at0 + (unsigned)(hx - 1 + (int)__mul24((int)Lo.px, hy - 1)));
     }
-    // halo of the window from the neighbours' rings: threads 0..67 the u
-    // grid, 68..135 the v grid
-    int hx, hy;
-    const int hcomp = tid >= 68 ? 1 : 0;
-    const int hh = tid < 136 ? tid - 68 * hcomp : 0;
-    halo_xy(hh, hx, hy);
-    // neighbour tile (dx, dy) and the slot in its ring
-    const int hdx = hx == 0 ? -1 : (hx == 17 ? 1 : 0), hdy = hy == 0 ? -1 : (hy == 17 ? 1 : 0);
-    const int hslot = hdy == -1 ? 16 + (hdx == -1 ? 15 : (hdx == 1 ? 0 : hx - 1))
-                    : hdy == 1 ? (hdx == -1 ? 15 : (hdx == 1 ? 0 : hx - 1))
-                    : hdx == -1 ? 48 + (hy - 1) : 32 + (hy - 1);
-    const int nbxx = bx + hdx, nbyy = by + hdy;
-    const int ntl = (nbxx >= 0 && nbxx < g.nbx && nbyy >= 0 && nbyy < g.nby) ? nbxx + g.nbx * nbyy : ntile;
-    const float *Rr = a.R;
-    const float hr = Rr[ring_at(PAR, ntile, ntl, 0, hcomp) + hslot];
-    float hs = 0.f, hw = 0.f;
-    if (!INIT) {
-        hs = Rr[ring_at(PAR, ntile, ntl, 1, hcomp) + hslot];
-        hw = Rr[ring_at(PAR, ntile, ntl, 2, hcomp) + hslot];
+    const float2 oH = cload(CGM_H, at);
+    const float2 cc = cload(CGM_CELL, at);
+    const float ch = elem32((const float *)Lo.corner(), at);
+    // the cells before the tile: (0, 0..16), (1..16, 0); lanes past them repeat the last
+    const int ex = l < 17 ? 0 : (l < 33 ? l - 16 : 16), ey = l < 17 ? l : 0;
+    float2 ec = make_float2(0.f, 0.f);
+    float eh = 0.f;
+    if (w == 0) {
+        const unsigned ea = at0 + (unsigned)(ex - 1 + (int)__mul24((int)Lo.px, ey - 1));
+        ec = cload(CGM_CELL, ea);
+        eh = elem32((const float *)Lo.corner(), ea);
     }
-    // thickness windows, entries q = tid and tid + 256 (< 324) of the 18 x 18 window
-    const int q1 = tid + 256 < 324 ? tid + 256 : tid;
-    const unsigned t0 = 4u * (wb + (unsigned)(tid % 18) + __umul24(px, (unsigned)(tid / 18)));
-    const unsigned t1 = 4u * (wb + (unsigned)(q1 % 18) + __umul24(px, (unsigned)(q1 / 18)));
-    const float thu0 = el(arr(CGM_HU), t0), thv0 = el(arr(CGM_HU + 1), t0);
-    const float thu1 = el(arr(CGM_HU), t1), thv1 = el(arr(CGM_HU + 1), t1);
-    // cell coefficients, cells q = tid and tid + 256 (< 289) of the 17 x 17 window
-    const int c1q = tid + 256 < 289 ? tid + 256 : tid;
-    const unsigned c0o = wb + (unsigned)(tid % 17) + __umul24(px, (unsigned)(tid / 17));
-    const unsigned c1o = wb + (unsigned)(c1q % 17) + __umul24(px, (unsigned)(c1q / 17));
-    const char *cell2 = reinterpret_cast<const char *>(arr(CGM_CELL));
-    const float2 cc0 = *reinterpret_cast<const float2 *>(cell2 + 8u * c0o);
-    const float2 cc1 = *reinterpret_cast<const float2 *>(cell2 + 8u * c1o);
-    const float ch0 = el(arr(CGM_CORNER), 4u * c0o), ch1 = el(arr(CGM_CORNER), 4u * c1o);
-    const float bu0 = el(arr(CGM_BU), ob), bv0 = el(arr(CGM_BU + 1), ob);
-    float dz_u = 1.f, dz_v = 1.f;
-    if constexpr (PRE) {
-        dz_u = el(arr(CGM_DINV), ob);
-        dz_v = el(arr(CGM_DINV + 1), ob);
-    }
-    const bool inu = mbu & 1, inv = mbv & 1, mwu = mbu & 2, mwv = mbv & 2;
+    const float2 oB = cload(CGM_B, at);
+    const bool inu = mb & CB_INNER_U, inv = mb & CB_INNER_V, mwu = mb & CB_WAVELET_U, mwv = mb & CB_WAVELET_V;
     // ---- scalars from the previous launch's partials (FP64 across workgroups)
     float fa = 0.f, fb = 0.f, fxp = 0.f;
     if (!INIT) {
@@ -3422,8 +3362,7 @@ __device__ __forceinline__ bool cgm_iter_tile(const CGMIterArgs &a, const int L)
             }
             if (XUPD && S.it > 0) {
                 const float fp = (float)S.alpha;
-                el(arr(CGM_X), ob) = x_u0 + fp * p_u0;
-                el(arr(CGM_X + 1), ob) = x_v0 + fp * p_v0;
+                cstore(CGM_X, make_float2(x0.x + fp * p0.x, x0.y + fp * p0.y));
             }
             return true;
         }
@@ -3445,158 +3384,122 @@ __device__ __forceinline__ bool cgm_iter_tile(const CGMIterArgs &a, const int L)
     }
     // ---- vector updates on the tile (zero past the ends of the grids); with
     // Jacobi the direction and x take u = D^-1 r where they take r
-    float s_u = 0.f, s_v = 0.f;
+    float2 s1 = make_float2(0.f, 0.f);
     if (!INIT) {
-        const float z_u = PRE ? dz_u * r_u : r_u, z_v = PRE ? dz_v * r_v : r_v;
-        const float p_u = z_u + fb * p_u0, p_v = z_v + fb * p_v0;
-        if (XUPD) {
-            st_nt(&el(arr(CGM_X), ob), (x_u0 + fxp * p_u0) + fa * z_u);
-            st_nt(&el(arr(CGM_X + 1), ob), (x_v0 + fxp * p_v0) + fa * z_v);
-        }
-        s_u = w_u0 + fb * s_u0;
-        s_v = w_v0 + fb * s_v0;
-        r_u = r_u - fa * s_u;
-        r_v = r_v - fa * s_v;
-        st_nt(&el(arr(CGM_P), ob), p_u);
-        st_nt(&el(arr(CGM_P + 1), ob), p_v);
-        st_nt(&el(arr(CGM_S), ob), s_u);
-        st_nt(&el(arr(CGM_S + 1), ob), s_v);
-        st_nt(&el(arr(CGM_R), ob), r_u);
-        st_nt(&el(arr(CGM_R + 1), ob), r_v);
+        const float z_u = PRE ? dz.x * r.x : r.x, z_v = PRE ? dz.y * r.y : r.y;
+        const float p_u = z_u + fb * p0.x, p_v = z_v + fb * p0.y;
+        if (XUPD) cstore(CGM_X, make_float2((x0.x + fxp * p0.x) + fa * z_u, (x0.y + fxp * p0.y) + fa * z_v));
+        s1 = make_float2(w0.x + fb * s0.x, w0.y + fb * s0.y);
+        r = make_float2(r.x - fa * s1.x, r.y - fa * s1.y);
+        cstore(CGM_P, make_float2(p_u, p_v));
+        cstore(CGM_S, s1);
+        cstore(CGM_R, r);
     }
     // ---- x pass of P r and P s (Jacobi: of D^-1 r and D^-1 s); halo and
     // thickness windows into LDS
     {
-        float a0 = mwu ? (PRE ? dz_u * r_u : r_u) : 0.f, a1 = mwv ? (PRE ? dz_v * r_v : r_v) : 0.f;
+        float a0 = mwu ? (PRE ? dz.x * r.x : r.x) : 0.f, a1 = mwv ? (PRE ? dz.y * r.y : r.y) : 0.f;
         haar_lines_P<LEV>(a0, a1, lx);
-        sm.T[0][ly][lx] = a0;
-        sm.T[1][ly][lx] = a1;
+        sm.T[0][ly][lx] = make_float2(a0, a1);
         if (!INIT) {
-            float a2 = mwu ? (PRE ? dz_u * s_u : s_u) : 0.f, a3 = mwv ? (PRE ? dz_v * s_v : s_v) : 0.f;
+            float a2 = mwu ? (PRE ? dz.x * s1.x : s1.x) : 0.f, a3 = mwv ? (PRE ? dz.y * s1.y : s1.y) : 0.f;
             haar_lines_P<LEV>(a2, a3, lx);
-            sm.T[2][ly][lx] = a2;
-            sm.T[3][ly][lx] = a3;
+            sm.T[1][ly][lx] = make_float2(a2, a3);
         }
     }
-    sm.mb[0][ly][lx] = mbu;
-    sm.mb[1][ly][lx] = mbv;
-    if constexpr (PRE) {
-        sm.dz[0][ly][lx] = dz_u;
-        sm.dz[1][ly][lx] = dz_v;
-    }
-    if (tid < 136) {
-        const float t = INIT ? hr : hr - fa * (hw + fb * hs);
-        if (!hcomp)
-            sm.U[hy][hx] = t;
-        else
-            sm.V[hy][hx] = t;
+    sm.mb[ly][lx] = (uint8_t)mb;
+    if constexpr (PRE) sm.dz[ly][lx] = dz;
+    sm.H[ly + 1][lx + 1] = oH;
+    if (halo) {
+        sm.UV[hy][hx] = INIT ? make_float2(hrs.x, hrs.y)
+                             : make_float2(hrs.x - fa * (hw.x + fb * hrs.z), hrs.y - fa * (hw.y + fb * hrs.w));
+        sm.H[hy][hx] = hH;
     }
     __syncthreads();
     // ---- y pass in the column-major lanes: P r into the window, rings of P r
-    // and P s; thickness windows into LDS (read after the next barrier)
-    sm.HU[tid / 18][tid % 18] = thu0;
-    sm.HV[tid / 18][tid % 18] = thv0;
-    if (tid + 256 < 324) {
-        sm.HU[q1 / 18][q1 % 18] = thu1;
-        sm.HV[q1 / 18][q1 % 18] = thv1;
-    }
+    // and P s
     {
-        const uint8_t m0 = sm.mb[0][cy][cx], m1 = sm.mb[1][cy][cx];
-        float y0 = sm.T[0][cy][cx], y1 = sm.T[1][cy][cx];
+        const unsigned m = sm.mb[cy][cx];
+        const float2 t0 = sm.T[0][cy][cx];
+        float y0 = t0.x, y1 = t0.y;
         haar_lines_P<LEV>(y0, y1, cy);
-        const float pr_u = (m0 & 1) ? y0 : 0.f, pr_v = (m1 & 1) ? y1 : 0.f;
-        sm.U[cy + 1][cx + 1] = pr_u;
-        sm.V[cy + 1][cx + 1] = pr_v;
-        float ps_u = 0.f, ps_v = 0.f;
+        const float2 pr = make_float2((m & CB_INNER_U) ? y0 : 0.f, (m & CB_INNER_V) ? y1 : 0.f);
+        sm.UV[cy + 1][cx + 1] = pr;
+        float2 ps = make_float2(0.f, 0.f);
         if (!INIT) {
-            float y2 = sm.T[2][cy][cx], y3 = sm.T[3][cy][cx];
+            const float2 t1 = sm.T[1][cy][cx];
+            float y2 = t1.x, y3 = t1.y;
             haar_lines_P<LEV>(y2, y3, cy);
-            ps_u = (m0 & 1) ? y2 : 0.f;
-            ps_v = (m1 & 1) ? y3 : 0.f;
+            ps = make_float2((m & CB_INNER_U) ? y2 : 0.f, (m & CB_INNER_V) ? y3 : 0.f);
         }
-        const RingSlots rs(cx, cy);
-        const unsigned rb = ring_at(NP, ntile, tile_id, 0, 0);
-        rs.put(a.R, rb, pr_u);
-        rs.put(a.R, rb + 64, pr_v);
-        rs.put(a.R, rb + 128, ps_u);
-        rs.put(a.R, rb + 192, ps_v);
+        RingSlots(cx, cy).put(a.R.rs + ring_at(NP, ntile, tile_id), make_float4(pr.x, pr.y, ps.x, ps.y));
     }
     __syncthreads();
-    // ---- intermediates on the 17 x 17 cells and corners
-#pragma unroll
-    for (int e = 0; e < 2; ++e) {
-        const int q = tid + 256 * e;
-        if (q < 289) {
-            const float hh = e ? cc1.x : cc0.x, dimp = e ? cc1.y : cc0.y, hc = e ? ch1 : ch0;
-            const int x = q % 17, y = q / 17;
-            const float u0 = sm.U[y][x], u1 = sm.U[y][x + 1], v0 = sm.V[y][x], v1 = sm.V[y + 1][x];
-            const float dudx = rdx * (u1 - u0), dvdy = rdy * (v1 - v0);
-            sm.rxx[y][x] = 2.f * hh * (2.f * dudx + dvdy);
-            sm.ryy[y][x] = 2.f * hh * (2.f * dvdy + dudx);
-            const float divq = rdx * (sm.HU[y][x + 1] * u1 - sm.HU[y][x] * u0) +
-                               rdy * (sm.HV[y + 1][x] * v1 - sm.HV[y][x] * v0);
-            sm.ext[y][x] = dimp * divq;
-            sm.rxy[y][x] = hc * (rdy * (sm.U[y + 1][x + 1] - sm.U[y][x + 1]) +
-                                 rdx * (sm.V[y + 1][x + 1] - sm.V[y + 1][x]));
-        }
-    }
+    // ---- intermediates of the cell (x, y) of the 17 x 17 window, whose own
+    // point has the value uv and the thickness h
+    auto intermediates = [&](int x, int y, float2 uv, float2 h, float2 hd, float hc) -> float4 {
+        const float u1 = sm.UV[y][x + 1].x, v1 = sm.UV[y + 1][x].y;
+        const float2 d = sm.UV[y + 1][x + 1];
+        const float dudx = rdx * (u1 - uv.x), dvdy = rdy * (v1 - uv.y);
+        const float divq = rdx * (sm.H[y][x + 1].x * u1 - h.x * uv.x) + rdy * (sm.H[y + 1][x].y * v1 - h.y * uv.y);
+        return make_float4(2.f * hd.x * (2.f * dudx + dvdy), 2.f * hd.x * (2.f * dvdy + dudx),
+                           hc * (rdy * (d.x - u1) + rdx * (d.y - v1)), hd.y * divq);
+    };
+    const float2 uv = sm.UV[ly + 1][lx + 1];
+    const float4 own = intermediates(lx + 1, ly + 1, uv, oH, cc, ch);
+    if (w == 0) sm.cell[ey][ex] = intermediates(ex, ey, sm.UV[ey][ex], sm.H[ey][ex], ec, eh);
+    sm.cell[ly + 1][lx + 1] = own;
     __syncthreads();
     // ---- A at the tile's points (zero off the inner masks), R x pass
     {
-        const int x = lx, y = ly;
-        const float d_rxx = rdx * (sm.rxx[y + 1][x + 1] - sm.rxx[y + 1][x]);
-        const float d_rxy_u = rdy * (sm.rxy[y + 1][x] - sm.rxy[y][x]);
-        const float d_ext_u = rdx * (sm.ext[y + 1][x + 1] - sm.ext[y + 1][x]);
-        const float Au = ((d_rxx + d_rxy_u) - bu0 * sm.U[y + 1][x + 1]) - sm.HU[y + 1][x + 1] * d_ext_u;
-        const float d_ryy = rdy * (sm.ryy[y + 1][x + 1] - sm.ryy[y][x + 1]);
-        const float d_rxy_v = rdx * (sm.rxy[y][x + 1] - sm.rxy[y][x]);
-        const float d_ext_v = rdy * (sm.ext[y + 1][x + 1] - sm.ext[y][x + 1]);
-        const float Av = ((d_ryy + d_rxy_v) - bv0 * sm.V[y + 1][x + 1]) - sm.HV[y + 1][x + 1] * d_ext_v;
+        const float4 left = sm.cell[ly + 1][lx], below = sm.cell[ly][lx + 1];
+        const float rxy00 = sm.cell[ly][lx].z;
+        const float d_rxx = rdx * (own.x - left.x);
+        const float d_rxy_u = rdy * (left.z - rxy00);
+        const float d_ext_u = rdx * (own.w - left.w);
+        const float Au = ((d_rxx + d_rxy_u) - oB.x * uv.x) - oH.x * d_ext_u;
+        const float d_ryy = rdy * (own.y - below.y);
+        const float d_rxy_v = rdx * (below.z - rxy00);
+        const float d_ext_v = rdy * (own.w - below.w);
+        const float Av = ((d_ryy + d_rxy_v) - oB.y * uv.y) - oH.y * d_ext_v;
         float a0 = inu ? Au : 0.f, a1 = inv ? Av : 0.f;
         haar_lines_R<LEV>(a0, a1, lx);
-        sm.T[0][ly][lx] = a0;
-        sm.T[1][ly][lx] = a1;
+        sm.T[0][ly][lx] = make_float2(a0, a1);
     }
     __syncthreads();
     // ---- R y pass, wavelet mask (w), P y pass
     {
-        float c0 = sm.T[0][cy][cx], c1 = sm.T[1][cy][cx];
+        const float2 t0 = sm.T[0][cy][cx];
+        float c0 = t0.x, c1 = t0.y;
         haar_lines_R<LEV>(c0, c1, cy);
-        const float w0 = (sm.mb[0][cy][cx] & 2) ? c0 : 0.f;
-        const float w1 = (sm.mb[1][cy][cx] & 2) ? c1 : 0.f;
-        float q0 = w0, q1v = w1;
+        const unsigned m = sm.mb[cy][cx];
+        const float2 wn = make_float2((m & CB_WAVELET_U) ? c0 : 0.f, (m & CB_WAVELET_V) ? c1 : 0.f);
+        float q0 = wn.x, q1 = wn.y;
         if constexpr (PRE) {
-            q0 = sm.dz[0][cy][cx] * w0;
-            q1v = sm.dz[1][cy][cx] * w1;
+            const float2 d = sm.dz[cy][cx];
+            q0 = d.x * wn.x;
+            q1 = d.y * wn.y;
         }
-        haar_lines_P<LEV>(q0, q1v, cy);
-        sm.T[0][cy][cx] = w0;
-        sm.T[1][cy][cx] = w1;
-        sm.T[2][cy][cx] = q0;
-        sm.T[3][cy][cx] = q1v;
+        haar_lines_P<LEV>(q0, q1, cy);
+        sm.T[0][cy][cx] = wn;
+        sm.T[1][cy][cx] = make_float2(q0, q1);
     }
     __syncthreads();
     // ---- P x pass, stores, partials of (r, r) and (w, r)
-    const float wn_u = sm.T[0][ly][lx], wn_v = sm.T[1][ly][lx];
-    float tw_u = sm.T[2][ly][lx], tw_v = sm.T[3][ly][lx];
+    const float2 wn = sm.T[0][ly][lx], tq = sm.T[1][ly][lx];
+    float tw_u = tq.x, tw_v = tq.y;
     haar_lines_P<LEV>(tw_u, tw_v, lx);
-    st_nt(&el(arr(CGM_W), ob), wn_u);
-    st_nt(&el(arr(CGM_W + 1), ob), wn_v);
-    {
-        const RingSlots rs(lx, ly);
-        const unsigned rb = ring_at(NP, ntile, tile_id, 2, 0);
-        rs.put(a.R, rb, inu ? tw_u : 0.f);
-        rs.put(a.R, rb + 64, inv ? tw_v : 0.f);
-    }
+    cstore(CGM_W, wn);
+    RingSlots(lx, ly).put(a.R.w + ring_at(NP, ntile, tile_id), make_float2(inu ? tw_u : 0.f, inv ? tw_v : 0.f));
     // (r, u) and (w, u) with u = D^-1 r under Jacobi, (r, r) and (w, r) without
-    const float zr_u = PRE ? dz_u * r_u : r_u, zr_v = PRE ? dz_v * r_v : r_v;
-    float gg = r_u * zr_u + r_v * zr_v;
-    float dd = wn_u * zr_u + wn_v * zr_v;
+    const float zr_u = PRE ? dz.x * r.x : r.x, zr_v = PRE ? dz.y * r.y : r.y;
+    float gg = r.x * zr_u + r.y * zr_v;
+    float dd = wn.x * zr_u + wn.y * zr_v;
     gg = wave_total_rows_f(row_sum16f(gg));
     dd = wave_total_rows_f(row_sum16f(dd));
-    if ((tid & 63) == 63) {
-        sm.red1[tid >> 6] = gg;
-        sm.red1[4 + (tid >> 6)] = dd;
+    if (l == 63) {
+        sm.red1[w] = gg;
+        sm.red1[4 + w] = dd;
     }
     __syncthreads();
     if (tid == 0)
