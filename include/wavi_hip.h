@@ -373,15 +373,18 @@ int wavi_set_smoother_tile(wavi_ctx *ctx, int tx, int ty);
 int wavi_smoother_tile(const wavi_ctx *ctx, int *tx, int *ty);
 
 /* How the coarse CG of the V-cycle runs (update_preconditioners.jl:73).
- * WAVI_CG_LAUNCHES: one launch per CG iteration over all tiles (three in
- * FP64, one in mixed precision), queued in chunks.  WAVI_CG_WORKGROUP: the
- * whole CG in one launch of one workgroup, which runs each iteration on the
- * tiles in turn, with no launch and no host round trip between iterations.
- * Both give the same bits.  WAVI_CG_AUTO (the default) is the library's
- * choice, at present WAVI_CG_LAUNCHES for every grid: measured on MI355X,
- * the workgroup is 3.4 to 3.6 times slower per iteration even on a grid of
- * six 16 x 16 tiles.  wavi_coarse_cg reports the mode in effect for the
- * context.  Lockstep batches (wavi_update_velocities_lockstep*) and the
+ * WAVI_CG_LAUNCHES: launches over all tiles per CG iteration (two in FP64,
+ * one in mixed precision), queued in chunks.  WAVI_CG_WORKGROUP: the whole CG
+ * in one launch of one workgroup, which runs each iteration on the tiles in
+ * turn, with no launch and no host round trip between iterations.
+ * WAVI_CG_AUTO (the default) is the library's choice: in FP64, while all tiles
+ * fit on the chip at once (up to 504 on MI355X), the whole CG in one launch
+ * of a workgroup per tile, which exchange sums and halos among themselves
+ * (7.1 us per iteration against 9.5 at 63 tiles); else WAVI_CG_LAUNCHES.  The
+ * workgroup is 3.4 to 3.6 times slower per iteration than the launches even on
+ * a grid of six 16 x 16 tiles.  All give the same bits.  wavi_coarse_cg
+ * reports the mode in effect for the context (WAVI_CG_LAUNCHES for
+ * WAVI_CG_AUTO).  Lockstep batches (wavi_update_velocities_lockstep*) and the
  * small members of wavi_misfit_gradient_batch share one launch per CG
  * iteration whatever the mode.  No reference counterpart. */
 #define WAVI_CG_AUTO 0
@@ -393,16 +396,17 @@ int wavi_coarse_cg(const wavi_ctx *ctx, int *mode);
 /* Kernel timing with HIP events on the context's stream, for measurement.
  * Sampled single launches (events around every 16th launch, so each time
  * includes the cost of the two event records): WAVI_KT_CG_APPLY (FP64
- * coarse CG: A then R on one tile, dot partials), WAVI_KT_CG_DIR (direction
- * update and prolongation), WAVI_KT_CG_UPDATE (axpys and norm partials),
+ * coarse CG: direction, P, A, R on one tile, dot partials), WAVI_KT_CG_DIR (no
+ * longer a launch of its own: 0), WAVI_KT_CG_UPDATE (axpys and norm partials),
  * WAVI_KT_COLOUR (one smoother iteration: its four colour sweeps in one
  * launch).  Bursts (events around each
  * chunk of 32 back-to-back iterations; only chunks in which every launch
  * still iterates are counted, and the count is of launches):
  * WAVI_KT_CG_ITER_MIXED (mixed-precision coarse CG, one whole iteration per
  * launch of k_cgm_iter) and WAVI_KT_CG_ITER_FP64 (FP64 coarse CG, one
- * iteration = k_cg_dir + k_cg_apply + k_cg_update).  FP64 chunks alternate
- * between burst timing and the sampled single launches.
+ * iteration = k_cg_step + k_cg_update).  FP64 chunks alternate between burst
+ * timing and the sampled single launches.  A CG in one launch is timed whole
+ * and counts its iterations.
  * enable=1 starts (and clears) the accumulation; wavi_profile_read returns
  * the total milliseconds and the number of timed launches (iterations).
  * No reference counterpart. */

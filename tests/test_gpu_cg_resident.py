@@ -1,0 +1,82 @@
+"""The FP64 coarse CG in one launch of resident workgroups: the same bits and
+the same iteration counts as the launches per iteration and as the oracle, on
+both sides of the tile counts where the folding of its sums (32 tiles) and its
+instance (two or four workgroups per CU) change, for every Haar level, and
+where its waits run out at once and the CG runs again in one workgroup."""
+import numpy as np
+import pytest
+
+
+def _mode(W, m, resident):
+    spec = m.parallel_spec
+    assert spec._lib.wavi_set_coarse_cg(spec.ctx, W._lib.WAVI_CG_AUTO if resident else W._lib.WAVI_CG_LAUNCHES) == 0
+
+
+def _solve(W, monkeypatch, nx, ny, levels=3, resident=True, polls=None, maxiter_coarse=40, calls=2, **kw):
+    if polls is not None:
+        monkeypatch.setenv("WAVI_CG_POLLS", str(polls))
+    m = W.workloads.channel_solve(nx=nx, ny=ny, nσ=4, maxiter_picard=3, **kw)
+    m.solver_params.levels = levels
+    m.solver_params.maxiter_coarse = maxiter_coarse
+    out = []
+    for _ in range(calls):
+        W.update_geometry(m)
+        _mode(W, m, resident)
+        W.update_velocities(m)
+        out.append((m.fields.gu.u.copy(), m.fields.gv.v.copy(), dict(m.last_report)))
+    monkeypatch.delenv("WAVI_CG_POLLS", raising=False)
+    return out
+
+
+def _equal(a, b):
+    for (u, v, r), (x, y, q) in zip(a, b):
+        np.testing.assert_array_equal(u, x)
+        np.testing.assert_array_equal(v, y)
+        assert r == q
+
+
+# 6 tiles; 31, 32 and 33 tiles in a row; 11 x 3; 246; 441 and 504 (two per CU); 512 and 891 (the launches)
+@pytest.mark.gpu
+@pytest.mark.parametrize("nx,ny", [(80, 10), (495, 14), (511, 15), (527, 12), (161, 33), (640, 80), (1007, 111), (1007, 120),
+                                   (1023, 127), (1280, 160)])
+def test_resident_cg_equals_the_launches(W, monkeypatch, nx, ny):
+    print("[gpu] resident CG %dx%d" % (nx, ny), flush=True)
+    _equal(_solve(W, monkeypatch, nx, ny), _solve(W, monkeypatch, nx, ny, resident=False))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nx,ny", [(77, 35), (250, 62)])
+@pytest.mark.parametrize("levels", [0, 1, 2])
+def test_resident_cg_at_every_level(W, monkeypatch, nx, ny, levels):
+    print("[gpu] resident CG %dx%d levels %d" % (nx, ny, levels), flush=True)
+    _equal(_solve(W, monkeypatch, nx, ny, levels), _solve(W, monkeypatch, nx, ny, levels, resident=False))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nx,ny", [(80, 10), (250, 62)])
+def test_waits_that_run_out_start_the_cg_over(W, monkeypatch, nx, ny):
+    """polls = 0: the first poll that does not find its words ends the launch;
+    the CG then runs in one workgroup from the same start, and the context
+    takes the launches per iteration from then on."""
+    print("[gpu] resident CG without polls %dx%d" % (nx, ny), flush=True)
+    _equal(_solve(W, monkeypatch, nx, ny, polls=0), _solve(W, monkeypatch, nx, ny, resident=False))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nx,ny", [(64, 16), (250, 62)])
+def test_resident_cg_in_the_adjoint(W, nx, ny):
+    """The Jacobi-preconditioned form, inside the linear solves."""
+    print("[gpu] resident CG in the adjoint %dx%d" % (nx, ny), flush=True)
+    res = []
+    for on in (True, False):
+        logc = W.workloads.inversion_logc_true(nx, ny, seed=4)
+        m = W.workloads.inversion_model(logc, "fp64", nσ=4, n_picard=2)
+        W.update_geometry(m)
+        _mode(W, m, on)
+        g = m.grid
+        rng = np.random.default_rng(1)
+        J, grad, rep = W.misfit_gradient(m, 2, 100 * rng.random(g.xxu.shape), 10 * rng.random(g.yyv.shape))
+        res.append((J, grad, rep))
+    assert res[0][0] == res[1][0]
+    np.testing.assert_array_equal(res[0][1], res[1][1])
+    assert res[0][2] == res[1][2]

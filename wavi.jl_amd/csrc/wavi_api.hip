@@ -65,6 +65,9 @@ struct VSet {
     DevVecT<T> h, beff, e, r, d, rho, t, cr, ct, xc;
 };
 
+// Polls of one wait of k_cg_resident, at least half a microsecond each.
+constexpr unsigned X_POLLS = 1u << 21;
+
 struct wavi_ctx {
     int device = 0;
     hipStream_t stream = nullptr;
@@ -99,6 +102,19 @@ struct wavi_ctx {
     double2 *arena64 = nullptr;
     uint8_t *marena64 = nullptr;
     unsigned px64 = 0, ns64 = 0;
+    // the CG in one launch (k_cg_resident): its exchange words (null: the grid
+    // does not fit on the chip), the next tag, and what it holds of the chip
+    // until the host has seen its end
+    xword *xwords = nullptr;
+    size_t n_xwords = 0;
+    unsigned xtag = 1;
+    unsigned x_polls = X_POLLS;
+    void (*x_fn[2])(CGArgs, CGExchange) = {};  // plain, Jacobi-preconditioned
+    int x_blocks = 0;               // workgroups of its launch
+    int x_units = 0;                // ... and their share of the chip (room_take)
+    bool x_off = false;             // a wait ran out once: the launches per iteration from then on
+    bool x_ran = false;             // the last CG ran so (k_cg_finish)
+    bool x_pending = false;         // ... and its report has not been read
     VSet<float> v32;
     // mixed-precision coarse CG: s, w, the parity-buffered images P r, P s,
     // P w and partials of (r, r) and (w, r)
@@ -245,6 +261,35 @@ static void burst_collect(wavi_ctx *ctx, int kid, int last_active)
         int rc_ = (expr);         \
         if (rc_ != WAVI_OK) return rc_; \
     } while (0)
+
+// How much of each GPU is taken by launches whose workgroups wait for one
+// another (k_cg_resident), in units of 1 / CU_UNITS of a CU.  A launch that waits
+// must have all its workgroups on the chip; alone it may take all of it.
+// Beside another one it may only bring the sum to half of the chip: a
+// workgroup takes at most half a CU, so then some CU always has room for the
+// next one, however the others lie.  Kernels that do not wait need no
+// place here: they end.  A launch that finds no room is not made: the CG then
+// takes a pair of launches per iteration.
+constexpr int CU_UNITS = 64;
+static std::mutex g_room_mu;
+static int g_room_used[MAX_DEVICES] = {};
+static int g_room[MAX_DEVICES] = {};  // CUs x CU_UNITS
+
+static bool room_take(int device, int units)
+{
+    if (device < 0 || device >= MAX_DEVICES) return false;
+    std::lock_guard<std::mutex> lock(g_room_mu);
+    const int used = g_room_used[device];
+    if (used + units > (used == 0 ? g_room[device] : g_room[device] / 2)) return false;
+    g_room_used[device] = used + units;
+    return true;
+}
+
+static void room_give(int device, int units)
+{
+    std::lock_guard<std::mutex> lock(g_room_mu);
+    g_room_used[device] -= units;
+}
 
 static inline dim3 flat(int n) { return dim3((unsigned)((n + 255) / 256)); }
 // workgroups of a launch over an nbx x nby tile grid with xcd_band_tile: a multiple of 8
@@ -430,6 +475,32 @@ static int run_members(wavi_ctx **ctxs, int n, int nthreads, int *codes, F &&fn)
 }
 
 // ---------------------------------------------------------------------------
+// Partials that a lane of the CG's folds loads with the kernels' other
+// inputs: all of them on grids of up to 2048 partials (npart: one per tile
+// and component).
+constexpr int CG_FOLD_LARGE = 8;
+
+// Tiles up to which every workgroup of k_cg_resident folds the partials itself.
+constexpr int X_FLAT_TILES = 32;
+// The instance of k_cg_resident for a grid of ntile tiles.
+typedef void (*CGResidentFn)(CGArgs, CGExchange);
+
+template <bool PRE, int LEV>
+static CGResidentFn cg_resident_fn_p(int ntile)
+{
+    return ntile <= X_FLAT_TILES ? k_cg_resident<PRE, LEV, true> : k_cg_resident<PRE, LEV, false>;
+}
+
+static CGResidentFn cg_resident_fn(int levels, bool pre, int ntile)
+{
+    switch (levels) {
+    case 0: return pre ? cg_resident_fn_p<true, 0>(ntile) : cg_resident_fn_p<false, 0>(ntile);
+    case 1: return pre ? cg_resident_fn_p<true, 1>(ntile) : cg_resident_fn_p<false, 1>(ntile);
+    case 2: return pre ? cg_resident_fn_p<true, 2>(ntile) : cg_resident_fn_p<false, 2>(ntile);
+    default: return pre ? cg_resident_fn_p<true, 3>(ntile) : cg_resident_fn_p<false, 3>(ntile);
+    }
+}
+
 extern "C" {
 #pragma GCC visibility push(default)
 
@@ -675,6 +746,27 @@ int wavi_ctx_create(const wavi_grid_desc *grid, const wavi_phys_params *phys, co
         CREATECHK(hipMemset(ctx->arena64, 0, bytes));
         CREATECHK(hipMalloc(&ctx->marena64, ns));
         CREATECHK(hipMemset(ctx->marena64, 0, ns));
+        const int ntile = g.nbx * g.nby;
+        int occ[2] = {}, cus = 0;
+        CREATECHK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device));
+        for (int pre = 0; pre < 2; ++pre) {
+            ctx->x_fn[pre] = cg_resident_fn(solver->levels, pre != 0, ntile);
+            CREATECHK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ[pre], ctx->x_fn[pre], 256, 0));
+        }
+        if (ctx->device < MAX_DEVICES) {
+            std::lock_guard<std::mutex> rlock(g_room_mu);
+            g_room[ctx->device] = cus * CU_UNITS;
+        }
+        ctx->x_blocks = ctx->nblk + (ntile <= X_FLAT_TILES ? 0 : 8);
+        const int per_cu = std::min(occ[0], occ[1]);
+        if (per_cu >= 2 && ctx->x_blocks <= cus * per_cu && g.npart <= 1024 && solver->maxiter_coarse < (1 << 28)) {
+            const char *polls = getenv("WAVI_CG_POLLS");  // the polls of a wait
+            if (polls) ctx->x_polls = (unsigned)std::max(0, atoi(polls));
+            ctx->x_units = ctx->x_blocks * ((CU_UNITS + per_cu - 1) / per_cu);
+            ctx->n_xwords = 4 * ns + 6 * (size_t)g.npart + 32 + X_COPIES * X_COPY;
+            CREATECHK(hipMalloc(&ctx->xwords, ctx->n_xwords * sizeof(xword)));
+            CREATECHK(hipMemset(ctx->xwords, 0, ctx->n_xwords * sizeof(xword)));
+        }
     }
     if (precision_mode == WAVI_PRECISION_MIXED) {
         VSet<float> &w = ctx->v32;
@@ -728,6 +820,7 @@ int wavi_ctx_destroy(wavi_ctx *ctx)
 static void ctx_free(wavi_ctx *ctx)
 {
     if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
+    if (ctx->x_pending) room_give(ctx->device, ctx->x_units);
     for (uint8_t *p : {ctx->hm, ctx->hfix, ctx->um, ctx->vm, ctx->cm, ctx->ui, ctx->vi, ctx->ufix, ctx->vfix,
                        ctx->mwu, ctx->mwv, ctx->saved_mwu, ctx->saved_mwv})
         if (p) (void)hipFree(p);
@@ -753,7 +846,7 @@ static void ctx_free(wavi_ctx *ctx)
         }
     }
     for (void *p : {(void *)ctx->arena, (void *)ctx->marena, (void *)ctx->Pgd, (void *)ctx->rings, (void *)ctx->arena64,
-                    (void *)ctx->marena64})
+                    (void *)ctx->marena64, (void *)ctx->xwords})
         if (p) (void)hipFree(p);
     if (ctx->stm) (void)hipFree(ctx->stm);
     if (ctx->h_flag) (void)hipHostFree(ctx->h_flag);
@@ -1262,6 +1355,8 @@ static CGIo cg_io(wavi_ctx *ctx, const VSet<double> &w)
     io.dinvv = ctx->cdinv.v;
     io.eu = w.e.u;
     io.ev = w.e.v;
+    io.abort = &ctx->st->abort;
+    io.resident = ctx->x_ran;
     return io;
 }
 
@@ -1302,7 +1397,8 @@ constexpr double CGM_FP32_RELTOL = 0x1p-19;
 constexpr double CGM_FP32_JACOBI_RELTOL = 0x1p-14;
 
 // The coarse CG runs in one workgroup (k_cg_solve1, k_cgm_solve1) only when
-// wavi_set_coarse_cg asks for it: on MI355X one workgroup spends about 3 us
+// wavi_set_coarse_cg asks for it, or in the place of a resident CG that gave
+// up (cg_try_resident): on MI355X one workgroup spends about 3 us
 // per tile and iteration (a tile's chain of loads, barriers and stores),
 // so even a 6-tile grid (80 x 10) takes 3.4 (mixed) to 3.6 (FP64) times as
 // long per CG iteration as the launches over all tiles, whose tiles run
@@ -1327,11 +1423,6 @@ static void launch_tile_haar(wavi_ctx *ctx, int dir, const T *inu, const T *inv,
 
 // The kernels of the FP64 coarse CG at the context's Haar level,
 // Jacobi-preconditioned inside a linear solve (ctx->cg_pre).
-// Partials that a lane of the CG's folds loads with the kernels' other
-// inputs: all of them on grids of up to 2048 partials (npart: one per tile
-// and component).
-constexpr int CG_FOLD_LARGE = 8;
-
 template <bool PRE, int FOLD>
 static void launch_cg_step_p(wavi_ctx *ctx, dim3 tb, const CGArgs &a, int par)
 {
@@ -1362,21 +1453,79 @@ static void launch_cg_update(wavi_ctx *ctx, dim3 tb, const CGArgs &a, int par)
 }
 
 template <bool PRE>
-static void launch_cg_solve1_p(wavi_ctx *ctx, const CGArgs &a)
+static void launch_cg_solve1_p(wavi_ctx *ctx, const CGArgs &a, const int *only_if = nullptr)
 {
     switch (ctx->S.levels) {
-    case 0: hipLaunchKernelGGL((k_cg_solve1<PRE, 0>), dim3(1), dim3(256), 0, ctx->stream, a); break;
-    case 1: hipLaunchKernelGGL((k_cg_solve1<PRE, 1>), dim3(1), dim3(256), 0, ctx->stream, a); break;
-    case 2: hipLaunchKernelGGL((k_cg_solve1<PRE, 2>), dim3(1), dim3(256), 0, ctx->stream, a); break;
-    default: hipLaunchKernelGGL((k_cg_solve1<PRE, 3>), dim3(1), dim3(256), 0, ctx->stream, a); break;
+    case 0: hipLaunchKernelGGL((k_cg_solve1<PRE, 0>), dim3(1), dim3(256), 0, ctx->stream, a, only_if); break;
+    case 1: hipLaunchKernelGGL((k_cg_solve1<PRE, 1>), dim3(1), dim3(256), 0, ctx->stream, a, only_if); break;
+    case 2: hipLaunchKernelGGL((k_cg_solve1<PRE, 2>), dim3(1), dim3(256), 0, ctx->stream, a, only_if); break;
+    default: hipLaunchKernelGGL((k_cg_solve1<PRE, 3>), dim3(1), dim3(256), 0, ctx->stream, a, only_if); break;
     }
+}
+
+// After the stream has been waited for: the iterations of a resident CG whose
+// report is still to be read, 0 if there is none.
+static int cg_collect(wavi_ctx *ctx, int *iters)
+{
+    *iters = 0;
+    if (!ctx->x_pending) return WAVI_OK;
+    ctx->x_pending = false;
+    room_give(ctx->device, ctx->x_units);
+    volatile CGMHostFlag *hf = ctx->h_flag;
+    if (!hf->done) {
+        ctx->err = "coarse CG did not terminate";
+        return WAVI_ESTATE;
+    }
+    if (hf->gave_up) ctx->x_off = true;
+    *iters = hf->iters;
+    for (wavi_ctx::Burst &b : ctx->bursts) b.n = hf->iters;
+    burst_collect(ctx, WAVI_KT_CG_ITER_FP64, hf->gave_up ? -1 : 0);
+    return WAVI_OK;
+}
+
+// The FP64 coarse CG in one launch if the context can have it now: then
+// queues it and what stands in for it should a wait run out, and returns
+// true; the report is read by cg_collect once the stream has got there.
+static bool cg_try_resident(wavi_ctx *ctx, const CGArgs &a)
+{
+    ctx->x_ran = false;
+    if (ctx->x_pending) {  // left by a call that ended with an error
+        int lost = 0;
+        if (hipStreamSynchronize(ctx->stream) != hipSuccess) return false;
+        (void)cg_collect(ctx, &lost);
+    }
+    if (!ctx->xwords || ctx->x_off || ctx->cg_mode != WAVI_CG_AUTO || !room_take(ctx->device, ctx->x_units)) return false;
+    if (ctx->xtag > 0xffffffffu - (unsigned)a.maxiter - 2u) {  // tags used up: clear the words and begin again
+        hipLaunchKernelGGL(k_fill<xword>, flat((int)ctx->n_xwords), dim3(256), 0, ctx->stream, ctx->xwords, (xword)0,
+                           (int)ctx->n_xwords);
+        ctx->xtag = 1;
+    }
+    CGExchange E;
+    E.c = ctx->xwords;
+    E.pd = E.c + 4 * (size_t)ctx->ns64;
+    E.pr = E.pd + 2 * ctx->g.npart;
+    E.root = ctx->xwords + (ctx->n_xwords / 32 * 32 - X_COPIES * X_COPY);  // whole lines at the end
+    E.abort = &ctx->st->abort;
+    E.tag = ctx->xtag;
+    E.limit = ctx->x_polls;
+    ctx->xtag += (unsigned)a.maxiter + 2u;
+    const int bev = burst_begin(ctx);
+    hipLaunchKernelGGL(ctx->x_fn[ctx->cg_pre], dim3(ctx->x_blocks), dim3(256), 0, ctx->stream, a, E);
+    burst_end(ctx, bev, 0, 0);
+    if (ctx->cg_pre)
+        launch_cg_solve1_p<true>(ctx, a, &ctx->st->abort);
+    else
+        launch_cg_solve1_p<false>(ctx, a, &ctx->st->abort);
+    ctx->x_ran = ctx->x_pending = true;
+    return true;
 }
 
 template <typename T>
 static int do_coarse_cg(wavi_ctx *ctx, const VSet<T> &w, int *iters);
 
 // FP64 coarse CG on b_c held in w.cr from the warm start w.xc; the solution
-// stays in the arena until k_cg_finish.
+// stays in the arena until k_cg_finish.  A resident CG is only queued, and
+// its iterations are not known yet (0): cg_collect has them.
 template <>
 int do_coarse_cg<double>(wavi_ctx *ctx, const VSet<double> &w, int *iters)
 {
@@ -1398,6 +1547,11 @@ int do_coarse_cg<double>(wavi_ctx *ctx, const VSet<double> &w, int *iters)
     else
         hipLaunchKernelGGL(k_cg_setup<false>, tb, dim3(256), 0, ctx->stream, a, io);
     HIPCHK(hipGetLastError());
+    *iters = 0;
+    if (cg_try_resident(ctx, a)) {
+        HIPCHK(hipGetLastError());
+        return WAVI_OK;
+    }
     volatile CGMHostFlag *hf = ctx->h_flag;
     if (cg_one_workgroup(ctx)) {
         if (pre)
@@ -1789,13 +1943,22 @@ static int vcycle_widen(wavi_ctx *ctx)
     return WAVI_OK;
 }
 
-static int do_vcycle(wavi_ctx *ctx, int *cg_iters)
+// A V-cycle, whose coarse CG's report may still be to be read (cg_collect).
+static int queue_vcycle(wavi_ctx *ctx, int *cg_iters)
 {
     if (ctx->precision == WAVI_PRECISION_FP64) return do_vcycle_t<double>(ctx, vset64(ctx), cg_iters);
     CHK(vcycle_narrow(ctx));
     VSet<float> &w = ctx->v32;
     CHK(do_vcycle_t<float>(ctx, w, cg_iters));
     return vcycle_widen(ctx);
+}
+
+static int do_vcycle(wavi_ctx *ctx, int *cg_iters)
+{
+    CHK(queue_vcycle(ctx, cg_iters));
+    if (!ctx->x_pending) return WAVI_OK;
+    HIPCHK(hipStreamSynchronize(ctx->stream));
+    return cg_collect(ctx, cg_iters);
 }
 
 // precondition!(model, ::BasicParallelSpec) (update_velocities.jl:50-83),
@@ -1862,16 +2025,37 @@ static int coarse_start(wavi_ctx *ctx, double rel)
     return WAVI_OK;
 }
 
-static int do_precondition(wavi_ctx *ctx, int *converged, double *rel, int *cg_iters)
+// *prev_iters: the iterations of the coarse CG before, if they were still to
+// be read (else 0); *cg_iters: those of this one, 0 if still to be read.
+static int do_precondition(wavi_ctx *ctx, int *converged, double *rel, int *prev_iters, int *cg_iters)
 {
     CHK(precondition_resid(ctx));
     CHK(precondition_decide(ctx, converged, rel));
+    CHK(cg_collect(ctx, prev_iters));
     *cg_iters = 0;
     if (!*converged) {
         CHK(coarse_start(ctx, *rel));
-        CHK(do_vcycle(ctx, cg_iters));
+        CHK(queue_vcycle(ctx, cg_iters));
         CHK(precondition_update(ctx));
     }
+    return WAVI_OK;
+}
+
+// coarse-CG iterations of Picard iteration it
+static void report_cg(wavi_solve_report *rep, int it, int cg)
+{
+    rep->coarse_cg_total += cg;
+    if (it <= WAVI_REPORT_MAX_PICARD) rep->coarse_cg_iters[it - 1] += cg;
+}
+
+// Waits for the stream and adds what the last coarse CG of rep's solve left
+// to be read.
+static int finish_report(wavi_ctx *ctx, wavi_solve_report *rep)
+{
+    int cg = 0;
+    HIPCHK(hipStreamSynchronize(ctx->stream));
+    CHK(cg_collect(ctx, &cg));
+    if (rep && rep->picard_iters > 0) report_cg(rep, rep->picard_iters, cg);
     return WAVI_OK;
 }
 
@@ -1882,24 +2066,21 @@ static int do_update_velocities(wavi_ctx *ctx, wavi_solve_report *rep, bool wait
     wavi_solve_report local;
     if (!rep) rep = &local;
     memset(rep, 0, sizeof(*rep));
-    int converged = 0, it = 0, total = 0;
+    int converged = 0, it = 0;
     double rel = INFINITY;
     while (!converged && it < ctx->S.maxiter_picard) {
         it = it + 1;
         CHK(do_inner_update(ctx));
-        int cg = 0;
-        CHK(do_precondition(ctx, &converged, &rel, &cg));
-        total += cg;
-        if (it <= WAVI_REPORT_MAX_PICARD) {
-            rep->coarse_cg_iters[it - 1] = cg;
-            rep->rel_resid_hist[it - 1] = rel;
-        }
+        int cg = 0, prev = 0;
+        CHK(do_precondition(ctx, &converged, &rel, &prev, &cg));
+        if (it > 1) report_cg(rep, it - 1, prev);  // before the first: an earlier call's
+        report_cg(rep, it, cg);
+        if (it <= WAVI_REPORT_MAX_PICARD) rep->rel_resid_hist[it - 1] = rel;
     }
-    if (wait) HIPCHK(hipStreamSynchronize(ctx->stream));
     rep->picard_iters = it;
     rep->converged = converged;
     rep->rel_resid = rel;
-    rep->coarse_cg_total = total;
+    if (wait) CHK(finish_report(ctx, rep));
     // mixed precision: every Picard iteration is one FP64 residual refinement
     rep->refinements = ctx->precision == WAVI_PRECISION_MIXED ? it : 0;
     return WAVI_OK;
@@ -3138,8 +3319,7 @@ int wavi_run_steps(wavi_ctx *ctx, int nsteps, wavi_solve_report *last_report)
         CHK(do_update_state(ctx, last_report, false));
         CHK(do_update_thickness(ctx, ctx->P.dt));
     }
-    HIPCHK(hipStreamSynchronize(ctx->stream));
-    return WAVI_OK;
+    return finish_report(ctx, nsteps > 0 ? last_report : nullptr);
 }
 
 int wavi_update_wavelets(wavi_ctx *ctx)

@@ -244,6 +244,115 @@ __device__ __forceinline__ void lanes_sum2(const double *P, const double *Q, int
 }
 
 // ---------------------------------------------------------------------------
+// Words that the workgroups of one launch exchange: 32 data bits below a
+// 32-bit tag, stored and loaded whole (relaxed atomics at agent scope, which
+// the caches of the XCDs do not hold back).  A reader that finds the tag it
+// waits for has the data too, so an exchange needs no fence and no flag, and
+// takes one store's and one load's way to memory.  Tags grow, so a word is
+// never taken for a later one.
+typedef unsigned long long xword;
+
+__device__ __forceinline__ void xput(xword *p, unsigned tag, unsigned v)
+{
+    __hip_atomic_store(p, ((xword)tag << 32) | v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+__device__ __forceinline__ xword xget(const xword *p)
+{
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// a double in two words, high half first
+__device__ __forceinline__ void xput2(xword *p, unsigned tag, double v, size_t stride = 1)
+{
+    const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+    xput(p, tag, (unsigned)(b >> 32));
+    xput(p + stride, tag, (unsigned)b);
+}
+
+__device__ __forceinline__ double xdouble(xword hi, xword lo)
+{
+    return __longlong_as_double((long long)((hi << 32) | (lo & 0xffffffffull)));
+}
+
+// A wait for N words in a row: load(), then check() until it holds.  A wait
+// that is over, or not wanted, loads nothing.
+template <int N>
+struct XWait {
+    xword v[N];
+    bool on;
+    __device__ __forceinline__ void want(bool w)
+    {
+        on = w;
+#pragma unroll
+        for (int k = 0; k < N; ++k) v[k] = 0;
+    }
+    __device__ __forceinline__ void load(const xword *p, size_t stride = 1)
+    {
+        if (!on) return;
+#pragma unroll
+        for (int k = 0; k < N; ++k) v[k] = xget(p + k * stride);
+    }
+    __device__ __forceinline__ bool check(unsigned tag)
+    {
+        if (!on) return true;
+        bool ok = true;
+#pragma unroll
+        for (int k = 0; k < N; ++k) ok &= (unsigned)(v[k] >> 32) == tag;
+        on = !ok;
+        return ok;
+    }
+    __device__ __forceinline__ double value(int k) const { return xdouble(v[2 * k], v[2 * k + 1]); }
+};
+
+// ... for all np <= 256 K partials, thread L taking L, L + 256, ... as
+// LaneFold does.
+template <int K>
+struct XFold {
+    xword v[K][2];
+    int np;  // 0: over or not wanted
+    __device__ __forceinline__ void want(bool w, int n) { np = w ? n : 0; }
+    __device__ __forceinline__ void load(const xword *p)
+    {
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            const int q = (int)threadIdx.x + 256 * k;
+            if (q < np) {
+                v[k][0] = xget(p + 2 * q);
+                v[k][1] = xget(p + 2 * q + 1);
+            }
+        }
+    }
+    __device__ __forceinline__ bool check(unsigned tag)
+    {
+        bool ok = true;
+#pragma unroll
+        for (int k = 0; k < K; ++k)
+            if ((int)threadIdx.x + 256 * k < np)
+                ok &= (unsigned)(v[k][0] >> 32) == tag && (unsigned)(v[k][1] >> 32) == tag;
+        if (ok) np = 0;
+        return ok;
+    }
+    __device__ __forceinline__ double sum(int n) const
+    {
+        double acc = (int)threadIdx.x < n ? xdouble(v[0][0], v[0][1]) : 0.0;
+#pragma unroll
+        for (int k = 1; k < K; ++k) acc = acc + ((int)threadIdx.x + 256 * k < n ? xdouble(v[k][0], v[k][1]) : 0.0);
+        return acc;
+    }
+};
+
+// After poll n of a wait: whether to give up, having raised the abort flag;
+// also when another workgroup has raised it.
+__device__ __forceinline__ bool x_give_up(unsigned n, unsigned limit, int *abort)
+{
+    if (n < limit && (n & 255u) != 255u) return false;
+    if (n < limit && __hip_atomic_load(abort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0) return false;
+    __hip_atomic_store(abort, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return true;
+}
+
+// ---------------------------------------------------------------------------
 // Non-temporal store (streamed past the caches).
 template <typename T>
 __device__ __forceinline__ void st_nt(T *p, T v)

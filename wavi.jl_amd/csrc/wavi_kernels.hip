@@ -2194,6 +2194,7 @@ __global__ void k_scale_uv(double *u, int nu, double *v, int nv, double a)
 struct CGMHostFlag {
     int done;
     int iters;
+    int gave_up;  // the resident CG did, and k_cg_solve1 ran in its place
 };
 
 struct CGScalars {
@@ -2204,6 +2205,7 @@ struct CGScalars {
     int done;         // sticky stop flag, written only by k_cg_step
     int iters;        // iterations at termination
     double rz[2];     // Jacobi-preconditioned CG: (r, D^-1 r) by parity (written by k_cg_step)
+    int abort;        // a workgroup of k_cg_resident gave up waiting
 };
 
 // The FP64 coarse CG works in an arena of zero-padded 2-D arrays shared by
@@ -2273,6 +2275,8 @@ struct CGIo {
     const double *tu, *tv;            // P x0
     const double *dinvu, *dinvv;      // Jacobi: 1 / |diag(A_c)|, 0 off the wavelet masks
     double *eu, *ev;                  // the V-cycle's correction, += P x
+    const int *abort;                 // CGScalars::abort
+    int resident;                     // the CG ran as k_cg_resident
 };
 
 // XCD-aware tile order: workgroups are dispatched round-robin over the 8
@@ -2310,11 +2314,13 @@ __global__ void __launch_bounds__(256) k_cg_setup(CGArgs a, CGIo io)
         a.st->it[0] = 0;
         a.st->it[1] = 0;
         a.st->alpha = 0.0;
+        a.st->abort = 0;
         // also reset on the stream: launches queued past the previous
         // CG's stop, which rewrite the report, may still have been running
         // when the host reset it
         a.hflag->done = 0;
         a.hflag->iters = 0;
+        a.hflag->gave_up = 0;
     }
     int bx, by;
     band_tile(g, L, bx, by);
@@ -2393,7 +2399,8 @@ __global__ void __launch_bounds__(256) k_cg_finish(CGArgs a, CGIo io)
     int bx, by;
     band_tile(a.g, L, bx, by);
     const unsigned at = a.Lo.at(bx * TILE + (int)(threadIdx.x & 15), by * TILE + (int)(threadIdx.x >> 4));
-    const double2 x = elem32(a.Lo.pair(CG_X), at);
+    const bool resident = io.resident && *io.abort == 0;  // the resident CG leaves x in CG_Q
+    const double2 x = elem32(a.Lo.pair(resident ? CG_Q : CG_X), at);
     cg_finish_tile<double>(a.g, io.levels, bx, by, x.x, x.y, elem32(a.Lo.M, at), io.xu, io.xv, io.eu, io.ev);
 }
 
@@ -2476,6 +2483,210 @@ __device__ __forceinline__ int haar_row_terms(int i, int (&off)[LEV + 2])
     return plus;
 }
 
+// The geometry and the coefficients of a thread's part of a tile, and the
+// tile's c = R A P u from its own direction and the coarse halo's.
+template <int LEV>
+struct CgTile {
+    using T = double;
+    static constexpr int N = LEV + 2;
+    int l, w, lx, ly;
+    unsigned at0, at, h0, h1;         // arena index of the tile, the own point, the two coarse halo points
+    bool rows, after, corner;
+    int cx, cy;                       // corner entry
+    HaloPos h;
+    OpOwn<T> o;
+    OpCoefRegs<T> cr;
+    unsigned mb, hmb;                 // mask bits of the own and the halo point
+    int hoff[N], hplus;               // the halo point's terms in the x pass (wavefronts 2, 3)
+
+    __device__ __forceinline__ void place(const CGLayout &Lo, int i0, int j0)
+    {
+        lx = threadIdx.x & 15;
+        ly = threadIdx.x >> 4;
+        l = threadIdx.x & 63;
+        w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+        at0 = Lo.at(i0, j0);
+        at = at0 + lx + __umul24(Lo.px, (unsigned)ly);
+        // the coarse halo, one side per wavefront (left, right, below, above):
+        // line k = l / 16 of N, point l % 16 along it; the fifth line and the
+        // corner blocks (u below right, v above left) in a second round
+        rows = w >= 2;
+        after = (w & 1) != 0;
+        int di, dj;
+        {
+            const int c = haar_halo_offset<LEV>(after, l >> 4), q = l & 15;
+            di = rows ? q : c;
+            dj = rows ? c : q;
+        }
+        h0 = at0 + (unsigned)(di + (int)__mul24((int)Lo.px, dj));
+        const int e = l - 16;  // corner entry of lanes 16..40 of wavefronts 0 (v) and 1 (u)
+        cx = e % 5;
+        cy = e / 5;
+        corner = w < 2 && e >= 0 && e < 25;
+        {
+            const int c = haar_halo_offset<LEV>(after, 4), q = l & 15;
+            di = corner ? haar_halo_offset<LEV>(after, cx) : (rows ? q : c);
+            dj = corner ? haar_halo_offset<LEV>(!after, cy) : (rows ? c : q);
+        }
+        h1 = at0 + (unsigned)(di + (int)__mul24((int)Lo.px, dj));
+        // halo points: wavefront 3 the sides' u, wavefront 2 their v, wavefront 1
+        // the corners (u lane 0, v lane 1)
+        h = HaloPos{17, 0, 0, 17, w == 3 || (w == 1 && l == 0), w == 2 || (w == 1 && l == 1)};
+        if (w >= 2) {
+            halo_side(l, h.ux, h.uy);
+            h.vx = h.ux;
+            h.vy = h.uy;
+        }
+    }
+    // the coefficients, in the order of their first use
+    __device__ __forceinline__ void load_coef(const CGLayout &Lo)
+    {
+        cr.hhu = cr.hhv = 0.0;
+        const double2 oh = elem32(Lo.pair(CG_H), at);
+        hmb = 0;
+        if (w >= 1) {
+            const int hx = h.hu ? h.ux : h.vx, hy = h.hu ? h.uy : h.vy;
+            const unsigned ha = at0 + (unsigned)(hx - 1 + (int)__mul24((int)Lo.px, hy - 1));
+            cr.hhu = cr.hhv = elem32(reinterpret_cast<const double *>(Lo.pair(CG_H)), 2 * ha + (h.hu ? 0 : 1));
+            hmb = elem32(Lo.M, ha);
+        }
+        const double2 cell = elem32(Lo.pair(CG_CELL), at);
+        o.hetac = elem32(Lo.corner(), at);
+        op_extra_cell(l, cr);
+        if (w == 0) {
+            const unsigned ea = at0 + (unsigned)(cr.ex - 1 + (int)__mul24((int)Lo.px, cr.ey - 1));
+            const double2 ce = elem32(Lo.pair(CG_CELL), ea);
+            cr.ec = elem32(Lo.corner(), ea);
+            cr.eh = ce.x;
+            cr.ed = ce.y;
+        }
+        const double2 ob = elem32(Lo.pair(CG_B), at);
+        o.hu = oh.x;
+        o.hv = oh.y;
+        o.bu = ob.x;
+        o.bv = ob.y;
+        o.heta = cell.x;
+        o.dimp = cell.y;
+        if (l < 32) {
+            haar_halo_terms<LEV>(17, hoff);
+            hplus = l < 16 ? LEV + 1 : 0;
+        } else {
+            hplus = haar_row_terms<LEV>(l & 15, hoff);
+        }
+    }
+    // un: the direction at the own point; n0, n1: at the coarse halo points.
+    // Six barriers; the first is followed by the rest only if go() holds.
+    template <class Go>
+    __device__ __forceinline__ bool apply(T rdx, T rdy, double2 un, double2 n0, double2 n1, OpLds<T> &s, double2 &c,
+                                          Go go)
+    {
+        s.p.t[0][ly][lx] = un.x;
+        s.p.t[1][ly][lx] = un.y;
+        {
+            const int k = (w & 1) * 5 + (l >> 4), q = l & 15;
+            if (rows) {
+                s.n.y[0][k][q] = n0.x;
+                s.n.y[1][k][q] = n0.y;
+                if (l < 16) {
+                    s.n.y[0][k + 4][q] = n1.x;
+                    s.n.y[1][k + 4][q] = n1.y;
+                }
+            } else {
+                s.n.x[0][k][q] = n0.x;
+                s.n.x[1][k][q] = n0.y;
+                if (l < 16) {
+                    s.n.x[0][k + 4][q] = n1.x;
+                    s.n.x[1][k + 4][q] = n1.y;
+                } else if (corner) {
+                    s.n.c[1 - w][cy][cx] = w == 1 ? n1.x : n1.y;
+                }
+            }
+        }
+        __syncthreads();
+        if (!go()) return false;
+        // y pass: the tile's lines; the columns' lines (40 half lines; lanes
+        // 40..63 repeat the first); rows -1 and 16 of the neighbours below and
+        // above (lanes 0..15) and the corners (16..20 of wavefronts 0, 1).  The
+        // operands of all three are read before the first is used.
+        {
+            const int q = l & 15, comp = (l >> 4) & 1, half = l >> 5;
+            const int hl = l < 40 ? l : l - 40, line = hl < 20 ? hl : hl - 20, lh = hl < 20 ? 0 : 1;
+            const int cp = w & 1, side = w >> 1;
+            const bool edge = l < 16;
+            const T *se = edge ? &s.n.y[cp][5 * side][l] : &s.n.c[cp][0][l < 20 ? l - 16 : 4];
+            int off[N];
+            haar_halo_terms<LEV>(edge ? 16 : 5, off);
+            HaarLineP<LEV, T> own, hal;
+            HaarRow<LEV, T> row;
+            own.load(&s.p.t[comp][0][q], TILE + 1, half, w);
+            hal.load(&s.n.x[0][0][0] + 17 * line, 1, lh, w);
+            row.load(se, off);
+            own.rows(&s.p.m[comp][0][q], TILE + 1, half, w);
+            hal.rows(&s.n.lx[0][0][0] + 17 * line, 1, lh, w);
+            const T y = row.sum((edge ? side != 0 : w == 1) ? 0 : LEV + 1);
+            if (edge)
+                s.n.ly[cp][side][l] = y;
+            else if (w < 2 && l < 21)
+                s.n.lc[w][l - 16] = y;
+        }
+        __syncthreads();
+        // x pass: the tile's lines and the halo points
+        T hu = 0.0, hv = 0.0;
+        {
+            const int q = l & 15, comp = (l >> 4) & 1, half = l >> 5;
+            HaarLineP<LEV, T> own;
+            own.load(&s.p.m[comp][q][0], 1, half, w);
+            if (w >= 2) {
+                const int cp = w == 3 ? 0 : 1, side = (l >> 4) & 1;
+                HaarRow<LEV, T> row;
+                row.load(l < 32 ? &s.n.lx[cp][5 * side][q] : &s.n.ly[cp][side][0], hoff);
+                own.rows(&s.p.t[comp][q][0], 1, half, w);
+                const T y = row.sum(hplus);
+                hu = hv = (hmb & (w == 3 ? CB_INNER_U : CB_INNER_V)) ? y : 0.0;
+            } else {
+                int off[N];
+                haar_halo_terms<LEV>(1, off);
+                HaarRow<LEV, T> row;
+                row.load(&s.n.lc[l == 0 ? 0 : 1][0], off);
+                own.rows(&s.p.t[comp][q][0], 1, half, w);
+                const T y = row.sum(l == 0 ? 0 : LEV + 1);
+                hu = hv = (hmb & (l == 0 ? CB_INNER_U : CB_INNER_V)) ? y : 0.0;  // staged by wavefront 1's lanes 0, 1
+            }
+        }
+        __syncthreads();
+        o.u = (mb & CB_INNER_U) ? s.p.t[0][ly][lx] : 0.0;
+        o.v = (mb & CB_INNER_V) ? s.p.t[1][ly][lx] : 0.0;
+        op_cells(rdx, rdy, h, hu, hv, o, cr, s);
+        s.h.t[0][ly][lx] = (mb & CB_INNER_U) ? op_out_u(rdx, rdy, s, o) : 0.0;
+        s.h.t[1][ly][lx] = (mb & CB_INNER_V) ? op_out_v(rdx, rdy, s, o) : 0.0;
+        __syncthreads();
+        haar_pair_lev<true, LEV, T>(s.h.t, s.h.m);
+        c = make_double2((mb & CB_WAVELET_U) ? s.h.t[0][ly][lx] : 0.0, (mb & CB_WAVELET_V) ? s.h.t[1][ly][lx] : 0.0);
+        return true;
+    }
+};
+
+// beta of iteration it, and the direction z + beta u (z = r, or D^-1 r)
+template <bool PRE>
+__device__ __forceinline__ double cg_beta(int it, double res, double prev_res, double rz, double prev_rz)
+{
+    if constexpr (PRE) {
+        return it == 0 ? 0.0 : rz / prev_rz;
+    } else {
+        const double prev = it == 0 ? 1.0 : prev_res;
+        return (res * res) / (prev * prev);
+    }
+}
+
+template <bool PRE>
+__device__ __forceinline__ double2 cg_direction(double beta, double2 r, double2 p, double2 dz)
+{
+    if constexpr (PRE)
+        return make_double2(dz.x * r.x + beta * p.x, dz.y * r.y + beta * p.y);
+    else
+        return make_double2(r.x + beta * p.x, r.y + beta * p.y);
+}
+
 // part 1 (iteration parity par): residual norm and stop test; x += alpha u
 // of the previous iteration; u = r + beta u with beta = res^2 / prev^2 (PRE:
 // u = D^-1 r + beta u with beta = rz / prev rz); c = R A P u and the partials
@@ -2498,18 +2709,16 @@ template <bool PRE, int LEV, int FOLD>
 __device__ __forceinline__ bool cg_step_tile(const CGArgs &a, int par, const int L)
 {
     using T = double;
-    constexpr int N = LEV + 2;
     __shared__ OpLds<T> s;
     __shared__ double lds[20];  // a slot per sum
     const GridDims &g = a.g;
     if (L >= g.nbx * g.nby) return false;
     int bx, by;
     band_tile(g, L, bx, by);
-    const int lx = threadIdx.x & 15, ly = threadIdx.x >> 4, l = threadIdx.x & 63;
-    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int i0 = bx * TILE, j0 = by * TILE;
     const CGLayout &Lo = a.Lo;
-    const unsigned at0 = Lo.at(i0, j0), at = at0 + lx + __umul24(Lo.px, (unsigned)ly);
+    CgTile<LEV> t;
+    t.place(Lo, bx * TILE, by * TILE);
+    const unsigned at = t.at;
     const double2 *R = Lo.pair(CG_R), *P = Lo.pair(CG_P + par), *D = Lo.pair(CG_DINV);
     // loads in the order of first use: scalars and partials, the tile's
     // vectors, the coarse halo, the coefficients
@@ -2525,72 +2734,10 @@ __device__ __forceinline__ bool cg_step_tile(const CGArgs &a, int par, const int
     }
     const double2 r = elem32(R, at), p = elem32(P, at), x = elem32(Lo.pair(CG_X), at);
     const double2 dz = PRE ? elem32(D, at) : make_double2(0.0, 0.0);
-    const unsigned mb = elem32(Lo.M, at);
-    // the coarse halo, one side per wavefront (left, right, below, above):
-    // line k = l / 16 of N, point l % 16 along it; the fifth line and the
-    // corner blocks (u below right, v above left) in a second round
-    const bool rows = w >= 2, after = (w & 1) != 0;
-    int di, dj;
-    {
-        const int c = haar_halo_offset<LEV>(after, l >> 4), q = l & 15;
-        di = rows ? q : c;
-        dj = rows ? c : q;
-    }
-    const unsigned h0 = at0 + (unsigned)(di + (int)__mul24((int)Lo.px, dj));
-    const double2 nr0 = elem32(R, h0), np0 = elem32(P, h0), nd0 = PRE ? elem32(D, h0) : make_double2(0.0, 0.0);
-    const int e = l - 16, cx = e % 5, cy = e / 5;  // corner entry of lanes 16..40 of wavefronts 0 (v) and 1 (u)
-    const bool corner = w < 2 && e >= 0 && e < 25;
-    {
-        const int c = haar_halo_offset<LEV>(after, 4), q = l & 15;
-        di = corner ? haar_halo_offset<LEV>(after, cx) : (rows ? q : c);
-        dj = corner ? haar_halo_offset<LEV>(!after, cy) : (rows ? c : q);
-    }
-    const unsigned h1 = at0 + (unsigned)(di + (int)__mul24((int)Lo.px, dj));
-    const double2 nr1 = elem32(R, h1), np1 = elem32(P, h1), nd1 = PRE ? elem32(D, h1) : make_double2(0.0, 0.0);
-    // halo points: wavefront 3 the sides' u, wavefront 2 their v, wavefront 1
-    // the corners (u lane 0, v lane 1)
-    HaloPos h{17, 0, 0, 17, w == 3 || (w == 1 && l == 0), w == 2 || (w == 1 && l == 1)};
-    if (w >= 2) {
-        halo_side(l, h.ux, h.uy);
-        h.vx = h.ux;
-        h.vy = h.uy;
-    }
-    OpOwn<T> o;
-    OpCoefRegs<T> cr;
-    cr.hhu = cr.hhv = 0.0;
-    const double2 oh = elem32(Lo.pair(CG_H), at);
-    unsigned hmb = 0;
-    if (w >= 1) {
-        const int hx = h.hu ? h.ux : h.vx, hy = h.hu ? h.uy : h.vy;
-        const unsigned ha = at0 + (unsigned)(hx - 1 + (int)__mul24((int)Lo.px, hy - 1));
-        cr.hhu = cr.hhv = elem32(reinterpret_cast<const double *>(Lo.pair(CG_H)), 2 * ha + (h.hu ? 0 : 1));
-        hmb = elem32(Lo.M, ha);
-    }
-    const double2 cell = elem32(Lo.pair(CG_CELL), at);
-    o.hetac = elem32(Lo.corner(), at);
-    op_extra_cell(l, cr);
-    if (w == 0) {
-        const unsigned ea = at0 + (unsigned)(cr.ex - 1 + (int)__mul24((int)Lo.px, cr.ey - 1));
-        const double2 ce = elem32(Lo.pair(CG_CELL), ea);
-        cr.ec = elem32(Lo.corner(), ea);
-        cr.eh = ce.x;
-        cr.ed = ce.y;
-    }
-    const double2 ob = elem32(Lo.pair(CG_B), at);
-    o.hu = oh.x;
-    o.hv = oh.y;
-    o.bu = ob.x;
-    o.bv = ob.y;
-    o.heta = cell.x;
-    o.dimp = cell.y;
-    // the halo point's terms in the x pass (wavefronts 2, 3)
-    int hoff[N], hplus;
-    if (l < 32) {
-        haar_halo_terms<LEV>(17, hoff);
-        hplus = l < 16 ? LEV + 1 : 0;
-    } else {
-        hplus = haar_row_terms<LEV>(l & 15, hoff);
-    }
+    t.mb = elem32(Lo.M, at);
+    const double2 nr0 = elem32(R, t.h0), np0 = elem32(P, t.h0), nd0 = PRE ? elem32(D, t.h0) : make_double2(0.0, 0.0);
+    const double2 nr1 = elem32(R, t.h1), np1 = elem32(P, t.h1), nd1 = PRE ? elem32(D, t.h1) : make_double2(0.0, 0.0);
+    t.load_coef(Lo);
     double res;
     if constexpr (PRE) {
         double r2 = fr.sum(a.Pr, g.npart);
@@ -2625,104 +2772,12 @@ __device__ __forceinline__ bool cg_step_tile(const CGArgs &a, int par, const int
     }
     if (alpha != 0.0) elem32(Lo.pair(CG_X), at) = make_double2(x.x + alpha * p.x, x.y + alpha * p.y);
     if (done) return true;
-    T beta;
-    if constexpr (PRE) {
-        beta = it == 0 ? T(0) : rz / prev_rz;
-    } else {
-        const double prev = it == 0 ? 1.0 : prev_res;
-        beta = (res * res) / (prev * prev);
-    }
-    auto direction = [&](double2 rr, double2 pp, double2 zz) -> double2 {
-        if constexpr (PRE)
-            return make_double2(zz.x * rr.x + beta * pp.x, zz.y * rr.y + beta * pp.y);
-        else
-            return make_double2(rr.x + beta * pp.x, rr.y + beta * pp.y);
-    };
-    const double2 un = direction(r, p, dz);
+    const T beta = cg_beta<PRE>(it, res, prev_res, rz, prev_rz);
+    const double2 un = cg_direction<PRE>(beta, r, p, dz);
     elem32(Lo.pair(CG_P + 1 - par), at) = un;
-    s.p.t[0][ly][lx] = un.x;
-    s.p.t[1][ly][lx] = un.y;
-    {
-        const int k = (w & 1) * 5 + (l >> 4), q = l & 15;
-        const double2 n0 = direction(nr0, np0, nd0), n1 = direction(nr1, np1, nd1);
-        if (rows) {
-            s.n.y[0][k][q] = n0.x;
-            s.n.y[1][k][q] = n0.y;
-            if (l < 16) {
-                s.n.y[0][k + 4][q] = n1.x;
-                s.n.y[1][k + 4][q] = n1.y;
-            }
-        } else {
-            s.n.x[0][k][q] = n0.x;
-            s.n.x[1][k][q] = n0.y;
-            if (l < 16) {
-                s.n.x[0][k + 4][q] = n1.x;
-                s.n.x[1][k + 4][q] = n1.y;
-            } else if (corner) {
-                s.n.c[1 - w][cy][cx] = w == 1 ? n1.x : n1.y;
-            }
-        }
-    }
-    __syncthreads();
-    // y pass: the tile's lines; the columns' lines (40 half lines; lanes
-    // 40..63 repeat the first); rows -1 and 16 of the neighbours below and
-    // above (lanes 0..15) and the corners (16..20 of wavefronts 0, 1).  The
-    // operands of all three are read before the first is used.
-    {
-        const int q = l & 15, comp = (l >> 4) & 1, half = l >> 5;
-        const int hl = l < 40 ? l : l - 40, line = hl < 20 ? hl : hl - 20, lh = hl < 20 ? 0 : 1;
-        const int cp = w & 1, side = w >> 1;
-        const bool edge = l < 16;
-        const T *se = edge ? &s.n.y[cp][5 * side][l] : &s.n.c[cp][0][l < 20 ? l - 16 : 4];
-        int off[N];
-        haar_halo_terms<LEV>(edge ? 16 : 5, off);
-        HaarLineP<LEV, T> own, hal;
-        HaarRow<LEV, T> row;
-        own.load(&s.p.t[comp][0][q], TILE + 1, half, w);
-        hal.load(&s.n.x[0][0][0] + 17 * line, 1, lh, w);
-        row.load(se, off);
-        own.rows(&s.p.m[comp][0][q], TILE + 1, half, w);
-        hal.rows(&s.n.lx[0][0][0] + 17 * line, 1, lh, w);
-        const T y = row.sum((edge ? side != 0 : w == 1) ? 0 : LEV + 1);
-        if (edge)
-            s.n.ly[cp][side][l] = y;
-        else if (w < 2 && l < 21)
-            s.n.lc[w][l - 16] = y;
-    }
-    __syncthreads();
-    // x pass: the tile's lines and the halo points
-    T hu = 0.0, hv = 0.0;
-    {
-        const int q = l & 15, comp = (l >> 4) & 1, half = l >> 5;
-        HaarLineP<LEV, T> own;
-        own.load(&s.p.m[comp][q][0], 1, half, w);
-        if (w >= 2) {
-            const int cp = w == 3 ? 0 : 1, side = (l >> 4) & 1;
-            HaarRow<LEV, T> row;
-            row.load(l < 32 ? &s.n.lx[cp][5 * side][q] : &s.n.ly[cp][side][0], hoff);
-            own.rows(&s.p.t[comp][q][0], 1, half, w);
-            const T y = row.sum(hplus);
-            hu = hv = (hmb & (w == 3 ? CB_INNER_U : CB_INNER_V)) ? y : 0.0;
-        } else {
-            int off[N];
-            haar_halo_terms<LEV>(1, off);
-            HaarRow<LEV, T> row;
-            row.load(&s.n.lc[l == 0 ? 0 : 1][0], off);
-            own.rows(&s.p.t[comp][q][0], 1, half, w);
-            const T y = row.sum(l == 0 ? 0 : LEV + 1);
-            hu = hv = (hmb & (l == 0 ? CB_INNER_U : CB_INNER_V)) ? y : 0.0;  // staged by wavefront 1's lanes 0, 1
-        }
-    }
-    __syncthreads();
-    o.u = (mb & CB_INNER_U) ? s.p.t[0][ly][lx] : 0.0;
-    o.v = (mb & CB_INNER_V) ? s.p.t[1][ly][lx] : 0.0;
-    op_cells(a.rdx, a.rdy, h, hu, hv, o, cr, s);
-    s.h.t[0][ly][lx] = (mb & CB_INNER_U) ? op_out_u(a.rdx, a.rdy, s, o) : 0.0;
-    s.h.t[1][ly][lx] = (mb & CB_INNER_V) ? op_out_v(a.rdx, a.rdy, s, o) : 0.0;
-    __syncthreads();
-    haar_pair_lev<true, LEV, T>(s.h.t, s.h.m);
-    const double2 c = make_double2((mb & CB_WAVELET_U) ? s.h.t[0][ly][lx] : 0.0,
-                                   (mb & CB_WAVELET_V) ? s.h.t[1][ly][lx] : 0.0);
+    double2 c;
+    (void)t.apply(a.rdx, a.rdy, un, cg_direction<PRE>(beta, nr0, np0, nd0), cg_direction<PRE>(beta, nr1, np1, nd1), s, c,
+                  [] { return true; });
     elem32(Lo.pair(CG_Q), at) = c;
     double du = un.x * c.x, dv = un.y * c.y;
     tree256x2_open(du, dv, lds + 12);
@@ -2885,10 +2940,15 @@ __global__ void __launch_bounds__(256) k_coarse_diag(GridDims g, OpCoef<double> 
 // partials and parity slots, so the results are those of the two
 // launches per iteration, bit for bit.  Ends at the stop, which every
 // thread of every tile decides alike from the same partials and scalars,
-// after maxiter + 1 iterations at most.
+// after maxiter + 1 iterations at most.  only_if: run only if it is set
+// (the resident CG below gave up; what it starts from is still in place).
 template <bool PRE, int LEV>
-__global__ void __launch_bounds__(256) k_cg_solve1(CGArgs a)
+__global__ void __launch_bounds__(256) k_cg_solve1(CGArgs a, const int *only_if)
 {
+    if (only_if) {
+        if (*only_if == 0) return;
+        if (threadIdx.x == 0) a.hflag->gave_up = 1;
+    }
     const int ntile = a.g.nbx * a.g.nby;
     for (int q = 0; q <= a.maxiter; ++q) {
         const int par = q & 1;
@@ -2901,6 +2961,284 @@ __global__ void __launch_bounds__(256) k_cg_solve1(CGArgs a)
         for (int L = 0; L < ntile; ++L) {
             cg_update_tile<PRE, true, 1>(a, par, L);
             __syncthreads();
+        }
+    }
+}
+
+// Copies of the folded sums, in lines of their own: with one copy all
+// wavefronts poll one line (3,564 of them at 1280 x 160), and the polls queue up.
+constexpr int X_COPIES = 64, X_COPY = 32;  // ... and words from one to the next
+
+// What the workgroups of the resident CG exchange, in tagged words (xput).
+struct CGExchange {
+    xword *c;       // c at every point: four planes of ns words (u, v), arena index, so that a
+                    // wavefront stores and a row of the halo loads whole lines
+    xword *pd;      // partials of (u, c): two words per partial
+    xword *pr;      // partials of ||r||^2, then (Jacobi) of (r, D^-1 r)
+    xword *root;    // the folded sums, if one workgroup folds, X_COPIES times: (u, c) at 0, the residual's at 8
+    int *abort;     // a wait ran out
+    unsigned tag;   // tag of iteration 0, larger than any used before
+    unsigned limit; // polls of one wait
+};
+
+// The whole FP64 coarse CG in one launch, a tile per workgroup, all of them
+// resident on the chip at once (after k_cg_setup; the host sees to it that
+// they fit).  Everything a tile owns (r, u, x, the coefficients, the coarse
+// halo's r and u) stays in registers; an iteration exchanges the partials of
+// (u, c) and ||r||^2, and c with the neighbours, which advance the halo's r
+// with it, so that the halo travels with the first sum and the second is
+// alone.  The same operations in the same order as the launches': the same
+// bits.
+//
+// What bounds it: two exchanges through the memory side of the chip and the
+// latency of one tile's chain of seven LDS passes.  FLAT: every workgroup folds
+// the partials itself (one hop).  Otherwise a workgroup without a tile does and
+// publishes the sums (two hops).  An exchange among 6 / 63 / 246 / 891
+// workgroups was measured at 1.2 / 2.0 / 2.7 / 18 us folding everywhere and
+// 1.75 / 2.3 / 3.5 us for the last three folding once.  Measured per iteration,
+// launches -> resident: 9.7 -> 5.4 us at 12 tiles, 9.5 -> 7.1 us at 63, 11.0 ->
+// 8.5 us at 246, 13.6 -> 10.8 us at 441.  Two
+// workgroups fit on a CU (165 to 193 registers).  With 128 registers four would,
+// for up to 1016 tiles, but 16 to 52 of them spill: 20 us at 891 tiles against
+// 18.6 us of the launches.
+//
+// Waits end: a wait that runs out of polls, or sees another's abort, raises
+// the abort flag and the whole workgroup returns at its next check.  A check
+// reads a flag that is written only in the waits before the barrier that
+// precedes it, so a workgroup's threads agree.  x leaves for CG_Q at the stop
+// and the arena is not written before, so k_cg_solve1 can start over.
+// The sums that the set-up left.
+template <bool PRE, int FOLD>
+__device__ __forceinline__ void cg_resident_sums(const CGArgs &a, double *lds, double &sum0, double &sum1, double &abstol)
+{
+    LaneFold<FOLD> f0, f1;
+    f0.load(a.Pr, a.g.npart);
+    if constexpr (PRE) f1.load(a.Pz, a.g.npart);
+    sum0 = f0.sum(a.Pr, a.g.npart);
+    sum1 = 0.0;
+    if constexpr (PRE) {
+        sum1 = f1.sum(a.Pz, a.g.npart);
+        tree256x2_open(sum0, sum1, lds);
+    } else {
+        sum0 = tree256_open(sum0, lds);
+    }
+    abstol = a.tol_coarse * sqrt(tree256(lane_fold(a.Pb, a.g.npart), lds + 8));
+}
+
+// The workgroup that folds: waits for all partials of a sum and publishes it.
+template <bool PRE, int FOLD>
+__device__ __forceinline__ void cg_resident_fold(const CGArgs &a, const CGExchange &E, double *lds, int *bad)
+{
+    const int np = a.g.npart;
+    double sum0, sum1, abstol, tol = 0.0;
+    cg_resident_sums<PRE, FOLD>(a, lds, sum0, sum1, abstol);
+    for (int it = 0;; ++it) {
+        const unsigned tag = E.tag + (unsigned)it;
+        const double res = sqrt(sum0);
+        if (it == 0) {
+            tol = a.reltol * res;
+            if (abstol > tol) tol = abstol;
+        }
+        if (it >= a.maxiter || res <= tol) return;
+        XFold<FOLD> f, fz;
+        f.want(true, np);
+        for (unsigned n = 0;; ++n) {
+            f.load(E.pd);
+            if (f.check(tag)) break;
+            if (x_give_up(n, E.limit, E.abort)) {
+                bad[0] = 1;
+                break;
+            }
+        }
+        const double dot = tree256_open(f.sum(np), lds + 12);
+        if (bad[0]) return;
+        if (threadIdx.x < X_COPIES) xput2(E.root + X_COPY * threadIdx.x, tag, dot);
+        f.want(true, np);
+        fz.want(PRE, np);
+        for (unsigned n = 0;; ++n) {
+            f.load(E.pr);
+            if constexpr (PRE) fz.load(E.pr + 2 * np);
+            if (f.check(tag) & fz.check(tag)) break;
+            if (x_give_up(n, E.limit, E.abort)) {
+                bad[1] = 1;
+                break;
+            }
+        }
+        sum0 = f.sum(np);
+        if constexpr (PRE) {
+            sum1 = fz.sum(np);
+            tree256x2_open(sum0, sum1, lds);
+        } else {
+            sum0 = tree256_open(sum0, lds);
+        }
+        if (bad[1]) return;
+        if (threadIdx.x < X_COPIES) {
+            xput2(E.root + X_COPY * threadIdx.x + 8, tag, sum0);
+            if constexpr (PRE) xput2(E.root + X_COPY * threadIdx.x + 10, tag, sum1);
+        }
+    }
+}
+
+template <bool PRE, int LEV, bool FLAT>
+__global__ void __launch_bounds__(256, 2) k_cg_resident(CGArgs a, CGExchange E)
+{
+    using T = double;
+    constexpr int K = PRE ? 2 : 1, FOLD = FLAT ? 1 : 4;
+    __shared__ OpLds<T> s;
+    __shared__ double lds[36];  // a slot per sum
+    __shared__ int bad[2];      // a wait of the first, second exchange ran out
+    const GridDims &g = a.g;
+    if (threadIdx.x < 2) bad[threadIdx.x] = 0;
+    if (!FLAT && (int)blockIdx.x >= a.nblk) {
+        if ((int)blockIdx.x == a.nblk) cg_resident_fold<PRE, FOLD>(a, E, lds, bad);
+        return;
+    }
+    const int L = xcd_tile(a.nblk);
+    if (L >= g.nbx * g.nby) return;
+    int bx, by;
+    band_tile(g, L, bx, by);
+    const int np = g.npart;
+    const CGLayout &Lo = a.Lo;
+    CgTile<LEV> t;
+    t.place(Lo, bx * TILE, by * TILE);
+    double sum0, sum1, abstol;
+    cg_resident_sums<PRE, FOLD>(a, lds, sum0, sum1, abstol);
+    // the tile's state; zero where there is no neighbour
+    const double2 *R = Lo.pair(CG_R), *D = Lo.pair(CG_DINV);
+    const double2 zero = make_double2(0.0, 0.0);
+    double2 r = elem32(R, t.at), x = elem32(Lo.pair(CG_X), t.at), u = zero;
+    double2 nr0 = elem32(R, t.h0), nr1 = elem32(R, t.h1), nu0 = zero, nu1 = zero;
+    const double2 dz = PRE ? elem32(D, t.at) : zero, nd0 = PRE ? elem32(D, t.h0) : zero, nd1 = PRE ? elem32(D, t.h1) : zero;
+    t.mb = elem32(Lo.M, t.at);
+    t.load_coef(Lo);
+    const bool west = bx > 0, east = bx + 1 < g.nbx, south = by > 0, north = by + 1 < g.nby;
+    const bool have0 = t.rows ? (t.after ? north : south) : (t.after ? east : west);
+    const bool have1 = t.corner ? (t.after ? east && south : west && north) : (t.l < 16 && have0);
+    const bool has_u = bx < g.nbxu && by < g.nbyu, has_v = bx < g.nbxv && by < g.nbyv;
+    const int pu = bx + g.nbxu * by, pv = g.nbxu * g.nbyu + bx + g.nbxv * by;
+    const xword *root = E.root + X_COPY * ((4 * L + t.w) & (X_COPIES - 1));
+    double tol = 0.0, prev_res = 1.0, prev_rz = 1.0, alpha = 0.0;
+    for (int it = 0;; ++it) {
+        const unsigned tag = E.tag + (unsigned)it;
+        const double res = sqrt(sum0), rz = sum1;
+        if (it == 0) {
+            tol = a.reltol * res;
+            if (abstol > tol) tol = abstol;
+        }
+        if (alpha != 0.0) x = make_double2(x.x + alpha * u.x, x.y + alpha * u.y);
+        if (it >= a.maxiter || res <= tol) {
+            elem32(Lo.pair(CG_Q), t.at) = x;
+            if (L == 0 && threadIdx.x == 0) {
+                a.hflag->iters = it;
+                a.hflag->done = 1;
+            }
+            return;
+        }
+        const double beta = cg_beta<PRE>(it, res, prev_res, rz, prev_rz);
+        u = cg_direction<PRE>(beta, r, u, dz);
+        nu0 = cg_direction<PRE>(beta, nr0, nu0, nd0);
+        nu1 = cg_direction<PRE>(beta, nr1, nu1, nd1);
+        double2 c;
+        if (!t.apply(a.rdx, a.rdy, u, nu0, nu1, s, c, [&] { return bad[1] == 0; })) return;
+        {
+            xword *q = &elem32(E.c, t.at);
+            xput2(q, tag, c.x, Lo.ns);
+            xput2(q + 2 * (size_t)Lo.ns, tag, c.y, Lo.ns);
+        }
+        double du = u.x * c.x, dv = u.y * c.y;
+        tree256x2_open(du, dv, lds + 12);
+        if (threadIdx.x == 0) {
+            if (has_u) xput2(E.pd + 2 * pu, tag, du);
+            if (has_v) xput2(E.pd + 2 * pv, tag, dv);
+        }
+        // first exchange: the halo's c and the sum
+        double2 nc0 = zero, nc1 = zero;
+        double dot;
+        {
+            XWait<4> w0, w1;
+            XFold<FOLD> wf;
+            XWait<2> wr;
+            w0.want(have0);
+            w1.want(have1);
+            wf.want(FLAT, np);
+            wr.want(!FLAT);
+            for (unsigned n = 0;; ++n) {
+                if (FLAT || n > 0) {  // two hops take longer than one: the halo is looked for after the first poll
+                    w0.load(&elem32(E.c, t.h0), Lo.ns);
+                    w1.load(&elem32(E.c, t.h1), Lo.ns);
+                }
+                if constexpr (FLAT) wf.load(E.pd);
+                if constexpr (!FLAT) wr.load(root);
+                const bool ok = w0.check(tag) & w1.check(tag) & wf.check(tag) & wr.check(tag);
+                if (ok) break;
+                if (x_give_up(n, E.limit, E.abort)) {
+                    bad[0] = 1;
+                    break;
+                }
+            }
+            if (have0) nc0 = make_double2(w0.value(0), w0.value(1));
+            if (have1) nc1 = make_double2(w1.value(0), w1.value(1));
+            if constexpr (FLAT)
+                dot = tree256_open(wf.sum(np), lds + 20);
+            else
+                dot = wr.value(0);
+        }
+        alpha = (PRE ? rz : res * res) / dot;
+        prev_res = res;
+        prev_rz = rz;
+        r = make_double2(r.x - alpha * c.x, r.y - alpha * c.y);
+        nr0 = make_double2(nr0.x - alpha * nc0.x, nr0.y - alpha * nc0.y);
+        nr1 = make_double2(nr1.x - alpha * nc1.x, nr1.y - alpha * nc1.y);
+        double r2u = r.x * r.x, r2v = r.y * r.y, z2u = 0.0, z2v = 0.0;
+        tree256x2_open(r2u, r2v, lds + 4);
+        if constexpr (PRE) {
+            z2u = r.x * (dz.x * r.x);
+            z2v = r.y * (dz.y * r.y);
+            tree256x2_open(z2u, z2v, lds + 28);
+        }
+        if (bad[0]) return;
+        if (threadIdx.x == 0) {
+            if (has_u) {
+                xput2(E.pr + 2 * pu, tag, r2u);
+                if constexpr (PRE) xput2(E.pr + 2 * (np + pu), tag, z2u);
+            }
+            if (has_v) {
+                xput2(E.pr + 2 * pv, tag, r2v);
+                if constexpr (PRE) xput2(E.pr + 2 * (np + pv), tag, z2v);
+            }
+        }
+        // second exchange: the residual norm
+        {
+            XFold<FOLD> wf, wz;
+            XWait<2 * K> wr;
+            wf.want(FLAT, np);
+            wz.want(PRE && FLAT, np);
+            wr.want(!FLAT);
+            bool lost = false;
+            for (unsigned n = 0;; ++n) {
+                if constexpr (FLAT) wf.load(E.pr);
+                if constexpr (FLAT && PRE) wz.load(E.pr + 2 * np);
+                if constexpr (!FLAT) wr.load(root + 8);
+                const bool ok = wf.check(tag) & wz.check(tag) & wr.check(tag);
+                if (ok) break;
+                if (x_give_up(n, E.limit, E.abort)) {
+                    bad[1] = 1;
+                    lost = true;
+                    break;
+                }
+            }
+            if constexpr (FLAT) {
+                sum0 = wf.sum(np);
+                if constexpr (PRE) {
+                    sum1 = wz.sum(np);
+                    tree256x2_open(sum0, sum1, lds);
+                } else {
+                    sum0 = tree256_open(sum0, lds);
+                }
+            } else {
+                sum0 = lost ? __builtin_nan("") : wr.value(0);  // NaN does not stop the loop before its check
+                if constexpr (PRE) sum1 = wr.value(1);
+            }
         }
     }
 }
