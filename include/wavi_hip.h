@@ -377,16 +377,18 @@ int wavi_smoother_tile(const wavi_ctx *ctx, int *tx, int *ty);
  * one in mixed precision), queued in chunks.  WAVI_CG_WORKGROUP: the whole CG
  * in one launch of one workgroup, which runs each iteration on the tiles in
  * turn, with no launch and no host round trip between iterations.
- * WAVI_CG_AUTO (the default) is the library's choice: in FP64, while all tiles
- * fit on the chip at once (up to 504 on MI355X), the whole CG in one launch
- * of a workgroup per tile, which exchange sums and halos among themselves
- * (7.1 us per iteration against 9.5 at 63 tiles); else WAVI_CG_LAUNCHES.  The
+ * WAVI_CG_AUTO (the default) is the library's choice: while all tiles fit on
+ * the chip at once (up to 504 in FP64, 256 in mixed precision on MI355X), the
+ * whole CG in one launch of a workgroup per tile, which exchange sums and
+ * halos among themselves (FP64, 63 tiles: 7.1 us per iteration against 9.5;
+ * mixed, 246 tiles: 4.2 against 5.1); else WAVI_CG_LAUNCHES.  The
  * workgroup is 3.4 to 3.6 times slower per iteration than the launches even on
  * a grid of six 16 x 16 tiles.  All give the same bits.  wavi_coarse_cg
  * reports the mode in effect for the context (WAVI_CG_LAUNCHES for
  * WAVI_CG_AUTO).  Lockstep batches (wavi_update_velocities_lockstep*) and the
- * small members of wavi_misfit_gradient_batch share one launch per CG
- * iteration whatever the mode.  No reference counterpart. */
+ * small members of wavi_misfit_gradient_batch share one launch for the whole
+ * CG where all members have WAVI_CG_AUTO and fit together, else one launch per
+ * CG iteration.  No reference counterpart. */
 #define WAVI_CG_AUTO 0
 #define WAVI_CG_LAUNCHES 1
 #define WAVI_CG_WORKGROUP 2

@@ -40,7 +40,8 @@ static std::mutex g_graph_mu;
 // its own address).  In host code `scratch` is only a stand-in for the
 // symbol: its device address on each GPU is looked up once, at the first
 // context creation on that GPU, and kept in g_scratch_ptr.
-static __device__ __align__(256) unsigned char scratch[WAVI_NOALLOC_SCRATCH_BYTES];
+// The members' exchanges (CGMExchange) follow the tables.
+static __device__ __align__(256) unsigned char scratch[WAVI_NOALLOC_SCRATCH_BYTES + WAVI_NOALLOC_MAX_MEMBERS * sizeof(CGMExchange)];
 constexpr int MAX_DEVICES = 64;
 // LDS the whole-grid smoother may take (at most the device's per-workgroup limit)
 constexpr size_t SMG_LDS_MAX = 65536;
@@ -110,6 +111,7 @@ struct wavi_ctx {
     unsigned xtag = 1;
     unsigned x_polls = X_POLLS;
     void (*x_fn[2])(CGArgs, CGExchange) = {};  // plain, Jacobi-preconditioned
+    void (*xm_fn[2])(CGMIterArgs, CGMExchange) = {};  // ... of the mixed CG
     int x_blocks = 0;               // workgroups of its launch
     int x_units = 0;                // ... and their share of the chip (room_take)
     bool x_off = false;             // a wait ran out once: the launches per iteration from then on
@@ -482,6 +484,9 @@ constexpr int CG_FOLD_LARGE = 8;
 
 // Tiles up to which every workgroup of k_cg_resident folds the partials itself.
 constexpr int X_FLAT_TILES = 32;
+// Tiles up to which the coarse CG is a resident launch: two workgroups per CU
+// in FP64, one partial per thread in mixed precision.
+constexpr int X_TILES_FP64 = 512, X_TILES_MIXED = 256;
 // The instance of k_cg_resident for a grid of ntile tiles.
 typedef void (*CGResidentFn)(CGArgs, CGExchange);
 
@@ -489,6 +494,18 @@ template <bool PRE, int LEV>
 static CGResidentFn cg_resident_fn_p(int ntile)
 {
     return ntile <= X_FLAT_TILES ? k_cg_resident<PRE, LEV, true> : k_cg_resident<PRE, LEV, false>;
+}
+
+typedef void (*CGMResidentFn)(CGMIterArgs, CGMExchange);
+
+static CGMResidentFn cgm_resident_fn(int levels, bool pre)
+{
+    switch (levels) {
+    case 0: return pre ? k_cgm_resident<0, true> : k_cgm_resident<0, false>;
+    case 1: return pre ? k_cgm_resident<1, true> : k_cgm_resident<1, false>;
+    case 2: return pre ? k_cgm_resident<2, true> : k_cgm_resident<2, false>;
+    default: return pre ? k_cgm_resident<3, true> : k_cgm_resident<3, false>;
+    }
 }
 
 static CGResidentFn cg_resident_fn(int levels, bool pre, int ntile)
@@ -499,6 +516,23 @@ static CGResidentFn cg_resident_fn(int levels, bool pre, int ntile)
     case 2: return pre ? cg_resident_fn_p<true, 2>(ntile) : cg_resident_fn_p<false, 2>(ntile);
     default: return pre ? cg_resident_fn_p<true, 3>(ntile) : cg_resident_fn_p<false, 3>(ntile);
     }
+}
+
+// Workgroups of a kernel that a CU holds at once, asked for once per kernel
+// (a property of the library's code).
+static hipError_t resident_occupancy(const void *fn, int *occ)
+{
+    static std::mutex mu;
+    static std::map<const void *, int> known;
+    std::lock_guard<std::mutex> lock(mu);
+    const auto it = known.find(fn);
+    if (it != known.end()) {
+        *occ = it->second;
+        return hipSuccess;
+    }
+    const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(occ, fn, 256, 0);
+    if (e == hipSuccess) known[fn] = *occ;
+    return e;
 }
 
 extern "C" {
@@ -733,6 +767,33 @@ int wavi_ctx_create(const wavi_grid_desc *grid, const wavi_phys_params *phys, co
     CREATECHK(hipEventCreateWithFlags(&ctx->ev_ls, hipEventDisableTiming));
     for (hipEvent_t &e : ctx->ev_tune) CREATECHK(hipEventCreate(&e));
     CREATECHK(hipEventCreateWithFlags(&ctx->ev_ls_done, hipEventDisableTiming));
+    {
+        // the coarse CG in one launch, if the grid's tiles fit on the chip at once
+        const int ntile = g.nbx * g.nby;
+        const bool fp64 = precision_mode == WAVI_PRECISION_FP64;
+        int occ[2] = {}, cus = 0;
+        CREATECHK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device));
+        for (int pre = 0; pre < 2; ++pre) {
+            ctx->x_fn[pre] = cg_resident_fn(solver->levels, pre != 0, ntile);
+            ctx->xm_fn[pre] = cgm_resident_fn(solver->levels, pre != 0);
+            CREATECHK(resident_occupancy(fp64 ? (const void *)ctx->x_fn[pre] : (const void *)ctx->xm_fn[pre], &occ[pre]));
+        }
+        if (ctx->device < MAX_DEVICES) {
+            std::lock_guard<std::mutex> rlock(g_room_mu);
+            g_room[ctx->device] = cus * CU_UNITS;
+        }
+        ctx->x_blocks = ctx->nblk + (fp64 && ntile > X_FLAT_TILES ? 8 : 0);  // the workgroup that folds
+        const int per_cu = std::min(std::min(occ[0], occ[1]), 4);  // 4: what k_cgm_resident_batch is built for
+        if (per_cu >= 2 && ctx->x_blocks <= cus * per_cu && ntile <= (fp64 ? X_TILES_FP64 : X_TILES_MIXED) &&
+            solver->maxiter_coarse < (1 << 28)) {
+            const char *polls = getenv("WAVI_CG_POLLS");  // the polls of a wait
+            if (polls) ctx->x_polls = (unsigned)std::max(0, atoi(polls));
+            ctx->x_units = ctx->x_blocks * ((CU_UNITS + per_cu - 1) / per_cu);
+            ctx->n_xwords = fp64 ? 4 * (size_t)(TILE * (g.nbx + 1)) * TILE * (g.nby + 2) + 6 * (size_t)g.npart + 64 +
+                                       X_COPIES * X_COPY
+                                 : (size_t)ntile * (2 * 6 * 64 + 4);
+        }
+    }
     if (precision_mode == WAVI_PRECISION_FP64) {
         const size_t px = (size_t)TILE * (g.nbx + 1), ns = px * TILE * (g.nby + 2);
         if (ns * sizeof(double2) > UINT32_MAX) {
@@ -741,32 +802,14 @@ int wavi_ctx_create(const wavi_grid_desc *grid, const wavi_phys_params *phys, co
         }
         ctx->px64 = (unsigned)px;
         ctx->ns64 = (unsigned)ns;
-        const size_t bytes = ns * (CG_NPAIR * sizeof(double2) + sizeof(double));
+        // the exchange words of a resident CG, if any, follow the arena, on a line of their own
+        const size_t arena = (ns * (CG_NPAIR * sizeof(double2) + sizeof(double)) + 255) / 256 * 256;
+        const size_t bytes = arena + ctx->n_xwords * sizeof(xword);
         CREATECHK(hipMalloc(&ctx->arena64, bytes));
         CREATECHK(hipMemset(ctx->arena64, 0, bytes));
+        if (ctx->n_xwords) ctx->xwords = (xword *)((char *)ctx->arena64 + arena);
         CREATECHK(hipMalloc(&ctx->marena64, ns));
         CREATECHK(hipMemset(ctx->marena64, 0, ns));
-        const int ntile = g.nbx * g.nby;
-        int occ[2] = {}, cus = 0;
-        CREATECHK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device));
-        for (int pre = 0; pre < 2; ++pre) {
-            ctx->x_fn[pre] = cg_resident_fn(solver->levels, pre != 0, ntile);
-            CREATECHK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ[pre], ctx->x_fn[pre], 256, 0));
-        }
-        if (ctx->device < MAX_DEVICES) {
-            std::lock_guard<std::mutex> rlock(g_room_mu);
-            g_room[ctx->device] = cus * CU_UNITS;
-        }
-        ctx->x_blocks = ctx->nblk + (ntile <= X_FLAT_TILES ? 0 : 8);
-        const int per_cu = std::min(occ[0], occ[1]);
-        if (per_cu >= 2 && ctx->x_blocks <= cus * per_cu && g.npart <= 1024 && solver->maxiter_coarse < (1 << 28)) {
-            const char *polls = getenv("WAVI_CG_POLLS");  // the polls of a wait
-            if (polls) ctx->x_polls = (unsigned)std::max(0, atoi(polls));
-            ctx->x_units = ctx->x_blocks * ((CU_UNITS + per_cu - 1) / per_cu);
-            ctx->n_xwords = 4 * ns + 6 * (size_t)g.npart + 32 + X_COPIES * X_COPY;
-            CREATECHK(hipMalloc(&ctx->xwords, ctx->n_xwords * sizeof(xword)));
-            CREATECHK(hipMemset(ctx->xwords, 0, ctx->n_xwords * sizeof(xword)));
-        }
     }
     if (precision_mode == WAVI_PRECISION_MIXED) {
         VSet<float> &w = ctx->v32;
@@ -784,8 +827,11 @@ int wavi_ctx_create(const wavi_grid_desc *grid, const wavi_phys_params *phys, co
         }
         ctx->px = (unsigned)(TILE * (g.nbx + 1));
         ctx->ns = ctx->px * (unsigned)(TILE * g.nby + 3);
-        CREATECHK(hipMalloc(&ctx->arena, (2 * CGM_NPAIR + 1) * (size_t)ctx->ns * sizeof(float)));
-        CREATECHK(hipMemset(ctx->arena, 0, (2 * CGM_NPAIR + 1) * (size_t)ctx->ns * sizeof(float)));
+        const size_t arena = ((2 * CGM_NPAIR + 1) * (size_t)ctx->ns * sizeof(float) + 255) / 256 * 256;
+        const size_t bytes = arena + ctx->n_xwords * sizeof(xword);  // as above
+        CREATECHK(hipMalloc(&ctx->arena, bytes));
+        CREATECHK(hipMemset(ctx->arena, 0, bytes));
+        if (ctx->n_xwords) ctx->xwords = (xword *)((char *)ctx->arena + arena);
         CREATECHK(hipMalloc(&ctx->marena, ctx->ns));
         CREATECHK(hipMemset(ctx->marena, 0, ctx->ns));
         ctx->npad = (g.nbx * g.nby + 1023) / 1024 * 1024;
@@ -846,7 +892,7 @@ static void ctx_free(wavi_ctx *ctx)
         }
     }
     for (void *p : {(void *)ctx->arena, (void *)ctx->marena, (void *)ctx->Pgd, (void *)ctx->rings, (void *)ctx->arena64,
-                    (void *)ctx->marena64, (void *)ctx->xwords})
+                    (void *)ctx->marena64})
         if (p) (void)hipFree(p);
     if (ctx->stm) (void)hipFree(ctx->stm);
     if (ctx->h_flag) (void)hipHostFree(ctx->h_flag);
@@ -1479,14 +1525,14 @@ static int cg_collect(wavi_ctx *ctx, int *iters)
     if (hf->gave_up) ctx->x_off = true;
     *iters = hf->iters;
     for (wavi_ctx::Burst &b : ctx->bursts) b.n = hf->iters;
-    burst_collect(ctx, WAVI_KT_CG_ITER_FP64, hf->gave_up ? -1 : 0);
+    burst_collect(ctx, ctx->precision == WAVI_PRECISION_FP64 ? WAVI_KT_CG_ITER_FP64 : WAVI_KT_CG_ITER_MIXED,
+                  hf->gave_up ? -1 : 0);
     return WAVI_OK;
 }
 
-// The FP64 coarse CG in one launch if the context can have it now: then
-// queues it and what stands in for it should a wait run out, and returns
-// true; the report is read by cg_collect once the stream has got there.
-static bool cg_try_resident(wavi_ctx *ctx, const CGArgs &a)
+// Whether the context's coarse CG can be a resident launch on `stream` now;
+// then takes its tags and (room) its room on the chip.
+static bool cg_resident_begin(wavi_ctx *ctx, unsigned *tag, hipStream_t stream, bool room = true)
 {
     ctx->x_ran = false;
     if (ctx->x_pending) {  // left by a call that ended with an error
@@ -1494,21 +1540,34 @@ static bool cg_try_resident(wavi_ctx *ctx, const CGArgs &a)
         if (hipStreamSynchronize(ctx->stream) != hipSuccess) return false;
         (void)cg_collect(ctx, &lost);
     }
-    if (!ctx->xwords || ctx->x_off || ctx->cg_mode != WAVI_CG_AUTO || !room_take(ctx->device, ctx->x_units)) return false;
-    if (ctx->xtag > 0xffffffffu - (unsigned)a.maxiter - 2u) {  // tags used up: clear the words and begin again
-        hipLaunchKernelGGL(k_fill<xword>, flat((int)ctx->n_xwords), dim3(256), 0, ctx->stream, ctx->xwords, (xword)0,
+    if (!ctx->xwords || ctx->x_off || ctx->cg_mode != WAVI_CG_AUTO) return false;
+    if (room && !room_take(ctx->device, ctx->x_units)) return false;
+    const unsigned need = (unsigned)ctx->S.maxiter_coarse + 2u;
+    if (ctx->xtag > 0xffffffffu - need) {  // tags used up: clear the words and begin again
+        hipLaunchKernelGGL(k_fill<xword>, flat((int)ctx->n_xwords), dim3(256), 0, stream, ctx->xwords, (xword)0,
                            (int)ctx->n_xwords);
         ctx->xtag = 1;
     }
+    *tag = ctx->xtag;
+    ctx->xtag += need;
+    return true;
+}
+
+// The FP64 coarse CG in one launch if the context can have it now: then
+// queues it and what stands in for it should a wait run out, and returns
+// true; the report is read by cg_collect once the stream has got there.
+static bool cg_try_resident(wavi_ctx *ctx, const CGArgs &a)
+{
+    unsigned tag;
+    if (!cg_resident_begin(ctx, &tag, ctx->stream)) return false;
     CGExchange E;
     E.c = ctx->xwords;
     E.pd = E.c + 4 * (size_t)ctx->ns64;
     E.pr = E.pd + 2 * ctx->g.npart;
     E.root = ctx->xwords + (ctx->n_xwords / 32 * 32 - X_COPIES * X_COPY);  // whole lines at the end
     E.abort = &ctx->st->abort;
-    E.tag = ctx->xtag;
+    E.tag = tag;
     E.limit = ctx->x_polls;
-    ctx->xtag += (unsigned)a.maxiter + 2u;
     const int bev = burst_begin(ctx);
     hipLaunchKernelGGL(ctx->x_fn[ctx->cg_pre], dim3(ctx->x_blocks), dim3(256), 0, ctx->stream, a, E);
     burst_end(ctx, bev, 0, 0);
@@ -1693,6 +1752,48 @@ static CGMIterArgs cgm_iter_args(wavi_ctx *ctx)
     return ia;
 }
 
+// The whole mixed CG in one workgroup (only_if: if it is set).
+static void launch_cgm_solve1(wavi_ctx *ctx, const CGMIterArgs &ia, const int *only_if = nullptr)
+{
+    const dim3 one(1), wg(256);
+    switch (ctx->S.levels + (ctx->cg_pre ? 4 : 0)) {
+    case 0: hipLaunchKernelGGL((k_cgm_solve1<0, false>), one, wg, 0, ctx->stream, ia, only_if); break;
+    case 1: hipLaunchKernelGGL((k_cgm_solve1<1, false>), one, wg, 0, ctx->stream, ia, only_if); break;
+    case 2: hipLaunchKernelGGL((k_cgm_solve1<2, false>), one, wg, 0, ctx->stream, ia, only_if); break;
+    case 3: hipLaunchKernelGGL((k_cgm_solve1<3, false>), one, wg, 0, ctx->stream, ia, only_if); break;
+    case 4: hipLaunchKernelGGL((k_cgm_solve1<0, true>), one, wg, 0, ctx->stream, ia, only_if); break;
+    case 5: hipLaunchKernelGGL((k_cgm_solve1<1, true>), one, wg, 0, ctx->stream, ia, only_if); break;
+    case 6: hipLaunchKernelGGL((k_cgm_solve1<2, true>), one, wg, 0, ctx->stream, ia, only_if); break;
+    default: hipLaunchKernelGGL((k_cgm_solve1<3, true>), one, wg, 0, ctx->stream, ia, only_if); break;
+    }
+}
+
+static CGMExchange cgm_exchange(const wavi_ctx *ctx, unsigned tag)
+{
+    const size_t ntile = (size_t)ctx->g.nbx * ctx->g.nby;
+    CGMExchange E;
+    E.ring = ctx->xwords;
+    E.part = E.ring + 2 * 6 * 64 * ntile;
+    E.abort = &ctx->stm->abort;
+    E.tag = tag;
+    E.limit = ctx->x_polls;
+    return E;
+}
+
+// The mixed coarse CG in one launch, as cg_try_resident.
+static bool cgm_try_resident(wavi_ctx *ctx, const CGMIterArgs &ia)
+{
+    unsigned tag;
+    if (!cg_resident_begin(ctx, &tag, ctx->stream)) return false;
+    const int bev = burst_begin(ctx);
+    hipLaunchKernelGGL(ctx->xm_fn[ctx->cg_pre], dim3(ctx->x_blocks), dim3(256), 0, ctx->stream, ia,
+                       cgm_exchange(ctx, tag));
+    burst_end(ctx, bev, 0, 0);
+    launch_cgm_solve1(ctx, ia, &ctx->stm->abort);
+    ctx->x_ran = ctx->x_pending = true;
+    return true;
+}
+
 static CGMArgs cgm_args(wavi_ctx *ctx, const VSet<float> &w)
 {
     CGMArgs sa;
@@ -1717,6 +1818,7 @@ static CGMArgs cgm_args(wavi_ctx *ctx, const VSet<float> &w)
     sa.st = ctx->stm;
     sa.hflag = ctx->d_flag;
     sa.nblk = ctx->nblk;
+    sa.resident = ctx->x_ran;
     return sa;
 }
 
@@ -1726,6 +1828,7 @@ static CGMArgs cgm_args(wavi_ctx *ctx, const VSet<float> &w)
 static int cgm_prepare(wavi_ctx *ctx, const VSet<float> &w)
 {
     launch_tile_haar<float>(ctx, 1, w.xc.u, w.xc.v, ctx->mwu, ctx->mwv, w.ct.u, w.ct.v, ctx->ui, ctx->vi);
+    ctx->x_ran = false;
     ctx->h_flag->done = 0;
     ctx->h_flag->iters = 0;
     const CGMArgs sa = cgm_args(ctx, w);
@@ -1750,18 +1853,13 @@ int do_coarse_cg<float>(wavi_ctx *ctx, const VSet<float> &w, int *iters)
     CHK(cgm_prepare(ctx, w));
     const CGMIterArgs ia = cgm_iter_args(ctx);
     volatile CGMHostFlag *hf = ctx->h_flag;
+    *iters = 0;
+    if (cgm_try_resident(ctx, ia)) {
+        HIPCHK(hipGetLastError());
+        return WAVI_OK;
+    }
     if (cg_one_workgroup(ctx)) {
-        const int sel = ctx->S.levels + (ctx->cg_pre ? 4 : 0);
-        switch (sel) {
-        case 0: hipLaunchKernelGGL((k_cgm_solve1<0, false>), dim3(1), dim3(256), 0, ctx->stream, ia); break;
-        case 1: hipLaunchKernelGGL((k_cgm_solve1<1, false>), dim3(1), dim3(256), 0, ctx->stream, ia); break;
-        case 2: hipLaunchKernelGGL((k_cgm_solve1<2, false>), dim3(1), dim3(256), 0, ctx->stream, ia); break;
-        case 3: hipLaunchKernelGGL((k_cgm_solve1<3, false>), dim3(1), dim3(256), 0, ctx->stream, ia); break;
-        case 4: hipLaunchKernelGGL((k_cgm_solve1<0, true>), dim3(1), dim3(256), 0, ctx->stream, ia); break;
-        case 5: hipLaunchKernelGGL((k_cgm_solve1<1, true>), dim3(1), dim3(256), 0, ctx->stream, ia); break;
-        case 6: hipLaunchKernelGGL((k_cgm_solve1<2, true>), dim3(1), dim3(256), 0, ctx->stream, ia); break;
-        default: hipLaunchKernelGGL((k_cgm_solve1<3, true>), dim3(1), dim3(256), 0, ctx->stream, ia); break;
-        }
+        launch_cgm_solve1(ctx, ia);
         HIPCHK(hipGetLastError());
         HIPCHK(hipStreamSynchronize(ctx->stream));
         if (!hf->done) {
@@ -2514,6 +2612,7 @@ static void launch_cgm_batch(hipStream_t s, int levels, int nwg, const CGMBatch 
 struct LockTables {
     CGMIterArgs *members = nullptr;
     int *group = nullptr, *first = nullptr;
+    CGMExchange *ex = nullptr;
     std::vector<hipEvent_t> ev;
 };
 
@@ -2525,6 +2624,7 @@ struct LockstepRes : LockTables {
             if (members) (void)hipFree(members);
             if (group) (void)hipFree(group);
             if (first) (void)hipFree(first);
+            if (ex) (void)hipFree(ex);
         }
         for (hipEvent_t e : ev)
             if (e) (void)hipEventDestroy(e);
@@ -2543,6 +2643,7 @@ static int lockstep_res_alloc(LockstepRes &R, wavi_ctx *const *ctxs, int n)
         HIPCHK(hipMalloc(&R.members, n * sizeof(CGMIterArgs)));
         HIPCHK(hipMalloc(&R.group, ngroups * sizeof(int)));
         HIPCHK(hipMalloc(&R.first, n * sizeof(int)));
+        HIPCHK(hipMalloc(&R.ex, n * sizeof(CGMExchange)));
     }
     R.ev.assign(n + 1, nullptr);
     for (hipEvent_t &e : R.ev) HIPCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
@@ -2556,11 +2657,51 @@ struct LockMember {
     double rel = INFINITY;
 };
 
+template <int LEV>
+static void launch_cgm_resident_batch_p(hipStream_t s, int nwg, int n, const CGMBatch &B, const CGMExchange *ex, bool pre)
+{
+    if (pre) {
+        hipLaunchKernelGGL((k_cgm_resident_batch<LEV, true>), dim3(nwg), dim3(256), 0, s, B, ex);
+        hipLaunchKernelGGL((k_cgm_solve1_batch<LEV, true>), dim3(n), dim3(256), 0, s, B, ex);
+    } else {
+        hipLaunchKernelGGL((k_cgm_resident_batch<LEV, false>), dim3(nwg), dim3(256), 0, s, B, ex);
+        hipLaunchKernelGGL((k_cgm_solve1_batch<LEV, false>), dim3(n), dim3(256), 0, s, B, ex);
+    }
+}
+
+static void launch_cgm_resident_batch(hipStream_t s, int levels, int nwg, int n, const CGMBatch &B,
+                                      const CGMExchange *ex, bool pre)
+{
+    switch (levels) {
+    case 0: launch_cgm_resident_batch_p<0>(s, nwg, n, B, ex, pre); break;
+    case 1: launch_cgm_resident_batch_p<1>(s, nwg, n, B, ex, pre); break;
+    case 2: launch_cgm_resident_batch_p<2>(s, nwg, n, B, ex, pre); break;
+    default: launch_cgm_resident_batch_p<3>(s, nwg, n, B, ex, pre); break;
+    }
+}
+
+// Room on the chip (room_take), given back at the end of the scope.
+struct RoomHold {
+    int device = 0, units = 0;
+    bool take(int d, int u)
+    {
+        if (!room_take(d, u)) return false;
+        device = d;
+        units = u;
+        return true;
+    }
+    ~RoomHold()
+    {
+        if (units) room_give(device, units);
+    }
+};
+
 // Coarse CGs of the members mem (each set up by cgm_prepare on its own
 // stream and marked there by the event pre[j]) run together on the stream of
-// mem[0]: one k_cgm_iter_batch launch per CG iteration over the tiles of all
-// of them, in chunks as for one member (cg_chunk_len), until every member's
-// CG has stopped.  On return the CGs are complete, iters[j] holds member j's
+// mem[0]: in one launch if their tiles fit on the chip at once
+// (k_cgm_resident_batch), else one k_cgm_iter_batch launch per CG iteration
+// over the tiles of all of them, in chunks as for one member (cg_chunk_len),
+// until every member's CG has stopped.  On return the CGs are complete, iters[j] holds member j's
 // iteration count, and every member's stream waits for the event done
 // before its next work.  On an error *bad names the member concerned.
 static int run_cg_batch(const std::vector<wavi_ctx *> &mem, const std::vector<hipEvent_t> &pre, hipEvent_t done,
@@ -2593,10 +2734,30 @@ static int run_cg_batch(const std::vector<wavi_ctx *> &mem, const std::vector<hi
     HIPCHK(hipMemcpyAsync(R.first, hf.data(), hf.size() * sizeof(int), hipMemcpyHostToDevice, cs));
     const CGMBatch B{R.members, R.group, R.first};
     const int levels = lead->S.levels;
-    launch_cgm_batch<0, true>(cs, levels, nwg, B, jac);
-    HIPCHK(hipGetLastError());
-    // launch q performs iteration q - 1 of every member whose CG has not stopped
+    // all of them in one launch if they fit on the chip at once
+    RoomHold hold;
+    std::vector<CGMExchange> hx(mem.size());
+    int units = 0;
+    for (wavi_ctx *m : mem) units += m->x_units;
+    bool resident = true;
+    for (wavi_ctx *m : mem) resident = resident && m->xwords && !m->x_off && m->cg_mode == WAVI_CG_AUTO;
+    resident = resident && hold.take(lead->device, units);
+    for (size_t j = 0; j < mem.size() && resident; ++j) {
+        unsigned tag = 0;
+        resident = cg_resident_begin(mem[j], &tag, cs, false);
+        if (resident) hx[j] = cgm_exchange(mem[j], tag);
+    }
     int q = 1, c = 0;
+    if (resident) {
+        HIPCHK(hipMemcpyAsync(R.ex, hx.data(), hx.size() * sizeof(CGMExchange), hipMemcpyHostToDevice, cs));
+        launch_cgm_resident_batch(cs, levels, nwg, (int)mem.size(), B, R.ex, jac);
+        HIPCHK(hipGetLastError());
+        q = qmax + 1;
+    } else {
+        launch_cgm_batch<0, true>(cs, levels, nwg, B, jac);
+        HIPCHK(hipGetLastError());
+    }
+    // launch q performs iteration q - 1 of every member whose CG has not stopped
     while (q <= qmax) {
         const int n = std::min(cg_chunk_len(c, 0), qmax - q + 1);
         for (int s = 0; s < n; ++s, ++q) {
@@ -2627,6 +2788,8 @@ static int run_cg_batch(const std::vector<wavi_ctx *> &mem, const std::vector<hi
             return WAVI_ESTATE;
         }
         iters[j] = f->iters;
+        ctx->x_ran = resident;
+        if (f->gave_up) ctx->x_off = true;
         if (j > 0) HIPCHK(hipStreamWaitEvent(ctx->stream, done, 0));
     }
     return WAVI_OK;
@@ -2910,6 +3073,7 @@ int wavi_update_velocities_lockstep_noalloc(wavi_ctx **ctxs, int n, wavi_solve_r
     T.members = (CGMIterArgs *)base;
     T.group = (int *)(base + off_group);
     T.first = (int *)(base + off_first);
+    T.ex = (CGMExchange *)(base + WAVI_NOALLOC_SCRATCH_BYTES);
     T.ev.resize(n + 1);
     for (int k = 0; k < n; ++k) T.ev[k] = ctxs[k]->ev_ls;
     T.ev[n] = ctxs[0]->ev_ls_done;

@@ -2507,6 +2507,10 @@ struct CgTile {
         w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
         at0 = Lo.at(i0, j0);
         at = at0 + lx + __umul24(Lo.px, (unsigned)ly);
+    }
+    // (apart, so that the first loads do not wait for its arithmetic)
+    __device__ __forceinline__ void place_halo(const CGLayout &Lo)
+    {
         // the coarse halo, one side per wavefront (left, right, below, above):
         // line k = l / 16 of N, point l % 16 along it; the fifth line and the
         // corner blocks (u below right, v above left) in a second round
@@ -2529,6 +2533,10 @@ struct CgTile {
             dj = corner ? haar_halo_offset<LEV>(!after, cy) : (rows ? c : q);
         }
         h1 = at0 + (unsigned)(di + (int)__mul24((int)Lo.px, dj));
+    }
+    // the coefficients, in the order of their first use
+    __device__ __forceinline__ void load_coef(const CGLayout &Lo)
+    {
         // halo points: wavefront 3 the sides' u, wavefront 2 their v, wavefront 1
         // the corners (u lane 0, v lane 1)
         h = HaloPos{17, 0, 0, 17, w == 3 || (w == 1 && l == 0), w == 2 || (w == 1 && l == 1)};
@@ -2537,10 +2545,6 @@ struct CgTile {
             h.vx = h.ux;
             h.vy = h.uy;
         }
-    }
-    // the coefficients, in the order of their first use
-    __device__ __forceinline__ void load_coef(const CGLayout &Lo)
-    {
         cr.hhu = cr.hhv = 0.0;
         const double2 oh = elem32(Lo.pair(CG_H), at);
         hmb = 0;
@@ -2735,6 +2739,7 @@ __device__ __forceinline__ bool cg_step_tile(const CGArgs &a, int par, const int
     const double2 r = elem32(R, at), p = elem32(P, at), x = elem32(Lo.pair(CG_X), at);
     const double2 dz = PRE ? elem32(D, at) : make_double2(0.0, 0.0);
     t.mb = elem32(Lo.M, at);
+    t.place_halo(Lo);
     const double2 nr0 = elem32(R, t.h0), np0 = elem32(P, t.h0), nd0 = PRE ? elem32(D, t.h0) : make_double2(0.0, 0.0);
     const double2 nr1 = elem32(R, t.h1), np1 = elem32(P, t.h1), nd1 = PRE ? elem32(D, t.h1) : make_double2(0.0, 0.0);
     t.load_coef(Lo);
@@ -3101,6 +3106,7 @@ __global__ void __launch_bounds__(256, 2) k_cg_resident(CGArgs a, CGExchange E)
     const CGLayout &Lo = a.Lo;
     CgTile<LEV> t;
     t.place(Lo, bx * TILE, by * TILE);
+    t.place_halo(Lo);
     double sum0, sum1, abstol;
     cg_resident_sums<PRE, FOLD>(a, lds, sum0, sum1, abstol);
     // the tile's state; zero where there is no neighbour
@@ -3282,6 +3288,7 @@ struct CGMScalars {
     CGMState s[2];  // by launch parity
     int done;       // sticky stop flag, read by the host only
     int iters;      // iterations at the stop
+    int abort;      // a workgroup of k_cgm_resident gave up waiting
 };
 
 // Arena arrays: (u, v) pairs, ns points each; then the corners' h*eta_av.
@@ -3329,6 +3336,11 @@ struct RingSlots {
         if (row >= 0) R[row] = v;
         if (col >= 0) R[col] = v;
     }
+    __device__ __forceinline__ void put_shared(xword *R, xword v) const
+    {
+        if (row >= 0) __hip_atomic_store(R + row, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (col >= 0) __hip_atomic_store(R + col, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
 };
 
 struct CGMLayout {
@@ -3362,6 +3374,7 @@ struct CGMArgs {
     CGMScalars *st;
     CGMHostFlag *hflag;      // host-mapped stop report, reset here
     int nblk;
+    int resident;            // the CG ran as k_cgm_resident
 };
 
 // setup (P x0 computed beforehand): r0 = b - R A P x0, p = s = 0, x = x0, the
@@ -3386,8 +3399,10 @@ __global__ void __launch_bounds__(256) k_cgm_setup(CGMArgs a)
         }
         a.st->done = 0;
         a.st->iters = 0;
+        a.st->abort = 0;
         a.hflag->done = 0;
         a.hflag->iters = 0;
+        a.hflag->gave_up = 0;
     }
     int bx, by;
     const int tile_id = band_tile(g, L, bx, by);
@@ -3443,7 +3458,8 @@ __global__ void __launch_bounds__(256) k_cgm_finish(CGMArgs a)
     int bx, by;
     band_tile(a.g, L, bx, by);
     const unsigned at = a.Lo.at(bx * TILE + (int)(threadIdx.x & 15), by * TILE + (int)(threadIdx.x >> 4));
-    const float2 x = elem32(a.Lo.pair(CGM_X), at);
+    const bool resident = a.resident && a.st->abort == 0;  // the resident CG leaves x in CGM_W
+    const float2 x = elem32(a.Lo.pair(resident ? CGM_W : CGM_X), at);
     cg_finish_tile<float>(a.g, a.levels, bx, by, x.x, x.y, elem32(a.Lo.M, at), a.xu, a.xv, a.eu, a.ev);
 }
 
@@ -3544,6 +3560,251 @@ struct CGMIterArgs {
     int maxiter, nblk;
 };
 
+template <bool PRE>
+struct CgmSmem {
+    float2 UV[18][19];               // window of P r (u and v points)
+    float2 H[18][19];                // thickness window, 0 off the masks
+    float4 cell[17][18];             // r_xx, r_yy, r_xy and the implicit term
+    float2 T[2][TILE][TILE + 1];     // transposes of the block transforms
+    float2 dz[PRE ? TILE : 1][TILE + 1];  // Jacobi: 1 / |diag(A_c)| of the tile
+    uint8_t mb[TILE][TILE + 4];      // mask bits of the tile
+    double red0[8];
+    float red1[8];
+    double red2[8];
+};
+
+// A thread's part of a tile in the mixed CG: its position, coefficients and
+// what the tile does with a new r and s.
+template <int LEV, bool PRE>
+struct CgmTile {
+    int tid, l, w, lx, ly, cx, cy;   // (lx, ly) row-major, (cx, cy) column-major (transposes)
+    unsigned at0, at, mb;
+    bool halo;
+    int hx, hy;                      // its halo point of the window
+    int ntl, hslot;                  // ... in the neighbour's ring (tile ntile: none)
+    int ex, ey;                      // its cell before the tile (wavefront 0)
+    float2 dz, hH, oH, cc, ec, oB;
+    float ch, eh;
+
+    __device__ __forceinline__ void place(const CGMLayout &Lo, int bx, int by)
+    {
+        tid = threadIdx.x;
+        l = tid & 63;
+        w = __builtin_amdgcn_readfirstlane(tid >> 6);
+        lx = tid & 15;
+        ly = tid >> 4;
+        cx = tid >> 4;
+        cy = tid & 15;
+        // (24-bit products: a 32-bit multiply-add is emitted as a 64-bit one whose
+        // unused high addend can be a register with a load in flight)
+        at0 = Lo.at(bx * TILE, by * TILE);
+        at = at0 + (unsigned)lx + __umul24(Lo.px, (unsigned)ly);
+        const bool corner = w == 2 && l < 2;  // lane 0: (17, 0), of which u is read; lane 1: (0, 17), v
+        halo = w == 3 || corner;
+        hx = l == 0 ? 17 : 0;
+        hy = l == 0 ? 0 : 17;
+        ntl = hslot = 0;
+        dz = make_float2(1.f, 1.f);
+        hH = ec = make_float2(0.f, 0.f);
+        eh = 0.f;
+    }
+    // Wavefronts 2 and 3: halo point (hx, hy) of the window from the
+    // neighbours' rings: slot hslot of the tile ntl, (bx + hdx, by + hdy)
+    __device__ __forceinline__ void place_halo(const GridDims &g, int bx, int by)
+    {
+        const int q = l & 15, side = l >> 4;
+        int hdx = l == 0 ? 1 : -1, hdy = -hdx;
+        hslot = l == 0 ? 16 : 15;
+        if (w == 3) {
+            halo_side(l, hx, hy);
+            hdx = side == 0 ? -1 : (side == 1 ? 1 : 0);
+            hdy = side == 2 ? -1 : (side == 3 ? 1 : 0);
+            hslot = q + (side == 0 ? 48 : (side == 1 ? 32 : (side == 2 ? 16 : 0)));
+        }
+        const int nbxx = bx + hdx, nbyy = by + hdy;
+        ntl = (nbxx >= 0 && nbxx < g.nbx && nbyy >= 0 && nbyy < g.nby) ? nbxx + g.nbx * nbyy : g.nbx * g.nby;
+    }
+    __device__ __forceinline__ float2 load(const CGMLayout &Lo, int A, unsigned k) const
+    {
+        return elem32((const float2 *)Lo.pair(A), k);
+    }
+    __device__ __forceinline__ float2 halo_thickness(const CGMLayout &Lo) const
+    {
+        return load(Lo, CGM_H, at0 + (unsigned)(hx - 1 + (int)__mul24((int)Lo.px, hy - 1)));
+    }
+    __device__ __forceinline__ void load_coef(const CGMLayout &Lo)
+    {
+        oH = load(Lo, CGM_H, at);
+        cc = load(Lo, CGM_CELL, at);
+        ch = elem32((const float *)Lo.corner(), at);
+        // the cells before the tile: (0, 0..16), (1..16, 0); lanes past them repeat the last
+        ex = l < 17 ? 0 : (l < 33 ? l - 16 : 16);
+        ey = l < 17 ? l : 0;
+        float2 c = make_float2(0.f, 0.f);
+        float h = 0.f;
+        if (w == 0) {
+            const unsigned ea = at0 + (unsigned)(ex - 1 + (int)__mul24((int)Lo.px, ey - 1));
+            c = load(Lo, CGM_CELL, ea);
+            h = elem32((const float *)Lo.corner(), ea);
+        }
+        ec = c;
+        eh = h;
+        oB = load(Lo, CGM_B, at);
+    }
+    // From r and s1 (S: there is one) of the tile and the halo's P r (hv): the
+    // own point's w = R A P r and P w, and P r, P s of the point (cx, cy),
+    // given to `images` as soon as they are known.
+    template <bool S, class Images>
+    __device__ __forceinline__ void operate(float rdx, float rdy, float2 r, float2 s1, float2 hv, CgmSmem<PRE> &sm,
+                                            float2 &wn, float2 &pw, Images images)
+    {
+        const bool inu = mb & CB_INNER_U, inv = mb & CB_INNER_V, mwu = mb & CB_WAVELET_U, mwv = mb & CB_WAVELET_V;
+        // ---- x pass of P r and P s (Jacobi: of D^-1 r and D^-1 s); halo and
+        // thickness windows into LDS
+        {
+            float a0 = mwu ? (PRE ? dz.x * r.x : r.x) : 0.f, a1 = mwv ? (PRE ? dz.y * r.y : r.y) : 0.f;
+            haar_lines_P<LEV>(a0, a1, lx);
+            sm.T[0][ly][lx] = make_float2(a0, a1);
+            if (S) {
+                float a2 = mwu ? (PRE ? dz.x * s1.x : s1.x) : 0.f, a3 = mwv ? (PRE ? dz.y * s1.y : s1.y) : 0.f;
+                haar_lines_P<LEV>(a2, a3, lx);
+                sm.T[1][ly][lx] = make_float2(a2, a3);
+            }
+        }
+        sm.mb[ly][lx] = (uint8_t)mb;
+        if constexpr (PRE) sm.dz[ly][lx] = dz;
+        sm.H[ly + 1][lx + 1] = oH;
+        if (halo) {
+            sm.UV[hy][hx] = hv;
+            sm.H[hy][hx] = hH;
+        }
+        __syncthreads();
+        // ---- y pass in the column-major lanes: P r into the window, rings of P r
+        // and P s
+        {
+            const unsigned m = sm.mb[cy][cx];
+            const float2 t0 = sm.T[0][cy][cx];
+            float y0 = t0.x, y1 = t0.y;
+            haar_lines_P<LEV>(y0, y1, cy);
+            const float2 pr = make_float2((m & CB_INNER_U) ? y0 : 0.f, (m & CB_INNER_V) ? y1 : 0.f);
+            sm.UV[cy + 1][cx + 1] = pr;
+            float2 ps = make_float2(0.f, 0.f);
+            if (S) {
+                const float2 t1 = sm.T[1][cy][cx];
+                float y2 = t1.x, y3 = t1.y;
+                haar_lines_P<LEV>(y2, y3, cy);
+                ps = make_float2((m & CB_INNER_U) ? y2 : 0.f, (m & CB_INNER_V) ? y3 : 0.f);
+            }
+            images(pr, ps);
+        }
+        __syncthreads();
+        // ---- intermediates of the cell (x, y) of the 17 x 17 window, whose own
+        // point has the value uv and the thickness h
+        auto intermediates = [&](int x, int y, float2 uv, float2 h, float2 hd, float hc) -> float4 {
+            const float u1 = sm.UV[y][x + 1].x, v1 = sm.UV[y + 1][x].y;
+            const float2 d = sm.UV[y + 1][x + 1];
+            const float dudx = rdx * (u1 - uv.x), dvdy = rdy * (v1 - uv.y);
+            const float divq = rdx * (sm.H[y][x + 1].x * u1 - h.x * uv.x) + rdy * (sm.H[y + 1][x].y * v1 - h.y * uv.y);
+            return make_float4(2.f * hd.x * (2.f * dudx + dvdy), 2.f * hd.x * (2.f * dvdy + dudx),
+                               hc * (rdy * (d.x - u1) + rdx * (d.y - v1)), hd.y * divq);
+        };
+        const float2 uv = sm.UV[ly + 1][lx + 1];
+        const float4 own = intermediates(lx + 1, ly + 1, uv, oH, cc, ch);
+        if (w == 0) sm.cell[ey][ex] = intermediates(ex, ey, sm.UV[ey][ex], sm.H[ey][ex], ec, eh);
+        sm.cell[ly + 1][lx + 1] = own;
+        __syncthreads();
+        // ---- A at the tile's points (zero off the inner masks), R x pass
+        {
+            const float4 left = sm.cell[ly + 1][lx], below = sm.cell[ly][lx + 1];
+            const float rxy00 = sm.cell[ly][lx].z;
+            const float d_rxx = rdx * (own.x - left.x);
+            const float d_rxy_u = rdy * (left.z - rxy00);
+            const float d_ext_u = rdx * (own.w - left.w);
+            const float Au = ((d_rxx + d_rxy_u) - oB.x * uv.x) - oH.x * d_ext_u;
+            const float d_ryy = rdy * (own.y - below.y);
+            const float d_rxy_v = rdx * (below.z - rxy00);
+            const float d_ext_v = rdy * (own.w - below.w);
+            const float Av = ((d_ryy + d_rxy_v) - oB.y * uv.y) - oH.y * d_ext_v;
+            float a0 = inu ? Au : 0.f, a1 = inv ? Av : 0.f;
+            haar_lines_R<LEV>(a0, a1, lx);
+            sm.T[0][ly][lx] = make_float2(a0, a1);
+        }
+        __syncthreads();
+        // ---- R y pass, wavelet mask (w), P y pass
+        {
+            const float2 t0 = sm.T[0][cy][cx];
+            float c0 = t0.x, c1 = t0.y;
+            haar_lines_R<LEV>(c0, c1, cy);
+            const unsigned m = sm.mb[cy][cx];
+            const float2 wc = make_float2((m & CB_WAVELET_U) ? c0 : 0.f, (m & CB_WAVELET_V) ? c1 : 0.f);
+            float q0 = wc.x, q1 = wc.y;
+            if constexpr (PRE) {
+                const float2 d = sm.dz[cy][cx];
+                q0 = d.x * wc.x;
+                q1 = d.y * wc.y;
+            }
+            haar_lines_P<LEV>(q0, q1, cy);
+            sm.T[0][cy][cx] = wc;
+            sm.T[1][cy][cx] = make_float2(q0, q1);
+        }
+        __syncthreads();
+        // ---- P x pass
+        wn = sm.T[0][ly][lx];
+        const float2 tq = sm.T[1][ly][lx];
+        float tw_u = tq.x, tw_v = tq.y;
+        haar_lines_P<LEV>(tw_u, tw_v, lx);
+        pw = make_float2(inu ? tw_u : 0.f, inv ? tw_v : 0.f);
+    }
+    // The tile's partials (r, u) and (w, u) with u = D^-1 r under Jacobi, (r, r)
+    // and (w, r) without; valid in thread 0 after its barrier.
+    __device__ __forceinline__ float2 partials(float2 r, float2 wn, CgmSmem<PRE> &sm) const
+    {
+        const float zr_u = PRE ? dz.x * r.x : r.x, zr_v = PRE ? dz.y * r.y : r.y;
+        float gg = r.x * zr_u + r.y * zr_v;
+        float dd = wn.x * zr_u + wn.y * zr_v;
+        gg = wave_total_rows_f(row_sum16f(gg));
+        dd = wave_total_rows_f(row_sum16f(dd));
+        if (l == 63) {
+            sm.red1[w] = gg;
+            sm.red1[4 + w] = dd;
+        }
+        __syncthreads();
+        return make_float2((sm.red1[0] + sm.red1[1]) + (sm.red1[2] + sm.red1[3]),
+                           (sm.red1[4] + sm.red1[5]) + (sm.red1[6] + sm.red1[7]));
+    }
+};
+
+// alpha and beta of an iteration from the sums (r, r) and (w, r) of the one
+// before (S: its state)
+__device__ __forceinline__ void cgm_scalars(const CGMState &S, double gamma, double delta, double &alpha, double &beta)
+{
+    beta = S.it == 0 ? 0.0 : gamma * S.igamma;
+    alpha = gamma / (S.it == 0 ? delta : delta - beta * gamma * S.ialpha);
+}
+
+// the state they leave
+__device__ __forceinline__ CGMState cgm_next(const CGMState &S, double gamma, double alpha, double tol2)
+{
+    CGMState n;
+    n.igamma = 1.0 / gamma;
+    n.alpha = alpha;
+    n.ialpha = 1.0 / alpha;
+    n.tol2 = tol2;
+    n.it = S.it + 1;
+    n.done = 0;
+    return n;
+}
+
+// square of the stopping tolerance, at iteration 0
+template <bool PRE>
+__device__ __forceinline__ double cgm_tol2(const CGMIterArgs &a, double gamma, CgmSmem<PRE> &sm)
+{
+    const double abstol = a.tol_coarse * sqrt(lanes_sum(a.Pb, a.g.npart, sm.red2));
+    double tol = a.reltol * sqrt(gamma);
+    if (abstol > tol) tol = abstol;
+    return tol * tol;
+}
+
 // One iteration (INIT: the launch before the first iteration, which only
 // computes w0 = A_c r0 and the rings of set 1: P r0, P s = 0, P w0, and the
 // partial (r0, r0), (w0, r0)).  All loads are issued up front, unconditional
@@ -3565,28 +3826,12 @@ template <int PAR, bool INIT, int LEV, bool PRE>
 __device__ __forceinline__ bool cgm_iter_tile(const CGMIterArgs &a, const int L)
 {
     static_assert(!INIT || PAR == 0, "the initial launch reads set 0");
-    struct Smem {
-        float2 UV[18][19];               // window of P r (u and v points)
-        float2 H[18][19];                // thickness window, 0 off the masks
-        float4 cell[17][18];             // r_xx, r_yy, r_xy and the implicit term
-        float2 T[2][TILE][TILE + 1];     // transposes of the block transforms
-        float2 dz[PRE ? TILE : 1][TILE + 1];  // Jacobi: 1 / |diag(A_c)| of the tile
-        uint8_t mb[TILE][TILE + 4];      // mask bits of the tile
-        double red0[8];
-        float red1[8];
-        double red2[8];
-    };
-    __shared__ Smem sm;
+    __shared__ CgmSmem<PRE> sm;
     const GridDims &g = a.g;
     const int ntile = g.nbx * g.nby;
     if (L >= ntile) return false;
-    const int tid = threadIdx.x, l = tid & 63;
-    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     int bx, by;
     const int tile_id = band_tile(g, L, bx, by);
-    const int i0 = bx * TILE, j0 = by * TILE;
-    const int lx = tid & 15, ly = tid >> 4;    // row-major position
-    const int cx = tid >> 4, cy = tid & 15;    // column-major position (transposes)
     constexpr int NP = 1 - PAR;
     // Launch q >= 1 performs iteration k = q - 1, so PAR == 0 iff k is odd.
     // x is advanced every other iteration: an even iteration leaves it, the
@@ -3595,13 +3840,11 @@ __device__ __forceinline__ bool cgm_iter_tile(const CGMIterArgs &a, const int L)
     // an even iteration applies the pending alpha_{k-1} p_{k-1}.
     constexpr bool XUPD = PAR == 0;
     const CGMLayout &Lo = a.Lo;
-    const float rdx = a.rdx, rdy = a.rdy;
-    // (24-bit products: a 32-bit multiply-add is emitted as a 64-bit one whose
-    // unused high addend can be a register with a load in flight)
-    const unsigned at0 = Lo.at(i0, j0), at = at0 + (unsigned)lx + __umul24(Lo.px, (unsigned)ly);
-    auto cload = [&](int A, unsigned k) -> float2 { return elem32((const float2 *)Lo.pair(A), k); };
+    CgmTile<LEV, PRE> t;
+    t.place(Lo, bx, by);
+    const int tid = t.tid;
     auto cstore = [&](int A, float2 v) {
-        st_nt(reinterpret_cast<double *>(&elem32(Lo.pair(A), at)),
+        st_nt(reinterpret_cast<double *>(&elem32(Lo.pair(A), t.at)),
               __hiloint2double(__float_as_int(v.y), __float_as_int(v.x)));
     };
     // ---- loads, all issued before the first use, in the order they are
@@ -3614,52 +3857,27 @@ __device__ __forceinline__ bool cgm_iter_tile(const CGMIterArgs &a, const int L)
 #pragma unroll
         for (int e = 0; e < 4; ++e) pv[e] = a.Pgd[PAR * a.npad + tid + 256 * e];
     }
-    const unsigned mb = elem32((const uint8_t *)Lo.M, at);
-    float2 r = cload(CGM_R, at), w0 = make_float2(0.f, 0.f), p0 = w0, s0 = w0, x0 = w0, dz = make_float2(1.f, 1.f);
+    t.mb = elem32((const uint8_t *)Lo.M, t.at);
+    float2 r = t.load(Lo, CGM_R, t.at), w0 = make_float2(0.f, 0.f), p0 = w0, s0 = w0, x0 = w0;
     if (!INIT) {
-        w0 = cload(CGM_W, at);
-        p0 = cload(CGM_P, at);
-        s0 = cload(CGM_S, at);
-        if (XUPD) x0 = cload(CGM_X, at);
+        w0 = t.load(Lo, CGM_W, t.at);
+        p0 = t.load(Lo, CGM_P, t.at);
+        s0 = t.load(Lo, CGM_S, t.at);
+        if (XUPD) x0 = t.load(Lo, CGM_X, t.at);
     }
-    if constexpr (PRE) dz = cload(CGM_DINV, at);
-    // halo point (hx, hy) of the window from the neighbours' rings: slot
-    // hslot of the tile (bx + hdx, by + hdy)
-    const bool corner = w == 2 && l < 2;  // lane 0: (17, 0), of which u is read; lane 1: (0, 17), v
-    const bool halo = w == 3 || corner;
-    int hx = l == 0 ? 17 : 0, hy = l == 0 ? 0 : 17;
+    if constexpr (PRE) t.dz = t.load(Lo, CGM_DINV, t.at);
+    const float2 dz = t.dz;
     float4 hrs = make_float4(0.f, 0.f, 0.f, 0.f);
     float2 hw = make_float2(0.f, 0.f), hH = hw;
-    if (w >= 2) {
-        const int q = l & 15, side = l >> 4;
-        int hdx = l == 0 ? 1 : -1, hdy = -hdx, hslot = l == 0 ? 16 : 15;
-        if (w == 3) {
-            halo_side(l, hx, hy);
-            hdx = side == 0 ? -1 : (side == 1 ? 1 : 0);
-            hdy = side == 2 ? -1 : (side == 3 ? 1 : 0);
-            hslot = q + (side == 0 ? 48 : (side == 1 ? 32 : (side == 2 ? 16 : 0)));
-        }
-        const int nbxx = bx + hdx, nbyy = by + hdy;
-        const int ntl = (nbxx >= 0 && nbxx < g.nbx && nbyy >= 0 && nbyy < g.nby) ? nbxx + g.nbx * nbyy : ntile;
-        const unsigned hr_at = ring_at(PAR, ntile, ntl) + (unsigned)hslot;
+    if (t.w >= 2) {
+        t.place_halo(g, bx, by);
+        const unsigned hr_at = ring_at(PAR, ntile, t.ntl) + (unsigned)t.hslot;
         hrs = elem32((const float4 *)a.R.rs, hr_at);
         if (!INIT) hw = elem32((const float2 *)a.R.w, hr_at);
-        hH = cload(CGM_H, at0 + (unsigned)(hx - 1 + (int)__mul24((int)Lo.px, hy - 1)));
+        hH = t.halo_thickness(Lo);
     }
-    const float2 oH = cload(CGM_H, at);
-    const float2 cc = cload(CGM_CELL, at);
-    const float ch = elem32((const float *)Lo.corner(), at);
-    // the cells before the tile: (0, 0..16), (1..16, 0); lanes past them repeat the last
-    const int ex = l < 17 ? 0 : (l < 33 ? l - 16 : 16), ey = l < 17 ? l : 0;
-    float2 ec = make_float2(0.f, 0.f);
-    float eh = 0.f;
-    if (w == 0) {
-        const unsigned ea = at0 + (unsigned)(ex - 1 + (int)__mul24((int)Lo.px, ey - 1));
-        ec = cload(CGM_CELL, ea);
-        eh = elem32((const float *)Lo.corner(), ea);
-    }
-    const float2 oB = cload(CGM_B, at);
-    const bool inu = mb & CB_INNER_U, inv = mb & CB_INNER_V, mwu = mb & CB_WAVELET_U, mwv = mb & CB_WAVELET_V;
+    t.hH = hH;
+    t.load_coef(Lo);
     // ---- scalars from the previous launch's partials (FP64 across workgroups)
     float fa = 0.f, fb = 0.f, fxp = 0.f;
     if (!INIT) {
@@ -3680,13 +3898,7 @@ __device__ __forceinline__ bool cgm_iter_tile(const CGMIterArgs &a, const int L)
             return true;
         }
         // stop when ||r|| <= tol, tested as ||r||^2 <= tol^2
-        double tol2 = S.tol2;
-        if (S.it == 0) {
-            const double abstol = a.tol_coarse * sqrt(lanes_sum(a.Pb, g.npart, sm.red2));
-            double tol = a.reltol * sqrt(gamma);
-            if (abstol > tol) tol = abstol;
-            tol2 = tol * tol;
-        }
+        const double tol2 = S.it == 0 ? cgm_tol2<PRE>(a, gamma, sm) : S.tol2;
         if (S.it >= a.maxiter || gamma <= tol2) {
             if (L == 0 && tid == 0) {
                 CGMState n = S;
@@ -3704,18 +3916,9 @@ __device__ __forceinline__ bool cgm_iter_tile(const CGMIterArgs &a, const int L)
             }
             return true;
         }
-        const double beta = S.it == 0 ? 0.0 : gamma * S.igamma;
-        const double alpha = gamma / (S.it == 0 ? delta : delta - beta * gamma * S.ialpha);
-        if (L == 0 && tid == 0) {
-            CGMState n;
-            n.igamma = 1.0 / gamma;
-            n.alpha = alpha;
-            n.ialpha = 1.0 / alpha;
-            n.tol2 = tol2;
-            n.it = S.it + 1;
-            n.done = 0;
-            a.st->s[NP] = n;
-        }
+        double alpha, beta;
+        cgm_scalars(S, gamma, delta, alpha, beta);
+        if (L == 0 && tid == 0) a.st->s[NP] = cgm_next(S, gamma, alpha, tol2);
         fa = (float)alpha;
         fb = (float)beta;
         fxp = XUPD ? (float)(S.alpha + alpha * beta) : 0.f;
@@ -3733,116 +3936,18 @@ __device__ __forceinline__ bool cgm_iter_tile(const CGMIterArgs &a, const int L)
         cstore(CGM_S, s1);
         cstore(CGM_R, r);
     }
-    // ---- x pass of P r and P s (Jacobi: of D^-1 r and D^-1 s); halo and
-    // thickness windows into LDS
-    {
-        float a0 = mwu ? (PRE ? dz.x * r.x : r.x) : 0.f, a1 = mwv ? (PRE ? dz.y * r.y : r.y) : 0.f;
-        haar_lines_P<LEV>(a0, a1, lx);
-        sm.T[0][ly][lx] = make_float2(a0, a1);
-        if (!INIT) {
-            float a2 = mwu ? (PRE ? dz.x * s1.x : s1.x) : 0.f, a3 = mwv ? (PRE ? dz.y * s1.y : s1.y) : 0.f;
-            haar_lines_P<LEV>(a2, a3, lx);
-            sm.T[1][ly][lx] = make_float2(a2, a3);
-        }
-    }
-    sm.mb[ly][lx] = (uint8_t)mb;
-    if constexpr (PRE) sm.dz[ly][lx] = dz;
-    sm.H[ly + 1][lx + 1] = oH;
-    if (halo) {
-        sm.UV[hy][hx] = INIT ? make_float2(hrs.x, hrs.y)
-                             : make_float2(hrs.x - fa * (hw.x + fb * hrs.z), hrs.y - fa * (hw.y + fb * hrs.w));
-        sm.H[hy][hx] = hH;
-    }
-    __syncthreads();
-    // ---- y pass in the column-major lanes: P r into the window, rings of P r
-    // and P s
-    {
-        const unsigned m = sm.mb[cy][cx];
-        const float2 t0 = sm.T[0][cy][cx];
-        float y0 = t0.x, y1 = t0.y;
-        haar_lines_P<LEV>(y0, y1, cy);
-        const float2 pr = make_float2((m & CB_INNER_U) ? y0 : 0.f, (m & CB_INNER_V) ? y1 : 0.f);
-        sm.UV[cy + 1][cx + 1] = pr;
-        float2 ps = make_float2(0.f, 0.f);
-        if (!INIT) {
-            const float2 t1 = sm.T[1][cy][cx];
-            float y2 = t1.x, y3 = t1.y;
-            haar_lines_P<LEV>(y2, y3, cy);
-            ps = make_float2((m & CB_INNER_U) ? y2 : 0.f, (m & CB_INNER_V) ? y3 : 0.f);
-        }
-        RingSlots(cx, cy).put(a.R.rs + ring_at(NP, ntile, tile_id), make_float4(pr.x, pr.y, ps.x, ps.y));
-    }
-    __syncthreads();
-    // ---- intermediates of the cell (x, y) of the 17 x 17 window, whose own
-    // point has the value uv and the thickness h
-    auto intermediates = [&](int x, int y, float2 uv, float2 h, float2 hd, float hc) -> float4 {
-        const float u1 = sm.UV[y][x + 1].x, v1 = sm.UV[y + 1][x].y;
-        const float2 d = sm.UV[y + 1][x + 1];
-        const float dudx = rdx * (u1 - uv.x), dvdy = rdy * (v1 - uv.y);
-        const float divq = rdx * (sm.H[y][x + 1].x * u1 - h.x * uv.x) + rdy * (sm.H[y + 1][x].y * v1 - h.y * uv.y);
-        return make_float4(2.f * hd.x * (2.f * dudx + dvdy), 2.f * hd.x * (2.f * dvdy + dudx),
-                           hc * (rdy * (d.x - u1) + rdx * (d.y - v1)), hd.y * divq);
-    };
-    const float2 uv = sm.UV[ly + 1][lx + 1];
-    const float4 own = intermediates(lx + 1, ly + 1, uv, oH, cc, ch);
-    if (w == 0) sm.cell[ey][ex] = intermediates(ex, ey, sm.UV[ey][ex], sm.H[ey][ex], ec, eh);
-    sm.cell[ly + 1][lx + 1] = own;
-    __syncthreads();
-    // ---- A at the tile's points (zero off the inner masks), R x pass
-    {
-        const float4 left = sm.cell[ly + 1][lx], below = sm.cell[ly][lx + 1];
-        const float rxy00 = sm.cell[ly][lx].z;
-        const float d_rxx = rdx * (own.x - left.x);
-        const float d_rxy_u = rdy * (left.z - rxy00);
-        const float d_ext_u = rdx * (own.w - left.w);
-        const float Au = ((d_rxx + d_rxy_u) - oB.x * uv.x) - oH.x * d_ext_u;
-        const float d_ryy = rdy * (own.y - below.y);
-        const float d_rxy_v = rdx * (below.z - rxy00);
-        const float d_ext_v = rdy * (own.w - below.w);
-        const float Av = ((d_ryy + d_rxy_v) - oB.y * uv.y) - oH.y * d_ext_v;
-        float a0 = inu ? Au : 0.f, a1 = inv ? Av : 0.f;
-        haar_lines_R<LEV>(a0, a1, lx);
-        sm.T[0][ly][lx] = make_float2(a0, a1);
-    }
-    __syncthreads();
-    // ---- R y pass, wavelet mask (w), P y pass
-    {
-        const float2 t0 = sm.T[0][cy][cx];
-        float c0 = t0.x, c1 = t0.y;
-        haar_lines_R<LEV>(c0, c1, cy);
-        const unsigned m = sm.mb[cy][cx];
-        const float2 wn = make_float2((m & CB_WAVELET_U) ? c0 : 0.f, (m & CB_WAVELET_V) ? c1 : 0.f);
-        float q0 = wn.x, q1 = wn.y;
-        if constexpr (PRE) {
-            const float2 d = sm.dz[cy][cx];
-            q0 = d.x * wn.x;
-            q1 = d.y * wn.y;
-        }
-        haar_lines_P<LEV>(q0, q1, cy);
-        sm.T[0][cy][cx] = wn;
-        sm.T[1][cy][cx] = make_float2(q0, q1);
-    }
-    __syncthreads();
-    // ---- P x pass, stores, partials of (r, r) and (w, r)
-    const float2 wn = sm.T[0][ly][lx], tq = sm.T[1][ly][lx];
-    float tw_u = tq.x, tw_v = tq.y;
-    haar_lines_P<LEV>(tw_u, tw_v, lx);
+    const float2 hv = INIT ? make_float2(hrs.x, hrs.y)
+                           : make_float2(hrs.x - fa * (hw.x + fb * hrs.z), hrs.y - fa * (hw.y + fb * hrs.w));
+    float2 wn, pw;
+    t.template operate<!INIT>(
+        a.rdx, a.rdy, r, s1, hv, sm, wn, pw,
+        [&](float2 pr, float2 ps) {
+            RingSlots(t.cx, t.cy).put(a.R.rs + ring_at(NP, ntile, tile_id), make_float4(pr.x, pr.y, ps.x, ps.y));
+        });
     cstore(CGM_W, wn);
-    RingSlots(lx, ly).put(a.R.w + ring_at(NP, ntile, tile_id), make_float2(inu ? tw_u : 0.f, inv ? tw_v : 0.f));
-    // (r, u) and (w, u) with u = D^-1 r under Jacobi, (r, r) and (w, r) without
-    const float zr_u = PRE ? dz.x * r.x : r.x, zr_v = PRE ? dz.y * r.y : r.y;
-    float gg = r.x * zr_u + r.y * zr_v;
-    float dd = wn.x * zr_u + wn.y * zr_v;
-    gg = wave_total_rows_f(row_sum16f(gg));
-    dd = wave_total_rows_f(row_sum16f(dd));
-    if (l == 63) {
-        sm.red1[w] = gg;
-        sm.red1[4 + w] = dd;
-    }
-    __syncthreads();
-    if (tid == 0)
-        a.Pgd[NP * a.npad + tile_id] = make_float2((sm.red1[0] + sm.red1[1]) + (sm.red1[2] + sm.red1[3]),
-                                             (sm.red1[4] + sm.red1[5]) + (sm.red1[6] + sm.red1[7]));
+    RingSlots(t.lx, t.ly).put(a.R.w + ring_at(NP, ntile, tile_id), pw);
+    const float2 part = t.partials(r, wn, sm);
+    if (tid == 0) a.Pgd[NP * a.npad + tile_id] = part;
     return false;
 }
 
@@ -3862,8 +3967,12 @@ __global__ void __launch_bounds__(256) k_cgm_iter(CGMIterArgs a)
 // iteration, bit for bit.  Every thread decides the stop alike (same
 // partials, same scalars); at most maxiter + 1 iterations.
 template <int LEV, bool PRE>
-__global__ void __launch_bounds__(256) k_cgm_solve1(CGMIterArgs a)
+__device__ __forceinline__ void cgm_solve1_run(const CGMIterArgs &a, const int *only_if)
 {
+    if (only_if) {  // the resident CG gave up; what it started from is still in place
+        if (*only_if == 0) return;
+        if (threadIdx.x == 0) a.hflag->gave_up = 1;
+    }
     const int ntile = a.g.nbx * a.g.nby;
     for (int L = 0; L < ntile; ++L) {
         (void)cgm_iter_tile<0, true, LEV, PRE>(a, L);
@@ -3877,6 +3986,154 @@ __global__ void __launch_bounds__(256) k_cgm_solve1(CGMIterArgs a)
         }
         if (stop) break;
     }
+}
+
+template <int LEV, bool PRE>
+__global__ void __launch_bounds__(256) k_cgm_solve1(CGMIterArgs a, const int *only_if)
+{
+    cgm_solve1_run<LEV, PRE>(a, only_if);
+}
+
+// What the workgroups of the resident mixed CG exchange, in tagged words.
+struct CGMExchange {
+    xword *ring;    // [2][6][tiles][64]: (P r)_u, (P r)_v, (P s)_u, (P s)_v, (P w)_u, (P w)_v of the ring slots
+    xword *part;    // [2][tiles][2]: the partials (r, r) and (w, r)
+    int *abort;     // a wait ran out
+    unsigned tag;   // tag of the first exchange, larger than any used before
+    unsigned limit; // polls of one wait
+};
+
+// The whole mixed coarse CG in one launch, a tile per workgroup, all of them
+// resident at once (after k_cgm_setup; k_cg_resident tells of the waits).  r,
+// w, p, s and x of a tile stay in registers; an iteration has one exchange: the
+// tiles' two sums, which every workgroup folds, and the ring images of the
+// neighbours, in two sets by parity, since a workgroup may be one exchange
+// ahead of another.  The same operations in the same order as the launches':
+// the same bits.
+// At most 256 tiles, one partial per thread: measured per iteration, launches
+// -> resident, 5.1 -> 3.5 us at 6 tiles, 5.2 -> 4.1 at 63, 5.9 -> 5.1 at 246.
+// With two partials per thread 7.1 -> 9.2 us at 357; with one workgroup
+// folding, as in FP64, 7.1 -> 7.2 us at 357 and 10.4 -> 10.1 at 891.
+template <int LEV, bool PRE>
+__device__ __forceinline__ void cgm_resident_tile(const CGMIterArgs &a, const CGMExchange &E, int blk)
+{
+    __shared__ CgmSmem<PRE> sm;
+    __shared__ int bad;  // a wait ran out; checked after the barrier that follows the wait
+    const GridDims &g = a.g;
+    const int ntile = g.nbx * g.nby, tid = threadIdx.x;
+    if (tid == 0) bad = 0;
+    CGMState S{};
+    const int L = (blk & 7) * (a.nblk >> 3) + (blk >> 3);
+    if (L >= ntile) return;
+    int bx, by;
+    const int tile_id = band_tile(g, L, bx, by);
+    const CGMLayout &Lo = a.Lo;
+    CgmTile<LEV, PRE> t;
+    t.place(Lo, bx, by);
+    const float2 zero = make_float2(0.f, 0.f);
+    t.mb = elem32((const uint8_t *)Lo.M, t.at);
+    float2 r = t.load(Lo, CGM_R, t.at), x = t.load(Lo, CGM_X, t.at), w = zero, p = zero, s = zero;
+    if constexpr (PRE) t.dz = t.load(Lo, CGM_DINV, t.at);
+    float4 hrs = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (t.w >= 2) {
+        t.place_halo(g, bx, by);
+        hrs = elem32((const float4 *)a.R.rs, ring_at(0, ntile, t.ntl) + (unsigned)t.hslot);
+        t.hH = t.halo_thickness(Lo);
+    }
+    t.load_coef(Lo);
+    const bool want = t.halo && t.ntl < ntile;
+    const size_t plane = (size_t)ntile * 64;
+    const size_t from = (size_t)t.ntl * 64 + t.hslot;
+    const RingSlots row_major(t.lx, t.ly), col_major(t.cx, t.cy);
+    float2 hv = make_float2(hrs.x, hrs.y), pw;
+    // images and sums of set par under a tag
+    auto images = [&](int par, unsigned tag, float2 pr, float2 ps) {
+        xword *R = E.ring + (size_t)(par * 6) * plane + (size_t)tile_id * 64;
+        const xword h = (xword)tag << 32;
+        col_major.put_shared(R, h | (unsigned)__float_as_int(pr.x));
+        col_major.put_shared(R + plane, h | (unsigned)__float_as_int(pr.y));
+        col_major.put_shared(R + 2 * plane, h | (unsigned)__float_as_int(ps.x));
+        col_major.put_shared(R + 3 * plane, h | (unsigned)__float_as_int(ps.y));
+    };
+    auto sums = [&](int par, unsigned tag) {
+        xword *R = E.ring + (size_t)(par * 6) * plane + (size_t)tile_id * 64;
+        const xword h = (xword)tag << 32;
+        row_major.put_shared(R + 4 * plane, h | (unsigned)__float_as_int(pw.x));
+        row_major.put_shared(R + 5 * plane, h | (unsigned)__float_as_int(pw.y));
+        const float2 part = t.partials(r, w, sm);
+        if (tid == 0) {
+            xword *P = E.part + (size_t)(par * ntile + tile_id) * 2;
+            xput(P, tag, (unsigned)__float_as_int(part.x));
+            xput(P + 1, tag, (unsigned)__float_as_int(part.y));
+        }
+    };
+    t.template operate<false>(
+        a.rdx, a.rdy, r, zero, hv, sm, w, pw, [&](float2 pr, float2 ps) { images(1, E.tag, pr, ps); });
+    sums(1, E.tag);
+    for (int q = 1;; ++q) {
+        const unsigned tag = E.tag + (unsigned)(q - 1);
+        const int par = q & 1;
+        // the exchange
+        double gamma, delta;
+        XWait<6> wh;
+        wh.want(want);
+        {
+            const xword *ring = E.ring + (size_t)(par * 6) * plane + from;
+            XWait<2> wp;
+            wp.want(tid < ntile);
+            for (unsigned n = 0;; ++n) {
+                wh.load(ring, plane);
+                wp.load(E.part + (size_t)(par * ntile + tid) * 2);
+                const bool ok = wh.check(tag) & wp.check(tag);
+                if (ok) break;
+                if (x_give_up(n, E.limit, E.abort)) {
+                    bad = 1;
+                    break;
+                }
+            }
+            gamma = tid < ntile ? (double)__int_as_float((int)wp.v[0]) : 0.0;
+            delta = tid < ntile ? (double)__int_as_float((int)wp.v[1]) : 0.0;
+            wg_sum2(gamma, delta, sm.red0);
+            if (bad) return;
+        }
+        const bool xupd = par == 0;
+        const double tol2 = S.it == 0 ? cgm_tol2<PRE>(a, gamma, sm) : S.tol2;
+        if (S.it >= a.maxiter || gamma <= tol2) {
+            if (xupd && S.it > 0) {
+                const float fp = (float)S.alpha;
+                x = make_float2(x.x + fp * p.x, x.y + fp * p.y);
+            }
+            elem32(Lo.pair(CGM_W), t.at) = x;
+            if (L == 0 && tid == 0) {
+                a.hflag->iters = S.it;
+                a.hflag->done = 1;
+            }
+            return;
+        }
+        double alpha, beta;
+        cgm_scalars(S, gamma, delta, alpha, beta);
+        const float fa = (float)alpha, fb = (float)beta;
+        const float z_u = PRE ? t.dz.x * r.x : r.x, z_v = PRE ? t.dz.y * r.y : r.y;
+        if (xupd) {
+            const float fxp = (float)(S.alpha + alpha * beta);
+            x = make_float2((x.x + fxp * p.x) + fa * z_u, (x.y + fxp * p.y) + fa * z_v);
+        }
+        S = cgm_next(S, gamma, alpha, tol2);
+        p = make_float2(z_u + fb * p.x, z_v + fb * p.y);
+        s = make_float2(w.x + fb * s.x, w.y + fb * s.y);
+        r = make_float2(r.x - fa * s.x, r.y - fa * s.y);
+        auto word = [&](int k) { return want ? __int_as_float((int)wh.v[k]) : 0.f; };
+        hv = make_float2(word(0) - fa * (word(4) + fb * word(2)), word(1) - fa * (word(5) + fb * word(3)));
+        t.template operate<true>(a.rdx, a.rdy, r, s, hv, sm, w, pw,
+                                       [&](float2 pr, float2 ps) { images(1 - par, tag + 1, pr, ps); });
+        sums(1 - par, tag + 1);
+    }
+}
+
+template <int LEV, bool PRE>
+__global__ void __launch_bounds__(256, 4) k_cgm_resident(CGMIterArgs a, CGMExchange E)
+{
+    cgm_resident_tile<LEV, PRE>(a, E, blockIdx.x);
 }
 
 // The same iteration of several independent CG problems (an ensemble's
@@ -3898,6 +4155,25 @@ __global__ void __launch_bounds__(256) k_cgm_iter_batch(CGMBatch B)
     const CGMIterArgs a = B.members[m];
     const int w = (int)blockIdx.x - B.first[m];
     (void)cgm_iter_tile<PAR, INIT, LEV, PRE>(a, (w & 7) * (a.nblk >> 3) + (w >> 3));
+}
+
+// The resident CGs of several problems in one launch; the workgroups of one
+// exchange nothing with those of another, so each stops by itself.
+template <int LEV, bool PRE>
+__global__ void __launch_bounds__(256, 4) k_cgm_resident_batch(CGMBatch B, const CGMExchange *ex)
+{
+    const int m = B.group_member[blockIdx.x >> 3];
+    const CGMIterArgs a = B.members[m];
+    const CGMExchange E = ex[m];
+    cgm_resident_tile<LEV, PRE>(a, E, (int)blockIdx.x - B.first[m]);
+}
+
+// ... and what stands in for those that gave up, a workgroup each.
+template <int LEV, bool PRE>
+__global__ void __launch_bounds__(256) k_cgm_solve1_batch(CGMBatch B, const CGMExchange *ex)
+{
+    const CGMIterArgs a = B.members[blockIdx.x];
+    cgm_solve1_run<LEV, PRE>(a, ex[blockIdx.x].abort);
 }
 
 // out = mask_out ? H(mask_in ? in : 0) : 0 on the u grid (comp 0) and v grid
