@@ -162,6 +162,10 @@ int wavi_set_dt(wavi_ctx *ctx, double dt);
 int wavi_field_size(const wavi_ctx *ctx, int field, size_t *n);
 int wavi_set_field(wavi_ctx *ctx, int field, const double *host, size_t n);
 int wavi_get_field(wavi_ctx *ctx, int field, double *host, size_t n);
+/* nfields fields at once, as so many calls of the above: field fields[k] from
+ * or to host[k], n[k] elements.  All are checked before the first is copied. */
+int wavi_set_fields(wavi_ctx *ctx, int nfields, const int *fields, const double *const *host, const size_t *n);
+int wavi_get_fields(wavi_ctx *ctx, int nfields, const int *fields, double *const *host, const size_t *n);
 /* quad_f2 = h/(3 eta_av) on the h mask (src/Fields/HGrid.jl:229). */
 int wavi_init_quad_f2(wavi_ctx *ctx);
 

@@ -124,6 +124,10 @@ SIGNATURES = {
     "wavi_field_size": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_int, ctypes.POINTER(ctypes.c_size_t)]),
     "wavi_set_field": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_int, _dp, ctypes.c_size_t]),
     "wavi_get_field": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_int, _dp, ctypes.c_size_t]),
+    "wavi_set_fields": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_int, ctypes.POINTER(ctypes.c_int),
+                                       ctypes.POINTER(ctypes.c_void_p), ctypes.POINTER(ctypes.c_size_t)]),
+    "wavi_get_fields": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_int, ctypes.POINTER(ctypes.c_int),
+                                       ctypes.POINTER(ctypes.c_void_p), ctypes.POINTER(ctypes.c_size_t)]),
     "wavi_init_quad_f2": (ctypes.c_int, [ctypes.c_void_p]),
     "wavi_state_save": (ctypes.c_int, [ctypes.c_void_p]),
     "wavi_state_restore": (ctypes.c_int, [ctypes.c_void_p]),

@@ -91,6 +91,9 @@ struct wavi_ctx {
     int rdv_rc = 0, rdv_iters = 0;    // that CG's return code and iteration count
     // fields (double, device); mask fields use mwu/mwv instead
     double *f[WAVI_NFIELDS] = {};
+    double *fields = nullptr;               // all of them in one allocation, with room for the mask fields as doubles
+    size_t field_at[WAVI_NFIELDS + 1] = {}; // where each begins in it (and its length)
+    std::vector<double> stage;              // host side of wavi_set_fields, wavi_get_fields on small grids
     // sigma-level constants
     double *zeta = nullptr, *qw = nullptr;
     // rheological coefficients
@@ -711,12 +714,12 @@ int wavi_ctx_create(const wavi_grid_desc *grid, const wavi_phys_params *phys, co
     CREATECHK(alloc8(&ctx->mwu, ones_u));  // UWavelets mask = trues (UWavelets.jl:38)
     CREATECHK(alloc8(&ctx->mwv, ones_v));
 
-    for (int id = 0; id < WAVI_NFIELDS; ++id) {
-        if (id == WAVI_WU_MASK || id == WAVI_WV_MASK) continue;
-        size_t n = (size_t)field_len(ctx, id);
-        CREATECHK(hipMalloc(&ctx->f[id], n * sizeof(double)));
-        CREATECHK(hipMemset(ctx->f[id], 0, n * sizeof(double)));
-    }
+    for (int id = 0; id < WAVI_NFIELDS; ++id)
+        ctx->field_at[id + 1] = ctx->field_at[id] + ((size_t)field_len(ctx, id) + 31) / 32 * 32;
+    CREATECHK(hipMalloc(&ctx->fields, ctx->field_at[WAVI_NFIELDS] * sizeof(double)));
+    CREATECHK(hipMemset(ctx->fields, 0, ctx->field_at[WAVI_NFIELDS] * sizeof(double)));
+    for (int id = 0; id < WAVI_NFIELDS; ++id)
+        if (id != WAVI_WU_MASK && id != WAVI_WV_MASK) ctx->f[id] = ctx->fields + ctx->field_at[id];
     // constructor defaults: dsdh = 1, gu/gv grounded_fraction = 1 (HGrid.jl:213, UGrid.jl:94)
     {
         std::vector<double> one(std::max(ctx->nh, std::max(ctx->nu, ctx->nv)), 1.0);
@@ -870,8 +873,7 @@ static void ctx_free(wavi_ctx *ctx)
     for (uint8_t *p : {ctx->hm, ctx->hfix, ctx->um, ctx->vm, ctx->cm, ctx->ui, ctx->vi, ctx->ufix, ctx->vfix,
                        ctx->mwu, ctx->mwv, ctx->saved_mwu, ctx->saved_mwv})
         if (p) (void)hipFree(p);
-    for (int id = 0; id < WAVI_NFIELDS; ++id)
-        if (ctx->f[id]) (void)hipFree(ctx->f[id]);
+    if (ctx->fields) (void)hipFree(ctx->fields);
     for (double *p : ctx->saved)
         if (p) (void)hipFree(p);
     for (double *p : {ctx->zeta, ctx->qw, ctx->heta_h, ctx->heta_c, ctx->dimp, ctx->Pr0, ctx->Pr1, ctx->Pd, ctx->Pb,
@@ -984,6 +986,117 @@ int wavi_get_field(wavi_ctx *ctx, int field, double *host, size_t n)
         return WAVI_OK;
     }
     HIPCHK(hipMemcpy(host, ctx->f[field], n * sizeof(double), hipMemcpyDeviceToHost));
+    return WAVI_OK;
+}
+
+// Several fields at once.  On small grids a transfer costs its latency, so the
+// fields are gathered on the host and each run of fields that follow one
+// another on the device goes in one copy (48 fields of the 80 x 10 channel:
+// 20 us each copied one by one).  Above FIELDS_STAGED bytes the copies' own
+// time prevails, and the gathering would add to it.
+constexpr size_t FIELDS_STAGED = 8u << 20;
+
+static int check_fields(wavi_ctx *ctx, int nfields, const int *fields, const double *const *host, const size_t *n)
+{
+    if (nfields < 0 || (nfields > 0 && (!fields || !host || !n))) {
+        ctx->err = "unknown field or null pointer";
+        return WAVI_EARG;
+    }
+    for (int k = 0; k < nfields; ++k) {
+        const int len = field_len(ctx, fields[k]);
+        if (len < 0 || !host[k]) {
+            ctx->err = "unknown field or null pointer";
+            return WAVI_EARG;
+        }
+        if ((size_t)len != n[k]) {
+            ctx->err = "field size mismatch: expected " + std::to_string(len) + ", got " + std::to_string(n[k]);
+            return WAVI_EDIM;
+        }
+    }
+    return WAVI_OK;
+}
+
+// Whether the fields go through the staging room, which then is there.
+static bool fields_staged(wavi_ctx *ctx)
+{
+    const size_t total = ctx->field_at[WAVI_NFIELDS];
+    if (total * sizeof(double) > FIELDS_STAGED) return false;
+    try {
+        ctx->stage.resize(total);
+    } catch (const std::bad_alloc &) {
+        return false;
+    }
+    return true;
+}
+
+// Copies the runs of fields present in `want` between the device and the
+// staging room.
+static int copy_runs(wavi_ctx *ctx, const bool *want, bool up)
+{
+    for (int a = 0; a < WAVI_NFIELDS;) {
+        if (!want[a]) {
+            ++a;
+            continue;
+        }
+        int b = a;
+        while (b < WAVI_NFIELDS && want[b]) ++b;
+        const size_t at = ctx->field_at[a], bytes = (ctx->field_at[b] - at) * sizeof(double);
+        if (up)
+            HIPCHK(hipMemcpyAsync(ctx->fields + at, ctx->stage.data() + at, bytes, hipMemcpyHostToDevice, ctx->stream));
+        else
+            HIPCHK(hipMemcpyAsync(ctx->stage.data() + at, ctx->fields + at, bytes, hipMemcpyDeviceToHost, ctx->stream));
+        a = b;
+    }
+    return WAVI_OK;
+}
+
+int wavi_set_fields(wavi_ctx *ctx, int nfields, const int *fields, const double *const *host, const size_t *n)
+{
+    if (!ctx) return WAVI_EARG;
+    CHK(check_fields(ctx, nfields, fields, host, n));
+    if (!fields_staged(ctx)) {
+        for (int k = 0; k < nfields; ++k) CHK(wavi_set_field(ctx, fields[k], host[k], n[k]));
+        return WAVI_OK;
+    }
+    std::lock_guard<std::mutex> lock(g_graph_mu);
+    HIPCHK(hipStreamSynchronize(ctx->stream));  // the staging room is free
+    bool want[WAVI_NFIELDS] = {};
+    for (int k = 0; k < nfields; ++k) {
+        want[fields[k]] = true;
+        memcpy(ctx->stage.data() + ctx->field_at[fields[k]], host[k], n[k] * sizeof(double));
+    }
+    CHK(copy_runs(ctx, want, true));
+    for (int id : {WAVI_WU_MASK, WAVI_WV_MASK})
+        if (want[id])
+            hipLaunchKernelGGL(k_mask_from_double, flat(field_len(ctx, id)), dim3(256), 0, ctx->stream,
+                               ctx->fields + ctx->field_at[id], id == WAVI_WU_MASK ? ctx->mwu : ctx->mwv,
+                               field_len(ctx, id));
+    HIPCHK(hipGetLastError());
+    HIPCHK(hipStreamSynchronize(ctx->stream));
+    return WAVI_OK;
+}
+
+int wavi_get_fields(wavi_ctx *ctx, int nfields, const int *fields, double *const *host, const size_t *n)
+{
+    if (!ctx) return WAVI_EARG;
+    CHK(check_fields(ctx, nfields, fields, host, n));
+    if (!fields_staged(ctx)) {
+        for (int k = 0; k < nfields; ++k) CHK(wavi_get_field(ctx, fields[k], host[k], n[k]));
+        return WAVI_OK;
+    }
+    std::lock_guard<std::mutex> lock(g_graph_mu);
+    bool want[WAVI_NFIELDS] = {};
+    for (int k = 0; k < nfields; ++k) want[fields[k]] = true;
+    for (int id : {WAVI_WU_MASK, WAVI_WV_MASK})
+        if (want[id])
+            hipLaunchKernelGGL(k_mask_to_double, flat(field_len(ctx, id)), dim3(256), 0, ctx->stream,
+                               id == WAVI_WU_MASK ? ctx->mwu : ctx->mwv, ctx->fields + ctx->field_at[id],
+                               field_len(ctx, id));
+    HIPCHK(hipGetLastError());
+    CHK(copy_runs(ctx, want, false));
+    HIPCHK(hipStreamSynchronize(ctx->stream));
+    for (int k = 0; k < nfields; ++k)
+        memcpy(host[k], ctx->stage.data() + ctx->field_at[fields[k]], n[k] * sizeof(double));
     return WAVI_OK;
 }
 

@@ -332,25 +332,41 @@ def update_preconditioner(model):
     return model
 
 
+_FIELD_IDS = (ctypes.c_int * len(FIELD_MAP))(*[_lib.FIELD[fid] for _, _, fid in FIELD_MAP])
+
+
+def _move_fields(model, move, arrays):
+    """One native call (wavi_set_fields, wavi_get_fields) for the arrays of all
+    fields, float64 in the memory order of the device."""
+    spec = model.parallel_spec
+    n = len(FIELD_MAP)
+    ptrs = (ctypes.c_void_p * n)(*[a.__array_interface__["data"][0] for a in arrays])
+    sizes = (ctypes.c_size_t * n)(*[a.size for a in arrays])
+    _check(spec._lib, spec.ctx, move(spec.ctx, n, _FIELD_IDS, ptrs, sizes))
+
+
 def push_fields(model):
     """Copy every field of model.fields to the device."""
-    spec = model.parallel_spec
-    lib = spec._lib
-    for cont, attr, fid in FIELD_MAP:
+    arrays = []
+    for cont, attr, _ in FIELD_MAP:
         a = model._array(cont, attr)
-        buf = np.ascontiguousarray(np.asarray(a, dtype=np.float64).ravel(order="F"))
-        _check(lib, spec.ctx, lib.wavi_set_field(spec.ctx, _lib.FIELD[fid], _lib.dptr(buf), buf.size))
+        if not (isinstance(a, np.ndarray) and a.dtype == np.float64 and a.flags.f_contiguous):
+            a = np.ascontiguousarray(np.asarray(a, dtype=np.float64).ravel(order="F"))
+        arrays.append(a)
+    _move_fields(model, model.parallel_spec._lib.wavi_set_fields, arrays)
 
 
 def pull_fields(model):
-    """Copy every field back from the device into model.fields."""
-    spec = model.parallel_spec
-    lib = spec._lib
-    for cont, attr, fid in FIELD_MAP:
-        a = model._array(cont, attr)
-        buf = np.empty(a.size, dtype=np.float64)
-        _check(lib, spec.ctx, lib.wavi_get_field(spec.ctx, _lib.FIELD[fid], _lib.dptr(buf), buf.size))
-        model._set_array(cont, attr, buf)
+    """Copy every field back from the device into model.fields, as new arrays."""
+    arrays = []
+    for cont, attr, _ in FIELD_MAP:
+        arrays.append(np.empty(model._array(cont, attr).shape, dtype=np.float64, order="F"))
+    _move_fields(model, model.parallel_spec._lib.wavi_get_fields, arrays)
+    for (cont, attr, _), a in zip(FIELD_MAP, arrays):
+        if model._array(cont, attr).dtype == np.float64:
+            setattr(model.params if cont == "params" else getattr(model.fields, cont), attr, a)
+        else:
+            model._set_array(cont, attr, a.ravel(order="F"))
 
 
 def _report_solve(model, rep, verbose):
