@@ -195,8 +195,9 @@ int wavi_update_velocities_batch(wavi_ctx **ctxs, int n, int nthreads,
  * the calling thread.  Each Picard iteration runs every member's inner
  * update and residual on the member's own stream; the members whose residual
  * asks for a V-cycle then run it up to the coarse right-hand side, and their
- * coarse CGs run together: one launch per CG iteration over the tiles of all
- * of them (k_cgm_iter_batch), until every member's CG has stopped; the rest
+ * coarse CGs run together: in one launch if their tiles fit on the chip at
+ * once (k_cgm_resident_batch), else one launch per CG iteration over the tiles
+ * of all of them (k_cgm_iter_batch), until every member's CG has stopped; the rest
  * of each V-cycle follows on the members' streams.  Every member is
  * bit-identical to its own wavi_update_velocities.  All contexts must be
  * mixed precision, on one device, with one Haar level count (else
@@ -316,8 +317,8 @@ int wavi_misfit_gradient(wavi_ctx *ctx, int n_picard, double tol_linear, int max
  * the first nonzero member code.  The small mixed-precision members (as in
  * wavi_update_velocities_batch) run on up to 32 threads of their own and
  * meet at every coarse CG: when all of them that are running wait there,
- * their CGs run as one batch (one launch per CG iteration over all their
- * tiles); every member stays bit-identical to its own call.  No reference
+ * their CGs run as one batch (one launch, or one per CG iteration, over all
+ * their tiles); every member stays bit-identical to its own call.  No reference
  * counterpart. */
 int wavi_misfit_gradient_batch(wavi_ctx **ctxs, int n, int nthreads, int n_picard, double tol_linear,
                                int maxit_linear, const double *const *u_obs, const double *const *v_obs,

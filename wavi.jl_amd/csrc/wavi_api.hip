@@ -1363,7 +1363,7 @@ static void launch_smooth_grid(wavi_ctx *ctx, const OpCoef<T> &c, const VSet<T> 
     const SmoothGridDims d(g);
     const size_t lds = d.elems() * sizeof(T);
     const T om = (T)ctx->S.smoother_omega;
-    if (d.points() <= SMG_THREADS)
+    if (d.inner() <= SMG_THREADS && d.cells() <= SMG_THREADS)
         hipLaunchKernelGGL((k_smooth_grid<T, 1>), dim3(1), dim3(SMG_THREADS), lds, ctx->stream, g, c, xu, xv, yu, yv,
                            w.r.u, w.r.v, w.d.u, w.d.v, om, packed, nsmooth);
     else
