@@ -59,16 +59,6 @@ def sizes(nx, ny):
     return (nx + 1) * ny, nx * (ny + 1), nx * ny, (nx - 1) * (ny - 1)
 
 
-def cg_apply_bytes(nx, ny, w=8):
-    """Algorithmic HBM bytes of one k_cg_apply launch (FP64 coarse CG, A then
-    R on a tile): t_u, t_v in; c_u, c_v out; u_u, u_v in for dot(u, c);
-    beta_eff on u, v; thickness on u, v; h*eta_av on h; dimp on h; h*eta_av
-    on c (w bytes each); masks (one byte each): inner u, v; wavelet u, v;
-    u, v masks; h and c masks."""
-    nu, nv, nh, nc = sizes(nx, ny)
-    return w * (5 * (nu + nv) + 2 * nh + nc) + 3 * (nu + nv) + nh + nc
-
-
 def cgm_iter_bytes(nx, ny, w=4):
     """Algorithmic HBM bytes of one k_cgm_iter launch (one whole iteration of
     the mixed-precision coarse CG), averaged over the two alternating
@@ -83,15 +73,16 @@ def cgm_iter_bytes(nx, ny, w=4):
 
 
 def cg_iteration_fp64_bytes(nx, ny, w=8):
-    """Algorithmic HBM bytes of one FP64 coarse-CG iteration (k_cg_dir +
-    k_cg_apply + k_cg_update).  k_cg_dir: r, u in, u, t out, wavelet and
-    inner masks; k_cg_apply as above; k_cg_update: x, u, r, c in, x, r out."""
+    """Algorithmic HBM bytes of one FP64 coarse-CG iteration (k_cg_step +
+    k_cg_update).  k_cg_step: r, u, x in, u, x, c out, thickness and beta_eff
+    on u and v; h*eta_av and dimp on h; h*eta_av on c; one byte of mask bits
+    per pair of a u and a v point; k_cg_update: r, c in, r out."""
     nu, nv, nh, nc = sizes(nx, ny)
-    return 4 * w * (nu + nv) + 2 * (nu + nv) + cg_apply_bytes(nx, ny, w) + 6 * w * (nu + nv)
+    return w * (11 * (nu + nv) + 2 * nh + nc) + (nu + nv) // 2
 
 
 DOMINANT = {  # precision -> (what is timed, timing id, profile name, bytes per launch)
-    "fp64": ("FP64 CG iteration (k_cg_dir + k_cg_apply + k_cg_update)", "cg_iter_fp64", "cg_iteration",
+    "fp64": ("FP64 CG iteration (k_cg_step + k_cg_update)", "cg_iter_fp64", "cg_iteration",
              lambda nx, ny: cg_iteration_fp64_bytes(nx, ny, 8)),
     "mixed": ("k_cgm_iter", "cg_iter_mixed", "k_cgm_iter", lambda nx, ny: cgm_iter_bytes(nx, ny, 4)),
 }

@@ -1155,7 +1155,7 @@ using TilePair = T[2][TILE][TILE + 1];
 // code of a wavefront is straight and the operands of a row are read from
 // LDS once, all before the first is used.  The rows as bit masks walked term
 // by term (one row per thread, 16 dependent LDS reads in the longest)
-// cost k_cg_apply 9,200 of its 16,600 cycles on a lone tile.
+// cost the operator's launch 9,200 of its 16,600 cycles on a lone tile.
 // Points past the grid's end must hold zero.  Ends with a barrier.
 template <bool R, int LEV, typename T>
 __device__ __forceinline__ void haar_pair_lev(TilePair<T> &t, TilePair<T> &m)
