@@ -2253,6 +2253,12 @@ struct CGLayout {
     {
         return (unsigned)(i + TILE) + __umul24(px, (unsigned)(j + TILE));
     }
+    // (dx, dy) from index k, dy >= -TILE: the product of what is not negative
+    // (a signed 24-bit one would end at a pitch of 2^23, half of the largest)
+    __device__ __forceinline__ unsigned from(unsigned k, int dx, int dy) const
+    {
+        return (k - (unsigned)TILE * px) + (unsigned)dx + __umul24(px, (unsigned)(dy + TILE));
+    }
     __device__ __forceinline__ double2 *pair(int a) const { return F + (size_t)a * ns; }
     __device__ __forceinline__ double *corner() const { return reinterpret_cast<double *>(F + (size_t)CG_NPAIR * ns); }
 };
@@ -2537,7 +2543,7 @@ struct CgTile {
             di = rows ? q : c;
             dj = rows ? c : q;
         }
-        h0 = at0 + (unsigned)(di + (int)__mul24((int)Lo.px, dj));
+        h0 = Lo.from(at0, di, dj);
         const int e = l - 16;  // corner entry of lanes 16..40 of wavefronts 0 (v) and 1 (u)
         cx = e % 5;
         cy = e / 5;
@@ -2547,7 +2553,7 @@ struct CgTile {
             di = corner ? haar_halo_offset<LEV>(after, cx) : (rows ? q : c);
             dj = corner ? haar_halo_offset<LEV>(!after, cy) : (rows ? c : q);
         }
-        h1 = at0 + (unsigned)(di + (int)__mul24((int)Lo.px, dj));
+        h1 = Lo.from(at0, di, dj);
     }
     // the coefficients, in the order of their first use
     __device__ __forceinline__ void load_coef(const CGLayout &Lo)
@@ -2565,7 +2571,7 @@ struct CgTile {
         hmb = 0;
         if (w >= 1) {
             const int hx = h.hu ? h.ux : h.vx, hy = h.hu ? h.uy : h.vy;
-            const unsigned ha = at0 + (unsigned)(hx - 1 + (int)__mul24((int)Lo.px, hy - 1));
+            const unsigned ha = Lo.from(at0, hx - 1, hy - 1);
             cr.hhu = cr.hhv = elem32(reinterpret_cast<const double *>(Lo.pair(CG_H)), 2 * ha + (h.hu ? 0 : 1));
             hmb = elem32(Lo.M, ha);
         }
@@ -2573,7 +2579,7 @@ struct CgTile {
         o.hetac = elem32(Lo.corner(), at);
         op_extra_cell(l, cr);
         if (w == 0) {
-            const unsigned ea = at0 + (unsigned)(cr.ex - 1 + (int)__mul24((int)Lo.px, cr.ey - 1));
+            const unsigned ea = Lo.from(at0, cr.ex - 1, cr.ey - 1);
             const double2 ce = elem32(Lo.pair(CG_CELL), ea);
             cr.ec = elem32(Lo.corner(), ea);
             cr.eh = ce.x;
@@ -3367,6 +3373,11 @@ struct CGMLayout {
     {
         return (unsigned)(i + TILE) + __umul24(px, (unsigned)(j + 1));
     }
+    // (dx, dy) from index k, dy >= -1 (as CGLayout::from)
+    __device__ __forceinline__ unsigned from(unsigned k, int dx, int dy) const
+    {
+        return (k - px) + (unsigned)dx + __umul24(px, (unsigned)(dy + 1));
+    }
     __device__ __forceinline__ float2 *pair(int a) const { return F + (size_t)a * ns; }
     __device__ __forceinline__ float *corner() const { return reinterpret_cast<float *>(F + (size_t)CGM_NPAIR * ns); }
 };
@@ -3645,7 +3656,7 @@ struct CgmTile {
     }
     __device__ __forceinline__ float2 halo_thickness(const CGMLayout &Lo) const
     {
-        return load(Lo, CGM_H, at0 + (unsigned)(hx - 1 + (int)__mul24((int)Lo.px, hy - 1)));
+        return load(Lo, CGM_H, Lo.from(at0, hx - 1, hy - 1));
     }
     __device__ __forceinline__ void load_coef(const CGMLayout &Lo)
     {
@@ -3658,7 +3669,7 @@ struct CgmTile {
         float2 c = make_float2(0.f, 0.f);
         float h = 0.f;
         if (w == 0) {
-            const unsigned ea = at0 + (unsigned)(ex - 1 + (int)__mul24((int)Lo.px, ey - 1));
+            const unsigned ea = Lo.from(at0, ex - 1, ey - 1);
             c = load(Lo, CGM_CELL, ea);
             h = elem32((const float *)Lo.corner(), ea);
         }
