@@ -1334,8 +1334,9 @@ __device__ __forceinline__ T optile_v(const OpCoef<T> &c, const S &s, const Poin
 // wavefront instead of 42 with the window walked by 256 threads and every
 // cell loading its four thicknesses and six masks.  The fluxes h u and h v
 // of the implicit term are formed once per point, masked, and staged.
-// heta_h, dimp and heta_c are zero off the h and c masks, so those masks are
-// not read.  The arithmetic is that of op_u / op_v.
+// The arithmetic and the masks are those of op_u / op_v: what lies off a mask
+// is selected away, not multiplied by a zero coefficient, so that a value that
+// is not finite there (missing data outside the ice) reaches no output.
 
 // Mask bits of a u or v point: 1 inner, 2 u / v mask, 4 wavelet mask.
 enum { MB_INNER = 1, MB_POINT = 2, MB_WAVELET = 4 };
@@ -1416,29 +1417,37 @@ struct OpOwn {
     T heta, dimp, hetac;
     OpCell<T> cell;   // the intermediates of its cell
     unsigned mu, mv;  // mask bits
+    unsigned mc;      // ... of its cell (CELL_*)
     bool oku, okv;
     int ku, kv;
 };
 
-// h cell (a, b) and its corner: 0 outside their grids
+// Mask bits of a cell: 1 on the grid, 2 h mask, 4 its corner on the c mask.
+enum { CELL_GRID = 1, CELL_H = 2, CELL_CORNER = 4 };
+
+// h cell (a, b) and its corner: 0 outside their grids.  Returns the mask bits.
 template <typename T>
-__device__ __forceinline__ void op_cell_load(const GridDims &g, const OpCoef<T> &c, int a, int b, T &heta, T &dimp,
-                                             T &hetac)
+__device__ __forceinline__ unsigned op_cell_load(const GridDims &g, const OpCoef<T> &c, int a, int b, T &heta, T &dimp,
+                                                 T &hetac)
 {
     const bool cell = a >= 0 && a < g.nx && b >= 0 && b < g.ny;
     const bool corner = a >= 0 && a < g.nx - 1 && b >= 0 && b < g.ny - 1;
     heta = ld_or(cell, c.heta_h, a + g.nx * b, T(0));
     dimp = ld_or(cell, c.dimp, a + g.nx * b, T(0));
     hetac = ld_or(corner, c.heta_c, a + (g.nx - 1) * b, T(0));
+    const uint8_t hm = ld_or(cell, c.hm, a + g.nx * b, (uint8_t)0);
+    const uint8_t cm = ld_or(corner, c.cm, a + (g.nx - 1) * b, (uint8_t)0);
+    return (cell ? CELL_GRID : 0u) | (hm ? CELL_H : 0u) | (cm ? CELL_CORNER : 0u);
 }
 
 // Intermediates of cell (x, y) (the expressions of op_rxx, op_ryy, op_extra,
 // op_rxy).  Cell (0, 0) reads one absent window point of each kind and corner
 // (16, 16) another; no output reads what they feed.
-// u, v, qx, qy: the window at (x, y)
-template <typename T>
+// u, v, qx, qy: the window at (x, y).  MASKED: by the cell's mask bits mc;
+// else its coefficients are zero off the masks and the window is finite there.
+template <bool MASKED, typename T>
 __device__ __forceinline__ OpCell<T> op_cell(T rdx, T rdy, const OpLds<T> &s, int x, int y, T u, T v, T qx, T qy,
-                                             T heta, T dimp, T hetac)
+                                             T heta, T dimp, T hetac, unsigned mc)
 {
     const T u1 = s.w.U[y][x + 1], v1 = s.w.V[y + 1][x];
     const T dudx = rdx * u1 - rdx * u;
@@ -1446,7 +1455,14 @@ __device__ __forceinline__ OpCell<T> op_cell(T rdx, T rdy, const OpLds<T> &s, in
     const T divq = (rdx * s.w.QX[y][x + 1] - rdx * qx) + (rdy * s.w.QY[y + 1][x] - rdy * qy);
     const T dudy = rdy * s.w.U[y + 1][x + 1] - rdy * u1;
     const T dvdx = rdx * s.w.V[y + 1][x + 1] - rdx * v1;
-    return {T(2) * (heta * (T(2) * dudx + dvdy)), T(2) * (heta * (T(2) * dvdy + dudx)), dimp * divq, hetac * (dudy + dvdx)};
+    OpCell<T> r{T(2) * (heta * (T(2) * dudx + dvdy)), T(2) * (heta * (T(2) * dvdy + dudx)), dimp * divq, hetac * (dudy + dvdx)};
+    if constexpr (MASKED) {
+        r.rxx = (mc & CELL_H) ? r.rxx : T(0);
+        r.ryy = (mc & CELL_H) ? r.ryy : T(0);
+        r.ext = (mc & CELL_GRID) ? r.ext : T(0);
+        r.rxy = (mc & CELL_CORNER) ? r.rxy : T(0);
+    }
+    return r;
 }
 
 // Halo points a thread stages: u at (ux, uy) and v at (vx, vy) of the window.
@@ -1481,7 +1497,9 @@ __device__ __forceinline__ HaloPos op_halo_sides(int w, int l)
 template <typename T>
 struct OpCoefRegs {
     T hhu, hhv;
+    bool hmu, hmv;    // the halo points are on the u, v mask
     T eh, ed, ec;
+    unsigned em;      // the cell's mask bits
     int ex, ey;
 };
 
@@ -1492,6 +1510,7 @@ __device__ __forceinline__ void op_extra_cell(int l, OpCoefRegs<T> &r)
     r.ex = l < 17 ? 0 : (l < 33 ? l - 16 : 16);
     r.ey = l < 17 ? l : 0;
     r.eh = r.ed = r.ec = T(0);
+    r.em = 0;
 }
 
 template <typename T, class M>
@@ -1502,17 +1521,20 @@ __device__ __forceinline__ void op_coef_load(const GridDims &g, const OpCoef<T> 
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const T ohu = ld_or(o.oku, c.hu, o.ku, T(0)), ohv = ld_or(o.okv, c.hv, o.kv, T(0));
     r.hhu = r.hhv = T(0);
+    r.hmu = r.hmv = false;
     if (halo_wave) {
         const int iu = i0 - 1 + h.ux, ju = j0 - 1 + h.uy, iv = i0 - 1 + h.vx, jv = j0 - 1 + h.vy;
         const bool oku = h.hu && iu >= 0 && iu < g.nxu && ju >= 0 && ju < g.nyu;
         const bool okv = h.hv && iv >= 0 && iv < g.nxv && jv >= 0 && jv < g.nyv;
         const T u = ld_or(oku, c.hu, iu + g.nxu * ju, T(0)), v = ld_or(okv, c.hv, iv + g.nxv * jv, T(0));
-        r.hhu = (mask.u(oku, iu + g.nxu * ju) & MB_POINT) ? u : T(0);
-        r.hhv = (mask.v(okv, iv + g.nxv * jv) & MB_POINT) ? v : T(0);
+        r.hmu = mask.u(oku, iu + g.nxu * ju) & MB_POINT;
+        r.hmv = mask.v(okv, iv + g.nxv * jv) & MB_POINT;
+        r.hhu = r.hmu ? u : T(0);
+        r.hhv = r.hmv ? v : T(0);
     }
-    op_cell_load(g, c, i0 + lx, j0 + ly, o.heta, o.dimp, o.hetac);
+    o.mc = op_cell_load(g, c, i0 + lx, j0 + ly, o.heta, o.dimp, o.hetac);
     op_extra_cell(l, r);
-    if (w == 0) op_cell_load(g, c, i0 - 1 + r.ex, j0 - 1 + r.ey, r.eh, r.ed, r.ec);
+    if (w == 0) r.em = op_cell_load(g, c, i0 - 1 + r.ex, j0 - 1 + r.ey, r.eh, r.ed, r.ec);
     const T obu = ld_or(o.oku, c.bu, o.ku, T(0)), obv = ld_or(o.okv, c.bv, o.kv, T(0));
     o.hu = (o.mu & MB_POINT) ? ohu : T(0);
     o.hv = (o.mv & MB_POINT) ? ohv : T(0);
@@ -1522,31 +1544,35 @@ __device__ __forceinline__ void op_coef_load(const GridDims &g, const OpCoef<T> 
 
 // Stage the window (the thread's own point and its halo points hu, hv) and
 // compute the cells' intermediates.  Ends with a barrier, after which the
-// window is free.
-template <typename T>
+// window is free.  MASKED: o and r hold the mask bits (op_coef_load).
+template <bool MASKED, typename T>
 __device__ __forceinline__ void op_cells(T rdx, T rdy, const HaloPos &h, T hu, T hv, OpOwn<T> &o,
                                          const OpCoefRegs<T> &r, OpLds<T> &s)
 {
     const int lx = threadIdx.x & 15, ly = threadIdx.x >> 4;
     s.w.U[ly + 1][lx + 1] = o.u;
     s.w.V[ly + 1][lx + 1] = o.v;
-    const T qx = o.hu * o.u, qy = o.hv * o.v;
+    T qx = o.hu * o.u, qy = o.hv * o.v;
+    if constexpr (MASKED) {
+        qx = (o.mu & MB_POINT) ? qx : T(0);
+        qy = (o.mv & MB_POINT) ? qy : T(0);
+    }
     s.w.QX[ly + 1][lx + 1] = qx;
     s.w.QY[ly + 1][lx + 1] = qy;
     if (h.hu) {
         s.w.U[h.uy][h.ux] = hu;
-        s.w.QX[h.uy][h.ux] = r.hhu * hu;
+        s.w.QX[h.uy][h.ux] = !MASKED || r.hmu ? r.hhu * hu : T(0);
     }
     if (h.hv) {
         s.w.V[h.vy][h.vx] = hv;
-        s.w.QY[h.vy][h.vx] = r.hhv * hv;
+        s.w.QY[h.vy][h.vx] = !MASKED || r.hmv ? r.hhv * hv : T(0);
     }
     __syncthreads();
-    o.cell = op_cell(rdx, rdy, s, lx + 1, ly + 1, o.u, o.v, qx, qy, o.heta, o.dimp, o.hetac);
+    o.cell = op_cell<MASKED>(rdx, rdy, s, lx + 1, ly + 1, o.u, o.v, qx, qy, o.heta, o.dimp, o.hetac, o.mc);
     if (__builtin_amdgcn_readfirstlane(threadIdx.x) == 0) {
         // lanes past the 33 cells before the tile repeat the last
-        const OpCell<T> first = op_cell(rdx, rdy, s, r.ex, r.ey, s.w.U[r.ey][r.ex], s.w.V[r.ey][r.ex],
-                                        s.w.QX[r.ey][r.ex], s.w.QY[r.ey][r.ex], r.eh, r.ed, r.ec);
+        const OpCell<T> first = op_cell<MASKED>(rdx, rdy, s, r.ex, r.ey, s.w.U[r.ey][r.ex], s.w.V[r.ey][r.ex],
+                                                s.w.QX[r.ey][r.ex], s.w.QY[r.ey][r.ex], r.eh, r.ed, r.ec, r.em);
         first.store(s, r.ex, r.ey);
     }
     o.cell.store(s, lx + 1, ly + 1);
@@ -1582,7 +1608,7 @@ __device__ __forceinline__ void op_tile(const GridDims &g, const OpCoef<T> &c, c
     }
     OpCoefRegs<T> r;
     op_coef_load(g, c, mask, i0, j0, h, w >= 2, o, r);
-    op_cells(c.rdx, c.rdy, h, hu, hv, o, r, s);
+    op_cells<true>(c.rdx, c.rdy, h, hu, hv, o, r, s);
 }
 
 // A x at the thread's u point and v point (inner or not)
@@ -2681,7 +2707,7 @@ struct CgTile {
         __syncthreads();
         o.u = (mb & CB_INNER_U) ? s.p.t[0][ly][lx] : 0.0;
         o.v = (mb & CB_INNER_V) ? s.p.t[1][ly][lx] : 0.0;
-        op_cells(rdx, rdy, h, hu, hv, o, cr, s);
+        op_cells<false>(rdx, rdy, h, hu, hv, o, cr, s);
         s.h.t[0][ly][lx] = (mb & CB_INNER_U) ? op_out_u(rdx, rdy, s, o) : 0.0;
         s.h.t[1][ly][lx] = (mb & CB_INNER_V) ? op_out_v(rdx, rdy, s, o) : 0.0;
         __syncthreads();
