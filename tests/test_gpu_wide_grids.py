@@ -1,5 +1,6 @@
-"""Row pitches of 2^23 points and more, the widest the coarse CG's arenas take:
-a V-cycle is compared with that of a narrow grid of the same columns."""
+"""Row pitches of 2^23 points and more, and arrays of 4 GiB and more in the FP64
+coarse CG's arena: a V-cycle is compared with that of a narrow grid of the same
+columns."""
 import numpy as np
 import pytest
 
@@ -34,9 +35,9 @@ def _vcycle(W, nx, first, precision):
 
 
 # the tiles' sums are the same; only their sum over the tiles, in FP64, is in
-# another order, which can move the FP32 step length by a rounding
+# another order, which can move the step length by roundings
 @pytest.mark.gpu
-@pytest.mark.parametrize("precision,tol", [("mixed", 1e-5)])
+@pytest.mark.parametrize("precision,tol", [("fp64", 1e-10), ("mixed", 1e-5)])
 def test_widest_pitch_equals_a_narrow_grid(W, precision, tol):
     nx = 1 << 23
     print("[gpu] V-cycle on %d x 2, %s" % (nx, precision), flush=True)

@@ -106,6 +106,7 @@ struct wavi_ctx {
     double2 *arena64 = nullptr;
     uint8_t *marena64 = nullptr;
     unsigned px64 = 0, ns64 = 0;
+    bool big64 = false;             // its arrays are too large for 32-bit byte offsets
     // the CG in one launch (k_cg_resident): its exchange words (null: the grid
     // does not fit on the chip), the next tag, and what it holds of the chip
     // until the host has seen its end
@@ -799,10 +800,8 @@ int wavi_ctx_create(const wavi_grid_desc *grid, const wavi_phys_params *phys, co
     }
     if (precision_mode == WAVI_PRECISION_FP64) {
         const size_t px = (size_t)TILE * (g.nbx + 1), ns = px * TILE * (g.nby + 2);
-        if (ns * sizeof(double2) > UINT32_MAX) {
-            ctx->err = "grid too large for the coarse solver's 32-bit offsets";
-            return fail(WAVI_EARG);
-        }
+        // the grids accepted above have fewer than 2^30 points here
+        ctx->big64 = ns * sizeof(double2) > UINT32_MAX;
         ctx->px64 = (unsigned)px;
         ctx->ns64 = (unsigned)ns;
         // the exchange words of a resident CG, if any, follow the arena, on a line of their own
@@ -1581,44 +1580,61 @@ static void launch_tile_haar(wavi_ctx *ctx, int dir, const T *inu, const T *inv,
 }
 
 // The kernels of the FP64 coarse CG at the context's Haar level,
-// Jacobi-preconditioned inside a linear solve (ctx->cg_pre).
-template <bool PRE, int FOLD>
+// Jacobi-preconditioned inside a linear solve (ctx->cg_pre), for arenas whose
+// arrays a 32-bit offset spans or not (ctx->big64).
+template <bool PRE, int FOLD, bool BIG>
 static void launch_cg_step_p(wavi_ctx *ctx, dim3 tb, const CGArgs &a, int par)
 {
     switch (ctx->S.levels) {
-    case 0: hipLaunchKernelGGL((k_cg_step<PRE, 0, FOLD>), tb, dim3(256), 0, ctx->stream, a, par); break;
-    case 1: hipLaunchKernelGGL((k_cg_step<PRE, 1, FOLD>), tb, dim3(256), 0, ctx->stream, a, par); break;
-    case 2: hipLaunchKernelGGL((k_cg_step<PRE, 2, FOLD>), tb, dim3(256), 0, ctx->stream, a, par); break;
-    default: hipLaunchKernelGGL((k_cg_step<PRE, 3, FOLD>), tb, dim3(256), 0, ctx->stream, a, par); break;
+    case 0: hipLaunchKernelGGL((k_cg_step<PRE, 0, FOLD, BIG>), tb, dim3(256), 0, ctx->stream, a, par); break;
+    case 1: hipLaunchKernelGGL((k_cg_step<PRE, 1, FOLD, BIG>), tb, dim3(256), 0, ctx->stream, a, par); break;
+    case 2: hipLaunchKernelGGL((k_cg_step<PRE, 2, FOLD, BIG>), tb, dim3(256), 0, ctx->stream, a, par); break;
+    default: hipLaunchKernelGGL((k_cg_step<PRE, 3, FOLD, BIG>), tb, dim3(256), 0, ctx->stream, a, par); break;
     }
 }
 
 template <bool PRE>
 static void launch_cg_step(wavi_ctx *ctx, dim3 tb, const CGArgs &a, int par)
 {
-    if (ctx->g.npart <= 256)
-        launch_cg_step_p<PRE, 1>(ctx, tb, a, par);
+    if (ctx->big64)
+        launch_cg_step_p<PRE, CG_FOLD_LARGE, true>(ctx, tb, a, par);
+    else if (ctx->g.npart <= 256)
+        launch_cg_step_p<PRE, 1, false>(ctx, tb, a, par);
     else
-        launch_cg_step_p<PRE, CG_FOLD_LARGE>(ctx, tb, a, par);
+        launch_cg_step_p<PRE, CG_FOLD_LARGE, false>(ctx, tb, a, par);
 }
 
 template <bool PRE, bool EARLY>
 static void launch_cg_update(wavi_ctx *ctx, dim3 tb, const CGArgs &a, int par)
 {
-    if (ctx->g.npart <= 256)
-        hipLaunchKernelGGL((k_cg_update<PRE, EARLY, 1>), tb, dim3(256), 0, ctx->stream, a, par);
+    if (ctx->big64)
+        hipLaunchKernelGGL((k_cg_update<PRE, EARLY, CG_FOLD_LARGE, true>), tb, dim3(256), 0, ctx->stream, a, par);
+    else if (ctx->g.npart <= 256)
+        hipLaunchKernelGGL((k_cg_update<PRE, EARLY, 1, false>), tb, dim3(256), 0, ctx->stream, a, par);
     else
-        hipLaunchKernelGGL((k_cg_update<PRE, EARLY, CG_FOLD_LARGE>), tb, dim3(256), 0, ctx->stream, a, par);
+        hipLaunchKernelGGL((k_cg_update<PRE, EARLY, CG_FOLD_LARGE, false>), tb, dim3(256), 0, ctx->stream, a, par);
 }
 
-template <bool PRE>
-static void launch_cg_solve1_p(wavi_ctx *ctx, const CGArgs &a, const int *only_if = nullptr)
+template <bool PRE, bool BIG>
+static void launch_cg_solve1_p(wavi_ctx *ctx, const CGArgs &a, const int *only_if)
 {
+    const dim3 one(1), wg(256);
     switch (ctx->S.levels) {
-    case 0: hipLaunchKernelGGL((k_cg_solve1<PRE, 0>), dim3(1), dim3(256), 0, ctx->stream, a, only_if); break;
-    case 1: hipLaunchKernelGGL((k_cg_solve1<PRE, 1>), dim3(1), dim3(256), 0, ctx->stream, a, only_if); break;
-    case 2: hipLaunchKernelGGL((k_cg_solve1<PRE, 2>), dim3(1), dim3(256), 0, ctx->stream, a, only_if); break;
-    default: hipLaunchKernelGGL((k_cg_solve1<PRE, 3>), dim3(1), dim3(256), 0, ctx->stream, a, only_if); break;
+    case 0: hipLaunchKernelGGL((k_cg_solve1<PRE, 0, BIG>), one, wg, 0, ctx->stream, a, only_if); break;
+    case 1: hipLaunchKernelGGL((k_cg_solve1<PRE, 1, BIG>), one, wg, 0, ctx->stream, a, only_if); break;
+    case 2: hipLaunchKernelGGL((k_cg_solve1<PRE, 2, BIG>), one, wg, 0, ctx->stream, a, only_if); break;
+    default: hipLaunchKernelGGL((k_cg_solve1<PRE, 3, BIG>), one, wg, 0, ctx->stream, a, only_if); break;
+    }
+}
+
+// The whole FP64 CG in one workgroup (only_if: if it is set).
+static void launch_cg_solve1(wavi_ctx *ctx, const CGArgs &a, const int *only_if = nullptr)
+{
+    switch ((ctx->cg_pre ? 2 : 0) + (ctx->big64 ? 1 : 0)) {
+    case 0: launch_cg_solve1_p<false, false>(ctx, a, only_if); break;
+    case 1: launch_cg_solve1_p<false, true>(ctx, a, only_if); break;
+    case 2: launch_cg_solve1_p<true, false>(ctx, a, only_if); break;
+    default: launch_cg_solve1_p<true, true>(ctx, a, only_if); break;
     }
 }
 
@@ -1684,10 +1700,7 @@ static bool cg_try_resident(wavi_ctx *ctx, const CGArgs &a)
     const int bev = burst_begin(ctx);
     hipLaunchKernelGGL(ctx->x_fn[ctx->cg_pre], dim3(ctx->x_blocks), dim3(256), 0, ctx->stream, a, E);
     burst_end(ctx, bev, 0, 0);
-    if (ctx->cg_pre)
-        launch_cg_solve1_p<true>(ctx, a, &ctx->st->abort);
-    else
-        launch_cg_solve1_p<false>(ctx, a, &ctx->st->abort);
+    launch_cg_solve1(ctx, a, &ctx->st->abort);
     ctx->x_ran = ctx->x_pending = true;
     return true;
 }
@@ -1714,10 +1727,12 @@ int do_coarse_cg<double>(wavi_ctx *ctx, const VSet<double> &w, int *iters)
     // launches queued past the stop are many.  Long CGs have
     // about one, and their launches do without the flag's round trip.
     const bool early = ctx->cg_prev < CG_CHUNK;
-    if (pre)
-        hipLaunchKernelGGL(k_cg_setup<true>, tb, dim3(256), 0, ctx->stream, a, io);
-    else
-        hipLaunchKernelGGL(k_cg_setup<false>, tb, dim3(256), 0, ctx->stream, a, io);
+    switch ((pre ? 2 : 0) + (ctx->big64 ? 1 : 0)) {
+    case 0: hipLaunchKernelGGL((k_cg_setup<false, false>), tb, dim3(256), 0, ctx->stream, a, io); break;
+    case 1: hipLaunchKernelGGL((k_cg_setup<false, true>), tb, dim3(256), 0, ctx->stream, a, io); break;
+    case 2: hipLaunchKernelGGL((k_cg_setup<true, false>), tb, dim3(256), 0, ctx->stream, a, io); break;
+    default: hipLaunchKernelGGL((k_cg_setup<true, true>), tb, dim3(256), 0, ctx->stream, a, io); break;
+    }
     HIPCHK(hipGetLastError());
     *iters = 0;
     if (cg_try_resident(ctx, a)) {
@@ -1726,10 +1741,7 @@ int do_coarse_cg<double>(wavi_ctx *ctx, const VSet<double> &w, int *iters)
     }
     volatile CGMHostFlag *hf = ctx->h_flag;
     if (cg_one_workgroup(ctx)) {
-        if (pre)
-            launch_cg_solve1_p<true>(ctx, a);
-        else
-            launch_cg_solve1_p<false>(ctx, a);
+        launch_cg_solve1(ctx, a);
         HIPCHK(hipGetLastError());
         HIPCHK(hipStreamSynchronize(ctx->stream));
         if (!hf->done) {
@@ -2080,9 +2092,12 @@ static int vcycle_post(wavi_ctx *ctx, const VSet<T> &w)
     const GridDims &g = ctx->g;
     dim3 tg(g.nbx, g.nby);
     // e += P x_c
-    if constexpr (std::is_same<T, double>::value)
-        hipLaunchKernelGGL(k_cg_finish, dim3(ctx->nblk), dim3(256), 0, ctx->stream, cg_args(ctx), cg_io(ctx, w));
-    else
+    if constexpr (std::is_same<T, double>::value) {
+        if (ctx->big64)
+            hipLaunchKernelGGL(k_cg_finish<true>, dim3(ctx->nblk), dim3(256), 0, ctx->stream, cg_args(ctx), cg_io(ctx, w));
+        else
+            hipLaunchKernelGGL(k_cg_finish<false>, dim3(ctx->nblk), dim3(256), 0, ctx->stream, cg_args(ctx), cg_io(ctx, w));
+    } else
         hipLaunchKernelGGL(k_cgm_finish, dim3(ctx->nblk), dim3(256), 0, ctx->stream, cgm_args(ctx, w));
     CHK(do_smoother(ctx, w, rev));
     HIPCHK(hipGetLastError());

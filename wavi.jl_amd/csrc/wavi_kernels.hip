@@ -2289,13 +2289,21 @@ struct CGLayout {
     __device__ __forceinline__ double *corner() const { return reinterpret_cast<double *>(F + (size_t)CG_NPAIR * ns); }
 };
 
-// Element k of an array below 4 GiB, addressed by a 32-bit byte offset from
-// its uniform base (the scalar-base form of the global loads and stores).
+// Element k of an array, addressed by a 32-bit byte offset from its uniform
+// base (the scalar-base form of the global loads and stores).  BIG: of an
+// array of 4 GiB and more, by a 64-bit address of each lane's own.
+template <bool BIG, typename V>
+__device__ __forceinline__ V &elem(V *p, unsigned k)
+{
+    if constexpr (BIG) return p[k];
+    typedef typename std::conditional<std::is_const<V>::value, const char, char>::type C;
+    return *reinterpret_cast<V *>(reinterpret_cast<C *>(p) + (size_t)(unsigned)(k * (unsigned)sizeof(V)));
+}
+
 template <typename V>
 __device__ __forceinline__ V &elem32(V *p, unsigned k)
 {
-    typedef typename std::conditional<std::is_const<V>::value, const char, char>::type C;
-    return *reinterpret_cast<V *>(reinterpret_cast<C *>(p) + (size_t)(unsigned)(k * (unsigned)sizeof(V)));
+    return elem<false>(p, k);
 }
 
 struct CGArgs {
@@ -2347,7 +2355,7 @@ __device__ __forceinline__ int band_tile(const GridDims &g, int L, int &bx, int 
 // setup (t = P x0 computed beforehand): r = b - R A t, x = x0, u = 0, the
 // coefficients and mask bits into the arena, partials of ||r0||^2 and ||b||^2
 // (PRE: also of (r0, D^-1 r0)); resets the scalars.
-template <bool PRE>
+template <bool PRE, bool BIG>
 __global__ void __launch_bounds__(256) k_cg_setup(CGArgs a, CGIo io)
 {
     __shared__ OpLds<double> s;
@@ -2383,15 +2391,15 @@ __global__ void __launch_bounds__(256) k_cg_setup(CGArgs a, CGIo io)
     op_restrict_tile(g, c, MaskSep<true>{c.ui, c.um, c.vi, c.vm, io.mwu, io.mwv}, io.levels, io.tu, io.tv, i0, j0, s, o);
     const double ru = (o.mu & MB_WAVELET) ? bu - s.h.t[0][ly][lx] : bu, rv = (o.mv & MB_WAVELET) ? bv - s.h.t[1][ly][lx] : bv;
     const unsigned at = a.Lo.at(i0 + lx, j0 + ly);
-    elem32(a.Lo.pair(CG_R), at) = make_double2(ru, rv);
-    elem32(a.Lo.pair(CG_P), at) = make_double2(0.0, 0.0);
-    elem32(a.Lo.pair(CG_X), at) = make_double2(xu, xv);
-    elem32(a.Lo.pair(CG_H), at) = make_double2(o.hu, o.hv);
-    elem32(a.Lo.pair(CG_B), at) = make_double2(o.bu, o.bv);
-    elem32(a.Lo.pair(CG_CELL), at) = make_double2(o.heta, o.dimp);
-    if constexpr (PRE) elem32(a.Lo.pair(CG_DINV), at) = make_double2(zu, zv);
-    elem32(a.Lo.corner(), at) = o.hetac;
-    elem32(a.Lo.M, at) = (uint8_t)(((o.mu & MB_INNER) ? CB_INNER_U : 0) | ((o.mv & MB_INNER) ? CB_INNER_V : 0) |
+    elem<BIG>(a.Lo.pair(CG_R), at) = make_double2(ru, rv);
+    elem<BIG>(a.Lo.pair(CG_P), at) = make_double2(0.0, 0.0);
+    elem<BIG>(a.Lo.pair(CG_X), at) = make_double2(xu, xv);
+    elem<BIG>(a.Lo.pair(CG_H), at) = make_double2(o.hu, o.hv);
+    elem<BIG>(a.Lo.pair(CG_B), at) = make_double2(o.bu, o.bv);
+    elem<BIG>(a.Lo.pair(CG_CELL), at) = make_double2(o.heta, o.dimp);
+    if constexpr (PRE) elem<BIG>(a.Lo.pair(CG_DINV), at) = make_double2(zu, zv);
+    elem<BIG>(a.Lo.corner(), at) = o.hetac;
+    elem<BIG>(a.Lo.M, at) = (uint8_t)(((o.mu & MB_INNER) ? CB_INNER_U : 0) | ((o.mv & MB_INNER) ? CB_INNER_V : 0) |
                            ((o.mu & MB_WAVELET) ? CB_WAVELET_U : 0) | ((o.mv & MB_WAVELET) ? CB_WAVELET_V : 0));
     double r2u = ru * ru, r2v = rv * rv, b2u = bu * bu, b2v = bv * bv;
     tree256x2(r2u, r2v, lds);
@@ -2439,6 +2447,7 @@ __device__ __forceinline__ void cg_finish_tile(const GridDims &g, int levels, in
     if (mb & CB_INNER_V) ev[kv] = e_v + t[1][ly][lx];
 }
 
+template <bool BIG>
 __global__ void __launch_bounds__(256) k_cg_finish(CGArgs a, CGIo io)
 {
     const int L = xcd_tile(a.nblk);
@@ -2447,8 +2456,8 @@ __global__ void __launch_bounds__(256) k_cg_finish(CGArgs a, CGIo io)
     band_tile(a.g, L, bx, by);
     const unsigned at = a.Lo.at(bx * TILE + (int)(threadIdx.x & 15), by * TILE + (int)(threadIdx.x >> 4));
     const bool resident = io.resident && *io.abort == 0;  // the resident CG leaves x in CG_Q
-    const double2 x = elem32(a.Lo.pair(resident ? CG_Q : CG_X), at);
-    cg_finish_tile<double>(a.g, io.levels, bx, by, x.x, x.y, elem32(a.Lo.M, at), io.xu, io.xv, io.eu, io.ev);
+    const double2 x = elem<BIG>(a.Lo.pair(resident ? CG_Q : CG_X), at);
+    cg_finish_tile<double>(a.g, io.levels, bx, by, x.x, x.y, elem<BIG>(a.Lo.M, at), io.xu, io.xv, io.eu, io.ev);
 }
 
 // A CG scalar written by an earlier kernel, read as a vector load: a scalar
@@ -2532,7 +2541,7 @@ __device__ __forceinline__ int haar_row_terms(int i, int (&off)[LEV + 2])
 
 // The geometry and the coefficients of a thread's part of a tile, and the
 // tile's c = R A P u from its own direction and the coarse halo's.
-template <int LEV>
+template <int LEV, bool BIG = false>
 struct CgTile {
     using T = double;
     static constexpr int N = LEV + 2;
@@ -2593,25 +2602,25 @@ struct CgTile {
             h.vy = h.uy;
         }
         cr.hhu = cr.hhv = 0.0;
-        const double2 oh = elem32(Lo.pair(CG_H), at);
+        const double2 oh = elem<BIG>(Lo.pair(CG_H), at);
         hmb = 0;
         if (w >= 1) {
             const int hx = h.hu ? h.ux : h.vx, hy = h.hu ? h.uy : h.vy;
             const unsigned ha = Lo.from(at0, hx - 1, hy - 1);
-            cr.hhu = cr.hhv = elem32(reinterpret_cast<const double *>(Lo.pair(CG_H)), 2 * ha + (h.hu ? 0 : 1));
-            hmb = elem32(Lo.M, ha);
+            cr.hhu = cr.hhv = elem<BIG>(reinterpret_cast<const double *>(Lo.pair(CG_H)), 2 * ha + (h.hu ? 0 : 1));
+            hmb = elem<BIG>(Lo.M, ha);
         }
-        const double2 cell = elem32(Lo.pair(CG_CELL), at);
-        o.hetac = elem32(Lo.corner(), at);
+        const double2 cell = elem<BIG>(Lo.pair(CG_CELL), at);
+        o.hetac = elem<BIG>(Lo.corner(), at);
         op_extra_cell(l, cr);
         if (w == 0) {
             const unsigned ea = Lo.from(at0, cr.ex - 1, cr.ey - 1);
-            const double2 ce = elem32(Lo.pair(CG_CELL), ea);
-            cr.ec = elem32(Lo.corner(), ea);
+            const double2 ce = elem<BIG>(Lo.pair(CG_CELL), ea);
+            cr.ec = elem<BIG>(Lo.corner(), ea);
             cr.eh = ce.x;
             cr.ed = ce.y;
         }
-        const double2 ob = elem32(Lo.pair(CG_B), at);
+        const double2 ob = elem<BIG>(Lo.pair(CG_B), at);
         o.hu = oh.x;
         o.hv = oh.y;
         o.bu = ob.x;
@@ -2756,7 +2765,7 @@ __device__ __forceinline__ double2 cg_direction(double beta, double2 r, double2 
 // iteration had a third kernel boundary (at least 2.5 us on this chip).
 // u and c are zero off the wavelet masks by construction (b, and with it r, u
 // and D^-1, are).
-template <bool PRE, int LEV, int FOLD>
+template <bool PRE, int LEV, int FOLD, bool BIG>
 __device__ __forceinline__ bool cg_step_tile(const CGArgs &a, int par, const int L)
 {
     using T = double;
@@ -2767,7 +2776,7 @@ __device__ __forceinline__ bool cg_step_tile(const CGArgs &a, int par, const int
     int bx, by;
     band_tile(g, L, bx, by);
     const CGLayout &Lo = a.Lo;
-    CgTile<LEV> t;
+    CgTile<LEV, BIG> t;
     t.place(Lo, bx * TILE, by * TILE);
     const unsigned at = t.at;
     const double2 *R = Lo.pair(CG_R), *P = Lo.pair(CG_P + par), *D = Lo.pair(CG_DINV);
@@ -2783,12 +2792,12 @@ __device__ __forceinline__ bool cg_step_tile(const CGArgs &a, int par, const int
         prev_rz = cg_scalar(&a.st->rz[1 - par]);
         fz.load(a.Pz, g.npart);
     }
-    const double2 r = elem32(R, at), p = elem32(P, at), x = elem32(Lo.pair(CG_X), at);
-    const double2 dz = PRE ? elem32(D, at) : make_double2(0.0, 0.0);
-    t.mb = elem32(Lo.M, at);
+    const double2 r = elem<BIG>(R, at), p = elem<BIG>(P, at), x = elem<BIG>(Lo.pair(CG_X), at);
+    const double2 dz = PRE ? elem<BIG>(D, at) : make_double2(0.0, 0.0);
+    t.mb = elem<BIG>(Lo.M, at);
     t.place_halo(Lo);
-    const double2 nr0 = elem32(R, t.h0), np0 = elem32(P, t.h0), nd0 = PRE ? elem32(D, t.h0) : make_double2(0.0, 0.0);
-    const double2 nr1 = elem32(R, t.h1), np1 = elem32(P, t.h1), nd1 = PRE ? elem32(D, t.h1) : make_double2(0.0, 0.0);
+    const double2 nr0 = elem<BIG>(R, t.h0), np0 = elem<BIG>(P, t.h0), nd0 = PRE ? elem<BIG>(D, t.h0) : make_double2(0.0, 0.0);
+    const double2 nr1 = elem<BIG>(R, t.h1), np1 = elem<BIG>(P, t.h1), nd1 = PRE ? elem<BIG>(D, t.h1) : make_double2(0.0, 0.0);
     t.load_coef(Lo);
     double res;
     if constexpr (PRE) {
@@ -2822,15 +2831,15 @@ __device__ __forceinline__ bool cg_step_tile(const CGArgs &a, int par, const int
             }
         }
     }
-    if (alpha != 0.0) elem32(Lo.pair(CG_X), at) = make_double2(x.x + alpha * p.x, x.y + alpha * p.y);
+    if (alpha != 0.0) elem<BIG>(Lo.pair(CG_X), at) = make_double2(x.x + alpha * p.x, x.y + alpha * p.y);
     if (done) return true;
     const T beta = cg_beta<PRE>(it, res, prev_res, rz, prev_rz);
     const double2 un = cg_direction<PRE>(beta, r, p, dz);
-    elem32(Lo.pair(CG_P + 1 - par), at) = un;
+    elem<BIG>(Lo.pair(CG_P + 1 - par), at) = un;
     double2 c;
     (void)t.apply(a.rdx, a.rdy, un, cg_direction<PRE>(beta, nr0, np0, nd0), cg_direction<PRE>(beta, nr1, np1, nd1), s, c,
                   [] { return true; });
-    elem32(Lo.pair(CG_Q), at) = c;
+    elem<BIG>(Lo.pair(CG_Q), at) = c;
     double du = un.x * c.x, dv = un.y * c.y;
     tree256x2_open(du, dv, lds + 12);
     if (threadIdx.x == 0) {
@@ -2847,7 +2856,7 @@ __device__ __forceinline__ bool cg_step_tile(const CGArgs &a, int par, const int
 // its partials and the count unchanged (selected by the flag, which is then
 // needed only at the stores), so that the flag's round trip does not precede
 // the loads.
-template <bool PRE, bool EARLY, int FOLD>
+template <bool PRE, bool EARLY, int FOLD, bool BIG>
 __device__ __forceinline__ void cg_update_tile(const CGArgs &a, int par, const int L)
 {
     __shared__ double lds[20];  // a slot per sum
@@ -2865,8 +2874,8 @@ __device__ __forceinline__ void cg_update_tile(const CGArgs &a, int par, const i
     const double res = cg_scalar(&a.st->res[par]);
     LaneFold<FOLD> fd;
     fd.load(a.Pd, g.npart);
-    const double2 r = elem32(a.Lo.pair(CG_R), at), q = elem32(a.Lo.pair(CG_Q), at);
-    const double2 dz = PRE ? elem32(a.Lo.pair(CG_DINV), at) : make_double2(0.0, 0.0);
+    const double2 r = elem<BIG>(a.Lo.pair(CG_R), at), q = elem<BIG>(a.Lo.pair(CG_Q), at);
+    const double2 dz = PRE ? elem<BIG>(a.Lo.pair(CG_DINV), at) : make_double2(0.0, 0.0);
     double rzc = 0.0;
     if constexpr (PRE) rzc = cg_scalar(&a.st->rz[par]);
     const double dot = tree256_open(fd.sum(a.Pd, g.npart), lds);
@@ -2877,7 +2886,7 @@ __device__ __forceinline__ void cg_update_tile(const CGArgs &a, int par, const i
     }
     double2 rn = make_double2(r.x - alpha * q.x, r.y - alpha * q.y);
     if (stopped) rn = r;
-    elem32(a.Lo.pair(CG_R), at) = rn;
+    elem<BIG>(a.Lo.pair(CG_R), at) = rn;
     double r2u = rn.x * rn.x, r2v = rn.y * rn.y, z2u = 0.0, z2v = 0.0;
     tree256x2_open(r2u, r2v, lds + 4);
     if constexpr (PRE) {
@@ -2898,16 +2907,16 @@ __device__ __forceinline__ void cg_update_tile(const CGArgs &a, int par, const i
     }
 }
 
-template <bool PRE, int LEV, int FOLD>
+template <bool PRE, int LEV, int FOLD, bool BIG>
 __global__ void __launch_bounds__(256) k_cg_step(CGArgs a, int par)
 {
-    (void)cg_step_tile<PRE, LEV, FOLD>(a, par, xcd_tile(a.nblk));
+    (void)cg_step_tile<PRE, LEV, FOLD, BIG>(a, par, xcd_tile(a.nblk));
 }
 
-template <bool PRE, bool EARLY, int FOLD>
+template <bool PRE, bool EARLY, int FOLD, bool BIG>
 __global__ void __launch_bounds__(256) k_cg_update(CGArgs a, int par)
 {
-    cg_update_tile<PRE, EARLY, FOLD>(a, par, xcd_tile(a.nblk));
+    cg_update_tile<PRE, EARLY, FOLD, BIG>(a, par, xcd_tile(a.nblk));
 }
 
 // Diagonal of the coarse-CG operator A_c = M_w R M_i A M_i P M_w
@@ -2994,7 +3003,7 @@ __global__ void __launch_bounds__(256) k_coarse_diag(GridDims g, OpCoef<double> 
 // thread of every tile decides alike from the same partials and scalars,
 // after maxiter + 1 iterations at most.  only_if: run only if it is set
 // (the resident CG below gave up; what it starts from is still in place).
-template <bool PRE, int LEV>
+template <bool PRE, int LEV, bool BIG>
 __global__ void __launch_bounds__(256) k_cg_solve1(CGArgs a, const int *only_if)
 {
     if (only_if) {
@@ -3006,12 +3015,12 @@ __global__ void __launch_bounds__(256) k_cg_solve1(CGArgs a, const int *only_if)
         const int par = q & 1;
         bool stop = false;
         for (int L = 0; L < ntile; ++L) {
-            stop = cg_step_tile<PRE, LEV, 1>(a, par, L);
+            stop = cg_step_tile<PRE, LEV, 1, BIG>(a, par, L);
             __syncthreads();
         }
         if (stop) break;
         for (int L = 0; L < ntile; ++L) {
-            cg_update_tile<PRE, true, 1>(a, par, L);
+            cg_update_tile<PRE, true, 1, BIG>(a, par, L);
             __syncthreads();
         }
     }
