@@ -400,6 +400,20 @@ int wavi_smoother_tile(const wavi_ctx *ctx, int *tx, int *ty);
 int wavi_set_coarse_cg(wavi_ctx *ctx, int mode);
 int wavi_coarse_cg(const wavi_ctx *ctx, int *mode);
 
+/* The coarse CGs of the context that have ended since its creation, by the
+ * form they took: runs[WAVI_CG_RAN_LAUNCHES] by launches per iteration,
+ * [.._RESIDENT] in one launch of a workgroup per tile, [.._WORKGROUP] in one
+ * workgroup, as WAVI_CG_WORKGROUP asks, [.._GAVE_UP] in one workgroup after a
+ * resident launch in which a wait ran out.  WAVI_CG_AUTO takes the launches on
+ * a grid that is too large for the resident form, and where other resident
+ * launches leave no room on the chip.  No reference counterpart. */
+#define WAVI_CG_RAN_LAUNCHES 0
+#define WAVI_CG_RAN_RESIDENT 1
+#define WAVI_CG_RAN_WORKGROUP 2
+#define WAVI_CG_RAN_GAVE_UP 3
+#define WAVI_CG_RAN_COUNT 4
+int wavi_coarse_cg_runs(const wavi_ctx *ctx, int64_t *runs);
+
 /* Kernel timing with HIP events on the context's stream, for measurement.
  * Sampled single launches (events around every 16th launch, so each time
  * includes the cost of the two event records): WAVI_KT_CG_APPLY (FP64

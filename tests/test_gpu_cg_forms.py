@@ -1,0 +1,99 @@
+"""Which form the coarse CG takes (wavi_coarse_cg_runs), and that its result is
+that of the launches per iteration, bit for bit."""
+import ctypes
+
+import numpy as np
+import pytest
+
+
+def runs(W, m):
+    """(launches, resident, workgroup, gave up) so far"""
+    got = (ctypes.c_int64 * W._lib.WAVI_CG_RAN_COUNT)()
+    assert m.parallel_spec._lib.wavi_coarse_cg_runs(m.parallel_spec.ctx, got) == 0
+    return tuple(got)
+
+
+def model(W, nx, ny, precision, maxiter_coarse=40, maxiter_picard=3, mode=None, seed=2):
+    m = W.workloads.channel_solve(nx=nx, ny=ny, nσ=4, maxiter_picard=maxiter_picard, precision=precision, seed=seed)
+    m.solver_params.maxiter_coarse = maxiter_coarse
+    W.update_geometry(m)
+    if mode is not None:
+        set_mode(m, mode)
+    return m
+
+
+def set_mode(m, mode):
+    assert m.parallel_spec._lib.wavi_set_coarse_cg(m.parallel_spec.ctx, mode) == 0
+
+
+def assert_same(m, ref):
+    np.testing.assert_array_equal(m.fields.gu.u, ref.fields.gu.u)
+    np.testing.assert_array_equal(m.fields.gv.v, ref.fields.gv.v)
+    assert m.last_report == ref.last_report
+
+
+# tiles: 6, 33, 246, 256, 260, 441, 504, 512, 891; resident up to 504 (FP64) and 256 (mixed)
+@pytest.mark.gpu
+@pytest.mark.parametrize("precision,most", [("fp64", 504), ("mixed", 256)])
+@pytest.mark.parametrize("nx,ny,tiles", [(80, 10, 6), (527, 12, 33), (640, 80, 246), (255, 255, 256), (1039, 63, 260),
+                                         (1007, 111, 441), (1007, 120, 504), (1023, 127, 512), (1280, 160, 891)])
+def test_form_by_the_number_of_tiles(W, nx, ny, tiles, precision, most):
+    print("[gpu] form of the coarse CG %s %dx%d" % (precision, nx, ny), flush=True)
+    m = model(W, nx, ny, precision)
+    W.update_velocities(m)
+    n = m.last_report["picard_iters"] - m.last_report["converged"]
+    assert n > 0 and runs(W, m) == ((0, n, 0, 0) if tiles <= most else (n, 0, 0, 0))
+    ref = model(W, nx, ny, precision, mode=W._lib.WAVI_CG_LAUNCHES)
+    W.update_velocities(ref)
+    assert runs(W, ref) == (n, 0, 0, 0)
+    assert_same(m, ref)
+    set_mode(ref, W._lib.WAVI_CG_WORKGROUP)
+    if tiles == 6:
+        W.update_velocities(ref)
+        assert runs(W, ref)[2] > 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_form_when_waits_run_out(W, monkeypatch, precision):
+    print("[gpu] form without polls %s" % precision, flush=True)
+    monkeypatch.setenv("WAVI_CG_POLLS", "0")
+    m = model(W, 250, 62, precision)
+    W.update_velocities(m)
+    n = m.last_report["picard_iters"] - m.last_report["converged"]
+    assert n > 1 and runs(W, m) == (n - 1, 0, 0, 1)
+
+
+@pytest.mark.gpu
+def test_form_in_a_gradient(W):
+    print("[gpu] form in a gradient", flush=True)
+    m = W.workloads.inversion_model(W.workloads.inversion_logc_true(64, 16, seed=4), "fp64", nσ=4, n_picard=2)
+    W.update_geometry(m)
+    rng = np.random.default_rng(1)
+    W.misfit_gradient(m, 2, 100 * rng.random(m.grid.xxu.shape), 10 * rng.random(m.grid.yyv.shape))
+    got = runs(W, m)
+    assert got[1] > 4 and got == (0, got[1], 0, 0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("polls", [None, "0"])
+def test_form_in_a_lockstep_batch(W, monkeypatch, polls):
+    """Every member resident, or every member's first CG started over; with one
+    member by launches, all are."""
+    print("[gpu] forms in a batch, polls %s" % polls, flush=True)
+    if polls is not None:
+        monkeypatch.setenv("WAVI_CG_POLLS", polls)
+    ms = [model(W, a, b, "mixed") for a, b in ((80, 10), (160, 20), (77, 35), (511, 15))]
+    W.update_velocities_batch(ms, lockstep=True)
+    for m in ms:
+        n = m.last_report["picard_iters"] - m.last_report["converged"]
+        assert n > 1 and runs(W, m) == ((0, n, 0, 0) if polls is None else (n - 1, 0, 0, 1))
+    if polls is None:
+        before = [runs(W, m) for m in ms]
+        set_mode(ms[1], W._lib.WAVI_CG_LAUNCHES)
+        for m in ms:
+            m.fields.gu.u[...] = 0.0
+            m.fields.gv.v[...] = 0.0
+        W.update_velocities_batch(ms, lockstep=True)
+        for m, b in zip(ms, before):
+            assert runs(W, m)[1:] == b[1:] and runs(W, m)[0] > b[0]

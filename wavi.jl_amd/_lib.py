@@ -21,6 +21,12 @@ WAVI_EHIP = 1
 WAVI_CG_AUTO = 0
 WAVI_CG_LAUNCHES = 1
 WAVI_CG_WORKGROUP = 2
+# forms of the coarse CGs that ran (wavi_coarse_cg_runs)
+WAVI_CG_RAN_LAUNCHES = 0
+WAVI_CG_RAN_RESIDENT = 1
+WAVI_CG_RAN_WORKGROUP = 2
+WAVI_CG_RAN_GAVE_UP = 3
+WAVI_CG_RAN_COUNT = 4
 
 PRECISION = {"fp64": 0, "mixed": 1}
 
@@ -173,6 +179,7 @@ SIGNATURES = {
     "wavi_set_linear_coarse_jacobi": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_int]),
     "wavi_coarse_diag": (ctypes.c_int, [ctypes.c_void_p, _dp, _dp]),
     "wavi_coarse_cg": (ctypes.c_int, [ctypes.c_void_p, ctypes.POINTER(ctypes.c_int)]),
+    "wavi_coarse_cg_runs": (ctypes.c_int, [ctypes.c_void_p, ctypes.POINTER(ctypes.c_int64)]),
     "wavi_profile_enable": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_int]),
     "wavi_profile_read": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_int, _dp, ctypes.POINTER(ctypes.c_int64)]),
     "wavi_math_probe": (ctypes.c_int, [ctypes.c_int, _dp, _dp, _dp, ctypes.c_size_t]),

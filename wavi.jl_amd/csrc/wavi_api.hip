@@ -121,6 +121,7 @@ struct wavi_ctx {
     bool x_off = false;             // a wait ran out once: the launches per iteration from then on
     bool x_ran = false;             // the last CG ran so (k_cg_finish)
     bool x_pending = false;         // ... and its report has not been read
+    int64_t cg_runs[WAVI_CG_RAN_COUNT] = {};  // coarse CGs that ended, by their form (wavi_coarse_cg_runs)
     VSet<float> v32;
     // mixed-precision coarse CG: s, w, the parity-buffered images P r, P s,
     // P w and partials of (r, r) and (w, r)
@@ -1652,6 +1653,7 @@ static int cg_collect(wavi_ctx *ctx, int *iters)
         return WAVI_ESTATE;
     }
     if (hf->gave_up) ctx->x_off = true;
+    ++ctx->cg_runs[hf->gave_up ? WAVI_CG_RAN_GAVE_UP : WAVI_CG_RAN_RESIDENT];
     *iters = hf->iters;
     for (wavi_ctx::Burst &b : ctx->bursts) b.n = hf->iters;
     burst_collect(ctx, ctx->precision == WAVI_PRECISION_FP64 ? WAVI_KT_CG_ITER_FP64 : WAVI_KT_CG_ITER_MIXED,
@@ -1748,6 +1750,7 @@ int do_coarse_cg<double>(wavi_ctx *ctx, const VSet<double> &w, int *iters)
             ctx->err = "coarse CG did not terminate";
             return WAVI_ESTATE;
         }
+        ++ctx->cg_runs[WAVI_CG_RAN_WORKGROUP];
         *iters = hf->iters;
         return WAVI_OK;
     }
@@ -1805,6 +1808,7 @@ int do_coarse_cg<double>(wavi_ctx *ctx, const VSet<double> &w, int *iters)
         ctx->err = "coarse CG did not terminate";
         return WAVI_ESTATE;
     }
+    ++ctx->cg_runs[WAVI_CG_RAN_LAUNCHES];
     *iters = hf->iters;
     ctx->cg_prev = hf->iters;
     return WAVI_OK;
@@ -1991,6 +1995,7 @@ int do_coarse_cg<float>(wavi_ctx *ctx, const VSet<float> &w, int *iters)
             ctx->err = "coarse CG did not terminate";
             return WAVI_ESTATE;
         }
+        ++ctx->cg_runs[WAVI_CG_RAN_WORKGROUP];
         *iters = hf->iters;
         return WAVI_OK;
     }
@@ -2055,6 +2060,7 @@ int do_coarse_cg<float>(wavi_ctx *ctx, const VSet<float> &w, int *iters)
         ctx->err = "coarse CG did not terminate";
         return WAVI_ESTATE;
     }
+    ++ctx->cg_runs[WAVI_CG_RAN_LAUNCHES];
     *iters = hf->iters;
     ctx->cg_prev = hf->iters;
     return WAVI_OK;
@@ -2918,6 +2924,7 @@ static int run_cg_batch(const std::vector<wavi_ctx *> &mem, const std::vector<hi
         iters[j] = f->iters;
         ctx->x_ran = resident;
         if (f->gave_up) ctx->x_off = true;
+        ++ctx->cg_runs[f->gave_up ? WAVI_CG_RAN_GAVE_UP : (resident ? WAVI_CG_RAN_RESIDENT : WAVI_CG_RAN_LAUNCHES)];
         if (j > 0) HIPCHK(hipStreamWaitEvent(ctx->stream, done, 0));
     }
     return WAVI_OK;
@@ -3788,6 +3795,13 @@ int wavi_coarse_cg(const wavi_ctx *ctx, int *mode)
 {
     if (!ctx || !mode) return WAVI_EARG;
     *mode = cg_one_workgroup(ctx) ? WAVI_CG_WORKGROUP : WAVI_CG_LAUNCHES;
+    return WAVI_OK;
+}
+
+int wavi_coarse_cg_runs(const wavi_ctx *ctx, int64_t *runs)
+{
+    if (!ctx || !runs) return WAVI_EARG;
+    for (int k = 0; k < WAVI_CG_RAN_COUNT; ++k) runs[k] = ctx->cg_runs[k];
     return WAVI_OK;
 }
 
