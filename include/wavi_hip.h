@@ -414,6 +414,13 @@ int wavi_coarse_cg(const wavi_ctx *ctx, int *mode);
 #define WAVI_CG_RAN_COUNT 4
 int wavi_coarse_cg_runs(const wavi_ctx *ctx, int64_t *runs);
 
+/* Test hook for the waits of the resident form: polls of a wait before it
+ * gives up (negative: unchanged; at most the default, 2^21), and the tag of the
+ * context's next exchange (0: unchanged; at least the present one).  Each CG
+ * takes maxiter_coarse + 2 of the 2^32 tags however few iterations it needs; the
+ * exchanged words are cleared and the tags begin again when they run out. */
+int wavi_set_coarse_cg_waits(wavi_ctx *ctx, int64_t polls, uint32_t tag);
+
 /* Kernel timing with HIP events on the context's stream, for measurement.
  * Sampled single launches (events around every 16th launch, so each time
  * includes the cost of the two event records): WAVI_KT_CG_APPLY (FP64

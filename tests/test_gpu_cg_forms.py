@@ -97,3 +97,43 @@ def test_form_in_a_lockstep_batch(W, monkeypatch, polls):
         W.update_velocities_batch(ms, lockstep=True)
         for m, b in zip(ms, before):
             assert runs(W, m)[1:] == b[1:] and runs(W, m)[0] > b[0]
+
+
+def set_waits(m, polls=-1, tag=0):
+    return m.parallel_spec._lib.wavi_set_coarse_cg_waits(m.parallel_spec.ctx, polls, tag)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("nx,ny", [(80, 10), (250, 62)])
+@pytest.mark.parametrize("maxiter_coarse", [1, 40])
+def test_tags_that_run_out(W, nx, ny, precision, maxiter_coarse):
+    """The words of the first call hold the first tags (1 with one iteration);
+    in the second call the tags run out and those come again, which is right only
+    if the words were cleared."""
+    print("[gpu] tags run out %s %dx%d, %d iterations" % (precision, nx, ny, maxiter_coarse), flush=True)
+    m, ref = (model(W, nx, ny, precision, maxiter_coarse=maxiter_coarse, maxiter_picard=1, mode=mode)
+              for mode in (None, W._lib.WAVI_CG_LAUNCHES))
+    for tag in (0, 2 ** 32 - 2 * (maxiter_coarse + 2), 0, 0, 0):
+        assert set_waits(m, tag=tag) == 0
+        for x in (m, ref):
+            W.update_velocities(x)
+        assert_same(m, ref)
+    assert runs(W, m) == (0, 5, 0, 0)
+    assert set_waits(m, tag=1) == W._lib.WAVI_EARG
+    assert set_waits(m, polls=2 ** 21 + 1) == W._lib.WAVI_EARG
+
+
+@pytest.mark.gpu
+def test_tags_that_run_out_in_a_batch(W):
+    print("[gpu] tags run out in a batch", flush=True)
+    sizes = ((80, 10), (160, 20), (77, 35))
+    ms = [model(W, a, b, "mixed", maxiter_coarse=1, maxiter_picard=1) for a, b in sizes]
+    refs = [model(W, a, b, "mixed", maxiter_coarse=1, maxiter_picard=1, mode=W._lib.WAVI_CG_LAUNCHES) for a, b in sizes]
+    for tag in (0, 2 ** 32 - 6, 0, 0, 0):
+        assert set_waits(ms[1], tag=tag) == 0
+        W.update_velocities_batch(ms, lockstep=True)
+        for m, ref in zip(ms, refs):
+            W.update_velocities(ref)
+            assert_same(m, ref)
+    assert all(runs(W, m) == (0, 5, 0, 0) for m in ms)

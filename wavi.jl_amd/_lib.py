@@ -180,6 +180,7 @@ SIGNATURES = {
     "wavi_coarse_diag": (ctypes.c_int, [ctypes.c_void_p, _dp, _dp]),
     "wavi_coarse_cg": (ctypes.c_int, [ctypes.c_void_p, ctypes.POINTER(ctypes.c_int)]),
     "wavi_coarse_cg_runs": (ctypes.c_int, [ctypes.c_void_p, ctypes.POINTER(ctypes.c_int64)]),
+    "wavi_set_coarse_cg_waits": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_int64, ctypes.c_uint32]),
     "wavi_profile_enable": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_int]),
     "wavi_profile_read": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_int, _dp, ctypes.POINTER(ctypes.c_int64)]),
     "wavi_math_probe": (ctypes.c_int, [ctypes.c_int, _dp, _dp, _dp, ctypes.c_size_t]),

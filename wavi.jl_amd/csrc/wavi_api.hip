@@ -3798,6 +3798,18 @@ int wavi_coarse_cg(const wavi_ctx *ctx, int *mode)
     return WAVI_OK;
 }
 
+int wavi_set_coarse_cg_waits(wavi_ctx *ctx, int64_t polls, uint32_t tag)
+{
+    if (!ctx) return WAVI_EARG;
+    if (polls > (int64_t)X_POLLS || (tag != 0 && tag < ctx->xtag)) {
+        ctx->err = "wavi_set_coarse_cg_waits: more polls than the default, or a tag that was used";
+        return WAVI_EARG;
+    }
+    if (polls >= 0) ctx->x_polls = (unsigned)polls;
+    if (tag != 0) ctx->xtag = tag;
+    return WAVI_OK;
+}
+
 int wavi_coarse_cg_runs(const wavi_ctx *ctx, int64_t *runs)
 {
     if (!ctx || !runs) return WAVI_EARG;
