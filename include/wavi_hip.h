@@ -388,7 +388,12 @@ int wavi_smoother_tile(const wavi_ctx *ctx, int *tx, int *ty);
  * halos among themselves (FP64, 63 tiles: 7.1 us per iteration against 9.5;
  * mixed, 246 tiles: 4.2 against 5.1); else WAVI_CG_LAUNCHES.  The
  * workgroup is 3.4 to 3.6 times slower per iteration than the launches even on
- * a grid of six 16 x 16 tiles.  All give the same bits.  wavi_coarse_cg
+ * a grid of six 16 x 16 tiles.  All give the same bits.  The one launch is
+ * made where its workgroups fit beside those of other such launches on the GPU,
+ * from this process or from others of the same user that share /dev/shm
+ * (an account of about 300 bytes per GPU there, /dev/shm/wavi_hip_room1.*).
+ * Beside processes that are not on that account its waits can run out, after a
+ * second or more: the CG is then done again in one workgroup.  wavi_coarse_cg
  * reports the mode in effect for the context (WAVI_CG_LAUNCHES for
  * WAVI_CG_AUTO).  Lockstep batches (wavi_update_velocities_lockstep*) and the
  * small members of wavi_misfit_gradient_batch share one launch for the whole

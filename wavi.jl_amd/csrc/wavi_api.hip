@@ -21,6 +21,7 @@
 #include <vector>
 
 #include "../../include/wavi_hip.h"
+#include "wavi_room.h"
 // all kernels of the library live in this translation unit
 #include "wavi_kernels.hip"
 
@@ -269,34 +270,34 @@ static void burst_collect(wavi_ctx *ctx, int kid, int last_active)
         if (rc_ != WAVI_OK) return rc_; \
     } while (0)
 
-// How much of each GPU is taken by launches whose workgroups wait for one
-// another (k_cg_resident), in units of 1 / CU_UNITS of a CU.  A launch that waits
-// must have all its workgroups on the chip; alone it may take all of it.
-// Beside another one it may only bring the sum to half of the chip: a
-// workgroup takes at most half a CU, so then some CU always has room for the
-// next one, however the others lie.  Kernels that do not wait need no
-// place here: they end.  A launch that finds no room is not made: the CG then
-// takes a pair of launches per iteration.
+// What launches whose workgroups wait for one another (k_cg_resident) take of
+// each GPU, in units of 1 / CU_UNITS of a CU (wavi_room.h).  Without room the
+// CG takes launches per iteration.
 constexpr int CU_UNITS = 64;
-static std::mutex g_room_mu;
-static int g_room_used[MAX_DEVICES] = {};
-static int g_room[MAX_DEVICES] = {};  // CUs x CU_UNITS
+static Room g_room[MAX_DEVICES];
+
+// Opens the account of the device at the first context on it.
+static hipError_t room_open(int device, int cus)
+{
+    static std::mutex mu;
+    static bool known[MAX_DEVICES] = {};
+    if (device < 0 || device >= MAX_DEVICES) return hipSuccess;
+    std::lock_guard<std::mutex> lock(mu);
+    if (known[device]) return hipSuccess;
+    char bus[64] = "";
+    const hipError_t e = hipDeviceGetPCIBusId(bus, sizeof(bus), device);
+    if (e != hipSuccess) return e;
+    g_room[device].open(bus, cus * CU_UNITS);
+    known[device] = true;
+    return hipSuccess;
+}
 
 static bool room_take(int device, int units)
 {
-    if (device < 0 || device >= MAX_DEVICES) return false;
-    std::lock_guard<std::mutex> lock(g_room_mu);
-    const int used = g_room_used[device];
-    if (used + units > (used == 0 ? g_room[device] : g_room[device] / 2)) return false;
-    g_room_used[device] = used + units;
-    return true;
+    return device >= 0 && device < MAX_DEVICES && g_room[device].take(units);
 }
 
-static void room_give(int device, int units)
-{
-    std::lock_guard<std::mutex> lock(g_room_mu);
-    g_room_used[device] -= units;
-}
+static void room_give(int device, int units) { g_room[device].give(units); }
 
 static inline dim3 flat(int n) { return dim3((unsigned)((n + 255) / 256)); }
 // workgroups of a launch over an nbx x nby tile grid with xcd_band_tile: a multiple of 8
@@ -783,10 +784,7 @@ int wavi_ctx_create(const wavi_grid_desc *grid, const wavi_phys_params *phys, co
             ctx->xm_fn[pre] = cgm_resident_fn(solver->levels, pre != 0);
             CREATECHK(resident_occupancy(fp64 ? (const void *)ctx->x_fn[pre] : (const void *)ctx->xm_fn[pre], &occ[pre]));
         }
-        if (ctx->device < MAX_DEVICES) {
-            std::lock_guard<std::mutex> rlock(g_room_mu);
-            g_room[ctx->device] = cus * CU_UNITS;
-        }
+        CREATECHK(room_open(ctx->device, cus));
         ctx->x_blocks = ctx->nblk + (fp64 && ntile > X_FLAT_TILES ? 8 : 0);  // the workgroup that folds
         const int per_cu = std::min(std::min(occ[0], occ[1]), 4);  // 4: what k_cgm_resident_batch is built for
         if (per_cu >= 2 && ctx->x_blocks <= cus * per_cu && ntile <= (fp64 ? X_TILES_FP64 : X_TILES_MIXED) &&
