@@ -393,7 +393,9 @@ int wavi_smoother_tile(const wavi_ctx *ctx, int *tx, int *ty);
  * from this process or from others of the same user that share /dev/shm
  * (an account of about 300 bytes per GPU there, /dev/shm/wavi_hip_room1.*).
  * Beside processes that are not on that account its waits can run out, after a
- * second or more: the CG is then done again in one workgroup.  wavi_coarse_cg
+ * second or more: the CG is then done again in one workgroup, and the context
+ * takes the launches for its next 256 CGs (twice as many after every further
+ * loss) before it tries again.  wavi_coarse_cg
  * reports the mode in effect for the context (WAVI_CG_LAUNCHES for
  * WAVI_CG_AUTO).  Lockstep batches (wavi_update_velocities_lockstep*) and the
  * small members of wavi_misfit_gradient_batch share one launch for the whole

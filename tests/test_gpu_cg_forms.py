@@ -137,3 +137,34 @@ def test_tags_that_run_out_in_a_batch(W):
             W.update_velocities(ref)
             assert_same(m, ref)
     assert all(runs(W, m) == (0, 5, 0, 0) for m in ms)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_resident_again_after_a_lost_wait(W, precision):
+    """256 CGs by launches after a loss, 512 after a second one in a row; then the
+    waits are polled again and the form is resident for good."""
+    print("[gpu] resident again after a lost wait, %s" % precision, flush=True)
+    m, ref = (model(W, 80, 10, precision, maxiter_coarse=4, maxiter_picard=1, mode=mode)
+              for mode in (None, W._lib.WAVI_CG_LAUNCHES))
+    rng = np.random.default_rng(0)
+    ru, rv = rng.standard_normal(m.fields.gu.u.shape), rng.standard_normal(m.fields.gv.v.shape)
+
+    def vcycles(n):
+        for _ in range(n):
+            got, want = W.vcycle(m, ru, rv), W.vcycle(ref, ru, rv)
+        for a, b in zip(got, want):
+            np.testing.assert_array_equal(a, b)
+        return runs(W, m)
+
+    assert vcycles(1) == (0, 1, 0, 0)
+    assert set_waits(m, polls=0) == 0
+    assert vcycles(1) == (0, 1, 0, 1)
+    assert vcycles(256) == (256, 1, 0, 1)
+    assert vcycles(1) == (256, 1, 0, 2)
+    assert set_waits(m, polls=2 ** 21) == 0
+    assert vcycles(512) == (768, 1, 0, 2)
+    assert vcycles(300) == (768, 301, 0, 2)
+    assert set_waits(m, polls=0) == 0
+    assert vcycles(1) == (768, 301, 0, 3)
+    assert vcycles(257) == (1024, 301, 0, 4)

@@ -69,6 +69,11 @@ struct VSet {
 
 // Polls of one wait of k_cg_resident, at least half a microsecond each.
 constexpr unsigned X_POLLS = 1u << 21;
+// CGs that take the launches after a wait ran out, doubled with every further
+// loss up to X_REST << X_REST_DOUBLED.  A loss costs the polls, a second or more,
+// and a CG in one workgroup; a resident CG of 1000 iterations on 441 tiles
+// saves 3 ms.  What held the chip may have been another program that has ended.
+constexpr int X_REST = 256, X_REST_DOUBLED = 10;
 
 struct wavi_ctx {
     int device = 0;
@@ -119,7 +124,8 @@ struct wavi_ctx {
     void (*xm_fn[2])(CGMIterArgs, CGMExchange) = {};  // ... of the mixed CG
     int x_blocks = 0;               // workgroups of its launch
     int x_units = 0;                // ... and their share of the chip (room_take)
-    bool x_off = false;             // a wait ran out once: the launches per iteration from then on
+    int x_lost = 0;                 // resident CGs in a row in which a wait ran out
+    int x_rest = 0;                 // CGs by launches before the next one is resident again (X_REST)
     bool x_ran = false;             // the last CG ran so (k_cg_finish)
     bool x_pending = false;         // ... and its report has not been read
     int64_t cg_runs[WAVI_CG_RAN_COUNT] = {};  // coarse CGs that ended, by their form (wavi_coarse_cg_runs)
@@ -1637,6 +1643,25 @@ static void launch_cg_solve1(wavi_ctx *ctx, const CGArgs &a, const int *only_if 
     }
 }
 
+// Whether the context's CGs take the launches for now after a lost wait; counts
+// one of them.
+static bool cg_rests(wavi_ctx *ctx)
+{
+    if (ctx->x_rest == 0) return false;
+    --ctx->x_rest;
+    return true;
+}
+
+// A resident CG has ended.
+static void cg_resident_ended(wavi_ctx *ctx, bool gave_up)
+{
+    ++ctx->cg_runs[gave_up ? WAVI_CG_RAN_GAVE_UP : WAVI_CG_RAN_RESIDENT];
+    if (gave_up)
+        ctx->x_rest = X_REST << std::min(ctx->x_lost++, X_REST_DOUBLED);
+    else
+        ctx->x_lost = 0;
+}
+
 // After the stream has been waited for: the iterations of a resident CG whose
 // report is still to be read, 0 if there is none.
 static int cg_collect(wavi_ctx *ctx, int *iters)
@@ -1650,8 +1675,7 @@ static int cg_collect(wavi_ctx *ctx, int *iters)
         ctx->err = "coarse CG did not terminate";
         return WAVI_ESTATE;
     }
-    if (hf->gave_up) ctx->x_off = true;
-    ++ctx->cg_runs[hf->gave_up ? WAVI_CG_RAN_GAVE_UP : WAVI_CG_RAN_RESIDENT];
+    cg_resident_ended(ctx, hf->gave_up != 0);
     *iters = hf->iters;
     for (wavi_ctx::Burst &b : ctx->bursts) b.n = hf->iters;
     burst_collect(ctx, ctx->precision == WAVI_PRECISION_FP64 ? WAVI_KT_CG_ITER_FP64 : WAVI_KT_CG_ITER_MIXED,
@@ -1669,7 +1693,7 @@ static bool cg_resident_begin(wavi_ctx *ctx, unsigned *tag, hipStream_t stream, 
         if (hipStreamSynchronize(ctx->stream) != hipSuccess) return false;
         (void)cg_collect(ctx, &lost);
     }
-    if (!ctx->xwords || ctx->x_off || ctx->cg_mode != WAVI_CG_AUTO) return false;
+    if (!ctx->xwords || ctx->cg_mode != WAVI_CG_AUTO || cg_rests(ctx)) return false;
     if (room && !room_take(ctx->device, ctx->x_units)) return false;
     const unsigned need = (unsigned)ctx->S.maxiter_coarse + 2u;
     if (ctx->xtag > 0xffffffffu - need) {  // tags used up: clear the words and begin again
@@ -2872,7 +2896,9 @@ static int run_cg_batch(const std::vector<wavi_ctx *> &mem, const std::vector<hi
     int units = 0;
     for (wavi_ctx *m : mem) units += m->x_units;
     bool resident = true;
-    for (wavi_ctx *m : mem) resident = resident && m->xwords && !m->x_off && m->cg_mode == WAVI_CG_AUTO;
+    for (wavi_ctx *m : mem) {
+        if (!m->xwords || m->cg_mode != WAVI_CG_AUTO || cg_rests(m)) resident = false;
+    }
     resident = resident && hold.take(lead->device, units);
     for (size_t j = 0; j < mem.size() && resident; ++j) {
         unsigned tag = 0;
@@ -2921,8 +2947,10 @@ static int run_cg_batch(const std::vector<wavi_ctx *> &mem, const std::vector<hi
         }
         iters[j] = f->iters;
         ctx->x_ran = resident;
-        if (f->gave_up) ctx->x_off = true;
-        ++ctx->cg_runs[f->gave_up ? WAVI_CG_RAN_GAVE_UP : (resident ? WAVI_CG_RAN_RESIDENT : WAVI_CG_RAN_LAUNCHES)];
+        if (resident)
+            cg_resident_ended(ctx, f->gave_up != 0);
+        else
+            ++ctx->cg_runs[WAVI_CG_RAN_LAUNCHES];
         if (j > 0) HIPCHK(hipStreamWaitEvent(ctx->stream, done, 0));
     }
     return WAVI_OK;
