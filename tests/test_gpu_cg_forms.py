@@ -168,3 +168,27 @@ def test_resident_again_after_a_lost_wait(W, precision):
     assert set_waits(m, polls=0) == 0
     assert vcycles(1) == (768, 301, 0, 3)
     assert vcycles(257) == (1024, 301, 0, 4)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("precision,timer,lockstep", [("fp64", "cg_iter_fp64", False), ("mixed", "cg_iter_mixed", False),
+                                                      ("mixed", "cg_iter_mixed", True)])
+def test_launches_know_the_length_of_a_resident_cg(W, precision, timer, lockstep):
+    """After a CG of 40 iterations the launches are queued in a first chunk of 32,
+    which is timed whole; without its length they begin with chunks of 2, 4, 8, 16."""
+    print("[gpu] launches after a resident CG, %s, lockstep %s" % (precision, lockstep), flush=True)
+    m = model(W, 80, 10, precision, maxiter_coarse=40, maxiter_picard=1)
+    lib, ctx = m.parallel_spec._lib, m.parallel_spec.ctx
+    if lockstep:
+        W.update_velocities_batch([m], lockstep=True)
+    else:
+        W.update_velocities(m)
+    assert m.last_report["coarse_cg_iters"] == [40] and runs(W, m) == (0, 1, 0, 0)
+    set_mode(m, W._lib.WAVI_CG_LAUNCHES)
+    assert lib.wavi_profile_enable(ctx, 1) == 0
+    W.update_velocities(m)
+    ms, n = ctypes.c_double(), ctypes.c_int64()
+    assert lib.wavi_profile_read(ctx, W._lib.KT[timer], ctypes.byref(ms), ctypes.byref(n)) == 0
+    assert lib.wavi_profile_enable(ctx, 0) == 0
+    assert m.last_report["coarse_cg_iters"] == [40] and runs(W, m) == (1, 1, 0, 0)
+    assert n.value == 32 and ms.value > 0.0

@@ -1652,9 +1652,11 @@ static bool cg_rests(wavi_ctx *ctx)
     return true;
 }
 
-// A resident CG has ended.
-static void cg_resident_ended(wavi_ctx *ctx, bool gave_up)
+// A resident CG has ended after `iters` iterations (cg_prev: the next CG may
+// find no room and go by launches).
+static void cg_resident_ended(wavi_ctx *ctx, bool gave_up, int iters)
 {
+    ctx->cg_prev = iters;
     ++ctx->cg_runs[gave_up ? WAVI_CG_RAN_GAVE_UP : WAVI_CG_RAN_RESIDENT];
     if (gave_up)
         ctx->x_rest = X_REST << std::min(ctx->x_lost++, X_REST_DOUBLED);
@@ -1675,7 +1677,7 @@ static int cg_collect(wavi_ctx *ctx, int *iters)
         ctx->err = "coarse CG did not terminate";
         return WAVI_ESTATE;
     }
-    cg_resident_ended(ctx, hf->gave_up != 0);
+    cg_resident_ended(ctx, hf->gave_up != 0, hf->iters);
     *iters = hf->iters;
     for (wavi_ctx::Burst &b : ctx->bursts) b.n = hf->iters;
     burst_collect(ctx, ctx->precision == WAVI_PRECISION_FP64 ? WAVI_KT_CG_ITER_FP64 : WAVI_KT_CG_ITER_MIXED,
@@ -2948,7 +2950,7 @@ static int run_cg_batch(const std::vector<wavi_ctx *> &mem, const std::vector<hi
         iters[j] = f->iters;
         ctx->x_ran = resident;
         if (resident)
-            cg_resident_ended(ctx, f->gave_up != 0);
+            cg_resident_ended(ctx, f->gave_up != 0, f->iters);
         else
             ++ctx->cg_runs[WAVI_CG_RAN_LAUNCHES];
         if (j > 0) HIPCHK(hipStreamWaitEvent(ctx->stream, done, 0));
