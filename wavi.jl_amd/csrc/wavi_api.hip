@@ -1572,16 +1572,13 @@ static bool cg_one_workgroup(const wavi_ctx *ctx)
 }
 
 // A +-1 Haar transform (dir 1: P, 2: R) of the u and v vectors on the tiles
-// (accu != nullptr: the result added into accu, accv at the output masks'
-// points instead, outu, outv untouched)
 template <typename T>
 static void launch_tile_haar(wavi_ctx *ctx, int dir, const T *inu, const T *inv, const uint8_t *min_u,
-                             const uint8_t *min_v, T *outu, T *outv, const uint8_t *mout_u, const uint8_t *mout_v,
-                             T *accu = nullptr, T *accv = nullptr)
+                             const uint8_t *min_v, T *outu, T *outv, const uint8_t *mout_u, const uint8_t *mout_v)
 {
     const GridDims &g = ctx->g;
     hipLaunchKernelGGL((k_tile_haar<T, T>), dim3(g.nbx, g.nby), dim3(256), 0, ctx->stream, g, ctx->tab, ctx->S.levels,
-                       dir, inu, inv, min_u, min_v, outu, outv, mout_u, mout_v, accu, accv);
+                       dir, inu, inv, min_u, min_v, outu, outv, mout_u, mout_v);
 }
 
 // The kernels of the FP64 coarse CG at the context's Haar level,

@@ -234,15 +234,6 @@ __device__ __forceinline__ double lanes_sum(const double *P, int np, double *lds
     return tree256(lane_fold(P, np), lds);
 }
 
-// lanes_sum of two partial arrays of the same length in one pass.
-__device__ __forceinline__ void lanes_sum2(const double *P, const double *Q, int np, double *lds, double &a,
-                                           double &b)
-{
-    a = lane_fold(P, np);
-    b = lane_fold(Q, np);
-    tree256x2(a, b, lds);
-}
-
 // ---------------------------------------------------------------------------
 // Words that the workgroups of one launch exchange: 32 data bits below a
 // 32-bit tag, stored and loaded whole (relaxed atomics at agent scope, which

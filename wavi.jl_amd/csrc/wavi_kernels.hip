@@ -1360,7 +1360,7 @@ struct MaskSep {
 };
 
 // The coarse values around a tile from which k_cg_step forms P u on the
-// halo (HALO_N of haar_halo_offset per side, 5 at three levels).
+// halo (LEV + 2 lines per side, haar_halo_offset; 5 at three levels).
 template <typename T>
 struct HaloLds {
     T x[2][10][17];   // component; columns left (0..4) and right (5..9), by y
@@ -4251,15 +4251,11 @@ __device__ __forceinline__ bool mask_or_all(const uint8_t *mask, const void *any
 }
 
 // Haar transform (dir 0 forward, 1 inverse, 2 transposed inverse) of the
-// masked u and v inputs into the masked outputs.  With accu != nullptr (a
-// +-1 transform only) the result is added into accu, accv at the points of
-// the output masks instead (x += P y, as an add of the masked output would
-// do), and outu, outv are not written.
+// masked u and v inputs into the masked outputs.
 template <typename Tin, typename Tout>
 __global__ void k_tile_haar(GridDims g, const HaarTable *tab, int levels, int dir,
                             const Tin *inu, const Tin *inv, const uint8_t *min_u, const uint8_t *min_v,
-                            Tout *outu, Tout *outv, const uint8_t *mout_u, const uint8_t *mout_v,
-                            Tout *accu = nullptr, Tout *accv = nullptr)
+                            Tout *outu, Tout *outv, const uint8_t *mout_u, const uint8_t *mout_v)
 {
     __shared__ TilePair<Tout> t, m;
     const int lx = threadIdx.x & 15, ly = threadIdx.x >> 4;
@@ -4275,14 +4271,6 @@ __global__ void k_tile_haar(GridDims g, const HaarTable *tab, int levels, int di
         const Tin xu = ld_or(oku, inu, ku, Tin(0)), xv = ld_or(okv, inv, kv, Tin(0));
         const bool iu = mask_or_all(min_u, inu, oku, ku), iv = mask_or_all(min_v, inv, okv, kv);
         const bool ou = mask_or_all(mout_u, inu, oku, ku), ov = mask_or_all(mout_v, inv, okv, kv);
-        // the accumulation target's values, loaded with the inputs (a uniform
-        // branch: their first use is after the transform)
-        const bool acc = accu != nullptr;
-        Tout au = Tout(0), av = Tout(0);
-        if (acc) {
-            au = ld_or(oku, accu, ku, Tout(0));
-            av = ld_or(okv, accv, kv, Tout(0));
-        }
         t[0][ly][lx] = (oku && iu) ? (Tout)xu : Tout(0);
         t[1][ly][lx] = (okv && iv) ? (Tout)xv : Tout(0);
         __syncthreads();
@@ -4290,13 +4278,8 @@ __global__ void k_tile_haar(GridDims g, const HaarTable *tab, int levels, int di
             haar_pair<false, Tout>(levels, t, m);
         else
             haar_pair<true, Tout>(levels, t, m);
-        if (acc) {
-            if (oku && ou) accu[ku] = au + t[0][ly][lx];
-            if (okv && ov) accv[kv] = av + t[1][ly][lx];
-        } else {
-            if (oku) outu[ku] = ou ? t[0][ly][lx] : Tout(0);
-            if (okv) outv[kv] = ov ? t[1][ly][lx] : Tout(0);
-        }
+        if (oku) outu[ku] = ou ? t[0][ly][lx] : Tout(0);
+        if (okv) outv[kv] = ov ? t[1][ly][lx] : Tout(0);
         return;
     }
     if (has_u) {
