@@ -387,7 +387,7 @@ int wavi_smoother_tile(const wavi_ctx *ctx, int *tx, int *ty);
  * whole CG in one launch of a workgroup per tile, which exchange sums and
  * halos among themselves (FP64, 63 tiles: 7.1 us per iteration against 9.5;
  * mixed, 246 tiles: 4.2 against 5.1); else WAVI_CG_LAUNCHES.  The
- * workgroup is 3.4 to 3.6 times slower per iteration than the launches even on
+ * workgroup is 2.5 to 3.3 times slower per iteration than the launches even on
  * a grid of six 16 x 16 tiles.  All give the same bits.  The one launch is
  * made where its workgroups fit beside those of other such launches on the GPU,
  * from this process or from others of the same user that share /dev/shm
@@ -432,7 +432,7 @@ int wavi_set_coarse_cg_waits(wavi_ctx *ctx, int64_t polls, uint32_t tag);
  * Sampled single launches (events around every 16th launch, so each time
  * includes the cost of the two event records): WAVI_KT_CG_APPLY (FP64
  * coarse CG: direction, P, A, R on one tile, dot partials), WAVI_KT_CG_DIR (no
- * longer a launch of its own: 0), WAVI_KT_CG_UPDATE (axpys and norm partials),
+ * longer a launch of its own: always 0), WAVI_KT_CG_UPDATE (axpys and norm partials),
  * WAVI_KT_COLOUR (one smoother iteration: its four colour sweeps in one
  * launch).  Bursts (events around each
  * chunk of 32 back-to-back iterations; only chunks in which every launch

@@ -32,6 +32,7 @@ PRECISION = {"fp64": 0, "mixed": 1}
 
 REPORT_MAX_PICARD = 64
 
+# timers (wavi_profile_read); cg_dir is no launch of its own any more and reads 0
 KT = {"cg_apply": 0, "cg_dir": 1, "cg_update": 2, "colour": 3, "cg_iter_mixed": 4, "cg_iter_fp64": 5}
 
 # enum wavi_field, in header order

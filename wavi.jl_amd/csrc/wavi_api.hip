@@ -1561,11 +1561,10 @@ constexpr double CGM_FP32_JACOBI_RELTOL = 0x1p-14;
 
 // The coarse CG runs in one workgroup (k_cg_solve1, k_cgm_solve1) only when
 // wavi_set_coarse_cg asks for it, or in the place of a resident CG that gave
-// up (cg_try_resident): on MI355X one workgroup spends about 3 us
-// per tile and iteration (a tile's chain of loads, barriers and stores),
-// so even a 6-tile grid (80 x 10) takes 3.4 (mixed) to 3.6 (FP64) times as
-// long per CG iteration as the launches over all tiles, whose tiles run
-// side by side.
+// up (cg_try_resident): on MI355X one workgroup spends 2.4 us (mixed) to 4.2
+// us (FP64) per tile and iteration (a tile's chain of loads, barriers and
+// stores), so even a 6-tile grid (80 x 10) takes 2.5 to 3.3 times as long per
+// CG iteration as the launches over all tiles, whose tiles run side by side.
 static bool cg_one_workgroup(const wavi_ctx *ctx)
 {
     return ctx->cg_mode == WAVI_CG_WORKGROUP;

@@ -1330,7 +1330,7 @@ __device__ __forceinline__ T optile_v(const OpCoef<T> &c, const S &s, const Poin
 // point (value, thickness, drag, mask bits) and its own h cell and corner;
 // wavefront 3 adds the 64 points of the four sides of the one-point halo,
 // wavefront 2 the two halo corners that are read (u at (16, -1), v at
-// (-1, 16)), wavefront 0 the 33 cells before the tile.  13 to 19 loads a
+// (-1, 16)), wavefront 0 the 33 cells before the tile.  15 to 21 loads a
 // wavefront instead of 42 with the window walked by 256 threads and every
 // cell loading its four thicknesses and six masks.  The fluxes h u and h v
 // of the implicit term are formed once per point, masked, and staged.
