@@ -283,19 +283,20 @@ constexpr int CU_UNITS = 64;
 static Room g_room[MAX_DEVICES];
 
 // Opens the account of the device at the first context on it.
-static hipError_t room_open(int device, int cus)
+static void room_open(int device, int cus)
 {
     static std::mutex mu;
     static bool known[MAX_DEVICES] = {};
-    if (device < 0 || device >= MAX_DEVICES) return hipSuccess;
+    if (device < 0 || device >= MAX_DEVICES) return;
     std::lock_guard<std::mutex> lock(mu);
-    if (known[device]) return hipSuccess;
+    if (known[device]) return;
     char bus[64] = "";
-    const hipError_t e = hipDeviceGetPCIBusId(bus, sizeof(bus), device);
-    if (e != hipSuccess) return e;
+    if (hipDeviceGetPCIBusId(bus, sizeof(bus), device) != hipSuccess) {
+        (void)hipGetLastError();
+        snprintf(bus, sizeof(bus), "device%d", device);  // by its number among the process's
+    }
     g_room[device].open(bus, cus * CU_UNITS);
     known[device] = true;
-    return hipSuccess;
 }
 
 static bool room_take(int device, int units)
@@ -790,7 +791,7 @@ int wavi_ctx_create(const wavi_grid_desc *grid, const wavi_phys_params *phys, co
             ctx->xm_fn[pre] = cgm_resident_fn(solver->levels, pre != 0);
             CREATECHK(resident_occupancy(fp64 ? (const void *)ctx->x_fn[pre] : (const void *)ctx->xm_fn[pre], &occ[pre]));
         }
-        CREATECHK(room_open(ctx->device, cus));
+        room_open(ctx->device, cus);
         ctx->x_blocks = ctx->nblk + (fp64 && ntile > X_FLAT_TILES ? 8 : 0);  // the workgroup that folds
         const int per_cu = std::min(std::min(occ[0], occ[1]), 4);  // 4: what k_cgm_resident_batch is built for
         if (per_cu >= 2 && ctx->x_blocks <= cus * per_cu && ntile <= (fp64 ? X_TILES_FP64 : X_TILES_MIXED) &&
