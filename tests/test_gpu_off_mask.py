@@ -56,3 +56,29 @@ def test_missing_dirichlet_data_off_the_ice(W, precision):
     np.testing.assert_array_equal(out[1][0], out[0][0])
     np.testing.assert_array_equal(out[1][1], out[0][1])
     assert out[0][2] == out[1][2]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_context_recovers_from_a_solve_that_ended_in_nan(W, precision):
+    """Nothing of a NaN solve stays in the context's work arrays: with its fields
+    put back it gives what a new context gives."""
+    print("[gpu] solve after a NaN solve, %s" % precision, flush=True)
+    out = []
+    for spoiled in (False, True):
+        m = ragged(W, precision=precision)
+        m.solver_params.maxiter_coarse = 60
+        if spoiled:
+            clean = {(c, a): m._array(c, a).copy(order="F") for c, a, _ in W.model.FIELD_MAP}
+            m.fields.gu.u[10, 10] = np.nan
+            W.update_geometry(m)
+            W.update_velocities(m)
+            assert np.isnan(m.fields.gu.u).mean() > 0.5
+            for (c, a), v in clean.items():
+                setattr(m.params if c == "params" else getattr(m.fields, c), a, v)
+        W.update_geometry(m)
+        W.update_velocities(m)
+        out.append((m.fields.gu.u, m.fields.gv.v, m.last_report))
+    np.testing.assert_array_equal(out[1][0], out[0][0])
+    np.testing.assert_array_equal(out[1][1], out[0][1])
+    assert out[1][2] == out[0][2] and np.isfinite(out[0][0]).all()
